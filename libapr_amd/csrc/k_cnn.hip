@@ -87,6 +87,19 @@ __device__ __forceinline__ void decompose(int v, int s, int& z, int& x, int& y) 
     y = r - x * s;
 }
 
+/* the four voxels vp .. vp + 3 of one channel of a planar activation, n of them inside the row: one
+   8-byte store (any alignment) where the row holds all four */
+__device__ __forceinline__ void store_planar4(uint16_t* p, const uint16_t (&h)[4], int n) {
+    if (n >= 4) {
+        const uint32_t w[2] = {pack2(h[0], h[1]), pack2(h[2], h[3])};
+        __builtin_memcpy(p, w, 8);
+    } else {
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+            if (i < n) p[i] = h[i];
+    }
+}
+
 /* ---------------- forward ---------------- */
 
 /* The forward layers run over bricks of 16 (y) x 8 (x) x 4 (z) output voxels.  A block stages the
@@ -232,14 +245,13 @@ __global__ __launch_bounds__(256) void k_l1_lds(const float* __restrict__ x, int
             const int vrow = ((z0 + kz) * s1 + x0 + kx) * s1 + y0 + g * 4;
             const int64_t vc = ((int64_t)t * nv + vrow) * CH + m;
             const int64_t vp = ((int64_t)t * CH + m) * nv + vrow;
+            uint16_t hv[4];
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                if (y0 + g * 4 + i < s1) {
-                    const uint16_t hv = f2bf_hw(fmaxf(acc[i] + bias, 0.0f));
-                    a_cl[vc + i * CH] = hv;
-                    if (a_pl) a_pl[vp + i] = hv;
-                }
+                hv[i] = f2bf_hw(fmaxf(acc[i] + bias, 0.0f));
+                if (y0 + g * 4 + i < s1) a_cl[vc + i * CH] = hv[i];
             }
+            if (a_pl) store_planar4(a_pl + vp, hv, s1 - (y0 + g * 4));
         }
     }
 }
@@ -273,17 +285,18 @@ __global__ __launch_bounds__(256) void k_conv16_lds(const uint16_t* __restrict__
             const int vrow = ((z0 + kz) * sout + x0 + kx) * sout + y0 + g * 4;
             const int64_t vc = ((int64_t)t * nv + vrow) * CH + m;
             const int64_t vp = ((int64_t)t * CH + m) * nv + vrow;
+            uint16_t hv[4] = {0, 0, 0, 0};
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 if (y0 + g * 4 + i < sout) {
                     float val = acc[i] + bv;
                     if (relu) val = fmaxf(val, 0.0f);
                     if (mask_cl && !(bf2f(mask_cl[vc + i * CH]) > 0.0f)) val = 0.0f;
-                    const uint16_t hv = f2bf_hw(val);
-                    if (out_cl) out_cl[vc + i * CH] = hv;
-                    if (out_pl) out_pl[vp + i] = hv;
+                    hv[i] = f2bf_hw(val);
+                    if (out_cl) out_cl[vc + i * CH] = hv[i];
                 }
             }
+            if (out_pl) store_planar4(out_pl + vp, hv, sout - (y0 + g * 4));
         }
     }
 }
@@ -389,116 +402,189 @@ __global__ __launch_bounds__(256) void k_l4_bwd(const float* __restrict__ g4, in
 #pragma unroll
             for (int c = 0; c < CH; ++c) acc[c] += w[tap * CH + c] * gv;
         }
-        const uint16_t* ap = a3_cl + i * CH;
+        /* the voxel's 16 channels as two 16-byte words each way (32-byte aligned) */
+        const u32x4* ap = (const u32x4*)(a3_cl + i * CH);
+        u32x4* gp = (u32x4*)(g3_cl + i * CH);
 #pragma unroll
-        for (int c = 0; c < CH; ++c) {
-            const uint16_t hv = f2bf(bf2f(ap[c]) > 0.0f ? acc[c] : 0.0f);
-            g3_cl[i * CH + c] = hv;
-            g3_pl[((int64_t)t * CH + c) * n3 + u] = hv;
+        for (int h = 0; h < 2; ++h) {
+            const u32x4 av = ap[h];
+            u32x4 o;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int c = h * 8 + 2 * q;
+                const uint16_t lo = f2bf(bf2f((uint16_t)(av[q] & 0xffffu)) > 0.0f ? acc[c] : 0.0f);
+                const uint16_t hi = f2bf(bf2f((uint16_t)(av[q] >> 16)) > 0.0f ? acc[c + 1] : 0.0f);
+                o[q] = pack2(lo, hi);
+                g3_pl[((int64_t)t * CH + c) * n3 + u] = lo;
+                g3_pl[((int64_t)t * CH + c + 1) * n3 + u] = hi;
+            }
+            gp[h] = o;
         }
     }
 }
 
-/* 8 consecutive planar bf16 values starting at y0 of a row (zero from y >= ylim) */
+/* Planar buffers end with this many readable bytes: the weight-gradient kernels load whole words
+   past the end of a row (and mask what they loaded), so the last row's loads leave the data */
+constexpr size_t PL_PAD = 32;
+
+/* 8 consecutive planar bf16 values starting at y0 of a row (zero from y >= ylim): one 16-byte load at
+   any alignment where all eight are inside */
 __device__ __forceinline__ u32x4 load8(const uint16_t* row, int y0, int ylim) {
-    uint16_t h[8];
+    u32x4 r = {0u, 0u, 0u, 0u};
+    if (y0 + 8 <= ylim) {
+        __builtin_memcpy(&r, row + y0, 16);
+    } else if (y0 < ylim) {
+        uint16_t h[8];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) h[j] = (y0 + j < ylim) ? row[y0 + j] : (uint16_t)0;
-    const u32x4 r = {pack2(h[0], h[1]), pack2(h[2], h[3]), pack2(h[4], h[5]), pack2(h[6], h[7])};
+        for (int j = 0; j < 8; ++j) h[j] = (y0 + j < ylim) ? row[y0 + j] : (uint16_t)0;
+        r = (u32x4){pack2(h[0], h[1]), pack2(h[2], h[3]), pack2(h[4], h[5]), pack2(h[6], h[7])};
+    }
     return r;
 }
 
-/* dW[tap][cin][cout] = sum_v a(v + tap)[cin] g(v)[cout], db[cout] = sum_v g(v)[cout];
-   one partial per wave: part[w][27 * 256 + 16] */
-__global__ __launch_bounds__(256) void k_dw16(const uint16_t* __restrict__ a_pl, const uint16_t* __restrict__ g_pl, int sg, float* part,
-                                              int T) {
-    const int lane = threadIdx.x & 63, m = lane & 15, g = lane >> 4;
-    const int64_t wid = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-    const int64_t nw = ((int64_t)gridDim.x * blockDim.x) >> 6;
+/* the values j < n of a word of two (element 2k and 2k + 1) */
+__device__ __forceinline__ uint32_t pair_mask(int k, int n) { return n >= 2 * k + 2 ? ~0u : n == 2 * k + 1 ? 0xffffu : 0u; }
+
+/* Weight gradients of a layer with 16 input channels:
+     dW[tap][cin][cout] = sum_v a(v + tap)[cin] g(v)[cout], db[cout] = sum_v g(v)[cout].
+   M = cin, N = cout, K = 32 voxels along y; lane (g, m) holds 8 consecutive voxels of channel m.  An item
+   is a run of xs rows along x of one (tile, z, 32 voxels of y): per row the wave loads the three new
+   windows of `a` (z, z + 1, z + 2 at x + 2; 10 voxels each: a 16-byte and a 4-byte load at any alignment),
+   keeps the windows of the two rows before in registers, and makes the taps' dy = 1, 2 operands by
+   shifting the 10 voxels by one and two.  27 MFMAs run per 3 window loads, and the next row's loads are
+   issued before them.  (Before: eight 2-byte loads per operand, 27 operands per row, 3.03 ms for 16
+   tiles of 64^3 against 0.33 ms.)  The block's four waves add up in LDS, in wave order, and leave one
+   partial: part[block][tap * 256 + cin * 16 + cout], then db.
+   ONE: the last layer, whose g is one f32 channel (column 0 of N; no db): part[block][tap * 16 + cin]. */
+template <bool ONE>
+__global__ __launch_bounds__(256, 2) void k_dw(const uint16_t* __restrict__ a_pl, const void* __restrict__ g_pl, int sg, int xs, int nseg,
+                                               int64_t items, float* part) {
+    constexpr int W = ONE ? NT * CH : NT * 256 + CH;
+    __shared__ float sum[W];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), m = lane & 15, g = lane >> 4;
+    const int64_t wid = (int64_t)blockIdx.x * 4 + wave;
+    const int64_t nw = (int64_t)gridDim.x * 4;
     const int sa = sg + 2;
-    const int ng = sg * sg * sg, na = sa * sa * sa;
+    const int64_t ng = (int64_t)sg * sg * sg, na = (int64_t)sa * sa * sa;
     const int nch = (sg + 31) / 32;
-    const int64_t items = (int64_t)T * sg * sg * nch;
     f32x4 acc[NT];
 #pragma unroll
     for (int k = 0; k < NT; ++k) acc[k] = (f32x4){0.f, 0.f, 0.f, 0.f};
     float dbs = 0.0f;
     for (int64_t it = wid; it < items; it += nw) {
         const int ch = (int)(it % nch);
-        const int64_t row = it / nch;
-        const int t = (int)(row / (sg * sg)), zx = (int)(row % (sg * sg));
-        const int z = zx / sg, x = zx % sg;
-        const int y0 = ch * 32 + g * 8;
-        const u32x4 bv = load8(g_pl + ((int64_t)t * CH + m) * ng + (z * sg + x) * sg, y0, sg);
+        int64_t r = it / nch;
+        const int seg = (int)(r % nseg);
+        r /= nseg;
+        const int z = (int)(r % sg), t = (int)(r / sg);
+        const int y0 = ch * 32 + g * 8, x0 = seg * xs, x1 = min(x0 + xs, sg);
+        const bool on = y0 < sg;
+        uint32_t am[5], bm[4];
 #pragma unroll
-        for (int q = 0; q < 4; ++q) dbs += bf2f((uint16_t)(bv[q] & 0xffffu)) + bf2f((uint16_t)(bv[q] >> 16));
-        const uint16_t* ab = a_pl + ((int64_t)t * CH + m) * na;
+        for (int k = 0; k < 5; ++k) am[k] = pair_mask(k, sa - y0);
 #pragma unroll
-        for (int tap = 0; tap < NT; ++tap) {
-            const int dz = tap / 9, dx = (tap / 3) % 3, dy = tap % 3;
-            const u32x4 av = load8(ab + ((z + dz) * sa + x + dx) * sa + dy, y0, sg);
-            acc[tap] = mfma(av, bv, acc[tap]);
+        for (int k = 0; k < 4; ++k) bm[k] = pair_mask(k, sg - y0);
+        const uint16_t* ap = a_pl + ((int64_t)t * CH + m) * na + (int64_t)z * sa * sa + y0;
+        /* the 10 voxels y0 .. y0 + 9 of row (z + dz, x) */
+        auto window = [&](int dz, int x, uint32_t (&w)[5]) {
+#pragma unroll
+            for (int k = 0; k < 5; ++k) w[k] = 0u;
+            if (on) {
+                const uint16_t* p = ap + (dz * sa + x) * sa;
+                __builtin_memcpy(w, p, 16);
+                __builtin_memcpy(w + 4, p + 8, 4);
+#pragma unroll
+                for (int k = 0; k < 5; ++k) w[k] &= am[k];
+            }
+        };
+        auto row_g = [&](int x) {
+            u32x4 v = {0u, 0u, 0u, 0u};
+            if constexpr (ONE) {
+                if (m == 0 && on) {
+                    const float* p = (const float*)g_pl + (int64_t)t * ng + ((int64_t)z * sg + x) * sg + y0;
+                    float f[8];
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) f[j] = y0 + j < sg ? p[j] : 0.0f;
+                    v = (u32x4){pack2_bf16(f[0], f[1]), pack2_bf16(f[2], f[3]), pack2_bf16(f[4], f[5]), pack2_bf16(f[6], f[7])};
+                }
+            } else if (on) {
+                __builtin_memcpy(&v, (const uint16_t*)g_pl + ((int64_t)t * CH + m) * ng + ((int64_t)z * sg + x) * sg + y0, 16);
+#pragma unroll
+                for (int k = 0; k < 4; ++k) v[k] &= bm[k];
+            }
+            return v;
+        };
+        uint32_t win[3][3][5];   /* [x slot][dz] */
+#pragma unroll
+        for (int dx = 0; dx < 3; ++dx)
+#pragma unroll
+            for (int dz = 0; dz < 3; ++dz) window(dz, x0 + dx, win[dx][dz]);
+        u32x4 bv = row_g(x0);
+        for (int x = x0; x < x1; ++x) {
+            uint32_t nxt[3][5];
+            u32x4 bn = {0u, 0u, 0u, 0u};
+            const bool more = x + 1 < x1;
+            if (more) {
+#pragma unroll
+                for (int dz = 0; dz < 3; ++dz) window(dz, x + 3, nxt[dz]);
+                bn = row_g(x + 1);
+            }
+            if constexpr (!ONE) {
+#pragma unroll
+                for (int q = 0; q < 4; ++q) dbs += bf2f((uint16_t)(bv[q] & 0xffffu)) + bf2f((uint16_t)(bv[q] >> 16));
+            }
+#pragma unroll
+            for (int dz = 0; dz < 3; ++dz)
+#pragma unroll
+                for (int dx = 0; dx < 3; ++dx) {
+                    const uint32_t* w = win[dx][dz];
+                    const u32x4 a0 = {w[0], w[1], w[2], w[3]};
+                    const u32x4 a1 = {__builtin_amdgcn_alignbit(w[1], w[0], 16), __builtin_amdgcn_alignbit(w[2], w[1], 16),
+                                      __builtin_amdgcn_alignbit(w[3], w[2], 16), __builtin_amdgcn_alignbit(w[4], w[3], 16)};
+                    const u32x4 a2 = {w[1], w[2], w[3], w[4]};
+                    const int k = dz * 9 + dx * 3;
+                    acc[k] = mfma(a0, bv, acc[k]);
+                    acc[k + 1] = mfma(a1, bv, acc[k + 1]);
+                    acc[k + 2] = mfma(a2, bv, acc[k + 2]);
+                }
+            if (more) {
+#pragma unroll
+                for (int dz = 0; dz < 3; ++dz)
+#pragma unroll
+                    for (int k = 0; k < 5; ++k) {
+                        win[0][dz][k] = win[1][dz][k];
+                        win[1][dz][k] = win[2][dz][k];
+                        win[2][dz][k] = nxt[dz][k];
+                    }
+                bv = bn;
+            }
         }
     }
-    float* pw = part + wid * (NT * 256 + CH);
-#pragma unroll
-    for (int tap = 0; tap < NT; ++tap)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) pw[tap * 256 + (g * 4 + i) * CH + m] = acc[tap][i];
     dbs += __shfl_xor(dbs, 16);
     dbs += __shfl_xor(dbs, 32);
-    if (lane < 16) pw[NT * 256 + m] = dbs;
-}
-
-/* dW4[tap][cin] = sum_u a3(u)[cin] g4(u - tap): M = cin, N = tap (two blocks of 16), K = voxels u */
-__global__ __launch_bounds__(256) void k_dw_l4(const uint16_t* __restrict__ a3_pl, const float* __restrict__ g4, int S, float* part, int T) {
-    const int lane = threadIdx.x & 63, m = lane & 15, g = lane >> 4;
-    const int64_t wid = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-    const int64_t nw = ((int64_t)gridDim.x * blockDim.x) >> 6;
-    const int s3 = S + 2;
-    const int n3 = s3 * s3 * s3, nv = S * S * S;
-    const int nch = (s3 + 31) / 32;
-    const int64_t items = (int64_t)T * s3 * s3 * nch;
-    f32x4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
-    for (int64_t it = wid; it < items; it += nw) {
-        const int ch = (int)(it % nch);
-        const int64_t row = it / nch;
-        const int t = (int)(row / (s3 * s3)), zx = (int)(row % (s3 * s3));
-        const int z = zx / s3, x = zx % s3;
-        const int y0 = ch * 32 + g * 8;
-        const u32x4 av = load8(a3_pl + ((int64_t)t * CH + m) * n3 + (z * s3 + x) * s3, y0, s3);
-        const float* gt = g4 + (int64_t)t * nv;
+    for (int w = 0; w < 4; ++w) {
+        if (wave == w) {
 #pragma unroll
-        for (int nb = 0; nb < 2; ++nb) {
-            const int tap = nb * 16 + m;
-            uint16_t h[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-            if (tap < NT) {
-                const int dz = tap / 9, dx = (tap / 3) % 3, dy = tap % 3;
-                const int vz = z - dz, vx = x - dx;
-                if (vz >= 0 && vz < S && vx >= 0 && vx < S) {
+            for (int k = 0; k < NT; ++k)
 #pragma unroll
-                    for (int j = 0; j < 8; ++j) {
-                        const int vy = y0 + j - dy;
-                        if (y0 + j < s3 && vy >= 0 && vy < S) h[j] = f2bf(gt[(vz * S + vx) * S + vy]);
-                    }
+                for (int i = 0; i < 4; ++i) {
+                    const int o = ONE ? k * CH + g * 4 + i : k * 256 + (g * 4 + i) * CH + m;
+                    if (!ONE || m == 0) sum[o] = w == 0 ? acc[k][i] : sum[o] + acc[k][i];
                 }
-            }
-            const u32x4 bv = {pack2(h[0], h[1]), pack2(h[2], h[3]), pack2(h[4], h[5]), pack2(h[6], h[7])};
-            acc[nb] = mfma(av, bv, acc[nb]);
+            if (!ONE && lane < 16) sum[NT * 256 + m] = w == 0 ? dbs : sum[NT * 256 + m] + dbs;
         }
+        __syncthreads();
     }
-    float* pw = part + wid * 512;
-#pragma unroll
-    for (int nb = 0; nb < 2; ++nb)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) pw[nb * 256 + (g * 4 + i) * CH + m] = acc[nb][i];
+    for (int i = threadIdx.x; i < W; i += 256) part[(int64_t)blockIdx.x * W + i] = sum[i];
 }
 
-/* dW1[tap][cout] = sum_v x(v + tap) g1(v)[cout], db1: M = tap (two blocks of 16), N = cout, K = voxels v */
+/* dW1[tap][cout] = sum_v x(v + tap) g1(v)[cout], db1: M = tap (two blocks of 16), N = cout, K = voxels v.
+   One partial per block: part[block][tap * 16 + cout], then db1 */
 __global__ __launch_bounds__(256) void k_dw_l1(const float* __restrict__ x, const uint16_t* __restrict__ g1_pl, int S, float* part, int T) {
-    const int lane = threadIdx.x & 63, m = lane & 15, g = lane >> 4;
-    const int64_t wid = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-    const int64_t nw = ((int64_t)gridDim.x * blockDim.x) >> 6;
+    __shared__ float sum[NT * CH + CH];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), m = lane & 15, g = lane >> 4;
+    const int64_t wid = (int64_t)blockIdx.x * 4 + wave;
+    const int64_t nw = (int64_t)gridDim.x * 4;
     const int s1 = S + 6, s0 = S + 8;
     const int n1 = s1 * s1 * s1, n0 = s0 * s0 * s0;
     const int nch = (s1 + 31) / 32;
@@ -518,49 +604,84 @@ __global__ __launch_bounds__(256) void k_dw_l1(const float* __restrict__ x, cons
 #pragma unroll
         for (int mb = 0; mb < 2; ++mb) {
             const int tap = mb * 16 + m;
-            uint16_t h[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+            float f[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
             if (tap < NT) {
                 const int dz = tap / 9, dx = (tap / 3) % 3, dy = tap % 3;
-                const float* xr = xt + ((z + dz) * s0 + x0 + dx) * s0 + dy;
+                const float* xr = xt + ((z + dz) * s0 + x0 + dx) * s0 + dy + y0;
+                if (y0 + 8 <= s1) {
+                    __builtin_memcpy(f, xr, 16);
+                    __builtin_memcpy(f + 4, xr + 4, 16);
+                } else {
 #pragma unroll
-                for (int j = 0; j < 8; ++j)
-                    if (y0 + j < s1) h[j] = f2bf(xr[y0 + j]);
+                    for (int j = 0; j < 8; ++j)
+                        if (y0 + j < s1) f[j] = xr[j];
+                }
             }
-            const u32x4 av = {pack2(h[0], h[1]), pack2(h[2], h[3]), pack2(h[4], h[5]), pack2(h[6], h[7])};
+            const u32x4 av = {pack2(f2bf(f[0]), f2bf(f[1])), pack2(f2bf(f[2]), f2bf(f[3])), pack2(f2bf(f[4]), f2bf(f[5])),
+                              pack2(f2bf(f[6]), f2bf(f[7]))};
             acc[mb] = mfma(av, bv, acc[mb]);
         }
     }
-    float* pw = part + wid * (512 + CH);
-#pragma unroll
-    for (int mb = 0; mb < 2; ++mb)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) pw[mb * 256 + (g * 4 + i) * CH + m] = acc[mb][i];
     dbs += __shfl_xor(dbs, 16);
     dbs += __shfl_xor(dbs, 32);
-    if (lane < 16) pw[512 + m] = dbs;
-}
-
-/* sum of per-wave partials in wave order into the gradient vector:
-   mode 0: grad[off + i] = sum_w part[w * stride + i] for i < count
-   mode 1 (layer 4): grad[OFF_W4 + tap * 16 + cin] = sum_w part[w * stride + nb * 256 + cin * 16 + n], tap = nb * 16 + n */
-__global__ void k_reduce_parts(const float* __restrict__ part, int64_t nwaves, int stride, int count, float* grad, int off, int mode) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= count) return;
-    int src = i;
-    if (mode == 1) {
-        const int tap = i / CH, cin = i % CH;
-        src = (tap / 16) * 256 + cin * CH + (tap % 16);
+    for (int w = 0; w < 4; ++w) {
+        if (wave == w) {
+#pragma unroll
+            for (int mb = 0; mb < 2; ++mb)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int tap = mb * 16 + g * 4 + i, o = tap * CH + m;
+                    if (tap < NT) sum[o] = w == 0 ? acc[mb][i] : sum[o] + acc[mb][i];
+                }
+            if (lane < 16) sum[NT * CH + m] = w == 0 ? dbs : sum[NT * CH + m] + dbs;
+        }
+        __syncthreads();
     }
-    float s = 0.0f;
-    for (int64_t w = 0; w < nwaves; ++w) s += part[w * stride + src];
-    grad[off + i] = s;
+    for (int i = threadIdx.x; i < NT * CH + CH; i += 256) part[(int64_t)blockIdx.x * (NT * CH + CH) + i] = sum[i];
 }
 
-__global__ void k_set_scalar(float* dst, const double* part, int nblocks, int which, double scale) {
-    if (blockIdx.x != 0 || threadIdx.x != 0) return;
-    double s = 0;
-    for (int i = 0; i < nblocks; ++i) s += part[2 * i + which];
-    dst[0] = (float)(s * scale);
+/* grad[off + i] = sum_p part[p * count + i] for i < count: 16 columns x 16 rows of partials a block, each
+   row's thread summing every 16th partial, the rows then added in order.  (One thread per column took
+   0.45 ms a layer for 2048 partials; 0.006 ms now.) */
+__global__ __launch_bounds__(256) void k_reduce_parts(const float* __restrict__ part, int64_t nparts, int count, float* grad, int off) {
+    __shared__ float sum[16][16];
+    const int c = threadIdx.x & 15, r = threadIdx.x >> 4;
+    const int i = blockIdx.x * 16 + c;
+    float s = 0.0f;
+    if (i < count) {
+#pragma unroll 8
+        for (int64_t p = r; p < nparts; p += 16) s += part[p * count + i];
+    }
+    sum[r][c] = s;
+    __syncthreads();
+    if (r == 0 && i < count) {
+        for (int k = 1; k < 16; ++k) s += sum[k][c];
+        grad[off + i] = s;
+    }
+}
+
+/* the loss and the last layer's bias gradient from the blocks' pairs of partial sums */
+__global__ __launch_bounds__(256) void k_loss(float* loss, float* db4, const double* __restrict__ part, int nblocks, double scale) {
+    __shared__ double red[2][256];
+    double s = 0, b = 0;
+    for (int i = threadIdx.x; i < nblocks; i += 256) {
+        s += part[2 * i];
+        b += part[2 * i + 1];
+    }
+    red[0][threadIdx.x] = s;
+    red[1][threadIdx.x] = b;
+    __syncthreads();
+    for (int o = 128; o > 0; o >>= 1) {
+        if ((int)threadIdx.x < o) {
+            red[0][threadIdx.x] += red[0][threadIdx.x + o];
+            red[1][threadIdx.x] += red[1][threadIdx.x + o];
+        }
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) {
+        loss[0] = (float)(red[0][0] * scale);
+        db4[0] = (float)red[1][0];
+    }
 }
 
 __global__ void k_adam(float* p, const float* __restrict__ g, float* m, float* v, int n, float lr, float b1, float b2, float eps, float bc1,
@@ -698,7 +819,12 @@ namespace aprh {
 
 namespace {
 
-constexpr int WAVES = 2048;   /* waves of the weight-gradient kernels (one partial each) */
+/* blocks of the weight-gradient kernels, one partial each: two waves on each SIMD (k_dw holds 27
+   accumulators), or as many as fit for the light first layer */
+constexpr int DW_BLOCKS = 512, DW1_BLOCKS = 2048;
+/* rows along x of one k_dw item: the two rows loaded ahead of it stay a small share, and 16 tiles of
+   64^3 give each wave about 8 items */
+constexpr int DW_ROWS = 16;
 
 /* the bricks of T tiles of output side s, and a grid of at most cap blocks over them */
 struct Bricks {
@@ -753,9 +879,9 @@ void forward(aprh_cnn* n, const float* x, int T, int S, float* y, Acts& A, bool 
     A.a2c.reset(n->ctx->pool, vox(s2) * CH * 2);
     A.a3c.reset(n->ctx->pool, vox(s3) * CH * 2);
     if (train) {
-        A.a1p.reset(n->ctx->pool, vox(s1) * CH * 2);
-        A.a2p.reset(n->ctx->pool, vox(s2) * CH * 2);
-        A.a3p.reset(n->ctx->pool, vox(s3) * CH * 2);
+        A.a1p.reset(n->ctx->pool, vox(s1) * CH * 2 + PL_PAD);
+        A.a2p.reset(n->ctx->pool, vox(s2) * CH * 2 + PL_PAD);
+        A.a3p.reset(n->ctx->pool, vox(s3) * CH * 2 + PL_PAD);
     }
     const float* P = n->P.as<float>();
     {
@@ -787,53 +913,49 @@ void train_step(aprh_cnn* n, const float* x, const float* tgt, int T, int S, flo
     const float* P = n->P.as<float>();
     /* loss and db4 */
     Buf dloss(pool, 4);
-    hipLaunchKernelGGL(k_set_scalar, dim3(1), dim3(64), 0, st, dloss.as<float>(), (const double*)part.as<double>(), nblk_l4, 0,
+    hipLaunchKernelGGL(k_loss, dim3(1), kBlk, 0, st, dloss.as<float>(), G + OFF_B4, (const double*)part.as<double>(), nblk_l4,
                        1.0 / (double)vox(S));
-    hipLaunchKernelGGL(k_set_scalar, dim3(1), dim3(64), 0, st, G + OFF_B4, (const double*)part.as<double>(), nblk_l4, 1, 1.0);
     HIP_LAUNCH_CHECK();
     /* layer 4 */
-    Buf g3c(pool, vox(s3) * CH * 2), g3p(pool, vox(s3) * CH * 2);
+    Buf g3c(pool, vox(s3) * CH * 2), g3p(pool, vox(s3) * CH * 2 + PL_PAD);
     hipLaunchKernelGGL(k_l4_bwd, dim3((unsigned)std::min<size_t>((vox(s3) + 255) / 256, 8192)), kBlk, 0, st, (const float*)g4.as<float>(), S,
                        P + OFF_W4, (const uint16_t*)A.a3c.as<uint16_t>(), g3c.as<uint16_t>(), g3p.as<uint16_t>(), T);
     HIP_LAUNCH_CHECK();
-    Buf pbuf(pool, (size_t)WAVES * (NT * 256 + CH) * 4);
-    const dim3 wgrid(WAVES / 4);
-    hipLaunchKernelGGL(k_dw_l4, wgrid, kBlk, 0, st, (const uint16_t*)A.a3p.as<uint16_t>(), (const float*)g4.as<float>(), S,
-                       pbuf.as<float>(), T);
-    HIP_LAUNCH_CHECK();
-    hipLaunchKernelGGL(k_reduce_parts, dim3((NT * CH + 255) / 256), kBlk, 0, st, (const float*)pbuf.as<float>(), (int64_t)WAVES, 512,
-                       NT * CH, G, OFF_W4, 1);
-    HIP_LAUNCH_CHECK();
+    Buf pbuf(pool, (size_t)std::max<int64_t>((int64_t)DW_BLOCKS * (NT * 256 + CH), (int64_t)DW1_BLOCKS * (NT * CH + CH)) * 4);
+    auto reduce = [&](int64_t nparts, int count, int off) {
+        hipLaunchKernelGGL(k_reduce_parts, dim3((unsigned)cdiv(count, 16)), kBlk, 0, st, (const float*)pbuf.as<float>(), nparts, count, G, off);
+        HIP_LAUNCH_CHECK();
+    };
+    /* weight gradients of a layer over gradients of side sg, into G + off */
+    auto dw = [&](const Buf& act, const Buf& grad, int sg, bool one, int off) {
+        const int nseg = (int)cdiv(sg, DW_ROWS);
+        const int64_t items = (int64_t)T * sg * nseg * cdiv(sg, 32);
+        const unsigned grid = (unsigned)std::min<int64_t>(DW_BLOCKS, cdiv(items, 4));
+        if (one)
+            hipLaunchKernelGGL(k_dw<true>, dim3(grid), kBlk, 0, st, (const uint16_t*)act.as<uint16_t>(), (const void*)grad.ptr(), sg, DW_ROWS,
+                               nseg, items, pbuf.as<float>());
+        else
+            hipLaunchKernelGGL(k_dw<false>, dim3(grid), kBlk, 0, st, (const uint16_t*)act.as<uint16_t>(), (const void*)grad.ptr(), sg, DW_ROWS,
+                               nseg, items, pbuf.as<float>());
+        HIP_LAUNCH_CHECK();
+        reduce(grid, one ? NT * CH : NT * 256 + CH, off);
+    };
+    dw(A.a3p, g4, S, true, OFF_W4);
     /* layer 3 weights, then the gradient of a2 */
-    hipLaunchKernelGGL(k_dw16, wgrid, kBlk, 0, st, (const uint16_t*)A.a2p.as<uint16_t>(), (const uint16_t*)g3p.as<uint16_t>(), s3,
-                       pbuf.as<float>(), T);
-    HIP_LAUNCH_CHECK();
-    hipLaunchKernelGGL(k_reduce_parts, dim3((NT * 256 + CH + 255) / 256), kBlk, 0, st, (const float*)pbuf.as<float>(), (int64_t)WAVES,
-                       NT * 256 + CH, NT * 256 + CH, G, OFF_W3, 0);
-    HIP_LAUNCH_CHECK();
-    auto grid = [&](size_t v) { return dim3((unsigned)std::min<size_t>((v / 16 + 3) / 4 + 1, 16384)); };
-    Buf g2c(pool, vox(s2) * CH * 2), g2p(pool, vox(s2) * CH * 2);
+    dw(A.a2p, g3p, s3, false, OFF_W3);
+    Buf g2c(pool, vox(s2) * CH * 2), g2p(pool, vox(s2) * CH * 2 + PL_PAD);
     conv16(st, g3c.as<uint16_t>(), s3, s2, -2, n->W3t.as<u32x4>(), nullptr, A.a2c.as<uint16_t>(), g2c.as<uint16_t>(), g2p.as<uint16_t>(),
            0, T);
     /* layer 2 weights, then the gradient of a1 */
-    hipLaunchKernelGGL(k_dw16, wgrid, kBlk, 0, st, (const uint16_t*)A.a1p.as<uint16_t>(), (const uint16_t*)g2p.as<uint16_t>(), s2,
-                       pbuf.as<float>(), T);
-    HIP_LAUNCH_CHECK();
-    hipLaunchKernelGGL(k_reduce_parts, dim3((NT * 256 + CH + 255) / 256), kBlk, 0, st, (const float*)pbuf.as<float>(), (int64_t)WAVES,
-                       NT * 256 + CH, NT * 256 + CH, G, OFF_W2, 0);
-    HIP_LAUNCH_CHECK();
-    Buf g1p(pool, vox(s1) * CH * 2);
+    dw(A.a1p, g2p, s2, false, OFF_W2);
+    Buf g1p(pool, vox(s1) * CH * 2 + PL_PAD);
     conv16(st, g2c.as<uint16_t>(), s2, s1, -2, n->W2t.as<u32x4>(), nullptr, A.a1c.as<uint16_t>(), nullptr, g1p.as<uint16_t>(), 0, T);
-    /* layer 1 */
-    hipLaunchKernelGGL(k_dw_l1, wgrid, kBlk, 0, st, x, (const uint16_t*)g1p.as<uint16_t>(), S, pbuf.as<float>(), T);
+    /* layer 1: its bias gradient follows its weights' in the partials as in the parameters */
+    static_assert(OFF_B1 == OFF_W1 + NT * CH && OFF_B2 == OFF_W2 + NT * 256 && OFF_B3 == OFF_W3 + NT * 256, "bias after weights");
+    const unsigned grid1 = (unsigned)std::min<int64_t>(DW1_BLOCKS, cdiv((int64_t)T * s1 * s1 * cdiv(s1, 32), 4));
+    hipLaunchKernelGGL(k_dw_l1, dim3(grid1), kBlk, 0, st, x, (const uint16_t*)g1p.as<uint16_t>(), S, pbuf.as<float>(), T);
     HIP_LAUNCH_CHECK();
-    hipLaunchKernelGGL(k_reduce_parts, dim3((NT * CH + CH + 255) / 256), kBlk, 0, st, (const float*)pbuf.as<float>(), (int64_t)WAVES,
-                       512 + CH, NT * CH, G, OFF_W1, 0);
-    HIP_LAUNCH_CHECK();
-    /* db1 sits after the 2 x 256 block */
-    hipLaunchKernelGGL(k_reduce_parts, dim3(1), kBlk, 0, st, (const float*)(pbuf.as<float>() + 512), (int64_t)WAVES, 512 + CH, CH, G, OFF_B1,
-                       0);
-    HIP_LAUNCH_CHECK();
+    reduce(grid1, NT * CH + CH, OFF_W1);
     if (grads_out) HIP_CHECK(hipMemcpyAsync(grads_out, G, N_PARAMS * 4, hipMemcpyDeviceToHost, st));
     if (lr > 0) {
         n->step += 1;

@@ -70,6 +70,17 @@ def test_forward_matches_oracle(oracle, ctx, S, T):
 
 @pytest.mark.parametrize("S,T", [(8, 2), (11, 1)])
 def test_gradients_match_oracle(oracle, ctx, S, T):
+    _gradients_against_oracle(oracle, ctx, S, T)
+
+
+@pytest.mark.parametrize("S,T", [(3, 2), (14, 1), (15, 1), (28, 1), (30, 1), (33, 1)])
+def test_gradients_at_item_edges(oracle, ctx, S, T):
+    """the weight-gradient kernels take 32 voxels along y and 16 rows along x at a time: gradient sides
+    S .. S + 6 just below, at and above those, in odd and even rows (2-byte and 4-byte aligned loads)"""
+    _gradients_against_oracle(oracle, ctx, S, T)
+
+
+def _gradients_against_oracle(oracle, ctx, S, T):
     L = oracle.load("oracle")
     p = rand_params(100 + S, last=0.3)
     net = A.WarmStartCNN(ctx, params=p)
