@@ -356,8 +356,9 @@ template <typename T>
 int richardson_lucy(aprh_context* ctx, aprh_apr& a, const T* in, float* u, const std::vector<HostStencil>& psf,
                     const std::vector<HostStencil>& psf_flipped, int max_iter, bool resume, double tol, double* last_rel);
 /* piecewise-constant image of level `level` (l_max: APRReconstruction::reconstruct_constant);
-   dtypes 0 = u16, 1 = f32 for particles (pdt) and image (idt) */
-void reconstruct_any(aprh_context* ctx, aprh_apr& a, const void* parts, int pdt, int level, void* img, int idt);
+   dtypes 0 = u16, 1 = f32 for particles (pdt) and image (idt); lev (optional): the level
+   of the particle covering each pixel, as bytes */
+void reconstruct_any(aprh_context* ctx, aprh_apr& a, const void* parts, int pdt, int level, void* img, int idt, uint8_t* lev = nullptr);
 /* level image at `level` (<= l_max) with pixels of finer particles set to `level` */
 void reconstruct_level(aprh_context* ctx, aprh_apr& a, int level, void* img, int idt);
 /* APRReconstruction::reconstruct_smooth of the whole image (scale3: y, x, z) */

@@ -309,6 +309,52 @@ def test_reconstruct_level(oracle, ctx, shape, nb, seed):
         assert got.dtype == out_dtype and np.array_equal(got, expect.astype(out_dtype))
 
 
+@pytest.mark.parametrize("shape,nb,seed,delta", [((3, 5, 1025), 6, 1, 0), ((5, 3, 2049), 6, 2, 0), ((4, 7, 4133), 9, 3, 0), ((5, 4, 4133), 9, 3, -1),
+                                                 ((2, 9, 2050), 4, 4, 0)])
+def test_reconstruct_long_rows(oracle, ctx, shape, nb, seed, delta):
+    """rows of more than one 4096-byte piece (1024 f32, 2048 u16), whose levels' entries are found by
+    search, at row starts of every alignment; and coarse cells wider than a piece"""
+    img, o, g = _pair(oracle, ctx, shape, nb, seed)
+    parts = o.sample(img)
+    for out_dtype in (np.uint16, np.float32):
+        assert np.array_equal(A.APRReconstruction.reconstruct_constant(g, parts, delta, out_dtype), o.reconstruct(parts, delta, out_dtype))
+    if delta == 0:
+        for out_dtype in (np.uint16, np.float32):
+            assert np.array_equal(A.APRReconstruction.reconstruct_level(g, out_dtype), _level_image(o).astype(out_dtype))
+
+
+def _level_image(o):
+    lev = np.concatenate([np.full(n, l, np.uint16) for l, n in _particles_per_level(o)])
+    return o.reconstruct(lev, 0, np.uint16)
+
+
+def _particles_per_level(o):
+    """(level, particles) of an oracle APR, from its row ends"""
+    ends = o.xz_end_vec
+    d = max(o.dims)
+    out, row = [], 1
+    for l in range(o.l_min, o.l_max + 1):
+        s = 1 << (o.l_max - l)
+        n = -(-o.dims[1] // s) * -(-o.dims[2] // s)
+        out.append((l, int(ends[row + n - 1] - ends[row - 1])))
+        row += n
+    assert d <= 1 << o.l_max and sum(n for _, n in out) == o.total
+    return out
+
+
+@pytest.mark.parametrize("shape,nb,seed", [((3, 3, 6200), 5, 1), ((2, 3, 40001), 9, 2), ((90, 5, 70), 6, 3), ((5, 91, 67), 6, 4)])
+def test_reconstruct_smooth_line_forms(oracle, ctx, shape, nb, seed):
+    """one line of y in LDS, a line longer than LDS holds (marched), and x / z lines long and short
+    against the ring of 42 sums"""
+    img, o, g = _pair(oracle, ctx, shape, nb, seed)
+    parts = o.sample(img)
+    for out_dtype in (np.uint16, np.float32):
+        for sc in ((2.0, 2.0, 2.0), (0.3, 0.5, 0.4)):
+            exp = o.reconstruct_smooth(parts, scale=sc, out_dtype=out_dtype)
+            got = A.APRReconstruction.reconstruct_smooth(g, parts, scale_d=sc, out_dtype=out_dtype)
+            assert np.array_equal(got.view(np.uint8), exp.view(np.uint8)), (out_dtype, sc, int((got != exp).sum()))
+
+
 @pytest.mark.parametrize("shape,nb,seed", CASES[:3] + [((3, 9, 40), 2, 8)])
 def test_reconstruct_smooth(oracle, ctx, shape, nb, seed):
     """reconstruct_smooth bit-equal to the oracle: u16 and f32 particles into u16 and f32 images,
