@@ -234,13 +234,18 @@ IIRCoeffs iir_coeffs(float lambda, float tol, int64_t len);
 /* ---- stage launchers (k_iir.hip) ---- */
 void launch_minmax_offset(aprh_context* ctx, const uint16_t* img, size_t n, float lambda, float* d_offset, uint32_t* d_minmax);
 void launch_offset_copy(aprh_context* ctx, const uint16_t* in, uint16_t* out, size_t n, const float* d_offset);
+/* elements of a row of y samples rounded up to whole 16-byte words: the pitch of the smoothed image
+   inside the pipeline */
+int64_t iir_pitch(int64_t y, size_t elem);
+/* packed rows of y in, rows of `pitch` out: iir_pitch (zeros past y), or y itself (also in place) */
 template <typename T>
 void launch_iir_y(aprh_context* ctx, const T* in, T* out, int64_t y, int64_t x, int64_t z, const IIRCoeffs& c,
-                  const float* d_offset, int* d_err);
-/* u16 y pass that also finds the bspline offset: it runs with the offset most images get, gathers
-   the input's (min, max) on the way, and runs again only when the true offset differs */
-bool iir_y_fuses_offset(int64_t y, const void* in, const void* out);
-/* pyr (optional): receives the first level of the input's mean pyramid (ceil(x/2) x ceil(z/2) rows
+                  const float* d_offset, int* d_err, int64_t pitch);
+/* whether the u16 y pass can write the first level of the mean pyramid on the way */
+bool iir_y_writes_pyramid(int64_t y, const void* in);
+/* u16 y pass (rows of iir_pitch out) that also finds the bspline offset: it runs with the offset most
+   images get, gathers the input's (min, max) on the way, and runs again only when the true offset
+   differs.  pyr (optional): receives the first level of the input's mean pyramid (ceil(x/2) x ceil(z/2) rows
    of y/2, 16-byte aligned) */
 void launch_iir_y_offset(aprh_context* ctx, const uint16_t* in, uint16_t* out, int64_t y, int64_t x, int64_t z, const IIRCoeffs& c,
                          float lambda, float* d_offset, uint32_t* d_mm, int* d_rerun, int* d_err, uint16_t* pyr);
@@ -249,9 +254,10 @@ void launch_iir_outer(aprh_context* ctx, T* img, int64_t y, int64_t x, int64_t z
 
 /* ---- gradient / inverse B-spline / LIS (k_grad_lis.hip) ---- */
 /* accum: take the existing grad values into the maximum (calc_bspline_fd_ds_mag semantics);
-   the pipeline passes false on a buffer it would otherwise have zero-filled */
+   the pipeline passes false on a buffer it would otherwise have zero-filled.  pitch: elements from
+   one image row to the next (y, or iir_pitch) */
 void launch_grad_ds_u16(aprh_context* ctx, const uint16_t* img, uint16_t* grad, float* mean, int64_t y, int64_t x, int64_t z,
-                        float hx, float hy, float hz, bool accum);
+                        float hx, float hy, float hz, bool accum, int64_t pitch);
 void launch_inv_bspline(aprh_context* ctx, float* m, float* tmp, int64_t y, int64_t x, int64_t z, bool ay, bool ax, bool az);
 /* the same passes alternating between a (input) and b; returns the buffer holding the result */
 float* launch_inv_bspline_pp(aprh_context* ctx, float* a, float* b, int64_t y, int64_t x, int64_t z, bool ay, bool ax, bool az);
@@ -285,7 +291,7 @@ void launch_levels_padded(aprh_context* ctx, const float* A, const LisParams& lp
                           const aprh_params& par, const float* d_offset, float mult, G* grad_keep);
 /* gradient magnitude + 2x2x2 max + mean downsample of a float image (APRConverter<float>) */
 void launch_grad_ds_f32(aprh_context* ctx, const float* img, float* grad, float* mean, int64_t y, int64_t x, int64_t z, float hx,
-                        float hy, float hz, bool accum);
+                        float hy, float hz, bool accum, int64_t pitch);
 
 /* ---- pulling scheme / structure / sampling (k_structure.hip) ---- */
 void build_structure(aprh_context* ctx, aprh_apr& a, const uint8_t* level_top, const aprh_params& par);

@@ -29,6 +29,13 @@ void keep_copy(aprh_context* ctx, Buf& dst, const void* src, size_t bytes) {
     HIP_CHECK(hipMemcpyAsync(dst.ptr(), src, bytes, hipMemcpyDeviceToDevice, ctx->stream));
 }
 
+/* rows of `bytes` out of rows of `pitch` bytes */
+void keep_rows(aprh_context* ctx, Buf& dst, const void* src, size_t pitch, size_t bytes, size_t rows) {
+    if (pitch == bytes) return keep_copy(ctx, dst, src, bytes * rows);
+    dst.reset(ctx->pool, bytes * rows);
+    HIP_CHECK(hipMemcpy2DAsync(dst.ptr(), bytes, src, pitch, bytes, rows, hipMemcpyDeviceToDevice, ctx->stream));
+}
+
 /* levels + pulling scheme + structure from a downsampled gradient, an unpadded
    scale (A with zero pads, var_rescale 1) or the padded LIS array */
 template <typename G>
@@ -87,16 +94,18 @@ void get_apr_u16(aprh_context* ctx, const uint16_t* image, int64_t y, int64_t x,
     int* d_err = flags + 4;
     int* d_rerun = flags + 8;
     launch_zero(ctx, d_err, 3 * sizeof(int));
-    Buf img(ctx->pool, n * 2);
+    /* the smoothed image's rows are whole 16-byte words once the y pass writes them */
+    const int64_t yq = par.lambda > 0 && y > 2 ? iir_pitch(y, 2) : y;
+    Buf img(ctx->pool, (size_t)(yq * x * z) * 2);
     uint16_t* I = img.as<uint16_t>();
     const float tol = 0.0001f;
-    if (par.lambda > 0 && y > 2 && iir_y_fuses_offset(y, in.ptr, I)) {
+    if (par.lambda > 0 && y > 2) {
         /* computeL's bspline offset (APRConverter.hpp:213-224) found by the y pass itself */
         mark(ctx, ST_SMOOTH_Y);
         /* with sampling requested, the pass also writes the first level of the image's mean pyramid */
         uint16_t* pyr_top = nullptr;
         SampleReq* sr = ctx->sample_req;
-        if (sr && !ctx->recorder && a->l_max - 1 >= a->l_min && a->l_max > 2) {
+        if (sr && !ctx->recorder && a->l_max - 1 >= a->l_min && a->l_max > 2 && iir_y_writes_pyramid(y, in.ptr)) {
             int64_t tot = 0;
             sr->pyr_off = pyramid_layout(*a, &tot);
             sr->pyr.reset(ctx->pool, (size_t)std::max<int64_t>(tot, 1) * 2);
@@ -106,20 +115,15 @@ void get_apr_u16(aprh_context* ctx, const uint16_t* image, int64_t y, int64_t x,
         launch_iir_y_offset(ctx, (const uint16_t*)in.ptr, I, y, x, z, iir_coeffs(par.lambda, tol, y), par.lambda, d_off, d_mm, d_rerun,
                             d_err + 0, pyr_top);
     } else {
-        /* computeL: bspline offset (APRConverter.hpp:213-224) */
+        /* computeL: bspline offset (APRConverter.hpp:213-224), no smoothing along y */
         launch_minmax_offset(ctx, (const uint16_t*)in.ptr, n, par.lambda, d_off, d_mm);
         mark(ctx, ST_SMOOTH_Y);
-        /* smoothing (ComputeGradient.hpp:173-205) with the offset copy fused into the first pass */
-        if (par.lambda > 0 && y > 2) {
-            launch_iir_y<uint16_t>(ctx, (const uint16_t*)in.ptr, I, y, x, z, iir_coeffs(par.lambda, tol, y), d_off, d_err + 0);
-        } else {
-            launch_offset_copy(ctx, (const uint16_t*)in.ptr, I, n, d_off);
-        }
+        launch_offset_copy(ctx, (const uint16_t*)in.ptr, I, n, d_off);
     }
     mark(ctx, ST_SMOOTH_X);
-    if (par.lambda > 0 && x > 2) launch_iir_outer<uint16_t>(ctx, I, y, x, z, 1, iir_coeffs(par.lambda, tol, x), d_err + 1);
+    if (par.lambda > 0 && x > 2) launch_iir_outer<uint16_t>(ctx, I, yq, x, z, 1, iir_coeffs(par.lambda, tol, x), d_err + 1);
     mark(ctx, ST_SMOOTH_Z);
-    if (par.lambda > 0 && z > 2) launch_iir_outer<uint16_t>(ctx, I, y, x, z, 2, iir_coeffs(par.lambda, tol, z), d_err + 2);
+    if (par.lambda > 0 && z > 2) launch_iir_outer<uint16_t>(ctx, I, yq, x, z, 2, iir_coeffs(par.lambda, tol, z), d_err + 2);
     mark(ctx, ST_GRADIENT);
     /* gradient magnitude + 2x2x2 max (ComputeGradient.hpp:92-93), mean downsample and inverse B-spline (:95-118) */
     Buf grad(ctx->pool, nd * 2);
@@ -129,12 +133,12 @@ void get_apr_u16(aprh_context* ctx, const uint16_t* image, int64_t y, int64_t x,
     Buf mean(ctx->pool, nd * 4), tmp;
     if (npass) tmp.reset(ctx->pool, nd * 4);
     float* mean_first = (npass & 1) ? tmp.as<float>() : mean.as<float>();
-    launch_grad_ds_u16(ctx, I, grad.as<uint16_t>(), mean_first, y, x, z, par.dx, par.dy, par.dz, false);
+    launch_grad_ds_u16(ctx, I, grad.as<uint16_t>(), mean_first, y, x, z, par.dx, par.dy, par.dz, false, yq);
     /* the overflow counters are read with the B-spline offset at the end of the call (one host
        synchronisation instead of a stall between the gradient and the inverse B-spline) */
     if (ctx->async_mode) launch_copy(ctx, ctx->slot_err, d_err, 3 * sizeof(int));
     if (ctx->keep_intermediates) {
-        keep_copy(ctx, a->smoothed, I, n * 2);
+        keep_rows(ctx, a->smoothed, I, yq * 2, y * 2, x * z);
         keep_copy(ctx, a->grad_raw, grad.ptr(), nd * 2);
     }
     img.release();
@@ -212,26 +216,27 @@ void get_apr_f32(aprh_context* ctx, const float* image, int64_t y, int64_t x, in
     int* d_err = ctx->d_flags + 4;
     launch_zero(ctx, ctx->d_flags, 8 * sizeof(int));   /* offset 0.0f, error counters 0 */
     mark(ctx, ST_SMOOTH_Y);
-    Buf img(ctx->pool, n * 4);
+    const int64_t yq = par.lambda > 0 && y > 2 ? iir_pitch(y, 4) : y;
+    Buf img(ctx->pool, (size_t)(yq * x * z) * 4);
     float* I = img.as<float>();
     const float tol = 0.0001f;
     if (par.lambda > 0 && y > 2)
-        launch_iir_y<float>(ctx, (const float*)in.ptr, I, y, x, z, iir_coeffs(par.lambda, tol, y), nullptr, d_err + 0);
+        launch_iir_y<float>(ctx, (const float*)in.ptr, I, y, x, z, iir_coeffs(par.lambda, tol, y), nullptr, d_err + 0, yq);
     else
         HIP_CHECK(hipMemcpyAsync(I, in.ptr, n * 4, hipMemcpyDeviceToDevice, st));
     mark(ctx, ST_SMOOTH_X);
-    if (par.lambda > 0 && x > 2) launch_iir_outer<float>(ctx, I, y, x, z, 1, iir_coeffs(par.lambda, tol, x), d_err + 1);
+    if (par.lambda > 0 && x > 2) launch_iir_outer<float>(ctx, I, yq, x, z, 1, iir_coeffs(par.lambda, tol, x), d_err + 1);
     mark(ctx, ST_SMOOTH_Z);
-    if (par.lambda > 0 && z > 2) launch_iir_outer<float>(ctx, I, y, x, z, 2, iir_coeffs(par.lambda, tol, z), d_err + 2);
+    if (par.lambda > 0 && z > 2) launch_iir_outer<float>(ctx, I, yq, x, z, 2, iir_coeffs(par.lambda, tol, z), d_err + 2);
     mark(ctx, ST_GRADIENT);
     Buf grad(ctx->pool, nd * 4);
     const int npass = par.lambda > 0 ? inv_bspline_launches(y > 2, x > 2, z > 2) : 0;
     Buf mean(ctx->pool, nd * 4), tmp;
     if (npass) tmp.reset(ctx->pool, nd * 4);
     float* mean_first = (npass & 1) ? tmp.as<float>() : mean.as<float>();
-    launch_grad_ds_f32(ctx, I, grad.as<float>(), mean_first, y, x, z, par.dx, par.dy, par.dz, false);
+    launch_grad_ds_f32(ctx, I, grad.as<float>(), mean_first, y, x, z, par.dx, par.dy, par.dz, false, yq);
     if (ctx->keep_intermediates) {
-        keep_copy(ctx, a->smoothed, I, n * 4);
+        keep_rows(ctx, a->smoothed, I, yq * 4, y * 4, x * z);
         keep_copy(ctx, a->grad_raw, grad.ptr(), nd * 4);
     }
     img.release();
@@ -554,7 +559,7 @@ int aprh_bspline_filt_rec_u16(aprh_context* ctx, uint16_t* image, int64_t y, int
     int* d_err = ctx->d_flags + 4;
     HIP_CHECK(hipMemsetAsync(d_err, 0, 4, ctx->stream));
     IIRCoeffs c = iir_coeffs(lambda, tol, len);
-    if (axis == 0) launch_iir_y<uint16_t>(ctx, (const uint16_t*)io.ptr, (uint16_t*)io.ptr, y, x, z, c, nullptr, d_err);
+    if (axis == 0) launch_iir_y<uint16_t>(ctx, (const uint16_t*)io.ptr, (uint16_t*)io.ptr, y, x, z, c, nullptr, d_err, y);
     else launch_iir_outer<uint16_t>(ctx, (uint16_t*)io.ptr, y, x, z, axis, c, d_err);
     int herr = 0;
     HIP_CHECK(hipMemcpyAsync(&herr, d_err, 4, hipMemcpyDeviceToHost, ctx->stream));
@@ -575,7 +580,7 @@ int aprh_bspline_filt_rec_f32(aprh_context* ctx, float* image, int64_t y, int64_
     if (io.host) HIP_CHECK(hipMemcpyAsync(io.ptr, image, n * 4, hipMemcpyHostToDevice, ctx->stream));
     int* d_err = ctx->d_flags + 4;
     IIRCoeffs c = iir_coeffs(lambda, tol, len);
-    if (axis == 0) launch_iir_y<float>(ctx, (const float*)io.ptr, (float*)io.ptr, y, x, z, c, nullptr, d_err);
+    if (axis == 0) launch_iir_y<float>(ctx, (const float*)io.ptr, (float*)io.ptr, y, x, z, c, nullptr, d_err, y);
     else launch_iir_outer<float>(ctx, (float*)io.ptr, y, x, z, axis, c, d_err);
     io.finish(ctx);
     APRH_CATCH
@@ -610,10 +615,10 @@ int aprh_gradient_ds_u16(aprh_context* ctx, const uint16_t* image, uint16_t* gra
     if (g.host) HIP_CHECK(hipMemcpyAsync(g.ptr, grad_ds, nd * 2, hipMemcpyHostToDevice, ctx->stream));
     if (mean_ds) {
         DevOut m(ctx, mean_ds, nd * 4);
-        launch_grad_ds_u16(ctx, (const uint16_t*)in.ptr, (uint16_t*)g.ptr, (float*)m.ptr, y, x, z, hx, hy, hz, true);
+        launch_grad_ds_u16(ctx, (const uint16_t*)in.ptr, (uint16_t*)g.ptr, (float*)m.ptr, y, x, z, hx, hy, hz, true, y);
         m.finish(ctx);
     } else {
-        launch_grad_ds_u16(ctx, (const uint16_t*)in.ptr, (uint16_t*)g.ptr, nullptr, y, x, z, hx, hy, hz, true);
+        launch_grad_ds_u16(ctx, (const uint16_t*)in.ptr, (uint16_t*)g.ptr, nullptr, y, x, z, hx, hy, hz, true, y);
     }
     g.finish(ctx);
     APRH_CATCH

@@ -2,14 +2,13 @@
  * k_iir.hip -- B-spline smoothing of the conversion pipeline on gfx950.
  *
  *  - min/max reduction + bspline offset     (AutoParameters.hpp:165-196)
- *  - y pass (ComputeGradient.hpp:248-413): one lane per y-line.  u16 lines of
- *    a multiple of 64 samples go through an LDS tile (64 lines x 64 samples)
- *    so global accesses stay coalesced, and do not store the causal result
- *    (per-chunk recursion states are saved and the chunk is recomputed for the
- *    anti-causal sweep); other lines whose length is a multiple of the 16-byte
- *    vector are streamed with 16-byte loads/stores, several vectors ahead of
- *    the recursion.  The offset copy of computeL (APRConverter.hpp:213-224) is
- *    fused into the first read.
+ *  - y pass (ComputeGradient.hpp:248-413): one lane per y-line.  Lines go
+ *    through an LDS tile (64 lines x 128 bytes) so global accesses stay
+ *    coalesced, and the causal result is not stored (per-chunk recursion states
+ *    are saved and the chunk is recomputed for the anti-causal sweep).  The
+ *    pipeline writes rows of whole 16-byte words, so the x and z passes and the
+ *    gradient take their vector forms for every y length.  The offset copy of
+ *    computeL (APRConverter.hpp:213-224) is fused into the first read.
  *  - x / z passes (ComputeGradient.hpp:415-599, 601-779): lanes run along y
  *    (8 u16 / 4 f32 samples per lane), so each recursion step is one
  *    coalesced 16-byte-per-lane row access.  Axes of 64 samples or more save
@@ -386,11 +385,7 @@ __device__ __forceinline__ void iir_outer_body(T* img, int64_t y_num, int64_t n,
 }
 
 
-/* ---------------- vector paths ----------------
- * y pass: lane = one y-line, streamed with 16-byte loads/stores (8 u16 or 4 f32
- * samples); D vectors are loaded ahead of the recursion so several HBM
- * requests per lane stay in flight.  Requires y_num % VEC == 0 and 16-byte
- * aligned lines. */
+/* ---------------- vector paths: 16 bytes, 8 u16 or 4 f32 samples ---------------- */
 template <typename T> struct Vec16;
 template <> struct Vec16<uint16_t> {
     static constexpr int N = 8;
@@ -428,118 +423,6 @@ __device__ __forceinline__ float vin(const uint4& v, int i, float off, bool has_
     const float x = Vec16<T>::get(v, i);
     /* x + offset lies in [-100, 65635]: the int32 conversion is the x86 one */
     return has_off ? (float)((uint32_t)(int)(x + off) & 0xFFFFu) : x;
-}
-
-template <typename T, int D>
-__device__ __forceinline__ void iir_y_vec_body(const T* __restrict__ in, T* out, int64_t y_num, int64_t n_lines, const IIRCoeffs& c,
-                                               const float* d_off, int* d_err, int64_t blk) {
-    constexpr int V = Vec16<T>::N;
-    const int64_t me = blk * blockDim.x + threadIdx.x;
-    if (me >= n_lines) return;
-    const bool has_off = d_off != nullptr;
-    const float off = has_off ? *d_off : 0.0f;
-    const float b1 = c.b1, b2 = c.b2, nf = c.nf;
-    const uint4* src = (const uint4*)(in + me * y_num);
-    uint4* dst = (uint4*)(out + me * y_num);
-    const int64_t nv = y_num / V;
-    int err = 0;
-    /* boundary sums over the first / last minLen samples (ComputeGradient.hpp:342-356) */
-    float t1 = 0, t2 = 0, t3 = 0, t4 = 0;
-    {
-        const int nb = (c.mL + V - 1) / V;
-        for (int b = 0; b < nb; ++b) {
-            const uint4 v = src[b];
-#pragma unroll
-            for (int i = 0; i < V; ++i) {
-                const int k = b * V + i;
-                if (k < c.mL) {
-                    const float x = vin<T>(v, i, off, has_off);
-                    t1 += c.bc1[k] * x;
-                    t2 += c.bc2[k] * x;
-                }
-            }
-        }
-        for (int b = 0; b < nb; ++b) {
-            const uint4 v = src[nv - 1 - b];
-#pragma unroll
-            for (int i = V - 1; i >= 0; --i) {
-                const int k = b * V + (V - 1 - i);   /* distance from the end */
-                if (k < c.mL) {
-                    const float x = vin<T>(v, i, off, has_off);
-                    t3 += c.bc3[k] * x;
-                    t4 += c.bc4[k] * x;
-                }
-            }
-        }
-    }
-    /* causal pass: state unrounded (ComputeGradient.hpp:359-373) */
-    float s1 = t1, s2 = t2;
-    /* y(0), y(1) are stored truncated, without the round<T> check (ComputeGradient.hpp:365-366) */
-    const float t2q = Val<T>::store(t2), t1q = Val<T>::store(t1);
-    for (int64_t b0 = 0; b0 < nv; b0 += D) {
-        uint4 buf[D];
-#pragma unroll
-        for (int d = 0; d < D; ++d)
-            if (b0 + d < nv) buf[d] = src[b0 + d];
-#pragma unroll
-        for (int d = 0; d < D; ++d) {
-            if (b0 + d >= nv) break;
-            uint4 o = buf[d];
-#pragma unroll
-            for (int i = 0; i < V; ++i) {
-                const int64_t k = (b0 + d) * V + i;
-                float r;
-                if (k == 0) {
-                    r = t2q;
-                } else if (k == 1) {
-                    r = t1q;
-                } else {
-                    const float t = s1 * b1 + s2 * b2 + vin<T>(buf[d], i, off, has_off);
-                    r = Val<T>::rnd(t, err);
-                    s2 = s1;
-                    s1 = t;
-                }
-                Vec16<T>::set_r(o, i, r);
-            }
-            dst[b0 + d] = o;
-        }
-    }
-    /* end values (ComputeGradient.hpp:375-376) */
-    const float e2 = Val<T>::rnd(t3 * nf, err);
-    const float e1 = Val<T>::rnd(t4 * nf, err);
-    const float bv_m2 = Val<T>::store(e2), bv_m1 = Val<T>::store(e1);
-    /* anti-causal pass: state from stored/norm (ComputeGradient.hpp:382-407) */
-    float r2 = bv_m1 / nf;
-    float r1 = bv_m2 / nf;
-    for (int64_t b0 = nv - 1; b0 >= 0; b0 -= D) {
-        uint4 buf[D];
-#pragma unroll
-        for (int d = 0; d < D; ++d)
-            if (b0 - d >= 0) buf[d] = dst[b0 - d];
-#pragma unroll
-        for (int d = 0; d < D; ++d) {
-            if (b0 - d < 0) break;
-            uint4 o = buf[d];
-#pragma unroll
-            for (int i = V - 1; i >= 0; --i) {
-                const int64_t k = (b0 - d) * V + i;
-                float r;
-                if (k == y_num - 1) {
-                    r = bv_m1;
-                } else if (k == y_num - 2) {
-                    r = bv_m2;
-                } else {
-                    const float t = r1 * b1 + r2 * b2 + Vec16<T>::get(buf[d], i);
-                    r = Val<T>::rnd(t * nf, err);
-                    r2 = r1;
-                    r1 = t;
-                }
-                Vec16<T>::set_r(o, i, r);
-            }
-            dst[b0 - d] = o;
-        }
-    }
-    if (Val<T>::failed(err)) atomicAdd(d_err, 1);
 }
 
 /* x / z pass, 16-byte vectors along y, D steps of the recursion loaded ahead */
@@ -868,21 +751,28 @@ __device__ __forceinline__ void iir_outer_ck_body(T* img, int64_t y_num, int64_t
     if (Val<T>::failed(err)) atomicAdd(d_err, 1);
 }
 
-/* y pass without storing the causal result (u16, y_num % 64 == 0): the causal sweep streams
+/* y pass without storing the causal result: the causal sweep streams
  * the lines once and saves each line's recursion state (two floats) at the start of every
- * chunk; the anti-causal sweep walks the chunks from the end, reloads each chunk of the input,
- * recomputes its causal outputs into the LDS row from the saved state and runs the
- * anti-causal recursion over the row before the chunk is written.  The same operations in the
- * same order as a plain causal-then-anti-causal sweep, so the outputs are identical; the line
- * moves 2 reads and one
- * write instead of 2 reads and 2 writes (plus 8 bytes of state per 64 samples).  In place is
- * safe: chunk ch is written after chunk ch - 1 has been loaded. */
-__device__ __forceinline__ void iir_y_lds_ck_body(const uint16_t* in, uint16_t* out, int64_t y_num, int64_t n_lines, const IIRCoeffs& c,
-                                                  const float* d_off, int* d_err, float2* __restrict__ ck, uint32_t* mm,
-                                                  const int* run_if, uint16_t* pyr, int64_t px_num, int64_t pz_num, int64_t blk) {
-    constexpr int CH = 64;
-    constexpr int PITCH = 72;
-    __shared__ __attribute__((aligned(16))) uint16_t tile[64 * PITCH];
+ * chunk of 128 bytes (64 u16, 32 f32); the anti-causal sweep walks the chunks from the end,
+ * reloads each chunk of the input, recomputes its causal outputs into the LDS row from the saved
+ * state and runs the anti-causal recursion over the row before the chunk is written.  The same
+ * operations in the same order as a plain causal-then-anti-causal sweep, so the outputs are
+ * identical; the line moves 2 reads and one write instead of 2 reads and 2 writes (plus 8 bytes of
+ * state per chunk).  In place is safe: chunk ch is written after chunk ch - 1 has been loaded.
+ * RAG: lines of any length and alignment, read with 16-byte loads at their own alignment and
+ * written to rows of pitch oq (whole 16-byte words; the samples past y_num become 0).  Only the
+ * last chunk, and the one before it where that holds sample y_num - 2, test their samples.  On
+ * 1001 x 777 x 203 u16 the pass took 2.41 ms with one sample per lane and load and the causal
+ * result stored, 0.30 ms this way. */
+template <typename T, bool RAG>
+__device__ __forceinline__ void iir_y_ck_body(const T* in, T* out, int64_t y_num, int64_t oq, int64_t n_lines, const IIRCoeffs& c,
+                                              const float* d_off, int* d_err, float2* __restrict__ ck, uint32_t* mm, const int* run_if,
+                                              uint16_t* pyr, int64_t px_num, int64_t pz_num, int64_t blk) {
+    constexpr bool U16 = std::is_same<T, uint16_t>::value;
+    constexpr int V = Vec16<T>::N;
+    constexpr int CH = 8 * V;
+    constexpr int PITCH = 9 * V;
+    __shared__ __attribute__((aligned(16))) T tile[64 * PITCH];
     if (run_if && *run_if == 0) return;
     const int lane = threadIdx.x;
     /* LDS row R -> line (z * x_num + x), or -1.  Plain: 64 consecutive lines.  With pyr: rows
@@ -901,27 +791,47 @@ __device__ __forceinline__ void iir_y_lds_ck_body(const uint16_t* in, uint16_t* 
     const bool has_off = d_off != nullptr;
     const float off = has_off ? *d_off : 0.0f;
     const float b1 = c.b1, b2 = c.b2, nf = c.nf;
-    const int64_t nch = y_num / CH;
+    const int64_t nch = RAG ? (y_num + CH - 1) / CH : y_num / CH;
+    const int tail = RAG ? (int)(y_num - (nch - 1) * CH) : CH;   /* samples of the last chunk */
     const int seg = lane & 7;
     int err = 0;
+    auto load16 = [](const T* p) -> uint4 {
+        uint4 v;
+        if constexpr (RAG) __builtin_memcpy(&v, p, 16);
+        else v = *(const uint4*)p;
+        return v;
+    };
 
     /* lines of the cooperative layout: load instruction i covers LDS rows 8i..8i+7 */
     int64_t lrow[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) lrow[i] = line_of(8 * i + (lane >> 3));
-    auto gload = [&](const uint16_t* base, int64_t ch, uint4* r) {
+    auto gload = [&](const T* base, int64_t ch, uint4* r) {
+        const bool whole = !RAG || ch + 1 < nch || seg * V + V <= tail;
 #pragma unroll
-        for (int i = 0; i < 8; ++i)
-            r[i] = (lrow[i] >= 0) ? *(const uint4*)(base + lrow[i] * y_num + ch * CH + seg * 8) : make_uint4(0, 0, 0, 0);
+        for (int i = 0; i < 8; ++i) {
+            r[i] = make_uint4(0, 0, 0, 0);
+            if (lrow[i] < 0) continue;
+            const T* p = base + lrow[i] * y_num + ch * CH + seg * V;
+            if (whole) {
+                r[i] = load16(p);
+            } else {
+                T e[V];
+#pragma unroll
+                for (int j = 0; j < V; ++j) e[j] = seg * V + j < tail ? p[j] : (T)0;
+                __builtin_memcpy(&r[i], e, 16);
+            }
+        }
     };
     auto lds_put = [&](const uint4* r) {
 #pragma unroll
-        for (int i = 0; i < 8; ++i) *(uint4*)(&tile[(8 * i + (lane >> 3)) * PITCH + seg * 8]) = r[i];
+        for (int i = 0; i < 8; ++i) *(uint4*)(&tile[(8 * i + (lane >> 3)) * PITCH + seg * V]) = r[i];
     };
-    auto gstore = [&](uint16_t* base, int64_t ch) {
+    auto gstore = [&](T* base, int64_t ch) {
+        if (RAG && ch * CH + seg * V >= oq) return;
 #pragma unroll
         for (int i = 0; i < 8; ++i)
-            if (lrow[i] >= 0) *(uint4*)(base + lrow[i] * y_num + ch * CH + seg * 8) = *(const uint4*)(&tile[(8 * i + (lane >> 3)) * PITCH + seg * 8]);
+            if (lrow[i] >= 0) *(uint4*)(base + lrow[i] * oq + ch * CH + seg * V) = *(const uint4*)(&tile[(8 * i + (lane >> 3)) * PITCH + seg * V]);
     };
     /* the mean pyramid's cells of one chunk (PixelData.hpp:944-962 with u16 storage): 16 x pairs
        x 32 y pairs of the plane pair; a lane sums 8 y pairs of one x pair over its 4 rows (eight
@@ -956,98 +866,103 @@ __device__ __forceinline__ void iir_y_lds_ck_body(const uint16_t* in, uint16_t* 
     /* boundary sums (ComputeGradient.hpp:342-356) */
     float t1 = 0, t2 = 0, t3 = 0, t4 = 0;
     if (valid) {
-        const uint4* src = (const uint4*)(in + me * y_num);
-        const int64_t nv = y_num / 8;
-        const int nb = (c.mL + 7) / 8;
-        for (int b = 0; b < nb; ++b) {
-            const uint4 v = src[b];
+        const T* line = in + me * y_num;
+        const int nb = (c.mL + V - 1) / V;
+        if (RAG && (int64_t)nb * V > y_num) {
+            /* a line shorter than the vectors that hold its boundary samples */
+            for (int k = 0; k < c.mL; ++k) {
+                const float x = load_in(line + k, off, has_off);
+                t1 += c.bc1[k] * x;
+                t2 += c.bc2[k] * x;
+            }
+            for (int k = 0; k < c.mL; ++k) {
+                const float x = load_in(line + (y_num - 1 - k), off, has_off);
+                t3 += c.bc3[k] * x;
+                t4 += c.bc4[k] * x;
+            }
+        } else {
+            for (int b = 0; b < nb; ++b) {
+                const uint4 v = load16(line + b * V);
 #pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                const int k = b * 8 + i;
-                if (k < c.mL) {
-                    const float x = vin<uint16_t>(v, i, off, has_off);
-                    t1 += c.bc1[k] * x;
-                    t2 += c.bc2[k] * x;
+                for (int i = 0; i < V; ++i) {
+                    const int k = b * V + i;
+                    if (k < c.mL) {
+                        const float x = vin<T>(v, i, off, has_off);
+                        t1 += c.bc1[k] * x;
+                        t2 += c.bc2[k] * x;
+                    }
                 }
             }
-        }
-        for (int b = 0; b < nb; ++b) {
-            const uint4 v = src[nv - 1 - b];
+            for (int b = 0; b < nb; ++b) {
+                const uint4 v = load16(line + (y_num - (int64_t)(b + 1) * V));
 #pragma unroll
-            for (int i = 7; i >= 0; --i) {
-                const int k = b * 8 + (7 - i);
-                if (k < c.mL) {
-                    const float x = vin<uint16_t>(v, i, off, has_off);
-                    t3 += c.bc3[k] * x;
-                    t4 += c.bc4[k] * x;
+                for (int i = V - 1; i >= 0; --i) {
+                    const int k = b * V + (V - 1 - i);
+                    if (k < c.mL) {
+                        const float x = vin<T>(v, i, off, has_off);
+                        t3 += c.bc3[k] * x;
+                        t4 += c.bc4[k] * x;
+                    }
                 }
             }
         }
     }
-    const float t2q = Val<uint16_t>::store(t2), t1q = Val<uint16_t>::store(t1);
-    /* causal recursion over one LDS row chunk from state (s1, s2); with `keep` the outputs
+    const float t2q = Val<T>::store(t2), t1q = Val<T>::store(t1);
+    /* causal recursion over one LDS row chunk of n samples from state (s1, s2); with `keep` the outputs
        replace the row's samples */
-    /* the first chunk holds samples 0 and 1, which take the boundary values; the others run
-       without per-sample tests.  Without `keep` (the first sweep) nothing is rounded: the
-       recursion carries the unrounded values, and the range check of the rounded outputs
+    /* the first chunk holds samples 0 and 1, which take the boundary values, and the last may be
+       short; the others run without per-sample tests.  Without `keep` (the first sweep) nothing is
+       rounded: the recursion carries the unrounded values, and the range check of the rounded outputs
        becomes a running min / max of the unrounded ones, since roundf(t) lies in [0, 65535]
        exactly when -0.5 < t < 65535.5.  The re-computing sweep rounds the same values again
        and skips the check. */
-    auto causal = [&](uint16_t* row, int64_t ch, float& s1, float& s2, bool keep, float& lo, float& hi) {
+    auto causal = [&](T* row, int64_t ch, float& s1, float& s2, bool keep, float& lo, float& hi) {
         int e = 0;
-        if (ch == 0) {
+        const int n = RAG && ch + 1 == nch ? tail : CH;
+        auto step = [&](const uint4& v, uint4& o, int i) {
+            const float t = s1 * b1 + s2 * b2 + vin<T>(v, i, off, has_off);
+            if (keep) {
+                Vec16<T>::set_r(o, i, Val<T>::rnd(t, e));
+            } else if (U16) {
+                lo = fminf(lo, t);
+                hi = fmaxf(hi, t);
+            }
+            s2 = s1;
+            s1 = t;
+        };
+        if (ch == 0 || (RAG && n < CH)) {
 #pragma unroll
-            for (int q = 0; q < CH / 8; ++q) {
-                uint4 v = *(uint4*)(row + q * 8);
+            for (int q = 0; q < CH / V; ++q) {
+                if (RAG && q * V >= n) break;
+                uint4 v = *(uint4*)(row + q * V);
                 uint4 o = make_uint4(0, 0, 0, 0);
 #pragma unroll
-                for (int i = 0; i < 8; ++i) {
-                    const int k = q * 8 + i;
-                    float r;
-                    if (k == 0) {
-                        r = t2q;
-                    } else if (k == 1) {
-                        r = t1q;
+                for (int i = 0; i < V; ++i) {
+                    const int k = q * V + i;
+                    if (RAG && k >= n) break;
+                    if (ch == 0 && k < 2) {
+                        if (keep) Vec16<T>::set_r(o, i, k == 0 ? t2q : t1q);
                     } else {
-                        const float t = s1 * b1 + s2 * b2 + vin<uint16_t>(v, i, off, has_off);
-                        if (keep) {
-                            r = Val<uint16_t>::rnd(t, e);
-                        } else {
-                            lo = fminf(lo, t);
-                            hi = fmaxf(hi, t);
-                            r = 0.0f;
-                        }
-                        s2 = s1;
-                        s1 = t;
+                        step(v, o, i);
                     }
-                    if (keep) Vec16<uint16_t>::set_r(o, i, r);
                 }
-                if (keep) *(uint4*)(row + q * 8) = o;
+                if (keep) *(uint4*)(row + q * V) = o;
             }
         } else {
 #pragma unroll
-            for (int q = 0; q < CH / 8; ++q) {
-                uint4 v = *(uint4*)(row + q * 8);
+            for (int q = 0; q < CH / V; ++q) {
+                uint4 v = *(uint4*)(row + q * V);
                 uint4 o = make_uint4(0, 0, 0, 0);
 #pragma unroll
-                for (int i = 0; i < 8; ++i) {
-                    const float t = s1 * b1 + s2 * b2 + vin<uint16_t>(v, i, off, has_off);
-                    if (keep) {
-                        Vec16<uint16_t>::set_r(o, i, Val<uint16_t>::rnd(t, e));
-                    } else {
-                        lo = fminf(lo, t);
-                        hi = fmaxf(hi, t);
-                    }
-                    s2 = s1;
-                    s1 = t;
-                }
-                if (keep) *(uint4*)(row + q * 8) = o;
+                for (int i = 0; i < V; ++i) step(v, o, i);
+                if (keep) *(uint4*)(row + q * V) = o;
             }
         }
     };
 
     /* causal sweep: states only; with mm, also the (min, max) of the raw samples (packed u16
-       min / max over the loaded vectors; lines past the end load zeros, so they are skipped) */
+       min / max over the loaded vectors; lines past the end and samples past a line's end load zeros, so
+       they are skipped) */
     {
         float s1 = t1, s2 = t2, tlo = 0.0f, thi = 0.0f;
         uint4 nxt[8];
@@ -1056,31 +971,45 @@ __device__ __forceinline__ void iir_y_lds_ck_body(const uint16_t* in, uint16_t* 
         gload(in, 0, nxt);
         for (int64_t ch = 0; ch < nch; ++ch) {
             __syncthreads();
-            if (mm) {
+            if (U16 && mm) {
+                const bool whole = !RAG || ch + 1 < nch || seg * V + V <= tail;
 #pragma unroll
                 for (int i = 0; i < 8; ++i) {
                     if (lrow[i] < 0) continue;
                     const uint32_t w[4] = {nxt[i].x, nxt[i].y, nxt[i].z, nxt[i].w};
+                    if (whole) {
 #pragma unroll
-                    for (int q = 0; q < 4; ++q) {
-                        us2 v;
-                        __builtin_memcpy(&v, &w[q], 4);
-                        lo = __builtin_elementwise_min(lo, v);
-                        hi = __builtin_elementwise_max(hi, v);
+                        for (int q = 0; q < 4; ++q) {
+                            us2 v;
+                            __builtin_memcpy(&v, &w[q], 4);
+                            lo = __builtin_elementwise_min(lo, v);
+                            hi = __builtin_elementwise_max(hi, v);
+                        }
+                    } else {
+#pragma unroll
+                        for (int j = 0; j < 8; ++j) {
+                            const uint16_t x = (uint16_t)(w[j >> 1] >> (16 * (j & 1)));
+                            if (seg * V + j < tail) {
+                                lo = __builtin_elementwise_min(lo, (us2){x, x});
+                                hi = __builtin_elementwise_max(hi, (us2){x, x});
+                            }
+                        }
                     }
                 }
             }
             lds_put(nxt);
             if (ch + 1 < nch) gload(in, ch + 1, nxt);
             __syncthreads();
-            if (pyr) pyr_chunk(ch);
+            if constexpr (U16 && !RAG) {
+                if (pyr) pyr_chunk(ch);
+            }
             if (valid) {
                 if (ch > 0) ck[(ch - 1) * n_lines + me] = make_float2(s1, s2);
                 causal(&tile[lane * PITCH], ch, s1, s2, false, tlo, thi);
             }
         }
-        if (!(tlo > -0.5f && thi < 65535.5f)) err |= 0x10000;
-        if (mm) {
+        if (U16 && !(tlo > -0.5f && thi < 65535.5f)) err |= 0x10000;
+        if (U16 && mm) {
             uint32_t l = min((uint32_t)lo.x, (uint32_t)lo.y), h = max((uint32_t)hi.x, (uint32_t)hi.y);
             for (int o = 32; o > 0; o >>= 1) {
                 l = min(l, (uint32_t)__shfl_xor((int)l, o));
@@ -1092,9 +1021,9 @@ __device__ __forceinline__ void iir_y_lds_ck_body(const uint16_t* in, uint16_t* 
             }
         }
     }
-    const float e2 = Val<uint16_t>::rnd(t3 * nf, err);
-    const float e1 = Val<uint16_t>::rnd(t4 * nf, err);
-    const float bv_m2 = Val<uint16_t>::store(e2), bv_m1 = Val<uint16_t>::store(e1);
+    const float e2 = Val<T>::rnd(t3 * nf, err);
+    const float e1 = Val<T>::rnd(t4 * nf, err);
+    const float bv_m2 = Val<T>::store(e2), bv_m1 = Val<T>::store(e1);
     float r2 = bv_m1 / nf;
     float r1 = bv_m2 / nf;
     /* anti-causal sweep: recompute each chunk's causal outputs, then run backwards over them */
@@ -1106,7 +1035,7 @@ __device__ __forceinline__ void iir_y_lds_ck_body(const uint16_t* in, uint16_t* 
         if (ch - 1 >= 0) gload(in, ch - 1, nxt);
         __syncthreads();
         if (valid) {
-            uint16_t* row = &tile[lane * PITCH];
+            T* row = &tile[lane * PITCH];
             float s1 = t1, s2 = t2;
             if (ch > 0) {
                 const float2 st = ck[(ch - 1) * n_lines + me];
@@ -1115,50 +1044,45 @@ __device__ __forceinline__ void iir_y_lds_ck_body(const uint16_t* in, uint16_t* 
             }
             float unused_lo = 0.0f, unused_hi = 0.0f;
             causal(row, ch, s1, s2, true, unused_lo, unused_hi);
-            if (ch == nch - 1) {
-                /* the last chunk holds samples y_num-2 and y_num-1, which take the boundary values */
+            auto back = [&](const uint4& v, uint4& o, int i) {
+                const float t = r1 * b1 + r2 * b2 + Vec16<T>::get(v, i);
+                Vec16<T>::set_r(o, i, Val<T>::rnd(t * nf, err));
+                r2 = r1;
+                r1 = t;
+            };
+            if ((ch + 1) * CH > y_num - 2) {
+                /* the chunk holds sample y_num - 2 or y_num - 1, which take the boundary values */
+                const int last = (int)(y_num - 1 - ch * CH);   /* sample y_num - 1 in this chunk's numbering */
 #pragma unroll
-                for (int q = CH / 8 - 1; q >= 0; --q) {
-                    uint4 v = *(uint4*)(row + q * 8);
+                for (int q = CH / V - 1; q >= 0; --q) {
+                    if (RAG && q * V > last) continue;
+                    uint4 v = *(uint4*)(row + q * V);
                     uint4 o = make_uint4(0, 0, 0, 0);
 #pragma unroll
-                    for (int i = 7; i >= 0; --i) {
-                        const int k = q * 8 + i;
-                        float r;
-                        if (k == CH - 1) {
-                            r = bv_m1;
-                        } else if (k == CH - 2) {
-                            r = bv_m2;
-                        } else {
-                            const float t = r1 * b1 + r2 * b2 + Vec16<uint16_t>::get(v, i);
-                            r = Val<uint16_t>::rnd(t * nf, err);
-                            r2 = r1;
-                            r1 = t;
-                        }
-                        Vec16<uint16_t>::set_r(o, i, r);
+                    for (int i = V - 1; i >= 0; --i) {
+                        const int k = q * V + i;
+                        if (RAG && k > last) continue;
+                        if (k == last) Vec16<T>::set_r(o, i, bv_m1);
+                        else if (k == last - 1) Vec16<T>::set_r(o, i, bv_m2);
+                        else back(v, o, i);
                     }
-                    *(uint4*)(row + q * 8) = o;
+                    *(uint4*)(row + q * V) = o;
                 }
             } else {
 #pragma unroll
-                for (int q = CH / 8 - 1; q >= 0; --q) {
-                    uint4 v = *(uint4*)(row + q * 8);
+                for (int q = CH / V - 1; q >= 0; --q) {
+                    uint4 v = *(uint4*)(row + q * V);
                     uint4 o = make_uint4(0, 0, 0, 0);
 #pragma unroll
-                    for (int i = 7; i >= 0; --i) {
-                        const float t = r1 * b1 + r2 * b2 + Vec16<uint16_t>::get(v, i);
-                        Vec16<uint16_t>::set_r(o, i, Val<uint16_t>::rnd(t * nf, err));
-                        r2 = r1;
-                        r1 = t;
-                    }
-                    *(uint4*)(row + q * 8) = o;
+                    for (int i = V - 1; i >= 0; --i) back(v, o, i);
+                    *(uint4*)(row + q * V) = o;
                 }
             }
         }
         __syncthreads();
         gstore(out, ch);
     }
-    if (Val<uint16_t>::failed(err)) atomicAdd(d_err, 1);
+    if (Val<T>::failed(err)) atomicAdd(d_err, 1);
 }
 
 /* per-volume arguments of the smoothing passes */
@@ -1167,7 +1091,7 @@ struct IirArgs {
     const T* in;          /* y pass input (may equal out) */
     T* out;               /* y pass output / image of the x, z passes */
     int64_t y_num, n;     /* y length; length of the filtered axis (x, z passes) or lines (y) */
-    int64_t s, outer_stride, gx;
+    int64_t s, outer_stride, gx;   /* s: axis stride (x, z passes) or output row pitch (y pass) */
     IIRCoeffs c;
     const float* d_off;
     int* d_err;
@@ -1186,19 +1110,13 @@ struct IirY {
     static const char* name() { return "bspline_y"; }
     static __device__ __forceinline__ void run(const Args& a, int64_t t) { iir_y_body<T>(a.in, a.out, a.y_num, a.n, a.c, a.d_off, a.d_err, t); }
 };
-template <typename T, int D>
-struct IirYVec {
+template <typename T, bool RAG>
+struct IirYCk {
     using Args = IirArgs<T>;
-    static constexpr int THREADS = 256;
-    static const char* name() { return "bspline_y_vec"; }
-    static __device__ __forceinline__ void run(const Args& a, int64_t t) { iir_y_vec_body<T, D>(a.in, a.out, a.y_num, a.n, a.c, a.d_off, a.d_err, t); }
-};
-struct IirYLdsCk {
-    using Args = IirArgs<uint16_t>;
     static constexpr int THREADS = 64;
-    static const char* name() { return "bspline_y_lds_ck"; }
+    static const char* name() { return RAG ? "bspline_y_ck_ragged" : "bspline_y_ck"; }
     static __device__ __forceinline__ void run(const Args& a, int64_t t) {
-        iir_y_lds_ck_body(a.in, a.out, a.y_num, a.n, a.c, a.d_off, a.d_err, (float2*)a.ck, a.mm, a.run_if, a.pyr, a.px, a.pz, t);
+        iir_y_ck_body<T, RAG>(a.in, a.out, a.y_num, a.s, a.n, a.c, a.d_off, a.d_err, (float2*)a.ck, a.mm, a.run_if, a.pyr, a.px, a.pz, t);
     }
 };
 template <typename T>
@@ -1248,14 +1166,30 @@ void launch_offset_copy(aprh_context* ctx, const uint16_t* in, uint16_t* out, si
     launch_tiles<OffsetCopy>(ctx, {in, out, n, d_offset, G}, G);
 }
 
-bool iir_y_fuses_offset(int64_t y, const void* in, const void* out) { return y % 64 == 0 && aligned16(in) && aligned16(out); }
+int64_t iir_pitch(int64_t y, size_t elem) {
+    const int64_t v = 16 / (int64_t)elem;
+    return cdiv(y, v) * v;
+}
+
+namespace {
+/* chunks of a y line (128 bytes each), and whether the pass reads and writes whole aligned chunks */
+template <typename T>
+int64_t y_chunks(int64_t y) { return cdiv(y, 8 * Vec16<T>::N); }
+template <typename T>
+bool y_whole(int64_t y, const void* in, const void* out) { return y % (8 * Vec16<T>::N) == 0 && aligned16(in) && aligned16(out); }
+}  // namespace
 
 void launch_iir_y_offset(aprh_context* ctx, const uint16_t* in, uint16_t* out, int64_t y, int64_t x, int64_t z, const IIRCoeffs& c,
                          float lambda, float* d_offset, uint32_t* d_mm, int* d_rerun, int* d_err, uint16_t* pyr) {
     const int64_t lines = x * z;
-    IirArgs<uint16_t> a{in, out, y, lines, 0, 0, 1, c, d_offset, d_err};
-    Buf ck(ctx->pool, (size_t)std::max<int64_t>(y / 64 - 1, 1) * (size_t)lines * 8);
+    const bool whole = y_whole<uint16_t>(y, in, out);
+    IirArgs<uint16_t> a{in, out, y, lines, iir_pitch(y, 2), 0, 1, c, d_offset, d_err};
+    Buf ck(ctx->pool, (size_t)std::max<int64_t>(y_chunks<uint16_t>(y) - 1, 1) * (size_t)lines * 8);
     a.ck = ck.as<uint4>();
+    auto pass = [&](int64_t tiles) {
+        if (whole) launch_tiles<IirYCk<uint16_t, false>>(ctx, a, tiles);
+        else launch_tiles<IirYCk<uint16_t, true>>(ctx, a, tiles);
+    };
     launch_tiles<OffsetGuess>(ctx, {d_mm, lambda, d_offset, d_rerun}, 1);
     a.mm = d_mm;
     if (pyr) {
@@ -1263,38 +1197,36 @@ void launch_iir_y_offset(aprh_context* ctx, const uint16_t* in, uint16_t* out, i
         a.pyr = pyr;
         a.px = x;
         a.pz = z;
-        launch_tiles<IirYLdsCk>(ctx, a, cdiv(z, 2) * cdiv(x, 32));
+        pass(cdiv(z, 2) * cdiv(x, 32));
     } else {
-        launch_tiles<IirYLdsCk>(ctx, a, cdiv(lines, 64));
+        pass(cdiv(lines, 64));
     }
     launch_tiles<OffsetVerify>(ctx, {d_mm, lambda, d_offset, d_rerun, d_err}, 1);
     /* the pass again with the true offset, as blocks that return at once unless the guess was wrong */
     a.mm = nullptr;
     a.pyr = nullptr;
     a.run_if = d_rerun;
-    launch_tiles<IirYLdsCk>(ctx, a, cdiv(lines, 64));
+    pass(cdiv(lines, 64));
 }
 
+bool iir_y_writes_pyramid(int64_t y, const void* in) { return y % 64 == 0 && aligned16(in); }
+
 template <typename T>
-void launch_iir_y(aprh_context* ctx, const T* in, T* out, int64_t y, int64_t x, int64_t z, const IIRCoeffs& c,
-                  const float* d_offset, int* d_err) {
+void launch_iir_y(aprh_context* ctx, const T* in, T* out, int64_t y, int64_t x, int64_t z, const IIRCoeffs& c, const float* d_offset,
+                  int* d_err, int64_t pitch) {
     const int64_t lines = x * z;
-    constexpr int V = Vec16<T>::N;
-    IirArgs<T> a{in, out, y, lines, 0, 0, 1, c, d_offset, d_err};
-    if constexpr (std::is_same<T, uint16_t>::value) {
-        if (y % 64 == 0 && aligned16(in) && aligned16(out)) {
-            /* line states at the start of chunks 1 .. y/64-1 */
-            Buf ck(ctx->pool, (size_t)std::max<int64_t>(y / 64 - 1, 1) * (size_t)lines * 8);
-            a.ck = ck.as<uint4>();
-            launch_tiles<IirYLdsCk>(ctx, a, cdiv(lines, 64));
-            return;
-        }
-    }
-    if (y % V == 0 && y >= 2 * V && aligned16(in) && aligned16(out)) {
-        launch_tiles<IirYVec<T, 4>>(ctx, a, cdiv(lines, 256));
-    } else {
+    IirArgs<T> a{in, out, y, lines, pitch, 0, 1, c, d_offset, d_err};
+    const bool whole = y_whole<T>(y, in, out) && pitch == y;
+    if (!whole && (pitch != iir_pitch(y, sizeof(T)) || !aligned16(out))) {
+        /* output rows that are no whole number of aligned 16-byte words (stage entry point) */
         launch_tiles<IirY<T>>(ctx, a, cdiv(lines, TL));
+        return;
     }
+    /* line states at the start of the chunks but the first */
+    Buf ck(ctx->pool, (size_t)std::max<int64_t>(y_chunks<T>(y) - 1, 1) * (size_t)lines * 8);
+    a.ck = ck.as<uint4>();
+    if (whole) launch_tiles<IirYCk<T, false>>(ctx, a, cdiv(lines, 64));
+    else launch_tiles<IirYCk<T, true>>(ctx, a, cdiv(lines, 64));
 }
 
 /* checkpointed x / z pass: chunk length and the shortest axis it is used for */
@@ -1339,9 +1271,9 @@ void launch_iir_outer(aprh_context* ctx, T* img, int64_t y, int64_t x, int64_t z
 }
 
 template void launch_iir_y<uint16_t>(aprh_context*, const uint16_t*, uint16_t*, int64_t, int64_t, int64_t, const IIRCoeffs&,
-                                     const float*, int*);
+                                     const float*, int*, int64_t);
 template void launch_iir_y<float>(aprh_context*, const float*, float*, int64_t, int64_t, int64_t, const IIRCoeffs&, const float*,
-                                  int*);
+                                  int*, int64_t);
 template void launch_iir_outer<uint16_t>(aprh_context*, uint16_t*, int64_t, int64_t, int64_t, int, const IIRCoeffs&, int*);
 template void launch_iir_outer<float>(aprh_context*, float*, int64_t, int64_t, int64_t, int, const IIRCoeffs&, int*);
 

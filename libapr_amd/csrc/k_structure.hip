@@ -84,10 +84,11 @@ __device__ __forceinline__ void seed_body(const uint8_t* __restrict__ lev, uint8
    one.  One lane per 8 consecutive y cells: the 3x3x3 neighbourhood
    predicates are formed as bit masks over the 9 neighbouring rows (10 bits: y0-1 .. y0+8),
    dilated along y by shifts, so a lane loads 9 row words instead of 27 bytes per cell. */
-__device__ __forceinline__ void load_row8(const uint8_t* row, int yn, int y0, bool aligned8, uint8_t b[10]) {
+__device__ __forceinline__ void load_row8(const uint8_t* row, int yn, int y0, uint8_t b[10]) {
     b[0] = (y0 > 0) ? row[y0 - 1] : (uint8_t)0;
-    if (aligned8 && y0 + 8 <= yn) {
-        const uint64_t w = *(const uint64_t*)(row + y0);
+    if (y0 + 8 <= yn) {   /* one 8-byte load at any alignment */
+        uint64_t w;
+        __builtin_memcpy(&w, row + y0, 8);
 #pragma unroll
         for (int j = 0; j < 8; ++j) b[1 + j] = (uint8_t)(w >> (8 * j));
     } else {
@@ -121,7 +122,6 @@ __device__ __forceinline__ void pull_level8_body(uint8_t* P, Dims d, uint8_t* Pc
     const int nwr = (yn + 7) >> 3;
     const int nzc = (zn + ZC - 1) / ZC;
     const int64_t total = (int64_t)nwr * xn * nzc;
-    const bool aligned8 = (yn & 7) == 0 && ((uintptr_t)P & 7) == 0;
     /* parent rows whose words never straddle two rows */
     const bool par_words = has_parent && (dp.y & 3) == 0 && ((uintptr_t)Pp & 3) == 0;
     for (int64_t i = t * blockDim.x + threadIdx.x; i < total; i += G * blockDim.x) {
@@ -140,7 +140,7 @@ __device__ __forceinline__ void pull_level8_body(uint8_t* P, Dims d, uint8_t* Pc
                 const int xx = x + dx;
                 if (xx < 0 || xx >= xn) continue;
                 uint8_t b[10];
-                load_row8(P + ((int64_t)zz * xn + xx) * yn, yn, y0, aligned8, b);
+                load_row8(P + ((int64_t)zz * xn + xx) * yn, yn, y0, b);
                 uint32_t a1, s1;
                 row_masks(b, a1, s1);
                 am |= a1;
@@ -176,11 +176,11 @@ __device__ __forceinline__ void pull_level8_body(uint8_t* P, Dims d, uint8_t* Pc
                 changed |= (nw != old) && (y0 + j < yn);
             }
             if (changed) {
-                if (aligned8) {
+                if (y0 + 8 <= yn) {
                     uint64_t v = 0;
 #pragma unroll
                     for (int j = 0; j < 8; ++j) v |= (uint64_t)nb[j] << (8 * j);
-                    *(uint64_t*)(row + y0) = v;
+                    __builtin_memcpy(row + y0, &v, 8);
                 } else {
 #pragma unroll
                     for (int j = 0; j < 8; ++j)
@@ -303,8 +303,9 @@ constexpr int CPL = 16;   /* cells per lane per chunk: a wave covers 1024 cells 
 /* weights of the CPL cells [c0, c0 + CPL) of a row (0 beyond its end) */
 __device__ __forceinline__ void chunk_weights(const RowTable& t, int li, const uint8_t* p, int ylen, int c0, int w[CPL]) {
     const bool top = (li == t.n_levels - 1);
-    if (c0 + CPL <= ylen && ((uintptr_t)(p + c0) & 15) == 0) {
-        const uint4 v = *(const uint4*)(p + c0);
+    if (c0 + CPL <= ylen) {   /* one 16-byte load at any alignment */
+        uint4 v;
+        __builtin_memcpy(&v, p + c0, 16);
         const uint32_t words[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
         for (int j = 0; j < CPL; ++j) w[j] = cell_weight(t, li, (uint8_t)(words[j >> 2] >> (8 * (j & 3))), c0 + j);
@@ -668,52 +669,75 @@ template <typename T> __device__ __forceinline__ T pyr_store(float m);
 template <> __device__ __forceinline__ uint16_t pyr_store<uint16_t>(float m) { return (uint16_t)(int32_t)m; }
 template <> __device__ __forceinline__ float pyr_store<float>(float m) { return m; }
 
+/* a lane takes the coarse cells of 16 bytes of a fine row (4 u16 cells, 2 float cells) from four fine
+   rows, loaded at any alignment; the sums of a u16 cell are exact in any order, those of a float cell
+   run in the order above.  fg, fx: division by the groups of a row and by cd.x (32-bit indices), or
+   fits == 0 */
+struct PyrDiv {
+    FastDiv fg, fx;
+    int fits;
+};
 template <typename T>
-__global__ void k_pyr_down(const T* __restrict__ fine, Dims fd, T* coarse, Dims cd) {
-    const size_t n = (size_t)(cd.y * cd.x * cd.z);
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
-        const int64_t y = (int64_t)(i % (size_t)cd.y);
-        const int64_t r = (int64_t)(i / (size_t)cd.y);
-        const int64_t x = r % cd.x, z = r / cd.x;
-        const int64_t y1 = min(2 * y + 1, fd.y - 1), x1 = min(2 * x + 1, fd.x - 1), z1 = min(2 * z + 1, fd.z - 1);
-        const int64_t y0 = 2 * y, x0 = 2 * x, z0 = 2 * z;
-        float s = (float)fine[(z0 * fd.x + x0) * fd.y + y0];
-        s = s + (float)fine[(z0 * fd.x + x0) * fd.y + y1];
-        s = s + (float)fine[(z0 * fd.x + x1) * fd.y + y0];
-        s = s + (float)fine[(z0 * fd.x + x1) * fd.y + y1];
-        s = s + (float)fine[(z1 * fd.x + x0) * fd.y + y0];
-        s = s + (float)fine[(z1 * fd.x + x0) * fd.y + y1];
-        s = s + (float)fine[(z1 * fd.x + x1) * fd.y + y0];
-        s = s + (float)fine[(z1 * fd.x + x1) * fd.y + y1];
-        const float m = s / 8.0f;
-        coarse[i] = pyr_store<T>(m);
-    }
-}
-
-/* the same mean for u16 with 8 fine y per lane (16-byte row loads, 4 coarse outputs); the
-   integer sum of eight u16 values is exact in float, so the order of the float additions
-   above does not matter and the result is identical */
-__global__ __launch_bounds__(256) void k_pyr_down_u16v(const uint16_t* __restrict__ fine, Dims fd, uint16_t* coarse, Dims cd) {
-    const int64_t ng = cd.y / 4;
+__global__ __launch_bounds__(256) void k_pyr_down(const T* __restrict__ fine, Dims fd, T* coarse, Dims cd, PyrDiv dv) {
+    constexpr int NF = 16 / sizeof(T), NC = NF / 2;
+    const int64_t ng = (cd.y + NC - 1) / NC;
     const int64_t total = ng * cd.x * cd.z;
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += (int64_t)gridDim.x * blockDim.x) {
-        const int64_t g = i % ng, r = i / ng;
-        const int64_t x = r % cd.x, z = r / cd.x;
-        const int64_t x0 = 2 * x, x1 = min(2 * x + 1, fd.x - 1), z0 = 2 * z, z1 = min(2 * z + 1, fd.z - 1);
-        const uint4 a = *(const uint4*)(fine + (z0 * fd.x + x0) * fd.y + 8 * g);
-        const uint4 b = *(const uint4*)(fine + (z0 * fd.x + x1) * fd.y + 8 * g);
-        const uint4 c = *(const uint4*)(fine + (z1 * fd.x + x0) * fd.y + 8 * g);
-        const uint4 d = *(const uint4*)(fine + (z1 * fd.x + x1) * fd.y + 8 * g);
-        const uint32_t wa[4] = {a.x, a.y, a.z, a.w}, wb[4] = {b.x, b.y, b.z, b.w}, wc[4] = {c.x, c.y, c.z, c.w},
-                       wd[4] = {d.x, d.y, d.z, d.w};
-        uint32_t o[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const uint32_t sum = (wa[j] & 0xFFFFu) + (wa[j] >> 16) + (wb[j] & 0xFFFFu) + (wb[j] >> 16) + (wc[j] & 0xFFFFu) +
-                                 (wc[j] >> 16) + (wd[j] & 0xFFFFu) + (wd[j] >> 16);
-            o[j] = (uint32_t)pyr_store<uint16_t>((float)sum / 8.0f);
+        int64_t g, x, z;
+        if (dv.fits) {
+            const uint32_t r = dv.fg.div((uint32_t)i), zz = dv.fx.div(r);
+            g = (uint32_t)i - r * (uint32_t)ng;
+            x = r - zz * (uint32_t)cd.x;
+            z = zz;
+        } else {
+            const int64_t r = i / ng;
+            g = i - r * ng;
+            z = r / cd.x;
+            x = r - z * cd.x;
         }
-        *(uint2*)(coarse + (z * cd.x + x) * cd.y + 4 * g) = make_uint2(o[0] | (o[1] << 16), o[2] | (o[3] << 16));
+        const int64_t x0 = 2 * x, x1 = min(2 * x + 1, fd.x - 1), z0 = 2 * z, z1 = min(2 * z + 1, fd.z - 1), y0 = NF * g;
+        const T* rows[4] = {fine + (z0 * fd.x + x0) * fd.y, fine + (z0 * fd.x + x1) * fd.y, fine + (z1 * fd.x + x0) * fd.y,
+                            fine + (z1 * fd.x + x1) * fd.y};
+        uint32_t w[4][4];
+        if (y0 + NF <= fd.y) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) __builtin_memcpy(w[q], rows[q] + y0, 16);
+        } else {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                T e[NF];
+#pragma unroll
+                for (int j = 0; j < NF; ++j) e[j] = rows[q][min(y0 + j, fd.y - 1)];
+                __builtin_memcpy(w[q], e, 16);
+            }
+        }
+        T o[NC];
+#pragma unroll
+        for (int j = 0; j < NC; ++j) {
+            if constexpr (std::is_same<T, uint16_t>::value) {
+                uint32_t s = 0;
+#pragma unroll
+                for (int q = 0; q < 4; ++q) s += (w[q][j] & 0xFFFFu) + (w[q][j] >> 16);
+                o[j] = pyr_store<T>((float)s / 8.0f);
+            } else {
+                float s = __uint_as_float(w[0][2 * j]);
+                s = s + __uint_as_float(w[0][2 * j + 1]);
+#pragma unroll
+                for (int q = 1; q < 4; ++q) {
+                    s = s + __uint_as_float(w[q][2 * j]);
+                    s = s + __uint_as_float(w[q][2 * j + 1]);
+                }
+                o[j] = pyr_store<T>(s / 8.0f);
+            }
+        }
+        T* dst = coarse + (z * cd.x + x) * cd.y + NC * g;
+        if (NC * g + NC <= cd.y) {
+            __builtin_memcpy(dst, o, NC * sizeof(T));
+        } else {
+#pragma unroll
+            for (int j = 0; j < NC - 1; ++j)
+                if (NC * g + j < cd.y) dst[j] = o[j];
+        }
     }
 }
 
@@ -1127,14 +1151,14 @@ void pyramid_levels(aprh_context* ctx, const aprh_apr& a, const T* img, T* Pyr, 
         const T* fine = (l == lmax - 1) ? img : Pyr + off[l + 1];
         const Dims fd{a.y_num[l + 1], a.x_num[l + 1], a.z_num[l + 1]}, cd{a.y_num[l], a.x_num[l], a.z_num[l]};
         T* coarse = Pyr + off[l];
-        if (std::is_same<T, uint16_t>::value && fd.y % 8 == 0 && cd.y * 2 == fd.y && ((uintptr_t)fine & 15u) == 0 &&
-            ((uintptr_t)coarse & 7u) == 0) {
-            const int64_t work = cd.y / 4 * cd.x * cd.z;
-            hipLaunchKernelGGL(k_pyr_down_u16v, dim3((unsigned)std::min<int64_t>(cdiv(work, 256), 16384)), dim3(256), 0, st,
-                               (const uint16_t*)fine, fd, (uint16_t*)coarse, cd);
-        } else {
-            hipLaunchKernelGGL(k_pyr_down<T>, dim3(4096), dim3(256), 0, st, fine, fd, coarse, cd);
+        const int64_t ng = cdiv(cd.y, 8 / (int64_t)sizeof(T)), work = ng * cd.x * cd.z;
+        PyrDiv dv;
+        dv.fits = fits32(work) ? 1 : 0;
+        if (dv.fits) {
+            dv.fg = FastDiv((uint64_t)ng);
+            dv.fx = FastDiv((uint64_t)cd.x);
         }
+        hipLaunchKernelGGL(k_pyr_down<T>, dim3((unsigned)std::min<int64_t>(cdiv(work, 256), 16384)), dim3(256), 0, st, fine, fd, coarse, cd, dv);
         HIP_LAUNCH_CHECK();
     }
 }

@@ -210,3 +210,45 @@ def test_get_apr_f32_matches_oracle(oracle, ctx, shape, nb, seed, scale):
     assert np.array_equal(xze, ref.xz_end_vec) and np.array_equal(yv, ref.y_vec)
     parts = A.ParticleData().sample_image(apr, img)
     assert np.array_equal(parts.view(np.uint32), ref.sample_f32(img).view(np.uint32))
+
+
+@pytest.mark.parametrize("y", [3, 4, 5, 7, 8, 9, 31, 33, 63, 65, 66, 71, 72, 127, 129, 190, 1025])
+@pytest.mark.parametrize("image_type", [np.uint16, np.float32])
+def test_ragged_y_lines(oracle, ctx, y, image_type):
+    """every stage at y lengths around the 16-byte words and 128-byte chunks of the y pass (u16: 8 and 64
+    samples, f32: 4 and 32), with odd x and z: the smoothed rows are padded inside the pipeline"""
+    shape = (13, 21, y)
+    img = A.synth_blobs(shape, y, 6)
+    if image_type == np.float32:
+        img = (img * np.float32(0.37) + np.float32(1.25)).astype(np.float32)
+    f32 = image_type == np.float32
+    ref = (oracle.get_apr_f32 if f32 else oracle.get_apr)(img, _par(oracle), "oracle")
+    conv = A.APRConverter(ctx, image_type=image_type)
+    conv.par = _apar()
+    apr = conv.get_apr(img)
+    print(f"y {y} {image_type.__name__} P={apr.total} oracle P={ref.total}", flush=True)
+    for w in range(6):
+        g, o = apr.intermediate(w), ref.intermediate(w)
+        assert np.array_equal(g.view(np.uint8), o.view(np.uint8)), (w, int((g != o).sum()), np.argwhere(g != o)[:3].tolist())
+    _, xze, yv = apr.structure()
+    assert apr.total == ref.total and np.array_equal(xze, ref.xz_end_vec) and np.array_equal(yv, ref.y_vec)
+    parts = A.ParticleData().sample_image(apr, img)
+    assert np.array_equal(parts, ref.sample_f32(img) if f32 else ref.sample(img))
+
+
+@pytest.mark.parametrize("lo,hi", [(20000, 47000), (30000, 35500)])
+@pytest.mark.parametrize("y", [65, 100])
+def test_ragged_y_offset_not_guessed(oracle, ctx, lo, hi, y):
+    """the smallest and largest sample of a short last chunk count for the offset, its zeros do not"""
+    z, x = 8, 24
+    img = A.synth_blobs((z, x, y), 5, 12).astype(np.float64)
+    img = (lo + 10 + (img - img.min()) * (hi - lo - 20) / max(img.max() - img.min(), 1.0)).round().astype(np.uint16)
+    img[3, 5, y - 1], img[2, 7, y - 1] = lo, hi
+    conv = A.APRConverter(ctx)
+    conv.par = A.APRParameters(rel_error=0.1, sigma_th=50, Ip_th=120, grad_th=10, lambda_=0.2)
+    ref = oracle.get_apr(img, oracle.params(rel_error=0.1, sigma_th=50, Ip_th=120, grad_th=10, lambda_=0.2), "oracle")
+    apr = conv.get_apr(img)
+    assert apr.bspline_offset == ref.bspline_offset
+    for w in range(6):
+        assert np.array_equal(apr.intermediate(w), ref.intermediate(w)), w
+    assert apr.total == ref.total
