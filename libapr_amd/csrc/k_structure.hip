@@ -28,110 +28,162 @@ namespace aprh {
 
 namespace {
 
+constexpr int MAXL = 24;
 enum : uint8_t { EMPTY = 0, SEED = 1, BOUNDARY = 2, FILLER = 3, UPSEED = 4, ASC = 8, PROP = 15, ASCN = 16 };
 
 struct Dims {
     int64_t y, x, z;
 };
 
-/* level map of level l from level l+1 (max of the clamped 2x2x2 block) + seeds of level l */
-__device__ __forceinline__ void level_down_body(const uint8_t* __restrict__ fine, Dims fd, uint8_t* coarse, Dims cd, uint8_t* pct,
-                                                int level, int mode, int64_t G, int64_t t) {
-    const size_t n = (size_t)(cd.y * cd.x * cd.z);
-    for (size_t i = (size_t)t * blockDim.x + threadIdx.x; i < n; i += (size_t)G * blockDim.x) {
-        const int64_t y = (int64_t)(i % (size_t)cd.y);
-        const int64_t r = (int64_t)(i / (size_t)cd.y);
-        const int64_t x = r % cd.x, z = r / cd.x;
-        const int64_t y1 = min(2 * y + 1, fd.y - 1), x1 = min(2 * x + 1, fd.x - 1), z1 = min(2 * z + 1, fd.z - 1);
-        const int64_t y0 = 2 * y, x0 = 2 * x, z0 = 2 * z;
-        uint8_t m = fine[(z0 * fd.x + x0) * fd.y + y0];
-        m = max(m, fine[(z0 * fd.x + x0) * fd.y + y1]);
-        m = max(m, fine[(z0 * fd.x + x1) * fd.y + y0]);
-        m = max(m, fine[(z0 * fd.x + x1) * fd.y + y1]);
-        m = max(m, fine[(z1 * fd.x + x0) * fd.y + y0]);
-        m = max(m, fine[(z1 * fd.x + x0) * fd.y + y1]);
-        m = max(m, fine[(z1 * fd.x + x1) * fd.y + y0]);
-        m = max(m, fine[(z1 * fd.x + x1) * fd.y + y1]);
-        if (coarse) coarse[i] = m;
-        bool seed = (mode == 0) ? (m >= level) : (mode == 1) ? (m <= level) : (m == level);
-        pct[i] = seed ? SEED : EMPTY;
-    }
+/* ---- four cells in a 32-bit word, one byte each ---- */
+__device__ __forceinline__ uint32_t rep4(uint32_t b) { return b * 0x01010101u; }
+/* 0x80 in every byte of w that is 0 */
+__device__ __forceinline__ uint32_t zero4(uint32_t w) { return ~(((w & 0x7f7f7f7fu) + 0x7f7f7f7fu) | w | 0x7f7f7f7fu); }
+/* bit k of the result <- bit 7 of byte k */
+__device__ __forceinline__ uint32_t bits4(uint32_t flags) { return (((flags >> 7) & 0x01010101u) * 0x10204080u) >> 28; }
+/* per byte, values below 128: the larger of two */
+__device__ __forceinline__ uint32_t max4(uint32_t a, uint32_t b) {
+    const uint32_t ge = (((a | 0x80808080u) - b) >> 7) & 0x01010101u;
+    const uint32_t m = ge * 0xFFu;
+    return (a & m) | (b & ~m);
 }
-
-/* seeds of the top level straight from the level map (PullingScheme::fill, k == l_max) */
+/* SEED or EMPTY per byte from four levels (below 32): >= level (mode 0), <= level (1), == level (2) */
+__device__ __forceinline__ uint32_t seed4(uint32_t w, int level, int mode) {
+    const uint32_t ge = w + rep4(128u - (uint32_t)level), le = rep4(128u + (uint32_t)level) - w;
+    const uint32_t t = mode == 0 ? ge : mode == 1 ? le : ge & le;
+    return (t >> 7) & 0x01010101u;
+}
 __device__ __forceinline__ uint8_t seed_of(uint8_t m, int level, int mode) {
     const bool seed = (mode == 0) ? (m >= level) : (mode == 1) ? (m <= level) : (m == level);
     return seed ? SEED : EMPTY;
 }
-/* eight cells per thread (8-byte loads and stores) over the 8-aligned body, then the tail */
-__device__ __forceinline__ void seed_body(const uint8_t* __restrict__ lev, uint8_t* pct, size_t n, int level, int mode, int64_t G,
-                                          int64_t t) {
-    const bool wide = (((uintptr_t)lev | (uintptr_t)pct) & 7u) == 0;
-    const size_t nw = wide ? n / 8 : 0;
-    const size_t stride = (size_t)G * blockDim.x;
-    for (size_t i = (size_t)t * blockDim.x + threadIdx.x; i < nw; i += stride) {
-        const uint64_t w = ((const uint64_t*)lev)[i];
-        uint64_t o = 0;
+
+/* level map of level l from level l + 1 (max of the clamped 2x2x2 block) and the seeds of level l; with
+   fpct, also the seeds of level l + 1 itself (the top level: every fine cell is in exactly one block).
+   A lane takes eight coarse cells along y: four 16-byte row loads at any alignment.  At the top of
+   1024 x 1024 x 256 maps, seeds and first level took 0.28 ms a byte at a time in two launches. */
+struct DownArgs {
+    const uint8_t* fine;
+    Dims fd;
+    uint8_t* coarse;   /* nullptr: not wanted */
+    Dims cd;
+    uint8_t* pct;
+    int level, mode;
+    uint8_t* fpct;     /* seeds of the fine level (mode 0), or nullptr */
+    int64_t G;
+    FastDiv fg, fx;    /* division by the groups of a row, by cd.x */
+    int i32;
+};
+__device__ __forceinline__ void level_down_body(const DownArgs& a, int64_t G, int64_t t) {
+    const Dims fd = a.fd, cd = a.cd;
+    const int64_t ng = (cd.y + 7) >> 3, total = ng * cd.x * cd.z;
+    for (int64_t i = t * blockDim.x + threadIdx.x; i < total; i += G * blockDim.x) {
+        int64_t g, x, z;
+        if (a.i32) {
+            const uint32_t r = a.fg.div((uint32_t)i), zz = a.fx.div(r);
+            g = (uint32_t)i - r * (uint32_t)ng;
+            x = r - zz * (uint32_t)cd.x;
+            z = zz;
+        } else {
+            const int64_t r = i / ng;
+            g = i - r * ng;
+            z = r / cd.x;
+            x = r - z * cd.x;
+        }
+        const int64_t y0 = 16 * g, c0 = 8 * g;
+        const int64_t x1 = min(2 * x + 1, fd.x - 1), z1 = min(2 * z + 1, fd.z - 1);
+        const int64_t rows[4] = {(2 * z * fd.x + 2 * x) * fd.y, (2 * z * fd.x + x1) * fd.y, (z1 * fd.x + 2 * x) * fd.y, (z1 * fd.x + x1) * fd.y};
+        const int64_t o = (z * cd.x + x) * cd.y + c0;
+        if (y0 + 16 <= fd.y) {
+            uint32_t w[4][4];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) o |= (uint64_t)seed_of((uint8_t)(w >> (8 * j)), level, mode) << (8 * j);
-        ((uint64_t*)pct)[i] = o;
+            for (int q = 0; q < 4; ++q) __builtin_memcpy(w[q], a.fine + rows[q] + y0, 16);
+            if (a.fpct) {
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    uint32_t f[4];
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) f[k] = seed4(w[q][k], a.level + 1, 0);
+                    __builtin_memcpy(a.fpct + rows[q] + y0, f, 16);   /* rows that coincide get the same bytes twice */
+                }
+            }
+            uint32_t m[2];
+#pragma unroll
+            for (int k = 0; k < 2; ++k) {
+                uint32_t h[2];
+#pragma unroll
+                for (int u = 0; u < 2; ++u) {
+                    const int q = 2 * k + u;
+                    const uint32_t v = max4(max4(w[0][q], w[1][q]), max4(w[2][q], w[3][q]));
+                    const uint32_t p = max4(v, v >> 8);
+                    h[u] = (p & 0xFFu) | ((p >> 8) & 0xFF00u);
+                }
+                m[k] = h[0] | (h[1] << 16);
+            }
+            const uint32_t sd[2] = {seed4(m[0], a.level, a.mode), seed4(m[1], a.level, a.mode)};
+            if (a.coarse) __builtin_memcpy(a.coarse + o, m, 8);
+            __builtin_memcpy(a.pct + o, sd, 8);
+        } else {
+            for (int j = 0; j < 8 && c0 + j < cd.y; ++j) {
+                const int64_t ya = y0 + 2 * j, yb = min(ya + 1, fd.y - 1);
+                uint8_t m = 0;
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const uint8_t va = a.fine[rows[q] + ya], vb = a.fine[rows[q] + yb];
+                    m = max(m, max(va, vb));
+                    if (a.fpct) {
+                        a.fpct[rows[q] + ya] = seed_of(va, a.level + 1, 0);
+                        a.fpct[rows[q] + yb] = seed_of(vb, a.level + 1, 0);
+                    }
+                }
+                if (a.coarse) a.coarse[o + j] = m;
+                a.pct[o + j] = seed_of(m, a.level, a.mode);
+            }
+        }
     }
-    for (size_t i = nw * 8 + (size_t)t * blockDim.x + threadIdx.x; i < n; i += stride) pct[i] = seed_of(lev[i], level, mode);
 }
 
 /* one pulling-scheme level (PullingScheme.hpp:111-132 loop body): set_ascendant_neighbours
    and fill_neighbours on this level, set_filler on the finer one, fill_parent on the coarser
-   one.  One lane per 8 consecutive y cells: the 3x3x3 neighbourhood
-   predicates are formed as bit masks over the 9 neighbouring rows (10 bits: y0-1 .. y0+8),
-   dilated along y by shifts, so a lane loads 9 row words instead of 27 bytes per cell. */
-__device__ __forceinline__ void load_row8(const uint8_t* row, int yn, int y0, uint8_t b[10]) {
-    b[0] = (y0 > 0) ? row[y0 - 1] : (uint8_t)0;
-    if (y0 + 8 <= yn) {   /* one 8-byte load at any alignment */
-        uint64_t w;
-        __builtin_memcpy(&w, row + y0, 8);
-#pragma unroll
-        for (int j = 0; j < 8; ++j) b[1 + j] = (uint8_t)(w >> (8 * j));
-    } else {
-#pragma unroll
-        for (int j = 0; j < 8; ++j) b[1 + j] = (y0 + j < yn) ? row[y0 + j] : (uint8_t)0;
-    }
-    b[9] = (y0 + 8 < yn) ? row[y0 + 8] : (uint8_t)0;
-}
-
-/* bit masks (bit k <-> y0 - 1 + k) of ASCENDANT and of SEED-or-PROPOGATE cells in a row */
-__device__ __forceinline__ void row_masks(const uint8_t b[10], uint32_t& am, uint32_t& sm) {
-    am = 0;
-    sm = 0;
-#pragma unroll
-    for (int k = 0; k < 10; ++k) {
-        am |= (uint32_t)(b[k] == ASC) << k;
-        sm |= (uint32_t)((b[k] == SEED) | (b[k] == PROP)) << k;
-    }
-}
-
-/* One lane owns 8 consecutive y cells of one (x) column over a run of ZC planes and marches
-   along z, keeping the ASCENDANT / SEED-or-PROPOGATE masks of the planes z-1, z, z+1 (each the
-   OR over rows x-1, x, x+1): every plane's three rows are loaded once instead of three times.
-   A cell's state is written only by its owner lane, so the cached bytes of the own row are
-   current. */
-constexpr int PULL_ZC = 4;   /* planes per lane of a single volume; a batch plan also times 8 */
-template <int ZC>
-__device__ __forceinline__ void pull_level8_body(uint8_t* P, Dims d, uint8_t* Pc, Dims dc, uint8_t* Pp, Dims dp, int is_top,
-                                                 int has_parent, int64_t G, int64_t t) {
-    const int yn = (int)d.y, xn = (int)d.x, zn = (int)d.z;
+   one.  One lane per 8 consecutive y cells: the 3x3x3 neighbourhood predicates are formed as bit masks
+   over the 9 neighbouring rows (10 bits: y0-1 .. y0+8), dilated along y by shifts.
+   A lane marches over a run of zc planes, keeping the ASCENDANT / SEED-or-PROPOGATE masks of the planes
+   z-1, z, z+1 (each the OR over rows x-1, x, x+1): every plane's three rows are loaded once instead of
+   three times.  A cell's state is written only by its owner lane, so the cached words of the own row are
+   current, and the 16 x 2 x 2 children of a lane's cells belong to it alone, so set_filler rewrites them
+   as whole words: four row loads at once, where one load and store after the other for every child made a
+   chain of up to 64 (28 us for a level of a few thousand cells, 10 us now).
+   atomics: fill_parent ORs whole parent words; else it stores the bytes it turns to ASCENDANT (inside one
+   block, where other waves read them after a barrier, and for parent rows that straddle words). */
+struct PullArgs {
+    uint8_t* P;
+    Dims d;
+    uint8_t* Pc;
+    Dims dc;
+    uint8_t* Pp;
+    Dims dp;
+    int is_top, has_parent;
+    int zc, atomics;
+    int64_t G;
+};
+__device__ __forceinline__ void pull_level8_body(const PullArgs& a, int64_t G, int64_t t) {
+    uint8_t* const P = a.P;
+    const Dims dc = a.dc, dp = a.dp;
+    const bool is_top = a.is_top, has_parent = a.has_parent;
+    const int yn = (int)a.d.y, xn = (int)a.d.x, zn = (int)a.d.z, ZC = a.zc;
     const int nwr = (yn + 7) >> 3;
     const int nzc = (zn + ZC - 1) / ZC;
     const int64_t total = (int64_t)nwr * xn * nzc;
     /* parent rows whose words never straddle two rows */
-    const bool par_words = has_parent && (dp.y & 3) == 0 && ((uintptr_t)Pp & 3) == 0;
+    const bool par_words = a.atomics && (dp.y & 3) == 0 && ((uintptr_t)a.Pp & 3) == 0;
     for (int64_t i = t * blockDim.x + threadIdx.x; i < total; i += G * blockDim.x) {
         const int w = (int)(i % nwr);
         const int64_t r = i / nwr;
         const int x = (int)(r % xn), zc = (int)(r / xn);
         const int y0 = w * 8;
         const int z_begin = zc * ZC, z_end = min(zn, z_begin + ZC);
-        /* masks of plane zz (0 outside the volume); own row bytes of that plane in own[] */
-        auto plane = [&](int zz, uint32_t& am, uint32_t& sm, uint8_t own[10]) {
+        /* masks of plane zz (0 outside the volume; bit k <-> y0 - 1 + k); own row's words in own[] */
+        auto plane = [&](int zz, uint32_t& am, uint32_t& sm, uint32_t own[2]) {
             am = 0;
             sm = 0;
             if (zz < 0 || zz >= zn) return;
@@ -139,19 +191,40 @@ __device__ __forceinline__ void pull_level8_body(uint8_t* P, Dims d, uint8_t* Pc
             for (int dx = -1; dx <= 1; ++dx) {
                 const int xx = x + dx;
                 if (xx < 0 || xx >= xn) continue;
-                uint8_t b[10];
-                load_row8(P + ((int64_t)zz * xn + xx) * yn, yn, y0, b);
-                uint32_t a1, s1;
-                row_masks(b, a1, s1);
-                am |= a1;
-                sm |= s1;
-                if (dx == 0)
+                const uint8_t* row = P + ((int64_t)zz * xn + xx) * yn;
+                uint32_t c[2], lf, rt;   /* the eight cells and the ones beside them */
+                if (y0 >= 4 && y0 + 12 <= yn) {   /* one 16-byte load at any alignment */
+                    uint32_t v[4];
+                    __builtin_memcpy(v, row + y0 - 4, 16);
+                    lf = v[0] >> 24;
+                    c[0] = v[1];
+                    c[1] = v[2];
+                    rt = v[3] & 0xFFu;
+                } else {
+                    lf = y0 > 0 ? row[y0 - 1] : 0u;
+                    rt = y0 + 8 < yn ? row[y0 + 8] : 0u;
+                    if (y0 + 8 <= yn) {
+                        __builtin_memcpy(c, row + y0, 8);
+                    } else {
+                        c[0] = c[1] = 0;
 #pragma unroll
-                    for (int k = 0; k < 10; ++k) own[k] = b[k];
+                        for (int j = 0; j < 8; ++j)
+                            if (y0 + j < yn) c[j >> 2] |= (uint32_t)row[y0 + j] << (8 * (j & 3));
+                    }
+                }
+                am |= (bits4(zero4(c[0] ^ rep4(ASC))) << 1) | (bits4(zero4(c[1] ^ rep4(ASC))) << 5) | (lf == ASC ? 1u : 0u) |
+                      (rt == ASC ? 0x200u : 0u);
+                sm |= (bits4(zero4(c[0] ^ rep4(SEED)) | zero4(c[0] ^ rep4(PROP))) << 1) |
+                      (bits4(zero4(c[1] ^ rep4(SEED)) | zero4(c[1] ^ rep4(PROP))) << 5) | (lf == SEED || lf == PROP ? 1u : 0u) |
+                      (rt == SEED || rt == PROP ? 0x200u : 0u);
+                if (dx == 0) {
+                    own[0] = c[0];
+                    own[1] = c[1];
+                }
             }
         };
         uint32_t pa0, ps0, pa1, ps1, pa2, ps2;
-        uint8_t cur[10], nxt[10];
+        uint32_t cur[2] = {0, 0}, nxt[2] = {0, 0};
         plane(z_begin - 1, pa0, ps0, nxt);
         plane(z_begin, pa1, ps1, cur);
         for (int z = z_begin; z < z_end; ++z) {
@@ -159,113 +232,167 @@ __device__ __forceinline__ void pull_level8_body(uint8_t* P, Dims d, uint8_t* Pc
             const uint32_t am = pa0 | pa1 | pa2, sm = ps0 | ps1 | ps2;
             const uint32_t ad = am | (am << 1) | (am >> 1), sd = sm | (sm << 1) | (sm >> 1);
             uint8_t* row = P + ((int64_t)z * xn + x) * yn;
-            uint8_t nb[8];
-            bool changed = false;
+            uint32_t nb[2] = {0, 0};
+            uint32_t fill = 0, up = 0;   /* cells whose children are filled; cells that raise their parent */
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
-                const uint8_t old = cur[1 + j];
+                const uint32_t old = (cur[j >> 2] >> (8 * (j & 3))) & 0xFFu;
                 const bool any_asc = (ad >> (j + 1)) & 1u, any_sp = (sd >> (j + 1)) & 1u;
-                uint8_t nw = old;
+                uint32_t nw = old;
                 if (!is_top) {
                     if (old == EMPTY) nw = any_asc ? ASCN : (any_sp ? BOUNDARY : EMPTY);
                     else if (old == SEED) nw = any_asc ? PROP : SEED;
                 } else if (old == EMPTY && any_sp) {
                     nw = BOUNDARY;
                 }
-                nb[j] = nw;
-                changed |= (nw != old) && (y0 + j < yn);
-            }
-            if (changed) {
-                if (y0 + 8 <= yn) {
-                    uint64_t v = 0;
-#pragma unroll
-                    for (int j = 0; j < 8; ++j) v |= (uint64_t)nb[j] << (8 * j);
-                    __builtin_memcpy(row + y0, &v, 8);
-                } else {
-#pragma unroll
-                    for (int j = 0; j < 8; ++j)
-                        if (y0 + j < yn && nb[j] != cur[1 + j]) row[y0 + j] = nb[j];
+                nb[j >> 2] |= nw << (8 * (j & 3));
+                if (y0 + j < yn) {
+                    fill |= (uint32_t)(!is_top && (nw == ASCN || nw == PROP)) << j;
+                    up |= (uint32_t)(nw == SEED || nw == PROP || nw == ASC) << j;
                 }
             }
-            /* fill_parent for the lane's 4 parent cells with one word: the parent level holds only
-               EMPTY, SEED and ASCENDANT now (its seeds, and ASCENDANT from this pass), so OR-ing
-               ASCENDANT's bits into the non-SEED bytes wanted gives each the reference's value, in
-               any order between lanes that share the word */
-            const bool word_parent = has_parent && par_words;
-            if (word_parent) {
-                uint32_t want = 0;
+            if (y0 + 8 <= yn) {
+                if (nb[0] != cur[0] || nb[1] != cur[1]) __builtin_memcpy(row + y0, nb, 8);
+            } else {
 #pragma unroll
                 for (int j = 0; j < 8; ++j) {
-                    const uint8_t nw = nb[j];
-                    if (y0 + j < yn && (nw == SEED || nw == PROP || nw == ASC)) want |= 0xFFu << (8 * (j >> 1));
-                }
-                if (want) {
-                    uint32_t* pw = (uint32_t*)&Pp[((int64_t)(z / 2) * dp.x + (x / 2)) * dp.y + (y0 / 2)];
-                    const uint32_t cur4 = *pw;
-                    uint32_t mask = 0;
-#pragma unroll
-                    for (int q = 0; q < 4; ++q)
-                        if (((want >> (8 * q)) & 0xFFu) && ((cur4 >> (8 * q)) & 0xFFu) != SEED) mask |= (uint32_t)ASC << (8 * q);
-                    if (mask) atomicOr(pw, mask);
+                    const uint8_t v = (uint8_t)(nb[j >> 2] >> (8 * (j & 3)));
+                    if (y0 + j < yn && v != (uint8_t)(cur[j >> 2] >> (8 * (j & 3)))) row[y0 + j] = v;
                 }
             }
+            /* fill_parent.  The parent level holds only EMPTY, SEED and ASCENDANT now (its seeds, and
+               ASCENDANT from this pass), so every non-SEED byte wanted becomes ASCENDANT, in any order
+               between lanes that share a parent cell or word */
+            if (has_parent && up) {
+                uint8_t* pp = a.Pp + ((int64_t)(z / 2) * dp.x + (x / 2)) * dp.y + (y0 / 2);
+                const uint32_t want = (up & 3u ? 0xFFu : 0u) | (up & 0xCu ? 0xFF00u : 0u) | (up & 0x30u ? 0xFF0000u : 0u) | (up & 0xC0u ? 0xFF000000u : 0u);
+                uint32_t cur4 = 0;
+                if (y0 / 2 + 4 <= dp.y) {
+                    __builtin_memcpy(&cur4, pp, 4);
+                } else {
 #pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const int y = y0 + j;
-                if (y >= yn) break;
-                const uint8_t nw = nb[j];
-                /* set_filler: empty children of ASCENDANTNEIGHBOUR / PROPOGATE become FILLER */
-                if (!is_top && (nw == ASCN || nw == PROP)) {
-                    const int cz = (z == zn - 1 && (dc.z & 1)) ? 1 : 2;
-                    const int cx = (x == xn - 1 && (dc.x & 1)) ? 1 : 2;
-                    const int cy = (y == yn - 1 && (dc.y & 1)) ? 1 : 2;
-                    for (int a = 0; a < cz; ++a)
-                        for (int bb = 0; bb < cx; ++bb)
-                            for (int c = 0; c < cy; ++c) {
-                                uint8_t* ch = &Pc[((int64_t)(2 * z + a) * dc.x + (2 * x + bb)) * dc.y + (2 * y + c)];
-                                if (*ch == EMPTY) *ch = FILLER;
-                            }
+                    for (int q = 0; q < 3; ++q)
+                        if (y0 / 2 + q < dp.y) cur4 |= (uint32_t)pp[q] << (8 * q);
                 }
-                /* fill_parent */
-                if (!word_parent && has_parent && (nw == SEED || nw == PROP || nw == ASC)) {
-                    uint8_t* pp = &Pp[((int64_t)(z / 2) * dp.x + (x / 2)) * dp.y + (y / 2)];
-                    if (*pp != SEED) *pp = ASC;
+                const uint32_t isseed = (zero4(cur4 ^ rep4(SEED)) >> 7) * 0xFFu, isasc = (zero4(cur4 ^ rep4(ASC)) >> 7) * 0xFFu;
+                const uint32_t turn = want & ~isseed & ~isasc;
+                if (turn) {
+                    if (par_words) {
+                        atomicOr((uint32_t*)pp, turn & rep4(ASC));
+                    } else {
+#pragma unroll
+                        for (int q = 0; q < 4; ++q)
+                            if ((turn >> (8 * q)) & 0xFFu) pp[q] = ASC;
+                    }
+                }
+            }
+            /* set_filler: empty children of ASCENDANTNEIGHBOUR / PROPOGATE become FILLER */
+            if (fill) {
+                const int cz = (z == zn - 1 && (dc.z & 1)) ? 1 : 2, cx = (x == xn - 1 && (dc.x & 1)) ? 1 : 2;
+                uint8_t* c00 = a.Pc + ((int64_t)(2 * z) * dc.x + 2 * x) * dc.y + 2 * y0;
+                uint8_t* crow[4] = {c00, c00 + (cx == 2 ? dc.y : 0), c00 + (cz == 2 ? dc.x * dc.y : 0),
+                                    c00 + (cx == 2 ? dc.y : 0) + (cz == 2 ? dc.x * dc.y : 0)};
+                if (2 * y0 + 16 <= dc.y) {
+                    uint32_t m[4];   /* FILLER in the two children of every such cell */
+#pragma unroll
+                    for (int q = 0; q < 4; ++q)
+                        m[q] = (((fill >> (2 * q)) & 1u) ? 0x0000FFFFu : 0u) | (((fill >> (2 * q + 1)) & 1u) ? 0xFFFF0000u : 0u);
+                    uint32_t v[4][4];
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) __builtin_memcpy(v[q], crow[q], 16);
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        uint32_t any = 0;
+#pragma unroll
+                        for (int k = 0; k < 4; ++k) {
+                            const uint32_t f = (zero4(v[q][k]) >> 7) * (uint32_t)FILLER & m[k];
+                            v[q][k] |= f;
+                            any |= f;
+                        }
+                        if (any) __builtin_memcpy(crow[q], v[q], 16);   /* rows that coincide get the same bytes twice */
+                    }
+                } else {
+                    for (int j = 0; j < 8; ++j) {
+                        if (!((fill >> j) & 1u)) continue;
+                        const int cy = (y0 + j == yn - 1 && (dc.y & 1)) ? 1 : 2;
+                        for (int q = 0; q < 4; ++q)
+                            for (int c = 0; c < cy; ++c)
+                                if (crow[q][2 * j + c] == EMPTY) crow[q][2 * j + c] = FILLER;
+                    }
                 }
             }
             pa0 = pa1;
             ps0 = ps1;
             pa1 = pa2;
             ps1 = ps2;
-#pragma unroll
-            for (int k = 0; k < 10; ++k) cur[k] = nxt[k];
+            cur[0] = nxt[0];
+            cur[1] = nxt[1];
         }
     }
 }
 
-/* equivalence optimisation step for one level (LinearAccess.hpp:265-294) */
-__device__ __forceinline__ void upseed_body(uint8_t* P, Dims d, const uint8_t* __restrict__ Pp, Dims dp, int min_type, int64_t G,
-                                            int64_t t, const FastDiv& fy, const FastDiv& fx, bool i32) {
-    const size_t n = (size_t)(d.y * d.x * d.z);
-    for (size_t i = (size_t)t * blockDim.x + threadIdx.x; i < n; i += (size_t)G * blockDim.x) {
-        int64_t y, x, z;
-        if (i32) {
-            const uint32_t r = fy.div((uint32_t)i), zz = fx.div(r);
-            y = (int64_t)((uint32_t)i - r * (uint32_t)d.y);
-            x = (int64_t)(r - zz * (uint32_t)d.x);
+/* equivalence optimisation step for one level (LinearAccess.hpp:265-294): a lane takes eight cells along
+   y, i.e. four parent cells, and writes only under parents of type 1 .. min_type.  (A cell per lane with
+   its own division: 0.37 ms over the levels of a 2048 x 2048 x 512 volume.) */
+struct UpseedArgs {
+    uint8_t* P;
+    Dims d;
+    const uint8_t* Pp;
+    Dims dp;
+    int min_type;
+    int64_t G;
+    FastDiv fg, fx;   /* division by the groups of a row, by d.x */
+    int i32;
+};
+__device__ __forceinline__ void upseed_body(const UpseedArgs& a, int64_t G, int64_t t) {
+    const Dims d = a.d, dp = a.dp;
+    const int64_t ng = (d.y + 7) >> 3, total = ng * d.x * d.z;
+    for (int64_t i = t * blockDim.x + threadIdx.x; i < total; i += G * blockDim.x) {
+        int64_t g, x, z;
+        if (a.i32) {
+            const uint32_t r = a.fg.div((uint32_t)i), zz = a.fx.div(r);
+            g = (uint32_t)i - r * (uint32_t)ng;
+            x = r - zz * (uint32_t)d.x;
             z = zz;
         } else {
-            y = (int64_t)(i % (size_t)d.y);
-            const int64_t r = (int64_t)(i / (size_t)d.y);
-            x = r % d.x;
+            const int64_t r = i / ng;
+            g = i - r * ng;
             z = r / d.x;
+            x = r - z * d.x;
         }
-        const uint8_t s = Pp[((z / 2) * dp.x + (x / 2)) * dp.y + (y / 2)];
-        if (s > 0 && s <= min_type) P[i] = UPSEED;
+        const uint8_t* pp = a.Pp + ((z / 2) * dp.x + (x / 2)) * dp.y + 4 * g;
+        uint32_t s = 0;
+        if (4 * g + 4 <= dp.y) {
+            __builtin_memcpy(&s, pp, 4);
+        } else {
+#pragma unroll
+            for (int q = 0; q < 3; ++q)
+                if (4 * g + q < dp.y) s |= (uint32_t)pp[q] << (8 * q);
+        }
+        uint32_t on = 0;   /* parents of type 1 .. min_type */
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const uint32_t v = (s >> (8 * q)) & 0xFFu;
+            on |= (uint32_t)(v > 0 && v <= (uint32_t)a.min_type) << q;
+        }
+        if (!on) continue;
+        const int64_t y0 = 8 * g;
+        uint8_t* p = a.P + (z * d.x + x) * d.y + y0;
+        if (on == 0xFu && y0 + 8 <= d.y) {
+            const uint32_t u[2] = {rep4(UPSEED), rep4(UPSEED)};
+            __builtin_memcpy(p, u, 8);
+        } else {
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                if ((on >> q) & 1u) {
+                    p[2 * q] = UPSEED;
+                    if (y0 + 2 * q + 1 < d.y) p[2 * q + 1] = UPSEED;
+                }
+        }
     }
 }
 
 /* row table of the APR levels l_min..l_max and the particle-cell maps that define them */
-constexpr int MAXL = 24;
 struct RowTable {
     int n_levels;                 /* APR levels l_min..l_max           */
     int l_min, l_max;
@@ -528,66 +655,94 @@ __device__ __forceinline__ void scan_add_body(uint64_t* out, const uint64_t* __r
 }
 
 /* tile bodies of the pulling scheme and the structure */
-struct Seed {
-    struct Args {
-        const uint8_t* lev;
-        uint8_t* pct;
-        size_t n;
-        int level, mode;
-        int64_t G;
-    };
-    static constexpr int THREADS = 256;
-    static const char* name() { return "pulling_seed"; }
-    static __device__ __forceinline__ void run(const Args& a, int64_t t) { seed_body(a.lev, a.pct, a.n, a.level, a.mode, a.G, t); }
-};
 struct LevelDown {
-    struct Args {
-        const uint8_t* fine;
-        Dims fd;
-        uint8_t* coarse;
-        Dims cd;
-        uint8_t* pct;
-        int level, mode;
-        int64_t G;
-    };
+    using Args = DownArgs;
     static constexpr int THREADS = 256;
     static const char* name() { return "pulling_level_down"; }
-    static __device__ __forceinline__ void run(const Args& a, int64_t t) { level_down_body(a.fine, a.fd, a.coarse, a.cd, a.pct, a.level, a.mode, a.G, t); }
+    static __device__ __forceinline__ void run(const Args& a, int64_t t) { level_down_body(a, a.G, t); }
 };
-struct PullLevelArgs {
-    uint8_t* P;
-    Dims d;
-    uint8_t* Pc;
-    Dims dc;
-    uint8_t* Pp;
-    Dims dp;
-    int is_top, has_parent;
-    int64_t G;
-};
-template <int ZC = PULL_ZC>
+/* planes per lane: a batch plan times the alternatives against each other */
+template <int ALT>
 struct PullLevel {
-    using Args = PullLevelArgs;
+    using Args = PullArgs;
     static constexpr int THREADS = 256;
     static const char* name() { return "pulling_level"; }
-    static __device__ __forceinline__ void run(const Args& a, int64_t t) {
-        pull_level8_body<ZC>(a.P, a.d, a.Pc, a.dc, a.Pp, a.dp, a.is_top, a.has_parent, a.G, t);
-    }
+    static __device__ __forceinline__ void run(const Args& a, int64_t t) { pull_level8_body(a, a.G, t); }
 };
 struct Upseed {
-    struct Args {
-        uint8_t* P;
-        Dims d;
-        const uint8_t* Pp;
-        Dims dp;
-        int min_type;
-        int64_t G;
-        FastDiv fy, fx;
-        int i32;
-    };
+    using Args = UpseedArgs;
     static constexpr int THREADS = 256;
     static const char* name() { return "upseed"; }
-    static __device__ __forceinline__ void run(const Args& a, int64_t t) {
-        upseed_body(a.P, a.d, a.Pp, a.dp, a.min_type, a.G, t, a.fy, a.fx, a.i32);
+    static __device__ __forceinline__ void run(const Args& a, int64_t t) { upseed_body(a, a.G, t); }
+};
+
+/* The coarsest levels (at most SMALL_CELLS cells each) in one block: a launch of their own costs each
+   of them more than its work.  The same bodies over one block, a barrier between levels (all waves of a
+   block run on one CU and share its vector L1, so a barrier makes their writes visible to each other). */
+constexpr int64_t SMALL_CELLS = 16384;
+constexpr int SMALL_THREADS = 1024;
+struct SmallLevels {
+    uint8_t* P;                /* particle-cell tree                                   */
+    uint8_t* LV;               /* level maps below the top (LevelDown)                 */
+    const uint8_t* level_top;  /* map of the top level                                 */
+    int lmin, s, top;          /* levels s .. lmin here; s <= top - 1                  */
+    int min_type;
+    int64_t off[MAXL + 1];
+    Dims d[MAXL + 1];
+};
+struct SmallDown {
+    using Args = SmallLevels;
+    static constexpr int THREADS = SMALL_THREADS;
+    static const char* name() { return "pulling_small_down"; }
+    static __device__ __forceinline__ void run(const Args& a, int64_t) {
+        for (int l = a.s; l >= a.lmin; --l) {
+            const uint8_t* fine = l + 1 == a.top ? a.level_top : a.LV + a.off[l + 1];
+            DownArgs d;
+            d.fine = fine;
+            d.fd = a.d[l + 1];
+            d.coarse = a.LV + a.off[l];
+            d.cd = a.d[l];
+            d.pct = a.P + a.off[l];
+            d.level = l;
+            d.mode = l == a.lmin ? 1 : 2;
+            d.fpct = l + 1 == a.top ? a.P + a.off[a.top] : nullptr;
+            d.i32 = 0;
+            level_down_body(d, 1, 0);
+            __syncthreads();
+        }
+    }
+};
+struct SmallPull {
+    using Args = SmallLevels;
+    static constexpr int THREADS = SMALL_THREADS;
+    static const char* name() { return "pulling_small"; }
+    static __device__ __forceinline__ void run(const Args& a, int64_t) {
+        for (int l = a.s; l >= a.lmin; --l) {
+            PullArgs p;
+            p.P = a.P + a.off[l];
+            p.d = a.d[l];
+            p.Pc = a.P + a.off[l + 1];
+            p.dc = a.d[l + 1];
+            p.has_parent = l > a.lmin;
+            p.Pp = p.has_parent ? a.P + a.off[l - 1] : nullptr;
+            p.dp = p.has_parent ? a.d[l - 1] : Dims{1, 1, 1};
+            p.is_top = 0;
+            p.zc = 1;
+            p.atomics = 0;
+            pull_level8_body(p, 1, 0);
+            __syncthreads();
+        }
+        for (int l = a.lmin + 1; l <= a.s; ++l) {
+            UpseedArgs u;
+            u.P = a.P + a.off[l];
+            u.d = a.d[l];
+            u.Pp = a.P + a.off[l - 1];
+            u.dp = a.d[l - 1];
+            u.min_type = a.min_type;
+            u.i32 = 0;
+            upseed_body(u, 1, 0);
+            __syncthreads();
+        }
     }
 };
 struct RowCount {
@@ -819,26 +974,56 @@ std::vector<int64_t> pct_layout(const aprh_apr& a) {
     return off;
 }
 
-/* PullingScheme::fill of every level (LocalParticleCellSet.hpp:58-91): seeds of the top level
-   straight from the level map, then the 2x2x2 max pyramid of the map with the seeds of each
-   coarser level.  zn: z extent per level (the APR's, or a patch's) */
+namespace {
+/* the largest level below the top that goes with the small ones (lmin - 1: none) */
+int small_level(const aprh_apr& a, const std::vector<int64_t>& zn) {
+    int s = a.l_min - 1;
+    while (s + 1 <= a.l_max - 2 && a.y_num[s + 1] * a.x_num[s + 1] * zn[s + 1] <= SMALL_CELLS) ++s;
+    return s;
+}
+SmallLevels small_levels(const aprh_apr& a, int s, const std::vector<int64_t>& zn, const std::vector<int64_t>& off, uint8_t* P) {
+    SmallLevels v;
+    std::memset(&v, 0, sizeof(v));
+    v.P = P;
+    v.lmin = a.l_min;
+    v.s = s;
+    v.top = a.l_max - 1;
+    if (v.top > MAXL) throw Error(APRH_ERR_UNSUPPORTED, "too many levels");
+    for (int l = a.l_min; l <= v.top; ++l) {
+        v.off[l] = off[l];
+        v.d[l] = Dims{a.y_num[l], a.x_num[l], zn[l]};
+    }
+    return v;
+}
+}  // namespace
+
+/* PullingScheme::fill of every level (LocalParticleCellSet.hpp:58-91): the 2x2x2 max pyramid of the level
+   map with the seeds of each level, the top level's straight from the map.  zn: z extent per level (the
+   APR's, or a patch's).  Levels below the top exist: l_max > 2 */
 void seed_levels(aprh_context* ctx, const aprh_apr& a, const uint8_t* level_top, const std::vector<int64_t>& zn, uint8_t* P,
                  const std::vector<int64_t>& off) {
     const int top = a.l_max - 1, lmin = a.l_min;
     auto D = [&](int l) { return Dims{a.y_num[l], a.x_num[l], zn[l]}; };
-    auto mode_of = [&](int l) { return l == top ? 0 : (l == lmin ? 1 : 2); };
     Buf lev(ctx->pool, (size_t)std::max<int64_t>(off[top + 1], 8));
     uint8_t* LV = lev.as<uint8_t>();
-    {
-        const size_t n = (size_t)(a.y_num[top] * a.x_num[top] * zn[top]);
-        const int64_t G = stride_tiles((int64_t)n, 256 * 4);
-        launch_tiles<Seed>(ctx, {level_top, P + off[top], n, top, mode_of(top), G}, G);
-    }
+    const int s = small_level(a, zn);
     const uint8_t* fine = level_top;
-    for (int l = top - 1; l >= lmin; --l) {
-        const int64_t G = stride_tiles(off[l + 1] - off[l], 256 * 4);
-        launch_tiles<LevelDown>(ctx, {fine, D(l + 1), LV + off[l], D(l), P + off[l], l, mode_of(l), G}, G);
+    for (int l = top - 1; l > s; --l) {
+        const int64_t ng = cdiv(a.y_num[l], 8), n = ng * a.x_num[l] * zn[l];
+        DownArgs d{fine, D(l + 1), LV + off[l], D(l), P + off[l], l, l == lmin ? 1 : 2, l + 1 == top ? P + off[top] : nullptr,
+                   stride_tiles(n, 256), FastDiv(), FastDiv(), fits32(n) ? 1 : 0};
+        if (d.i32) {
+            d.fg = FastDiv((uint64_t)ng);
+            d.fx = FastDiv((uint64_t)a.x_num[l]);
+        }
+        launch_tiles<LevelDown>(ctx, d, d.G);
         fine = LV + off[l];
+    }
+    if (s >= lmin) {
+        SmallLevels v = small_levels(a, s, zn, off, P);
+        v.LV = LV;
+        v.level_top = level_top;
+        launch_tiles<SmallDown>(ctx, v, 1);
     }
 }
 
@@ -1011,35 +1196,47 @@ void build_structure_seeded(aprh_context* ctx, aprh_apr& a, const uint8_t* level
         P = pct.as<uint8_t>();
         seed_levels(ctx, a, level_top, a.z_num, P, off);
     }
-    /* pulling scheme, top to bottom */
-    for (int l = top; l >= lmin; --l) {
+    const int min_type = par.neighborhood_optimization ? 1 : 2;
+    const int small = small_level(a, a.z_num);
+    /* pulling scheme, top to bottom; the coarsest levels' equivalence optimisation with their own */
+    for (int l = top; l > std::max(small, lmin - 1); --l) {
         const bool has_parent = (l - 1) >= lmin;
         const bool is_top = (l == top);
         uint8_t* Pc = is_top ? nullptr : P + off[l + 1];
         uint8_t* Pp = has_parent ? P + off[l - 1] : nullptr;
         auto pargs = [&](int zc) {
-            const int64_t G = stride_tiles(cdiv(a.y_num[l], 8) * a.x_num[l] * cdiv(a.z_num[l], zc), 256 * 2);
-            return PullLevelArgs{P + off[l], D(l), Pc, is_top ? Dims{1, 1, 1} : D(l + 1), Pp, has_parent ? D(l - 1) : Dims{1, 1, 1},
-                                 is_top ? 1 : 0, has_parent ? 1 : 0, G};
+            const int64_t G = stride_tiles(cdiv(a.y_num[l], 8) * a.x_num[l] * cdiv(a.z_num[l], zc), 256);
+            return PullArgs{P + off[l], D(l), Pc, is_top ? Dims{1, 1, 1} : D(l + 1), Pp, has_parent ? D(l - 1) : Dims{1, 1, 1},
+                            is_top ? 1 : 0, has_parent ? 1 : 0, zc, 1, G};
         };
-        const PullLevelArgs p4 = pargs(PULL_ZC);
+        /* runs of 4 planes load each row half as often as single planes; levels of fewer than about 256
+           thousand lanes that way take shorter runs, since a lane walks its planes one after another */
+        const int64_t lanes1 = cdiv(a.y_num[l], 8) * a.x_num[l] * a.z_num[l];
+        const int zc = lanes1 >= 4 * 262144 ? 4 : lanes1 >= 2 * 262144 ? 2 : 1;
+        const PullArgs p = pargs(zc);
         if (ctx->recorder) {
-            const PullLevelArgs p8 = pargs(8);
-            launch_tiles_alts(ctx, {tile_alt<PullLevel<PULL_ZC>>(p4, p4.G, "4 planes per lane"), tile_alt<PullLevel<8>>(p8, p8.G, "8 planes per lane")},
+            const PullArgs p4 = pargs(4);
+            launch_tiles_alts(ctx, {tile_alt<PullLevel<0>>(p, p.G, "planes per lane by size"), tile_alt<PullLevel<4>>(p4, p4.G, "4 planes per lane")},
                               0);
         } else {
-            launch_tiles<PullLevel<>>(ctx, p4, p4.G);
+            launch_tiles<PullLevel<0>>(ctx, p, p.G);
         }
     }
-    const int min_type = par.neighborhood_optimization ? 1 : 2;
+    if (small >= lmin) {
+        SmallLevels v = small_levels(a, small, a.z_num, off, P);
+        v.min_type = min_type;
+        launch_tiles<SmallPull>(ctx, v, 1);
+    }
     mark(ctx, ST_STRUCTURE);
     /* equivalence optimisation, levels upward in order */
-    for (int l = lmin + 1; l <= top; ++l) {
-        const int64_t G = stride_tiles(off[l + 1] - off[l], 256 * 4);
-        const int i32 = fits32(off[l + 1] - off[l]) ? 1 : 0;
-        launch_tiles<Upseed>(ctx, {P + off[l], D(l), P + off[l - 1], D(l - 1), min_type, G, i32 ? FastDiv((uint64_t)a.y_num[l]) : FastDiv(),
-                                   i32 ? FastDiv((uint64_t)a.x_num[l]) : FastDiv(), i32},
-                             G);
+    for (int l = std::max(small, lmin) + 1; l <= top; ++l) {
+        const int64_t ng = cdiv(a.y_num[l], 8), n = ng * a.x_num[l] * a.z_num[l];
+        UpseedArgs u{P + off[l], D(l), P + off[l - 1], D(l - 1), min_type, stride_tiles(n, 256), FastDiv(), FastDiv(), fits32(n) ? 1 : 0};
+        if (u.i32) {
+            u.fg = FastDiv((uint64_t)ng);
+            u.fx = FastDiv((uint64_t)a.x_num[l]);
+        }
+        launch_tiles<Upseed>(ctx, u, u.G);
     }
     /* segment table over APR levels lmin..lmax */
     RowTable t;
