@@ -139,7 +139,7 @@ __device__ __forceinline__ int u16at(const uint4& v, int i) {
  * rows and its down rows, so a step loads 8 rows instead of 12.  RAG: y_num is no multiple of 8: the
  * samples past y_num are left out, and the outputs are stored at their own alignment (the gradient of
  * 1001 x 777 x 203 u16: 0.64 ms a cell per lane, 0.15 ms this way). */
-constexpr int GZC = 8;
+constexpr int GZC = 8;   /* fewer in small volumes (grad_zc) */
 template <typename E>
 __device__ __forceinline__ void store_cells(E* p, const E* v, int n, int left) {
     /* n cells, `left` of them inside the row */
@@ -152,7 +152,7 @@ __device__ __forceinline__ void store_cells(E* p, const E* v, int n, int left) {
 template <bool UNIT, bool RAG>
 __device__ __forceinline__ void grad_ds_vec_body(const uint16_t* __restrict__ img, uint16_t* grad, float* mean, int64_t y_num, int64_t yq,
                                                  int64_t x_num, int64_t z_num, int64_t yd_num, float h2x, float h2y, float h2z,
-                                                 int accum, int64_t yg, int64_t xd, int64_t zc, int64_t xd_num, int64_t zd_num) {
+                                                 int accum, int64_t yg, int64_t xd, int64_t zc, int64_t xd_num, int64_t zd_num, int64_t gzc) {
     /* yg: group of 8 y */
     if (yg * 8 >= y_num) return;
     const int64_t xy = x_num * yq;
@@ -170,7 +170,7 @@ __device__ __forceinline__ void grad_ds_vec_body(const uint16_t* __restrict__ im
         if (which == 0) return y0 > 0 ? (int)p[y0 - 1] : -1;
         return y0 + 8 < y_num ? (int)p[y0 + 8] : -1;
     };
-    const int64_t zd_begin = zc * GZC, zd_end = min(zd_num, zd_begin + GZC);
+    const int64_t zd_begin = zc * gzc, zd_end = min(zd_num, zd_begin + gzc);
     uint4 keep_u0 = make_uint4(0, 0, 0, 0), keep_u1 = keep_u0, keep_c0 = keep_u0, keep_c1 = keep_u0;
     int64_t keep_uz = -1, keep_cz = -1;   /* planes the kept rows belong to */
     for (int64_t zd = zd_begin; zd < zd_end; ++zd) {
@@ -273,7 +273,7 @@ __device__ __forceinline__ void grad_ds_vec_body(const uint16_t* __restrict__ im
 template <bool UNIT>
 __device__ __forceinline__ void grad_ds_vecf_body(const float* __restrict__ img, float* grad, float* mean, int64_t y_num, int64_t yq,
                                                   int64_t x_num, int64_t z_num, int64_t yd_num, float h2x, float h2y, float h2z, int accum,
-                                                  int64_t yg, int64_t xd, int64_t zc, int64_t xd_num, int64_t zd_num) {
+                                                  int64_t yg, int64_t xd, int64_t zc, int64_t xd_num, int64_t zd_num, int64_t gzc) {
     const int64_t xy = x_num * yq;
     const int64_t y0 = yg * 4, x0 = 2 * xd;
     const bool hx1 = x0 + 1 < x_num;
@@ -291,7 +291,7 @@ __device__ __forceinline__ void grad_ds_vecf_body(const float* __restrict__ img,
         const double q = (double)(UNIT ? d * 0.5f : d / h2);
         return q * q;
     };
-    const int64_t zd_begin = zc * GZC, zd_end = min(zd_num, zd_begin + GZC);
+    const int64_t zd_begin = zc * gzc, zd_end = min(zd_num, zd_begin + gzc);
     F4 keep_u0 = {}, keep_u1 = {}, keep_c0 = {}, keep_c1 = {};
     int64_t keep_uz = -1, keep_cz = -1;
     for (int64_t zd = zd_begin; zd < zd_end; ++zd) {
@@ -362,7 +362,7 @@ __device__ __forceinline__ void grad_ds_vecf_body(const float* __restrict__ img,
 
 /* ---------------- inverse cubic B-spline, [1 4 1]/6 (ComputeGradient.hpp:784-964) ---------------- */
 /* All active passes of the inverse B-spline in one sweep.  A block owns a 64 (y) x 16 (x) tile
- * and marches along a run of INV_ZC z planes: each plane is loaded once with a one-sample halo
+ * and marches along a run of up to INV_ZC z planes: each plane is loaded once with a one-sample halo
  * into LDS, the y pass is applied to the 18 rows of the tile (the halo rows' y outputs are the
  * x neighbours), then the x pass, and the x-y result of three consecutive planes gives the z
  * pass of the middle one.  Each value is formed by the same operations in the same order as the
@@ -405,6 +405,7 @@ struct InvFusedArgs {
     int64_t y, x, z;
     int ay, ax, az;
     int64_t nty, ntx;   /* tiles along y and x */
+    int64_t zc;         /* planes per block    */
 };
 
 __device__ __forceinline__ void inv_fused_body(const InvFusedArgs& a, int64_t t) {
@@ -414,7 +415,7 @@ __device__ __forceinline__ void inv_fused_body(const InvFusedArgs& a, int64_t t)
     __shared__ float s_y[NR][INV_TY + 1];
     const int64_t Y = a.y, X = a.x, Z = a.z;
     const int64_t ty = t % a.nty, r0 = t / a.nty, tx = r0 % a.ntx, tz = r0 / a.ntx;
-    const int64_t y0 = ty * INV_TY, x0 = tx * INV_TX, zs = tz * INV_ZC, ze = min(zs + INV_ZC, Z);
+    const int64_t y0 = ty * INV_TY, x0 = tx * INV_TX, zs = tz * a.zc, ze = min(zs + a.zc, Z);
     const int ly = threadIdx.x & 63, lx = threadIdx.x >> 6;
     const int64_t yy = y0 + ly;
     /* the plane's halo'd tile, loaded cooperatively into registers */
@@ -1011,6 +1012,7 @@ struct GradArgs {
     int accum;
     int64_t gx, xd_num, zd_num;
     int64_t yq;   /* image row pitch (vector forms) */
+    int64_t gzc;  /* downsampled planes per lane (vector forms) */
 };
 template <typename T>
 struct GradDs {
@@ -1032,12 +1034,12 @@ struct GradDsVec {
         /* lanes numbered densely over (y group, x column pair, run of GZC z planes), so short y
            rows still fill the blocks */
         /* rows of whole 16-byte words, which launch_grad_ds_u16 checks before choosing it */
-        const int64_t ny = (a.y_num + 7) / 8, nz = (a.zd_num + GZC - 1) / GZC;
+        const int64_t ny = (a.y_num + 7) / 8, nz = (a.zd_num + a.gzc - 1) / a.gzc;
         const int64_t L = t * blockDim.x + threadIdx.x;
         if (L >= ny * a.xd_num * nz) return;
         const int64_t yg = L % ny, r = L / ny;
         grad_ds_vec_body<UNIT, RAG>((const uint16_t*)a.img, (uint16_t*)a.grad, a.mean, a.y_num, a.yq, a.x_num, a.z_num, a.yd_num, a.h2x,
-                                    a.h2y, a.h2z, a.accum, yg, r % a.xd_num, r / a.xd_num, a.xd_num, a.zd_num);
+                                    a.h2y, a.h2z, a.accum, yg, r % a.xd_num, r / a.xd_num, a.xd_num, a.zd_num, a.gzc);
     }
 };
 template <bool UNIT>
@@ -1046,12 +1048,12 @@ struct GradDsVecF {
     static constexpr int THREADS = 256;
     static const char* name() { return "gradient_ds_vec_f32"; }
     static __device__ __forceinline__ void run(const Args& a, int64_t t) {
-        const int64_t ny = (a.y_num + 3) / 4, nz = (a.zd_num + GZC - 1) / GZC;
+        const int64_t ny = (a.y_num + 3) / 4, nz = (a.zd_num + a.gzc - 1) / a.gzc;
         const int64_t L = t * blockDim.x + threadIdx.x;
         if (L >= ny * a.xd_num * nz) return;
         const int64_t yg = L % ny, r = L / ny;
         grad_ds_vecf_body<UNIT>((const float*)a.img, (float*)a.grad, a.mean, a.y_num, a.yq, a.x_num, a.z_num, a.yd_num, a.h2x, a.h2y, a.h2z,
-                                a.accum, yg, r % a.xd_num, r / a.xd_num, a.xd_num, a.zd_num);
+                                a.accum, yg, r % a.xd_num, r / a.xd_num, a.xd_num, a.zd_num, a.gzc);
     }
 };
 template <typename G>
@@ -1119,14 +1121,25 @@ PadGeom pad_geom(int64_t yd, int64_t xd, int64_t zd, const LisParams& lp) {
 
 }  // namespace
 
+namespace {
+/* planes per lane of a vector gradient with `columns` (y group, x) columns: GZC, halved while that leaves
+   fewer than 65536 lanes, since a lane walks its planes one after another (60 x 52 x 36: 27 -> 8 us); a
+   batch's launch has the lanes of all its volumes (12 volumes: 0.21 ms with 8, 0.25 with fewer) */
+int64_t grad_zc(const aprh_context* ctx, int64_t columns, int64_t zd) {
+    int64_t g = GZC;
+    while (!ctx->recorder && g > 1 && columns * cdiv(zd, g) < 65536) g >>= 1;
+    return g;
+}
+}  // namespace
+
 void launch_grad_ds_u16(aprh_context* ctx, const uint16_t* img, uint16_t* grad, float* mean, int64_t y, int64_t x, int64_t z,
                         float hx, float hy, float hz, bool accum, int64_t pitch) {
     const int64_t yd = cdiv(y, 2), xd = cdiv(x, 2), zd = cdiv(z, 2);
     const bool unit = hx == 1.0f && hy == 1.0f && hz == 1.0f;
     const bool whole = y % 8 == 0 && (((uintptr_t)grad | (uintptr_t)mean) & 15u) == 0;
-    GradArgs a{img, grad, mean, y, x, z, yd, 2.0f * hx, 2.0f * hy, 2.0f * hz, accum ? 1 : 0, 0, xd, zd, pitch};
+    GradArgs a{img, grad, mean, y, x, z, yd, 2.0f * hx, 2.0f * hy, 2.0f * hz, accum ? 1 : 0, 0, xd, zd, pitch, grad_zc(ctx, cdiv(y, 8) * xd, zd)};
     if (pitch % 8 == 0 && ((uintptr_t)img & 15u) == 0 && y >= 2) {
-        const int64_t tiles = cdiv(cdiv(y, 8) * xd * cdiv(zd, GZC), 256);   /* 256 lanes per tile */
+        const int64_t tiles = cdiv(cdiv(y, 8) * xd * cdiv(zd, a.gzc), 256);   /* 256 lanes per tile */
         if (whole && unit) launch_tiles<GradDsVec<true, false>>(ctx, a, tiles);
         else if (whole) launch_tiles<GradDsVec<false, false>>(ctx, a, tiles);
         else if (unit) launch_tiles<GradDsVec<true, true>>(ctx, a, tiles);
@@ -1144,8 +1157,13 @@ float* launch_inv_bspline_pp(aprh_context* ctx, float* a, float* b, int64_t y, i
     if (ay || ax || az) {
         /* one sweep for all active axes: a -> b */
         if ((ay && y < 2) || (ax && x < 2) || (az && z < 2)) throw Error(APRH_ERR_UNSUPPORTED, "inverse B-spline over an axis shorter than 2");
-        const int64_t nty = cdiv(y, INV_TY), ntx = cdiv(x, INV_TX), ntz = cdiv(z, INV_ZC);
-        launch_tiles<InvFused>(ctx, InvFusedArgs{a, b, y, x, z, ay ? 1 : 0, ax ? 1 : 0, az ? 1 : 0, nty, ntx}, nty * ntx * ntz);
+        const int64_t nty = cdiv(y, INV_TY), ntx = cdiv(x, INV_TX);
+        /* runs of INV_ZC planes read 2 more; small volumes take shorter runs, down to 2 planes, while
+           there are fewer than 512 blocks (30 x 26 x 18: 42 -> 11 us); a batch's launch has the blocks of
+           all its volumes (12 volumes: 0.16 ms with 16 planes, 0.18 with fewer) */
+        int64_t zc = INV_ZC;
+        while (!ctx->recorder && zc > 2 && nty * ntx * cdiv(z, zc) < 512) zc >>= 1;
+        launch_tiles<InvFused>(ctx, InvFusedArgs{a, b, y, x, z, ay ? 1 : 0, ax ? 1 : 0, az ? 1 : 0, nty, ntx, zc}, nty * ntx * cdiv(z, zc));
         return b;
     }
     return a;
@@ -1280,9 +1298,9 @@ template void launch_levels_padded<float>(aprh_context*, const float*, const Lis
 void launch_grad_ds_f32(aprh_context* ctx, const float* img, float* grad, float* mean, int64_t y, int64_t x, int64_t z, float hx,
                         float hy, float hz, bool accum, int64_t pitch) {
     const int64_t yd = cdiv(y, 2), xd = cdiv(x, 2), zd = cdiv(z, 2);
-    GradArgs a{img, grad, mean, y, x, z, yd, 2.0f * hx, 2.0f * hy, 2.0f * hz, accum ? 1 : 0, 0, xd, zd, pitch};
+    GradArgs a{img, grad, mean, y, x, z, yd, 2.0f * hx, 2.0f * hy, 2.0f * hz, accum ? 1 : 0, 0, xd, zd, pitch, grad_zc(ctx, cdiv(y, 4) * xd, zd)};
     if (pitch % 4 == 0 && ((uintptr_t)img & 15u) == 0 && y >= 2) {
-        const int64_t tiles = cdiv(cdiv(y, 4) * xd * cdiv(zd, GZC), 256);
+        const int64_t tiles = cdiv(cdiv(y, 4) * xd * cdiv(zd, a.gzc), 256);
         if (hx == 1.0f && hy == 1.0f && hz == 1.0f) launch_tiles<GradDsVecF<true>>(ctx, a, tiles);
         else launch_tiles<GradDsVecF<false>>(ctx, a, tiles);
     } else {

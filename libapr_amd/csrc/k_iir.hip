@@ -10,10 +10,11 @@
  *    gradient take their vector forms for every y length.  The offset copy of
  *    computeL (APRConverter.hpp:213-224) is fused into the first read.
  *  - x / z passes (ComputeGradient.hpp:415-599, 601-779): lanes run along y
- *    (8 u16 / 4 f32 samples per lane), so each recursion step is one
- *    coalesced 16-byte-per-lane row access.  Axes of 64 samples or more save
+ *    (16 bytes of samples per lane, less in volumes of few lines), so each
+ *    recursion step is one coalesced row access.  Axes of 64 samples or more save
  *    the causal state every 16 steps instead of storing the causal result and
- *    recompute each chunk in the anti-causal sweep, one chunk loaded ahead.
+ *    recompute each chunk in the anti-causal sweep, one chunk loaded ahead;
+ *    shorter lines stay in LDS between the sweeps.
  *
  * Every lane keeps the reference's per-line FP32 operation order; the build
  * disables FP contraction, so results are bit-identical to the CPU path.
@@ -418,6 +419,28 @@ template <> struct Vec16<float> {
     static __device__ __forceinline__ void set_r(uint4& v, int i, float f) { set(v, i, f); }
 };
 
+/* V consecutive samples as one aligned memory word of 4, 8 or 16 bytes */
+template <typename T, int V>
+struct alignas(V * sizeof(T)) Pack {
+    static constexpr int NW = V * (int)sizeof(T) / 4;
+    uint32_t w[NW];
+    __device__ __forceinline__ float get(int i) const {
+        if constexpr (std::is_same<T, uint16_t>::value) return (float)((i & 1) ? (w[i >> 1] >> 16) : (w[i >> 1] & 0xFFFFu));
+        else return __uint_as_float(w[i]);
+    }
+    /* an integral value that is in [0, 65535] unless the pass reports an overflow; the word starts as 0 */
+    __device__ __forceinline__ void set_r(int i, float f) {
+        if constexpr (std::is_same<T, uint16_t>::value) w[i >> 1] |= ((uint32_t)clamp_q(f) & 0xFFFFu) << (16 * (i & 1));
+        else w[i] = __float_as_uint(f);
+    }
+    static __device__ __forceinline__ Pack zero() {
+        Pack p;
+#pragma unroll
+        for (int k = 0; k < NW; ++k) p.w[k] = 0;
+        return p;
+    }
+};
+
 template <typename T>
 __device__ __forceinline__ float vin(const uint4& v, int i, float off, bool has_off) {
     const float x = Vec16<T>::get(v, i);
@@ -425,102 +448,94 @@ __device__ __forceinline__ float vin(const uint4& v, int i, float off, bool has_
     return has_off ? (float)((uint32_t)(int)(x + off) & 0xFFFFu) : x;
 }
 
-/* x / z pass, 16-byte vectors along y, D steps of the recursion loaded ahead */
-template <typename T, int D>
-__device__ __forceinline__ void iir_outer_vec_body(T* img, int64_t y_num, int64_t n, int64_t s, int64_t outer_stride, const IIRCoeffs& c,
-                                                   int64_t lanes, int* d_err, int64_t t) {
-    constexpr int V = Vec16<T>::N;
-    const int64_t ny = y_num / V;
-    /* lanes are numbered densely over (line, y vector), so short y rows still fill the blocks */
-    const int64_t lane = t * blockDim.x + threadIdx.x;
-    if (lane >= lanes) return;
-    const int64_t by = lane / ny, yv = lane - by * ny;
-    T* basep = img + by * outer_stride + yv * V;
-    const int64_t sv = s / V;   /* stride in vectors */
-    uint4* base = (uint4*)basep;
+/* x / z pass over lines of fewer than 64 samples: a lane takes 4 bytes of y (two u16, one float) and keeps
+   its whole line in an LDS column, so the line is read once (16 loads in flight) and written once and
+   both recursions run from LDS.  (With 16 bytes per lane, eight steps loaded ahead and the causal result
+   stored: 32 us for lines of 52 and 36 samples in a small volume, 12 us this way.) */
+constexpr int LINE_LEN = 64;
+template <typename T>
+__device__ __forceinline__ void iir_outer_line_body(T* img, int64_t y_num, int64_t n64, int64_t s, int64_t outer_stride, const IIRCoeffs& c,
+                                                    int64_t lanes, int* d_err, int64_t t) {
+    constexpr int V = 4 / (int)sizeof(T);
+    using P = Pack<T, V>;
+    __shared__ uint32_t lines[LINE_LEN][64];
+    const int64_t lane = t * 64 + threadIdx.x;
+    if (lane >= lanes) return;   /* columns are private: no barrier */
+    const int n = (int)n64;
+    const int64_t ny = y_num / V, by = lane / ny, yv = lane - by * ny;
+    uint32_t* base = (uint32_t*)(img + by * outer_stride + yv * V);
+    const int64_t sv = s / V;
     const float b1 = c.b1, b2 = c.b2, nf = c.nf;
     int err = 0;
-    float v1[V], v2[V], v3[V], v4[V];
+    auto at = [&](int j) -> P { return P{{lines[j][threadIdx.x]}}; };
+    for (int j0 = 0; j0 < n; j0 += 16) {
+        uint32_t r[16];
+#pragma unroll
+        for (int d = 0; d < 16; ++d)
+            if (j0 + d < n) r[d] = base[(j0 + d) * sv];
+#pragma unroll
+        for (int d = 0; d < 16; ++d)
+            if (j0 + d < n) lines[j0 + d][threadIdx.x] = r[d];
+    }
+    float v1[V], v2[V], v3[V], v4[V], p1[V], p2[V];
 #pragma unroll
     for (int i = 0; i < V; ++i) v1[i] = v2[i] = v3[i] = v4[i] = 0.0f;
+#pragma unroll 4
     for (int j = 0; j < c.mL; ++j) {
-        const uint4 a = base[(int64_t)j * sv];
-        const uint4 b = base[(n - 1 - j) * sv];
-        const float w1 = c.bc1[j], w2 = c.bc2[j], w3 = c.bc3[j], w4 = c.bc4[j];
+        const P a = at(j), b = at(n - 1 - j);
 #pragma unroll
         for (int i = 0; i < V; ++i) {
-            const float xa = Vec16<T>::get(a, i), xb = Vec16<T>::get(b, i);
-            v1[i] += w1 * xa;
-            v2[i] += w2 * xa;
-            v3[i] += w3 * xb;
-            v4[i] += w4 * xb;
+            v1[i] += c.bc1[j] * a.get(i);
+            v2[i] += c.bc2[j] * a.get(i);
+            v3[i] += c.bc3[j] * b.get(i);
+            v4[i] += c.bc4[j] * b.get(i);
         }
-    }
-    {
-        uint4 o0 = make_uint4(0, 0, 0, 0), o1 = make_uint4(0, 0, 0, 0);
-#pragma unroll
-        for (int i = 0; i < V; ++i) {
-            Vec16<T>::set_r(o0, i, Val<T>::rnd(v2[i], err));
-            Vec16<T>::set_r(o1, i, Val<T>::rnd(v1[i], err));
-        }
-        base[0] = o0;
-        base[sv] = o1;
     }
     /* causal: state becomes the rounded output after the first step */
-    float p1[V], p2[V];
+    P o0 = P::zero(), o1 = P::zero();
 #pragma unroll
     for (int i = 0; i < V; ++i) {
+        o0.set_r(i, Val<T>::rnd(v2[i], err));
+        o1.set_r(i, Val<T>::rnd(v1[i], err));
         p1[i] = v1[i];
         p2[i] = v2[i];
     }
-    for (int64_t j0 = 2; j0 < n; j0 += D) {
-        uint4 buf[D];
-#pragma unroll
-        for (int d = 0; d < D; ++d)
-            if (j0 + d < n) buf[d] = base[(j0 + d) * sv];
-#pragma unroll
-        for (int d = 0; d < D; ++d) {
-            if (j0 + d >= n) break;
-            uint4 o = make_uint4(0, 0, 0, 0);
-#pragma unroll
-            for (int i = 0; i < V; ++i) {
-                const float t = Val<T>::rnd(Vec16<T>::get(buf[d], i) + b1 * p1[i] + b2 * p2[i], err);
-                Vec16<T>::set_r(o, i, t);
-                p2[i] = p1[i];
-                p1[i] = t;
-            }
-            base[(j0 + d) * sv] = o;
-        }
-    }
-    /* anti-causal: state from the unrounded boundary sums */
-    {
-        uint4 oa = make_uint4(0, 0, 0, 0), ob = make_uint4(0, 0, 0, 0);
+    lines[0][threadIdx.x] = o0.w[0];
+    lines[1][threadIdx.x] = o1.w[0];
+#pragma unroll 4
+    for (int j = 2; j < n; ++j) {
+        const P x = at(j);
+        P o = P::zero();
 #pragma unroll
         for (int i = 0; i < V; ++i) {
-            Vec16<T>::set_r(oa, i, Val<T>::rnd(v4[i] * nf, err));
-            Vec16<T>::set_r(ob, i, Val<T>::rnd(v3[i] * nf, err));
+            const float v = Val<T>::rnd(x.get(i) + b1 * p1[i] + b2 * p2[i], err);
+            o.set_r(i, v);
+            p2[i] = p1[i];
+            p1[i] = v;
         }
-        base[(n - 1) * sv] = oa;
-        base[(n - 2) * sv] = ob;
+        lines[j][threadIdx.x] = o.w[0];
     }
-    for (int64_t j0 = n - 3; j0 >= 0; j0 -= D) {
-        uint4 buf[D];
+    /* anti-causal: boundary values and state from the unrounded sums */
+    P oa = P::zero(), ob = P::zero();
 #pragma unroll
-        for (int d = 0; d < D; ++d)
-            if (j0 - d >= 0) buf[d] = base[(j0 - d) * sv];
+    for (int i = 0; i < V; ++i) {
+        oa.set_r(i, Val<T>::rnd(v4[i] * nf, err));
+        ob.set_r(i, Val<T>::rnd(v3[i] * nf, err));
+    }
+    base[(n - 1) * sv] = oa.w[0];
+    base[(n - 2) * sv] = ob.w[0];
+#pragma unroll 4
+    for (int j = n - 3; j >= 0; --j) {
+        const P x = at(j);
+        P o = P::zero();
 #pragma unroll
-        for (int d = 0; d < D; ++d) {
-            if (j0 - d < 0) break;
-            uint4 o = make_uint4(0, 0, 0, 0);
-#pragma unroll
-            for (int i = 0; i < V; ++i) {
-                const float t = (Vec16<T>::get(buf[d], i) + b1 * v3[i]) + b2 * v4[i];
-                Vec16<T>::set_r(o, i, Val<T>::rnd(t * nf, err));
-                v4[i] = v3[i];
-                v3[i] = t;
-            }
-            base[(j0 - d) * sv] = o;
+        for (int i = 0; i < V; ++i) {
+            const float v = (x.get(i) + b1 * v3[i]) + b2 * v4[i];
+            o.set_r(i, Val<T>::rnd(v * nf, err));
+            v4[i] = v3[i];
+            v3[i] = v;
         }
+        base[j * sv] = o.w[0];
     }
     if (Val<T>::failed(err)) atomicAdd(d_err, 1);
 }
@@ -531,22 +546,23 @@ __device__ __forceinline__ void iir_outer_vec_body(T* img, int64_t y_num, int64_
  * input, recomputes its causal outputs from the saved state into registers and runs the
  * anti-causal recursion over them.  Per sample the line moves 2 reads and 1 write instead of
  * 2 reads and 2 writes, plus 4/C bytes of saved state.  Every value is computed by the same
- * operations in the same order as iir_outer_vec_body, so the outputs are identical; the causal
+ * operations in the same order as a plain causal-then-anti-causal sweep, so the outputs are identical; the causal
  * outputs held in registers are packed like the stored ones, and saved states are packed the
  * same way (exact for u16 unless the pass reports an overflow, where the reference throws).
  * In place: chunk k is written only after its input was read, and chunks below k are read
  * later but written later still. */
-template <typename T, int C>
+template <typename T, int C, int V>
 __device__ __forceinline__ void iir_outer_ck_body(T* img, int64_t y_num, int64_t n, int64_t s, int64_t outer_stride, const IIRCoeffs& c,
-                                                  int* d_err, uint4* __restrict__ ck, int64_t ck_lanes, int64_t t) {
-    constexpr int V = Vec16<T>::N;
+                                                  int* d_err, void* __restrict__ ckv, int64_t ck_lanes, int64_t t) {
+    using P = Pack<T, V>;
+    P* __restrict__ ck = (P*)ckv;
     const int64_t ny = y_num / V;
     /* lanes are numbered densely over (line, y vector), so short y rows still fill the blocks */
     const int64_t lane = t * blockDim.x + threadIdx.x;
     if (lane >= ck_lanes) return;
     /* lane counts stay below 2^32 (the launcher checks): 32-bit division */
     const uint32_t by = (uint32_t)lane / (uint32_t)ny, yv = (uint32_t)lane - by * (uint32_t)ny;
-    uint4* base = (uint4*)(img + (int64_t)by * outer_stride + (int64_t)yv * V);
+    P* base = (P*)(img + (int64_t)by * outer_stride + (int64_t)yv * V);
     const int64_t sv = s / V;
     const float b1 = c.b1, b2 = c.b2, nf = c.nf;
     /* causal steps j = 2 .. n-1; the anti-causal sweep consumes j = 2 .. n-3 in chunks
@@ -554,35 +570,23 @@ __device__ __forceinline__ void iir_outer_ck_body(T* img, int64_t y_num, int64_t
        starts of chunks 1 .. K-1, then the four boundary sums (unrounded floats), which are
        parked there between the sweeps to keep registers free for the chunk buffers. */
     const int64_t K = (n - 4 + C - 1) / C;
-    uint4* sums = ck + (K - 1) * ck_lanes * 2 + lane * V;
-    auto put_f = [&](uint4* dst, const float* v) {
-#pragma unroll
-        for (int q = 0; q < V / 4; ++q) dst[q] = make_uint4(__float_as_uint(v[4 * q]), __float_as_uint(v[4 * q + 1]),
-                                                             __float_as_uint(v[4 * q + 2]), __float_as_uint(v[4 * q + 3]));
-    };
-    auto get_f = [&](const uint4* src, float* v) {
-#pragma unroll
-        for (int q = 0; q < V / 4; ++q) {
-            const uint4 w = src[q];
-            v[4 * q] = __uint_as_float(w.x);
-            v[4 * q + 1] = __uint_as_float(w.y);
-            v[4 * q + 2] = __uint_as_float(w.z);
-            v[4 * q + 3] = __uint_as_float(w.w);
-        }
-    };
+    float* sums = (float*)(ck + (K - 1) * ck_lanes * 2) + lane * 4 * V;
+    auto put_f = [&](float* dst, const float* v) { __builtin_memcpy(dst, v, V * 4); };
+    auto get_f = [&](const float* src, float* v) { __builtin_memcpy(v, src, V * 4); };
     int err = 0;
     float p1[V], p2[V];
     {
         float v1[V], v2[V], v3[V], v4[V];
 #pragma unroll
         for (int i = 0; i < V; ++i) v1[i] = v2[i] = v3[i] = v4[i] = 0.0f;
+#pragma unroll 4
         for (int j = 0; j < c.mL; ++j) {
-            const uint4 a = base[(int64_t)j * sv];
-            const uint4 b = base[(n - 1 - j) * sv];
+            const P a = base[(int64_t)j * sv];
+            const P b = base[(n - 1 - j) * sv];
             const float w1 = c.bc1[j], w2 = c.bc2[j], w3 = c.bc3[j], w4 = c.bc4[j];
 #pragma unroll
             for (int i = 0; i < V; ++i) {
-                const float xa = Vec16<T>::get(a, i), xb = Vec16<T>::get(b, i);
+                const float xa = a.get(i), xb = b.get(i);
                 v1[i] += w1 * xa;
                 v2[i] += w2 * xa;
                 v3[i] += w3 * xb;
@@ -590,9 +594,9 @@ __device__ __forceinline__ void iir_outer_ck_body(T* img, int64_t y_num, int64_t
             }
         }
         put_f(sums, v1);
-        put_f(sums + V / 4, v2);
-        put_f(sums + 2 * (V / 4), v3);
-        put_f(sums + 3 * (V / 4), v4);
+        put_f(sums + V, v2);
+        put_f(sums + 2 * V, v3);
+        put_f(sums + 3 * V, v4);
 #pragma unroll
         for (int i = 0; i < V; ++i) {
             p1[i] = v1[i];
@@ -600,12 +604,12 @@ __device__ __forceinline__ void iir_outer_ck_body(T* img, int64_t y_num, int64_t
         }
     }
     /* chunk loads are issued one chunk ahead of the recursion */
-    auto load_chunk = [&](uint4* dst, int64_t j0, int cnt) {
+    auto load_chunk = [&](P* dst, int64_t j0, int cnt) {
 #pragma unroll
         for (int d = 0; d < C; ++d)
             if (d < cnt) dst[d] = base[(j0 + d) * sv];
     };
-    uint4 cur[C], nxt[C];
+    P cur[C], nxt[C];
     {
         int cnt = (int)min((int64_t)C, n - 2);
         load_chunk(cur, 2, cnt);
@@ -614,13 +618,13 @@ __device__ __forceinline__ void iir_outer_ck_body(T* img, int64_t y_num, int64_t
             const int cn = jn < n ? (int)min((int64_t)C, n - jn) : 0;
             load_chunk(nxt, jn, cn);
             if (k > 0 && k < K) {
-                uint4 q1 = make_uint4(0, 0, 0, 0), q2 = make_uint4(0, 0, 0, 0);
+                P q1 = P::zero(), q2 = q1;
 #pragma unroll
                 for (int i = 0; i < V; ++i) {
-                    Vec16<T>::set_r(q1, i, p1[i]);
-                    Vec16<T>::set_r(q2, i, p2[i]);
+                    q1.set_r(i, p1[i]);
+                    q2.set_r(i, p2[i]);
                 }
-                uint4* cp = ck + ((k - 1) * ck_lanes + lane) * 2;
+                P* cp = ck + ((k - 1) * ck_lanes + lane) * 2;
                 cp[0] = q1;
                 cp[1] = q2;
             }
@@ -629,7 +633,7 @@ __device__ __forceinline__ void iir_outer_ck_body(T* img, int64_t y_num, int64_t
                 if (d < cnt) {
 #pragma unroll
                     for (int i = 0; i < V; ++i) {
-                        const float t = Val<T>::rnd(Vec16<T>::get(cur[d], i) + b1 * p1[i] + b2 * p2[i], err);
+                        const float t = Val<T>::rnd(cur[d].get(i) + b1 * p1[i] + b2 * p2[i], err);
                         p2[i] = p1[i];
                         p1[i] = t;
                     }
@@ -642,55 +646,39 @@ __device__ __forceinline__ void iir_outer_ck_body(T* img, int64_t y_num, int64_t
     }
     /* anti-causal: boundary values from the unrounded sums */
     float v3[V], v4[V];
-    get_f(sums + 2 * (V / 4), v3);
-    get_f(sums + 3 * (V / 4), v4);
+    get_f(sums + 2 * V, v3);
+    get_f(sums + 3 * V, v4);
     {
-        uint4 oa = make_uint4(0, 0, 0, 0), ob = make_uint4(0, 0, 0, 0);
+        P oa = P::zero(), ob = oa;
 #pragma unroll
         for (int i = 0; i < V; ++i) {
-            Vec16<T>::set_r(oa, i, Val<T>::rnd(v4[i] * nf, err));
-            Vec16<T>::set_r(ob, i, Val<T>::rnd(v3[i] * nf, err));
+            oa.set_r(i, Val<T>::rnd(v4[i] * nf, err));
+            ob.set_r(i, Val<T>::rnd(v3[i] * nf, err));
         }
         base[(n - 1) * sv] = oa;
         base[(n - 2) * sv] = ob;
     }
-    auto back = [&](const uint4& f, int64_t j) {
-        uint4 o = make_uint4(0, 0, 0, 0);
+    auto back = [&](const P& f, int64_t j) {
+        P o = P::zero();
 #pragma unroll
         for (int i = 0; i < V; ++i) {
-            const float t = (Vec16<T>::get(f, i) + b1 * v3[i]) + b2 * v4[i];
-            Vec16<T>::set_r(o, i, Val<T>::rnd(t * nf, err));
+            const float t = (f.get(i) + b1 * v3[i]) + b2 * v4[i];
+            o.set_r(i, Val<T>::rnd(t * nf, err));
             v4[i] = v3[i];
             v3[i] = t;
         }
         base[j * sv] = o;
     };
-    /* two anti-causal steps (j, then j - 1) with the states swapping roles instead of moving */
-    auto back2 = [&](const uint4& f, const uint4& g, int64_t j) {
-        uint4 o = make_uint4(0, 0, 0, 0), u = o;
-#pragma unroll
-        for (int i = 0; i < V; ++i) {
-            v4[i] = (Vec16<T>::get(f, i) + b1 * v3[i]) + b2 * v4[i];
-            Vec16<T>::set_r(o, i, Val<T>::rnd(v4[i] * nf, err));
-        }
-        base[j * sv] = o;
-#pragma unroll
-        for (int i = 0; i < V; ++i) {
-            v3[i] = (Vec16<T>::get(g, i) + b1 * v4[i]) + b2 * v3[i];
-            Vec16<T>::set_r(u, i, Val<T>::rnd(v3[i] * nf, err));
-        }
-        base[(j - 1) * sv] = u;
-    };
     /* causal outputs of chunk `buf` from state (p1, p2), then the anti-causal sweep over it */
-    auto chunk = [&](uint4* buf, int64_t j0, int cnt) {
+    auto chunk = [&](P* buf, int64_t j0, int cnt) {
 #pragma unroll
         for (int d = 0; d < C; ++d) {
             if (d < cnt) {
-                uint4 o = make_uint4(0, 0, 0, 0);
+                P o = P::zero();
 #pragma unroll
                 for (int i = 0; i < V; ++i) {
-                    const float t = Val<T>::rnd(Vec16<T>::get(buf[d], i) + b1 * p1[i] + b2 * p2[i], err);
-                    Vec16<T>::set_r(o, i, t);
+                    const float t = Val<T>::rnd(buf[d].get(i) + b1 * p1[i] + b2 * p2[i], err);
+                    o.set_r(i, t);
                     p2[i] = p1[i];
                     p1[i] = t;
                 }
@@ -705,25 +693,25 @@ __device__ __forceinline__ void iir_outer_ck_body(T* img, int64_t y_num, int64_t
         int64_t j0 = 2 + (K - 1) * C;
         int cnt = (int)min((int64_t)C, n - 2 - j0);
         load_chunk(cur, j0, cnt);
-        uint4 q1 = make_uint4(0, 0, 0, 0), q2 = q1;
+        P q1 = P::zero(), q2 = q1;
         if (K > 1) {
-            const uint4* cp = ck + ((K - 2) * ck_lanes + lane) * 2;
+            const P* cp = ck + ((K - 2) * ck_lanes + lane) * 2;
             q1 = cp[0];
             q2 = cp[1];
         }
         /* chunks K-1 .. 1 start from packed states; chunk 0 from the boundary sums */
         for (int64_t k = K - 1; k >= 1; --k, j0 -= C) {
-            uint4 n1 = make_uint4(0, 0, 0, 0), n2 = n1;
+            P n1 = P::zero(), n2 = n1;
             load_chunk(nxt, j0 - C, C);
             if (k > 1) {
-                const uint4* cp = ck + ((k - 2) * ck_lanes + lane) * 2;
+                const P* cp = ck + ((k - 2) * ck_lanes + lane) * 2;
                 n1 = cp[0];
                 n2 = cp[1];
             }
 #pragma unroll
             for (int i = 0; i < V; ++i) {
-                p1[i] = Vec16<T>::get(q1, i);
-                p2[i] = Vec16<T>::get(q2, i);
+                p1[i] = q1.get(i);
+                p2[i] = q2.get(i);
             }
             chunk(cur, j0, cnt);
 #pragma unroll
@@ -733,18 +721,18 @@ __device__ __forceinline__ void iir_outer_ck_body(T* img, int64_t y_num, int64_t
             cnt = C;
         }
         get_f(sums, p1);
-        get_f(sums + V / 4, p2);
+        get_f(sums + V, p2);
         chunk(cur, 2, cnt);
     }
     /* causal outputs at 0 and 1, as they would be stored */
     float v1[V], v2[V];
     get_f(sums, v1);
-    get_f(sums + V / 4, v2);
-    uint4 f0 = make_uint4(0, 0, 0, 0), f1 = make_uint4(0, 0, 0, 0);
+    get_f(sums + V, v2);
+    P f0 = P::zero(), f1 = f0;
 #pragma unroll
     for (int i = 0; i < V; ++i) {
-        Vec16<T>::set_r(f0, i, Val<T>::rnd(v2[i], err));
-        Vec16<T>::set_r(f1, i, Val<T>::rnd(v1[i], err));
+        f0.set_r(i, Val<T>::rnd(v2[i], err));
+        f1.set_r(i, Val<T>::rnd(v1[i], err));
     }
     if (n - 3 >= 1) back(f1, 1);
     back(f0, 0);
@@ -1128,24 +1116,25 @@ struct IirOuter {
         iir_outer_body<T>(a.out, a.y_num, a.n, a.s, a.outer_stride, a.c, a.d_err, t % a.gx, t / a.gx);
     }
 };
-template <typename T, int D>
-struct IirOuterVec {
+template <typename T>
+struct IirOuterLine {
     using Args = IirArgs<T>;
-    static constexpr int THREADS = 256;
-    static const char* name() { return "bspline_outer_vec"; }
+    static constexpr int THREADS = 64;
+    static const char* name() { return "bspline_outer_line"; }
     static __device__ __forceinline__ void run(const Args& a, int64_t t) {
-        iir_outer_vec_body<T, D>(a.out, a.y_num, a.n, a.s, a.outer_stride, a.c, a.ck_lanes, a.d_err, t);
+        iir_outer_line_body<T>(a.out, a.y_num, a.n, a.s, a.outer_stride, a.c, a.ck_lanes, a.d_err, t);
     }
 };
 
-template <typename T, int C>
+/* V samples of y per lane: 16 bytes, or less where a volume has few lines */
+template <typename T, int C, int V>
 struct IirOuterCk {
     using Args = IirArgs<T>;
     static constexpr int THREADS = 256;
     static constexpr int MIN_WAVES = 2;   /* two chunk buffers in registers; one wave per SIMD hides too little latency */
     static const char* name() { return "bspline_outer_ck"; }
     static __device__ __forceinline__ void run(const Args& a, int64_t t) {
-        iir_outer_ck_body<T, C>(a.out, a.y_num, a.n, a.s, a.outer_stride, a.c, a.d_err, a.ck, a.ck_lanes, t);
+        iir_outer_ck_body<T, C, V>(a.out, a.y_num, a.n, a.s, a.outer_stride, a.c, a.d_err, a.ck, a.ck_lanes, t);
     }
 };
 
@@ -1231,7 +1220,8 @@ void launch_iir_y(aprh_context* ctx, const T* in, T* out, int64_t y, int64_t x, 
 
 /* checkpointed x / z pass: chunk length and the shortest axis it is used for */
 constexpr int OUTER_CK = 16;
-constexpr int64_t OUTER_CK_MIN = 64;
+constexpr int64_t OUTER_CK_MIN = LINE_LEN;
+constexpr int64_t OUTER_LANES = 131072;
 
 template <typename T>
 void launch_iir_outer(aprh_context* ctx, T* img, int64_t y, int64_t x, int64_t z, int axis, const IIRCoeffs& c, int* d_err) {
@@ -1239,35 +1229,54 @@ void launch_iir_outer(aprh_context* ctx, T* img, int64_t y, int64_t x, int64_t z
     /* x pass: lines along x (stride y), one per (y, z); z pass: along z (stride x*y), one per (y, x) */
     const int64_t n = axis == 1 ? x : z, s = axis == 1 ? y : x * y, outer = axis == 1 ? z : x;
     const int64_t ostride = axis == 1 ? x * y : y;
+    IirArgs<T> a{img, img, y, n, s, ostride, 1, c, nullptr, d_err};
     if (y % V == 0 && aligned16(img)) {
-        const int64_t lanes = (y / V) * outer;
-        IirArgs<T> a{img, img, y, n, s, ostride, 1, c, nullptr, d_err};
-        a.ck_lanes = lanes;
-        if (n >= OUTER_CK_MIN && lanes < (int64_t(1) << 32)) {
-            /* a batch plan also times checkpoints every 8 and every 32 steps (the buffer then
-               holds the states of the densest spacing) */
-            const bool alts = std::is_same<T, uint16_t>::value && ctx->recorder;
-            const int64_t chunks = (n - 4 + (alts ? 8 : OUTER_CK) - 1) / (alts ? 8 : OUTER_CK);
-            /* the chunk states live until the launch ends: from the pool, returned after the
-               launch is queued (stream order keeps later users behind it) */
-            Buf ck(ctx->pool, ((size_t)(chunks - 1) * 2 + V) * (size_t)lanes * 16);
-            a.ck = ck.as<uint4>();
-            const int64_t tiles = cdiv(lanes, 256);
-            if (alts)
-                launch_tiles_alts(ctx,
-                                  {tile_alt<IirOuterCk<T, 8>>(a, tiles, "checkpoint every 8"),
-                                   tile_alt<IirOuterCk<T, OUTER_CK>>(a, tiles, "checkpoint every 16"),
-                                   tile_alt<IirOuterCk<T, 32>>(a, tiles, "checkpoint every 32")},
-                                  1);
-            else
-                launch_tiles<IirOuterCk<T, OUTER_CK>>(ctx, a, tiles);
-        } else {
-            launch_tiles<IirOuterVec<T, 8>>(ctx, a, cdiv(lanes, 256));
+        if (n < OUTER_CK_MIN) {
+            a.ck_lanes = y / (4 / (int64_t)sizeof(T)) * outer;
+            launch_tiles<IirOuterLine<T>>(ctx, a, cdiv(a.ck_lanes, 64));
+            return;
         }
-        return;
+        if ((y / V) * outer < (int64_t(1) << 30)) {
+            /* a lane takes 16 bytes of y; with fewer than OUTER_LANES lanes that way (2 waves for each of
+               the chip's 1024 SIMDs) it takes 8, and with fewer than half of them 4: the pass waits on
+               memory, and a wave has 16 loads in flight whatever their width.  1001 x 777 x 203 u16: x (26
+               thousand lanes of 16 bytes) and z (98 thousand) 0.86 ms together with 16 bytes, 0.47 this way */
+            int vl = V;
+            while (vl > 4 / (int)sizeof(T) && (y / vl) * outer < OUTER_LANES) vl >>= 1;
+            auto pass = [&](auto cc, auto vv, int chunk) {
+                constexpr int C = decltype(cc)::value, VL = decltype(vv)::value;
+                IirArgs<T> q = a;
+                q.ck_lanes = (y / VL) * outer;
+                /* the chunk states live until the launch ends: from the pool, returned after the
+                   launch is queued (stream order keeps later users behind it) */
+                const int64_t chunks = (n - 4 + chunk - 1) / chunk;
+                Buf ck(ctx->pool, ((size_t)(chunks - 1) * 2 * sizeof(Pack<T, VL>) + 16 * VL) * (size_t)q.ck_lanes);
+                q.ck = ck.as<uint4>();
+                return tile_alt<IirOuterCk<T, C, VL>>(q, cdiv(q.ck_lanes, 256), C == 8 ? "checkpoint every 8, 16 bytes"
+                                                                                : VL == V ? "checkpoint every 16, 16 bytes"
+                                                                                          : "checkpoint every 16, fewer bytes");
+            };
+            auto run = [&](const TileAlt& alt) { launch_tiles_alts(ctx, {alt}, 0); };
+            using C16 = std::integral_constant<int, OUTER_CK>;
+            if (ctx->recorder && std::is_same<T, uint16_t>::value) {
+                /* a batch plan times the widths and a denser spacing over all its volumes */
+                launch_tiles_alts(ctx,
+                                  {pass(C16{}, std::integral_constant<int, V>{}, OUTER_CK), pass(std::integral_constant<int, 8>{}, std::integral_constant<int, V>{}, 8),
+                                   pass(C16{}, std::integral_constant<int, V / 2>{}, OUTER_CK)},
+                                  0);
+            } else if (vl == V) {
+                run(pass(C16{}, std::integral_constant<int, V>{}, OUTER_CK));
+            } else if (vl == V / 2) {
+                run(pass(C16{}, std::integral_constant<int, V / 2>{}, OUTER_CK));
+            } else {
+                run(pass(C16{}, std::integral_constant<int, V / 4>{}, OUTER_CK));
+            }
+            return;
+        }
     }
     const int64_t gx = cdiv(y, 256);
-    launch_tiles<IirOuter<T>>(ctx, IirArgs<T>{img, img, y, n, s, ostride, gx, c, nullptr, d_err}, gx * outer);
+    a.gx = gx;
+    launch_tiles<IirOuter<T>>(ctx, a, gx * outer);
 }
 
 template void launch_iir_y<uint16_t>(aprh_context*, const uint16_t*, uint16_t*, int64_t, int64_t, int64_t, const IIRCoeffs&,

@@ -252,3 +252,30 @@ def test_ragged_y_offset_not_guessed(oracle, ctx, lo, hi, y):
     for w in range(6):
         assert np.array_equal(apr.intermediate(w), ref.intermediate(w)), w
     assert apr.total == ref.total
+
+
+@pytest.mark.parametrize("dtype", [np.uint16, np.float32])
+@pytest.mark.parametrize("axis", [1, 2])
+@pytest.mark.parametrize("n", [2, 3, 4, 15, 16, 17, 33, 63, 64, 65])
+def test_bspline_outer_short_lines(oracle, ctx, dtype, axis, n):
+    """lines kept in LDS (below 64 samples) and the first checkpointed ones, 4 bytes of y per lane"""
+    shape = (5, n, 72) if axis == 1 else (n, 5, 72)
+    _bspline_outer_against_oracle(oracle, ctx, dtype, axis, shape)
+
+
+@pytest.mark.parametrize("dtype,x", [(np.uint16, 512), (np.uint16, 256), (np.float32, 256), (np.float32, 128)])
+def test_bspline_outer_lane_widths(oracle, ctx, dtype, x):
+    """enough lines for 16 bytes of y per lane (131072 lanes), and just half as many, which take 8"""
+    _bspline_outer_against_oracle(oracle, ctx, dtype, 2, (67, x, 2048))
+
+
+def _bspline_outer_against_oracle(oracle, ctx, dtype, axis, shape):
+    lib = oracle.load("oracle")
+    rng = np.random.default_rng(shape[0] * 1000 + shape[1])
+    img = rng.integers(200, 3200, shape).astype(dtype)
+    z, x, y = shape
+    print(f"axis {axis} {shape} {np.dtype(dtype)}", flush=True)
+    g = A.bspline_filt_rec(img.copy(), axis, ctx=ctx)
+    o = img.copy()
+    (lib.orc_bspline_u16 if dtype == np.uint16 else lib.orc_bspline_f32)(o.reshape(-1), y, x, z, axis, 3.0, 1e-4)
+    assert np.array_equal(g.view(np.uint8), o.view(np.uint8))
