@@ -751,7 +751,8 @@ __device__ __forceinline__ void iir_outer_ck_body(T* img, int64_t y_num, int64_t
  * written to rows of pitch oq (whole 16-byte words; the samples past y_num become 0).  Only the
  * last chunk, and the one before it where that holds sample y_num - 2, test their samples.  On
  * 1001 x 777 x 203 u16 the pass took 2.41 ms with one sample per lane and load and the causal
- * result stored, 0.30 ms this way. */
+ * result stored, 0.35 ms this way; at two waves per SIMD instead of three its 2464 waves took a second
+ * round, 0.60 ms. */
 template <typename T, bool RAG>
 __device__ __forceinline__ void iir_y_ck_body(const T* in, T* out, int64_t y_num, int64_t oq, int64_t n_lines, const IIRCoeffs& c,
                                               const float* d_off, int* d_err, float2* __restrict__ ck, uint32_t* mm, const int* run_if,
@@ -790,28 +791,48 @@ __device__ __forceinline__ void iir_y_ck_body(const T* in, T* out, int64_t y_num
         return v;
     };
 
-    /* lines of the cooperative layout: load instruction i covers LDS rows 8i..8i+7 */
-    int64_t lrow[8];
+    /* lines of the cooperative layout: load instruction i covers LDS rows 8i..8i+7 (dims are at most
+       65535, so a line's number fits 32 bits with room for "none") */
+    constexpr uint32_t NONE = 0xFFFFFFFFu;
+    uint32_t lrow[8];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) lrow[i] = line_of(8 * i + (lane >> 3));
+    for (int i = 0; i < 8; ++i) {
+        const int64_t l = line_of(8 * i + (lane >> 3));
+        lrow[i] = l < 0 ? NONE : (uint32_t)l;
+    }
+    /* a chunk's words; of a short last chunk the word that holds the line's end is loaded as the line's
+       last V samples (so it stays inside the line), which settle() moves down to their place */
+    const int have = RAG ? tail - seg * V : V;   /* samples of this lane's word in the last chunk */
+    const bool tiny = RAG && y_num < V;          /* a line shorter than a word: one sample after the other */
     auto gload = [&](const T* base, int64_t ch, uint4* r) {
-        const bool whole = !RAG || ch + 1 < nch || seg * V + V <= tail;
+        if (tiny) return;
+        const bool end = RAG && ch + 1 == nch && have < V;
+        const int64_t o = end ? y_num - V : ch * CH + seg * V;
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+            r[i] = lrow[i] != NONE ? load16(base + (int64_t)lrow[i] * y_num + o) : make_uint4(0, 0, 0, 0);
+    };
+    auto settle = [&](int64_t ch, uint4* r) {
+        if (!RAG || tiny || ch + 1 != nch || tail == CH) return;
+        const int sh = have >= V ? 0 : have <= 0 ? 128 : (V - have) * 8 * (int)sizeof(T);
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
-            r[i] = make_uint4(0, 0, 0, 0);
-            if (lrow[i] < 0) continue;
-            const T* p = base + lrow[i] * y_num + ch * CH + seg * V;
-            if (whole) {
-                r[i] = load16(p);
-            } else {
-                T e[V];
-#pragma unroll
-                for (int j = 0; j < V; ++j) e[j] = seg * V + j < tail ? p[j] : (T)0;
-                __builtin_memcpy(&r[i], e, 16);
-            }
+            const uint64_t lo = ((uint64_t)r[i].y << 32) | r[i].x, hi = ((uint64_t)r[i].w << 32) | r[i].z;
+            const uint64_t nl = sh >= 128 ? 0 : sh >= 64 ? hi >> (sh - 64) : (lo >> sh) | (hi << (63 - sh) << 1);
+            const uint64_t nh = sh >= 64 ? 0 : hi >> sh;
+            r[i] = make_uint4((uint32_t)nl, (uint32_t)(nl >> 32), (uint32_t)nh, (uint32_t)(nh >> 32));
         }
     };
-    auto lds_put = [&](const uint4* r) {
+    auto lds_put = [&](const T* base, const uint4* r) {
+        if (tiny) {
+#pragma unroll 1
+            for (int i = 0; i < 8; ++i) {
+                const int R = 8 * i + (lane >> 3);
+                const int64_t l = line_of(R);
+                for (int j = 0; j < V; ++j) tile[R * PITCH + seg * V + j] = (l >= 0 && seg == 0 && j < y_num) ? base[l * y_num + j] : (T)0;
+            }
+            return;
+        }
 #pragma unroll
         for (int i = 0; i < 8; ++i) *(uint4*)(&tile[(8 * i + (lane >> 3)) * PITCH + seg * V]) = r[i];
     };
@@ -819,7 +840,7 @@ __device__ __forceinline__ void iir_y_ck_body(const T* in, T* out, int64_t y_num
         if (RAG && ch * CH + seg * V >= oq) return;
 #pragma unroll
         for (int i = 0; i < 8; ++i)
-            if (lrow[i] >= 0) *(uint4*)(base + lrow[i] * oq + ch * CH + seg * V) = *(const uint4*)(&tile[(8 * i + (lane >> 3)) * PITCH + seg * V]);
+            if (lrow[i] != NONE) *(uint4*)(base + (int64_t)lrow[i] * oq + ch * CH + seg * V) = *(const uint4*)(&tile[(8 * i + (lane >> 3)) * PITCH + seg * V]);
     };
     /* the mean pyramid's cells of one chunk (PixelData.hpp:944-962 with u16 storage): 16 x pairs
        x 32 y pairs of the plane pair; a lane sums 8 y pairs of one x pair over its 4 rows (eight
@@ -919,7 +940,7 @@ __device__ __forceinline__ void iir_y_ck_body(const T* in, T* out, int64_t y_num
             s1 = t;
         };
         if (ch == 0 || (RAG && n < CH)) {
-#pragma unroll
+#pragma unroll 1
             for (int q = 0; q < CH / V; ++q) {
                 if (RAG && q * V >= n) break;
                 uint4 v = *(uint4*)(row + q * V);
@@ -937,7 +958,7 @@ __device__ __forceinline__ void iir_y_ck_body(const T* in, T* out, int64_t y_num
                 if (keep) *(uint4*)(row + q * V) = o;
             }
         } else {
-#pragma unroll
+#pragma unroll 2
             for (int q = 0; q < CH / V; ++q) {
                 uint4 v = *(uint4*)(row + q * V);
                 uint4 o = make_uint4(0, 0, 0, 0);
@@ -959,33 +980,38 @@ __device__ __forceinline__ void iir_y_ck_body(const T* in, T* out, int64_t y_num
         gload(in, 0, nxt);
         for (int64_t ch = 0; ch < nch; ++ch) {
             __syncthreads();
+            settle(ch, nxt);
             if (U16 && mm) {
-                const bool whole = !RAG || ch + 1 < nch || seg * V + V <= tail;
+                const int n = tiny ? 0 : RAG && ch + 1 == nch ? min(max(have, 0), V) : V;   /* samples of each word */
 #pragma unroll
                 for (int i = 0; i < 8; ++i) {
-                    if (lrow[i] < 0) continue;
+                    if (lrow[i] == NONE || n == 0) continue;
                     const uint32_t w[4] = {nxt[i].x, nxt[i].y, nxt[i].z, nxt[i].w};
-                    if (whole) {
 #pragma unroll
-                        for (int q = 0; q < 4; ++q) {
-                            us2 v;
-                            __builtin_memcpy(&v, &w[q], 4);
-                            lo = __builtin_elementwise_min(lo, v);
-                            hi = __builtin_elementwise_max(hi, v);
-                        }
-                    } else {
-#pragma unroll
-                        for (int j = 0; j < 8; ++j) {
-                            const uint16_t x = (uint16_t)(w[j >> 1] >> (16 * (j & 1)));
-                            if (seg * V + j < tail) {
-                                lo = __builtin_elementwise_min(lo, (us2){x, x});
-                                hi = __builtin_elementwise_max(hi, (us2){x, x});
-                            }
-                        }
+                    for (int q = 0; q < 4; ++q) {
+                        /* past the word's samples: its first one again */
+                        const uint32_t f = w[0] & 0xFFFFu;
+                        uint32_t x = w[q];
+                        if (RAG) x = (2 * q < n ? x & 0xFFFFu : f) | (2 * q + 1 < n ? x & 0xFFFF0000u : f << 16);
+                        us2 v;
+                        __builtin_memcpy(&v, &x, 4);
+                        lo = __builtin_elementwise_min(lo, v);
+                        hi = __builtin_elementwise_max(hi, v);
                     }
                 }
             }
-            lds_put(nxt);
+            lds_put(in, nxt);
+            if (U16 && mm && tiny && seg == 0) {
+                for (int i = 0; i < 8; ++i)
+                    for (int j = 0; j < (int)y_num; ++j) {
+                        const int R = 8 * i + (lane >> 3);
+                        const unsigned short x = (unsigned short)tile[R * PITCH + j];
+                        if (line_of(R) >= 0) {
+                            lo = __builtin_elementwise_min(lo, (us2){x, x});
+                            hi = __builtin_elementwise_max(hi, (us2){x, x});
+                        }
+                    }
+            }
             if (ch + 1 < nch) gload(in, ch + 1, nxt);
             __syncthreads();
             if constexpr (U16 && !RAG) {
@@ -1019,7 +1045,8 @@ __device__ __forceinline__ void iir_y_ck_body(const T* in, T* out, int64_t y_num
     gload(in, nch - 1, nxt);
     for (int64_t ch = nch - 1; ch >= 0; --ch) {
         __syncthreads();
-        lds_put(nxt);
+        settle(ch, nxt);
+        lds_put(in, nxt);
         if (ch - 1 >= 0) gload(in, ch - 1, nxt);
         __syncthreads();
         if (valid) {
@@ -1041,7 +1068,7 @@ __device__ __forceinline__ void iir_y_ck_body(const T* in, T* out, int64_t y_num
             if ((ch + 1) * CH > y_num - 2) {
                 /* the chunk holds sample y_num - 2 or y_num - 1, which take the boundary values */
                 const int last = (int)(y_num - 1 - ch * CH);   /* sample y_num - 1 in this chunk's numbering */
-#pragma unroll
+#pragma unroll 1
                 for (int q = CH / V - 1; q >= 0; --q) {
                     if (RAG && q * V > last) continue;
                     uint4 v = *(uint4*)(row + q * V);
@@ -1057,7 +1084,7 @@ __device__ __forceinline__ void iir_y_ck_body(const T* in, T* out, int64_t y_num
                     *(uint4*)(row + q * V) = o;
                 }
             } else {
-#pragma unroll
+#pragma unroll 2
                 for (int q = CH / V - 1; q >= 0; --q) {
                     uint4 v = *(uint4*)(row + q * V);
                     uint4 o = make_uint4(0, 0, 0, 0);
@@ -1102,6 +1129,7 @@ template <typename T, bool RAG>
 struct IirYCk {
     using Args = IirArgs<T>;
     static constexpr int THREADS = 64;
+    static constexpr int MIN_WAVES = 3;
     static const char* name() { return RAG ? "bspline_y_ck_ragged" : "bspline_y_ck"; }
     static __device__ __forceinline__ void run(const Args& a, int64_t t) {
         iir_y_ck_body<T, RAG>(a.in, a.out, a.y_num, a.s, a.n, a.c, a.d_off, a.d_err, (float2*)a.ck, a.mm, a.run_if, a.pyr, a.px, a.pz, t);

@@ -182,53 +182,73 @@ __device__ __forceinline__ void pull_level8_body(const PullArgs& a, int64_t G, i
         const int x = (int)(r % xn), zc = (int)(r / xn);
         const int y0 = w * 8;
         const int z_begin = zc * ZC, z_end = min(zn, z_begin + ZC);
+        /* the rows x - 1, x, x + 1 of plane zz at y0 - 4 .. y0 + 11, one 16-byte load each at any alignment
+           (x and zz clamped: the loads carry no branches, and masks() leaves out what lies outside); near
+           the row's ends only the ten cells y0 - 1 .. y0 + 8, zeros past them */
+        auto load3 = [&](int zz, uint32_t (&v)[3][4]) {
+            const int zc2 = min(max(zz, 0), zn - 1);
+            const uint8_t* rows[3];
+#pragma unroll
+            for (int k = 0; k < 3; ++k) rows[k] = P + ((int64_t)zc2 * xn + min(max(x + k - 1, 0), xn - 1)) * yn;
+            if (y0 >= 4 && y0 + 12 <= yn) {
+#pragma unroll
+                for (int k = 0; k < 3; ++k) __builtin_memcpy(v[k], rows[k] + y0 - 4, 16);
+            } else if (y0 + 8 <= yn) {
+                uint8_t l[3], r[3];
+#pragma unroll
+                for (int k = 0; k < 3; ++k) {
+                    __builtin_memcpy(&v[k][1], rows[k] + y0, 8);
+                    l[k] = rows[k][max(y0 - 1, 0)];
+                    r[k] = rows[k][min(y0 + 8, yn - 1)];
+                }
+#pragma unroll
+                for (int k = 0; k < 3; ++k) {
+                    v[k][0] = y0 > 0 ? (uint32_t)l[k] << 24 : 0u;
+                    v[k][3] = y0 + 8 < yn ? r[k] : 0u;
+                }
+            } else {
+                uint8_t c[3][9];
+#pragma unroll
+                for (int k = 0; k < 3; ++k)
+#pragma unroll
+                    for (int j = 0; j < 9; ++j) c[k][j] = rows[k][min(max(y0 - 1 + j, 0), yn - 1)];
+#pragma unroll
+                for (int k = 0; k < 3; ++k) {
+                    v[k][0] = y0 > 0 ? (uint32_t)c[k][0] << 24 : 0u;
+                    v[k][1] = v[k][2] = v[k][3] = 0u;
+#pragma unroll
+                    for (int j = 0; j < 8; ++j)
+                        if (y0 + j < yn) v[k][1 + (j >> 2)] |= (uint32_t)c[k][1 + j] << (8 * (j & 3));
+                }
+            }
+        };
         /* masks of plane zz (0 outside the volume; bit k <-> y0 - 1 + k); own row's words in own[] */
-        auto plane = [&](int zz, uint32_t& am, uint32_t& sm, uint32_t own[2]) {
+        auto masks = [&](int zz, const uint32_t (&v)[3][4], uint32_t& am, uint32_t& sm, uint32_t own[2]) {
             am = 0;
             sm = 0;
+            own[0] = v[1][1];
+            own[1] = v[1][2];
             if (zz < 0 || zz >= zn) return;
 #pragma unroll
-            for (int dx = -1; dx <= 1; ++dx) {
-                const int xx = x + dx;
-                if (xx < 0 || xx >= xn) continue;
-                const uint8_t* row = P + ((int64_t)zz * xn + xx) * yn;
-                uint32_t c[2], lf, rt;   /* the eight cells and the ones beside them */
-                if (y0 >= 4 && y0 + 12 <= yn) {   /* one 16-byte load at any alignment */
-                    uint32_t v[4];
-                    __builtin_memcpy(v, row + y0 - 4, 16);
-                    lf = v[0] >> 24;
-                    c[0] = v[1];
-                    c[1] = v[2];
-                    rt = v[3] & 0xFFu;
-                } else {
-                    lf = y0 > 0 ? row[y0 - 1] : 0u;
-                    rt = y0 + 8 < yn ? row[y0 + 8] : 0u;
-                    if (y0 + 8 <= yn) {
-                        __builtin_memcpy(c, row + y0, 8);
-                    } else {
-                        c[0] = c[1] = 0;
-#pragma unroll
-                        for (int j = 0; j < 8; ++j)
-                            if (y0 + j < yn) c[j >> 2] |= (uint32_t)row[y0 + j] << (8 * (j & 3));
-                    }
-                }
-                am |= (bits4(zero4(c[0] ^ rep4(ASC))) << 1) | (bits4(zero4(c[1] ^ rep4(ASC))) << 5) | (lf == ASC ? 1u : 0u) |
-                      (rt == ASC ? 0x200u : 0u);
-                sm |= (bits4(zero4(c[0] ^ rep4(SEED)) | zero4(c[0] ^ rep4(PROP))) << 1) |
-                      (bits4(zero4(c[1] ^ rep4(SEED)) | zero4(c[1] ^ rep4(PROP))) << 5) | (lf == SEED || lf == PROP ? 1u : 0u) |
-                      (rt == SEED || rt == PROP ? 0x200u : 0u);
-                if (dx == 0) {
-                    own[0] = c[0];
-                    own[1] = c[1];
-                }
+            for (int k = 0; k < 3; ++k) {
+                if ((k == 0 && x == 0) || (k == 2 && x == xn - 1)) continue;
+                const uint32_t lf = v[k][0] >> 24, c0 = v[k][1], c1 = v[k][2], rt = v[k][3] & 0xFFu;
+                am |= (bits4(zero4(c0 ^ rep4(ASC))) << 1) | (bits4(zero4(c1 ^ rep4(ASC))) << 5) | (lf == ASC ? 1u : 0u) | (rt == ASC ? 0x200u : 0u);
+                sm |= (bits4(zero4(c0 ^ rep4(SEED)) | zero4(c0 ^ rep4(PROP))) << 1) | (bits4(zero4(c1 ^ rep4(SEED)) | zero4(c1 ^ rep4(PROP))) << 5) |
+                      (lf == SEED || lf == PROP ? 1u : 0u) | (rt == SEED || rt == PROP ? 0x200u : 0u);
             }
         };
         uint32_t pa0, ps0, pa1, ps1, pa2, ps2;
         uint32_t cur[2] = {0, 0}, nxt[2] = {0, 0};
-        plane(z_begin - 1, pa0, ps0, nxt);
-        plane(z_begin, pa1, ps1, cur);
+        uint32_t v0[3][4], v1[3][4], v2[3][4];
+        load3(z_begin - 1, v0);
+        load3(z_begin, v1);
+        load3(z_begin + 1, v2);
+        masks(z_begin - 1, v0, pa0, ps0, nxt);
+        masks(z_begin, v1, pa1, ps1, cur);
         for (int z = z_begin; z < z_end; ++z) {
-            plane(z + 1, pa2, ps2, nxt);
+            masks(z + 1, v2, pa2, ps2, nxt);
+            if (z + 1 < z_end) load3(z + 2, v2);
             const uint32_t am = pa0 | pa1 | pa2, sm = ps0 | ps1 | ps2;
             const uint32_t ad = am | (am << 1) | (am >> 1), sd = sm | (sm << 1) | (sm >> 1);
             uint8_t* row = P + ((int64_t)z * xn + x) * yn;
