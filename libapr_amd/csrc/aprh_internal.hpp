@@ -361,6 +361,10 @@ void fill_f32(aprh_context* ctx, float* p, size_t n, float v);
 template <typename T>
 int richardson_lucy(aprh_context* ctx, aprh_apr& a, const T* in, float* u, const std::vector<HostStencil>& psf,
                     const std::vector<HostStencil>& psf_flipped, int max_iter, bool resume, double tol, double* last_rel);
+/* the piecewise-constant float image at every level l_min .. l_max (out[l], packed): the level's particles,
+   coarser particles, and the tree values where finer particles live */
+template <typename T>
+void level_images(aprh_context* ctx, const aprh_apr& a, const T* parts, const float* tree, const std::vector<float*>& out);
 /* piecewise-constant image of level `level` (l_max: APRReconstruction::reconstruct_constant);
    dtypes 0 = u16, 1 = f32 for particles (pdt) and image (idt); lev (optional): the level
    of the particle covering each pixel, as bytes */

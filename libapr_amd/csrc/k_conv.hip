@@ -9,7 +9,9 @@
  * update_lower_level, :743-849; reflective or zero ends, :384-504), summing taps
  * in (z, x, y) order (run_convolution_pencil, :705-736).
  *
- * Here one launch per level walks tiles of TX x 64 cells (x, y) through a run of
+ * Cubic stencils: k_conv_dense over dense images of all levels (see there).
+ *
+ * Other stencils (k_conv_tile): one launch per level walks tiles of TX x 64 cells (x, y) through a run of
  * z planes.  For each plane the block assembles the tile and its halo in LDS:
  *   1. the coarser level's image V(l-1) upsampled (every cell not covered by a
  *      level-l particle or tree node lies inside a coarser particle),
@@ -464,311 +466,243 @@ __global__ __launch_bounds__(CT) void k_conv_tile(ConvArgs<TIn> a) {
     }
 }
 
-/* smallest power of two above n */
-constexpr int pow2_above(int n) {
-    int p = 1;
-    while (p <= n) p <<= 1;
-    return p;
-}
+/* ---- convolution of dense level images ----
+ * Cubic stencils of up to 13 taps a side run over the level images that level_images() makes in one launch
+ * (k_conv_tile assembles its windows from particle rows instead, level after level).  A block takes 16
+ * x-rows x 64 y and marches through a run of z planes.  Each plane's window comes from the image with plain
+ * coalesced loads issued one plane ahead; reflected ends are taken from the reflected row, column or
+ * plane.  Each thread owns one y in four rows:
+ *   - reference order: a plane's values meet the stencil's taps of every output plane they belong to, in
+ *     (x, y) order, in one accumulator per output plane; planes arrive in z order, so each sum runs in the
+ *     reference's (z, x, y) order, multiply then add, and a value read from LDS serves S taps;
+ *   - separable (SEP): the y pass into LDS, the x pass into the registers, which hold the last S planes,
+ *     and the z pass there.
+ * A row's particles in the 64 cells are at most 64: one lane each fetches its result from the lane of its
+ * y.  Their rows are looked up one plane ahead, and their y and epilogue inputs are loaded before the
+ * plane's arithmetic.  What bounds it: the reference order its multiplies and adds (2 S^3 a cell: 125 taps
+ * over 1000 x 1024 x 250, 1.6 ms of them), the separable form instruction issue and the latency left
+ * between two barriers a plane.  Levels of one stencil size share a launch.  With windows assembled from
+ * the particle rows in every block, level after level: 5x5x5 in reference order on 1000 x 1024 x 250 6.7 ms
+ * for the levels' launches, now 2.05 and 0.74 for the images; 9x9x9 separable on 1024 x 1024 x 256 3.2 ms,
+ * now 1.45 and 0.77; 3x3x3 on 256 x 256 x 128 0.39 ms in eight launches, now 0.047 and 0.036. */
+constexpr int CONV_LEVELS = 24;
+struct DenseLevel {
+    int64_t Y, X, Z;
+    int64_t row_begin;            /* xz_end index of row (z=0, x=0)                        */
+    int64_t yidx_off;
+    const float* V;
+    int nyb, ntx, ntz, zc;
+    int64_t w_off;                /* weights: reference order S^3; separable fy|fx|fz      */
+    int64_t block0;               /* first block of the launch                             */
+};
+struct DenseArgs {
+    int n;
+    DenseLevel L[CONV_LEVELS];
+    const uint64_t* xz_end;
+    const uint16_t* y_vec;
+    const uint16_t* yidx;
+    const float* W;
+    float* out;
+    const void* epi_in;
+    double* part;
+    int reflect, epi_in_u16;
+};
 
-/* Separable mode with the z pass in registers.  Each thread owns one y (its lane) in TX / 4
-   rows of the tile and keeps the x-passed values of the last SZ planes of those cells in
-   registers; a per-plane map from interior cells to their particle (offset in the row's block,
-   0xFF for none) sits in an LDS ring of SZ + 1 planes, so the tile needs no LDS ring of planes
-   and more blocks fit on a CU.  Per plane: assemble the window (as k_conv_tile), y pass into A,
-   x pass into the registers, and the outputs of plane z - hz at the cells that hold particles. */
-template <typename TIn, int TX, int SZ, int EPI, bool TOP>
-__global__ __launch_bounds__(CT) void k_conv_sep(ConvArgs<TIn> a) {
-    extern __shared__ __align__(16) uint8_t smem[];
-    constexpr int SZR = SZ + 1;
-    constexpr int HZ = (SZ - 1) / 2;
-    constexpr int RPT = TX / NWAVE;
-    const LevelDesc& L = a.L;
-    constexpr int hy = HZ, hx = HZ;
-    constexpr int WX = TX + 2 * hx, WY = TY + 2 * hy, WYS = WY;
-    uint8_t* p = smem;
-    uint64_t* sbase = (uint64_t*)p;      /* SZR x TX: first particle of each interior row's block */
-    p += (size_t)SZR * TX * 8;
-    uint64_t* mlo = (uint64_t*)p;        /* 2 WX */
-    p += (size_t)2 * WX * 8;
-    /* exclusive prefix of the window rows' load counts, then the total, then INT_MAX up to a
-       power of two: the row search runs a fixed number of steps */
-    constexpr int NPM = pow2_above(2 * WX);
-    int* mpre = (int*)p;                 /* NPM + 2 */
-    p += (size_t)(NPM + 2) * 4;
-    float* V = (float*)p;                /* WX x WYS */
-    p += (size_t)WX * WYS * 4;
-    float* Ab = (float*)p;               /* WX x TY */
-    p += (size_t)WX * TY * 4;
-    int32_t* cxo = (int32_t*)p;          /* WX: coarse-plane offset of each window row, -1 none */
-    p += (size_t)((WX + 3) & ~3) * 4;
-    uint8_t* pidx = p;                   /* SZR x TX x TY */
-
-    const int64_t ntiles = (int64_t)L.ntx * L.nty * L.ntz;
-    const int64_t tile = xcd_block(blockIdx.x, gridDim.x);
-    if (tile >= ntiles) return;
-    /* y tiles fastest: consecutive blocks (one XCD's run) cover whole rows, so the partial
-       cache lines of a row's particle chunks meet in one L2 */
-    const int ty = (int)(tile % L.nty);
-    const int tx = (int)((tile / L.nty) % L.ntx);
-    const int tz = (int)(tile / ((int64_t)L.ntx * L.nty));
+template <int S, bool SEP, int EPI>
+__global__ __launch_bounds__(CT) void k_conv_dense(DenseArgs a) {
+    constexpr int H = (S - 1) / 2, TX = 16, WX = TX + 2 * H, WY = TY + 2 * H, RPT = TX / NWAVE;
+    constexpr int RW = (WX + NWAVE - 1) / NWAVE;            /* window rows per wave            */
+    constexpr int NT = (2 * H * WX + CT - 1) / CT;          /* columns 64 .. per thread        */
+    constexpr int NTA = NT > 0 ? NT : 1;
+    __shared__ float win[SEP ? 1 : 2][WX * WY];
+    __shared__ float ypass[SEP ? WX * TY : 1];
+    __shared__ double red[EPI == 2 ? 2 * CT : 1];
+    const int64_t t = xcd_block(blockIdx.x, gridDim.x);
+    int li = 0;
+    while (li + 1 < a.n && t >= a.L[li + 1].block0) ++li;
+    const DenseLevel& L = a.L[li];
+    /* y tiles fastest: consecutive blocks (one XCD's run) cover whole rows */
+    const int64_t tile = t - L.block0;
+    const int ty = (int)(tile % L.nyb);
+    const int64_t tr = tile / L.nyb;
+    const int tx = (int)(tr % L.ntx), tz = (int)(tr / L.ntx);
+    const int64_t X = L.X, Y = L.Y, Z = L.Z;
     const int64_t x0 = (int64_t)tx * TX, y0 = (int64_t)ty * TY;
-    const int yb0 = ty;
-    const int64_t z_lo = (int64_t)tz * L.zc, z_hi = min(z_lo + L.zc, L.Z);
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    float fy[SZ], fx[SZ], fz[SZ];
-    {
-        const CWeights w = (CWeights)(a.W + L.w_off);
+    const int64_t z_lo = (int64_t)tz * L.zc, z_hi = min(z_lo + L.zc, Z);
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const CWeights w = (CWeights)(a.W + L.w_off);
+    const bool reflect = a.reflect != 0;
+
+    /* where the window's values come from within a plane: this lane's column and the wave's rows, then the
+       threads' columns past the 64th (offsets below 2^32: dims are at most 65535); NONE reads 0 */
+    constexpr uint32_t NONE = 0xFFFFFFFFu;
+    auto source = [&](int64_t q, int64_t n) -> uint32_t { return reflect ? (uint32_t)refl_c(q, n) : (q >= 0 && q < n) ? (uint32_t)q : NONE; };
+    const uint32_t col = source(y0 - H + lane, Y);
+    uint32_t row[RW], tail[NTA];
 #pragma unroll
-        for (int k = 0; k < SZ; ++k) {
+    for (int k = 0; k < RW; ++k) {
+        const uint32_t xs = source(x0 - H + wv + NWAVE * k, X);
+        row[k] = xs == NONE ? NONE : xs * (uint32_t)Y;
+    }
+#pragma unroll
+    for (int k = 0; k < NT; ++k) {
+        const int e = threadIdx.x + CT * k, xw = e / (2 * H > 0 ? 2 * H : 1), yw = 64 + e - xw * 2 * H;
+        const uint32_t xs = xw < WX ? source(x0 - H + xw, X) : NONE, ys = source(y0 - H + yw, Y);
+        tail[k] = xs == NONE || ys == NONE ? NONE : xs * (uint32_t)Y + ys;
+    }
+    float main_v[RW], tail_v[NTA];
+    auto load = [&](int64_t zq) {
+        const bool in = reflect || (zq >= 0 && zq < Z);
+        const float* p = L.V + (in ? (reflect ? refl_c(zq, Z) : zq) : 0) * X * Y;
+#pragma unroll
+        for (int k = 0; k < RW; ++k) main_v[k] = (in && col != NONE && row[k] != NONE) ? p[row[k] + col] : 0.0f;
+#pragma unroll
+        for (int k = 0; k < NT; ++k) tail_v[k] = (in && tail[k] != NONE) ? p[tail[k]] : 0.0f;
+    };
+    /* lane j < RPT of each wave: the particles of row wv + 4 j of plane z in this block's 64 cells */
+    uint64_t pb = 0;
+    int pc = 0;
+    auto lookup = [&](int64_t z) {
+        pc = 0;
+        const int64_t x = x0 + wv + NWAVE * lane;
+        if (lane < RPT && x < X && z >= z_lo && z < z_hi) {
+            const int64_t r = z * X + x;
+            uint64_t b, e, s0, s1;
+            row_block(a.xz_end, a.yidx + L.yidx_off, r, L.nyb, L.row_begin + r, ty, b, e, s0, s1);
+            pb = s0;
+            pc = (int)(s1 - s0);
+        }
+    };
+    float fy[SEP ? S : 1], fx[SEP ? S : 1], fz[SEP ? S : 1];
+    if constexpr (SEP) {
+#pragma unroll
+        for (int k = 0; k < S; ++k) {
             fy[k] = w[k];
-            fx[k] = w[SZ + k];
-            fz[k] = w[2 * SZ + k];
+            fx[k] = w[S + k];
+            fz[k] = w[2 * S + k];
         }
     }
-    constexpr int nmd = TOP ? WX : 2 * WX;   /* window rows looked up: particle rows, tree rows */
-    constexpr int NP = pow2_above(nmd);
-    for (int t = nmd + 1 + threadIdx.x; t < NP; t += CT) mpre[t] = 0x7FFFFFFF;
-
-    /* plane-invariant coarse geometry: each window row's offset in a coarse plane (LDS), and
-       this lane's two window columns' coarse y (-1 outside the level) */
-    for (int t = threadIdx.x; t < WX; t += CT) {
-        const int64_t x = x0 - hx + t;
-        const bool ok = a.coarse && (a.reflect || (x >= 0 && x < L.X));
-        cxo[t] = ok ? (int32_t)(((a.reflect ? refl_c(x, L.X) : x) >> 1) * L.cY) : -1;
-    }
-    int32_t cyo[2];
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-        const int yw = lane + 64 * h;
-        const int64_t y = y0 - hy + yw;
-        cyo[h] = (yw < WY && y >= 0 && y < L.Y) ? (int32_t)(y >> 1) : -1;
-    }
-    const int64_t cplane = L.cX * L.cY;
-    __syncthreads();
-
-    double n1 = 0.0, n2 = 0.0;
-    float breg[RPT][SZ];
+    /* SEP: the x-passed values of the last S planes; else the sums of the S output planes in progress,
+       acc[j][k] having met the stencil's planes 0 .. k - 1 */
+    float acc[RPT][S];
 #pragma unroll
     for (int j = 0; j < RPT; ++j)
 #pragma unroll
-        for (int k = 0; k < SZ; ++k) breg[j][k] = 0.0f;
+        for (int k = 0; k < S; ++k) acc[j][k] = 0.0f;
+    double n1 = 0.0, n2 = 0.0;
 
-    const int64_t nq = (z_hi - z_lo) + 2 * HZ;
-    for (int64_t q = 0; q < nq; ++q) {
-        const int64_t zq = z_lo - HZ + q;
-        const int slot = (int)(q % SZR);
-        uint8_t* pid = pidx + (size_t)slot * TX * TY;
-        uint64_t* bs = sbase + (size_t)slot * TX;
-        const bool zin = zq >= 0 && zq < L.Z;
-        const bool plane_zero = !a.reflect && !zin;
-        const int64_t zs = a.reflect ? refl_c(zq, L.Z) : zq;
-        /* 1. wave 0: row lookups and the exclusive prefix of the load counts; every thread:
-           clear this plane's particle map; all waves: the coarse image under the window */
-        for (int c = threadIdx.x * 8; c < TX * TY; c += CT * 8) *(uint64_t*)(pid + c) = ~(uint64_t)0;
-        if (wv == 0) {
-            int carry = 0;
-            for (int t0 = 0; t0 < nmd; t0 += 64) {
-                const int t = t0 + lane;
-                uint64_t lo = 0;
-                int n = 0;
-                if (t < nmd) {
-                    const bool trow = t >= WX;
-                    const int xw = trow ? t - WX : t;
-                    const int64_t x = x0 - hx + xw;
-                    const bool xin = x >= 0 && x < L.X;
-                    const bool interior = !trow && xw >= hx && xw < hx + TX;
-                    if (!(plane_zero || (!a.reflect && !xin) || (trow && (TOP || L.t_row_begin < 0)))) {
-                        const int64_t xs = a.reflect ? refl_c(x, L.X) : x;
-                        const int64_t row = zs * L.X + xs;
-                        uint64_t b, e, s0, s1;
-                        if (TOP || !trow) row_block(a.xz_end, a.yidx + L.yidx_off, row, L.nyb, L.row_begin + row, yb0, b, e, s0, s1);
-                        else row_block(a.t_xz_end, a.t_yidx + L.t_yidx_off, row, L.nyb, L.t_row_begin + row, yb0, b, e, s0, s1);
-                        lo = (s0 - b > (uint64_t)hy) ? s0 - hy : b;
-                        const uint64_t hi = (e - s1 > (uint64_t)hy) ? s1 + hy : e;
-                        n = (int)(hi - lo);
-                        /* interior rows of planes inside the level list their block's particles */
-                        if (interior) bs[xw - hx] = (zin && xin) ? s0 : ~(uint64_t)0;
-                    } else if (interior) {
-                        bs[xw - hx] = ~(uint64_t)0;
-                    }
-                    mlo[t] = lo;
-                }
-                int inc = n;
+    const int nq = (int)(z_hi - z_lo) + 2 * H;
+    load(z_lo - H);
+    lookup(z_lo - 2 * H);
+    for (int q = 0; q < nq; ++q) {
+        const int64_t zq = z_lo - H + q;
+        float* V = win[SEP ? 0 : q & 1];
 #pragma unroll
-                for (int o = 1; o < 64; o <<= 1) {
-                    const int u = __shfl_up(inc, o, 64);
-                    if (lane >= o) inc += u;
-                }
-                if (t < nmd) mpre[t] = carry + inc - n;
-                carry += __shfl(inc, 63, 64);
-            }
-            if (lane == 0) mpre[nmd] = carry;
-        }
-        /* the coarse image under the window: a wave per window row, lanes along y (a second
-           pass for the y halo beyond 64 cells), four rows' loads in flight before their stores;
-           offsets within the coarse plane come from the plane-invariant tables */
-        const float* cpl = (plane_zero || !a.coarse) ? nullptr : a.coarse + (zs >> 1) * cplane;
-        for (int xb = wv; xb < WX; xb += 4 * NWAVE) {
-            float cv[4][2];
+        for (int k = 0; k < RW; ++k)
+            if (WX % NWAVE == 0 || wv + NWAVE * k < WX) V[(wv + NWAVE * k) * WY + lane] = main_v[k];
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const int xw = xb + u * NWAVE;
-                const int32_t xo = (cpl && xw < WX) ? cxo[xw] : -1;
-#pragma unroll
-                for (int h = 0; h < 2; ++h) cv[u][h] = (xo >= 0 && cyo[h] >= 0) ? cpl[xo + cyo[h]] : 0.0f;
-            }
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const int xw = xb + u * NWAVE;
-                if (xw >= WX) break;
-                V[xw * WYS + lane] = cv[u][0];
-                if (lane + 64 < WY) V[xw * WYS + lane + 64] = cv[u][1];
-            }
+        for (int k = 0; k < NT; ++k) {
+            const int e = threadIdx.x + CT * k, xw = e / (2 * H > 0 ? 2 * H : 1);
+            if (xw < WX) V[xw * WY + 64 + e - xw * 2 * H] = tail_v[k];
         }
         __syncthreads();
-        /* 2. particles and tree nodes of the level over the coarse image; interior particles of
-           planes inside the level enter the plane's particle map */
-        {
-            const int total = mpre[nmd];
-            for (int k0 = threadIdx.x; k0 < total; k0 += 4 * CT) {
-                int rr[4];
-                uint64_t ii[4];
-                int yy[4];
-                float vv[4];
-#pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                    const int k = k0 + u * CT;
-                    /* the last row r with mpre[r] <= k, in log2(NP) fixed steps */
-                    int lo = 0;
-#pragma unroll
-                    for (int st = NP / 2; st >= 1; st >>= 1)
-                        if (mpre[lo + st] <= k) lo += st;
-                    rr[u] = k < total ? lo : -1;
-                    ii[u] = k < total ? mlo[lo] + (uint64_t)(k - mpre[lo]) : 0;
-                }
-#pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                    if (rr[u] < 0) continue;
-                    if (TOP || rr[u] < WX) {
-                        yy[u] = a.y_vec[ii[u]];
-                        vv[u] = tof(a.in[ii[u]]);
-                    } else {
-                        yy[u] = a.t_y_vec[ii[u]];
-                        vv[u] = a.tree[ii[u]];
-                    }
-                }
-#pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                    if (rr[u] < 0) continue;
-                    const int xw = rr[u] < WX ? rr[u] : rr[u] - WX;
-                    const int yw = yy[u] - (int)(y0 - hy);
-                    if (yw >= 0 && yw < WY) V[xw * WYS + yw] = vv[u];
-                    if (rr[u] < WX && xw >= hx && xw < hx + TX) {
-                        const uint64_t b0 = bs[xw - hx];
-                        const uint64_t d = ii[u] - b0;
-                        const int yo = yy[u] - (int)y0;
-                        if (b0 != ~(uint64_t)0 && d < (uint64_t)TY && yo >= 0 && yo < TY) pid[(xw - hx) * TY + yo] = (uint8_t)d;
-                    }
-                }
-            }
-        }
-        __syncthreads();
-        /* 3. y ends: mirror inside the window */
-        if (a.reflect && (y0 - hy < 0 || y0 + TY + hy > L.Y)) {
-            for (int xw = wv; xw < WX; xw += NWAVE) {
-                float* vrow = V + xw * WYS;
-                for (int yw = lane; yw < WY; yw += 64) {
-                    const int64_t y = y0 - hy + yw;
-                    if ((y < 0 || y >= L.Y) && y < L.Y + hy) {
-                        const int64_t src = refl_c(y, L.Y) - (y0 - hy);
-                        if (src >= 0 && src < WY) vrow[yw] = vrow[src];
-                    }
-                }
-            }
-            __syncthreads();
-        }
-        /* the assembled interior is the next level's coarse image */
-        if (!TOP && a.vout && zq >= z_lo && zq < z_hi) {
-            for (int r = wv; r < TX; r += NWAVE) {
-                const int64_t x = x0 + r;
-                const int64_t y = y0 + lane;
-                if (x < L.X && y < L.Y) a.vout[(zq * L.X + x) * L.Y + y] = V[(r + hx) * WYS + hy + lane];
-            }
-        }
-        /* 4. y pass of every window row */
-        for (int xw = wv; xw < WX; xw += NWAVE) {
-            const float* vrow = V + xw * WYS + lane;
-            float acc = 0.0f;
-#pragma unroll
-            for (int k = 0; k < SZ; ++k) acc = fmaf(fy[k], vrow[k], acc);
-            Ab[xw * TY + lane] = acc;
-        }
-        __syncthreads();
-        /* 5. x pass of the thread's rows into the register ring; then the outputs of plane
-           zq - HZ, whose z neighbourhood is now in the ring */
-        const bool emit = q >= 2 * HZ;
-        const int oslot = (int)((q - HZ + SZR) % SZR);
-        const uint8_t* opid = pidx + (size_t)oslot * TX * TY;
-        const uint64_t* obs = sbase + (size_t)oslot * TX;
+        if (q + 1 < nq) load(zq + 1);
+        /* the particles of output plane zq - H, looked up in the previous step */
+        const bool emit = q >= 2 * H;
+        uint64_t ob[RPT];
+        int oc[RPT], oy[RPT];
+        float ov[RPT];
 #pragma unroll
         for (int j = 0; j < RPT; ++j) {
-            const int r = wv + j * NWAVE;
-            float acc = 0.0f;
-#pragma unroll
-            for (int k = 0; k < SZ; ++k) acc = fmaf(fx[k], Ab[(r + k) * TY + lane], acc);
-#pragma unroll
-            for (int k = 0; k + 1 < SZ; ++k) breg[j][k] = breg[j][k + 1];
-            breg[j][SZ - 1] = acc;
+            ob[j] = ((uint64_t)__builtin_amdgcn_readlane((int)(pb >> 32), j) << 32) | (uint32_t)__builtin_amdgcn_readlane((int)pb, j);
+            oc[j] = emit ? __builtin_amdgcn_readlane(pc, j) : 0;
+            oy[j] = 0;
+            ov[j] = 0.0f;
+            if (lane < oc[j]) {
+                const uint64_t i = ob[j] + (uint64_t)lane;
+                oy[j] = a.y_vec[i];
+                if constexpr (EPI == 1) ov[j] = a.epi_in_u16 ? (float)((const uint16_t*)a.epi_in)[i] : ((const float*)a.epi_in)[i];
+                if constexpr (EPI == 2) ov[j] = a.out[i];
+            }
         }
-        if (emit) {
-            uint64_t oi[RPT];
-            float ov[RPT];
-            bool on[RPT];
+        lookup(zq + 1 - H);
+        float val[RPT];
+        if constexpr (SEP) {
+#pragma unroll
+            for (int k = 0; k < RW; ++k) {
+                const int xw = wv + NWAVE * k;
+                if (WX % NWAVE != 0 && xw >= WX) break;
+                const float* v = V + xw * WY + lane;
+                float s = 0.0f;
+#pragma unroll
+                for (int i = 0; i < S; ++i) s = fmaf(fy[i], v[i], s);
+                ypass[xw * TY + lane] = s;
+            }
+            __syncthreads();
 #pragma unroll
             for (int j = 0; j < RPT; ++j) {
-                const int r = wv + j * NWAVE;
-                const int d = opid[r * TY + lane];
-                on[j] = d != 0xFF;
-                oi[j] = on[j] ? obs[r] + (uint64_t)d : 0;
-                float val = 0.0f;
-                if (on[j]) {
+                const float* v = ypass + (wv + NWAVE * j) * TY + lane;
+                float s = 0.0f;
 #pragma unroll
-                    for (int k = 0; k < SZ; ++k) val = fmaf(fz[k], breg[j][k], val);
-                }
-                ov[j] = val;
+                for (int i = 0; i < S; ++i) s = fmaf(fx[i], v[i * TY], s);
+#pragma unroll
+                for (int k = 0; k + 1 < S; ++k) acc[j][k] = acc[j][k + 1];
+                acc[j][S - 1] = s;
+                val[j] = 0.0f;
             }
-            if constexpr (EPI == 0) {
+            if (emit) {
 #pragma unroll
                 for (int j = 0; j < RPT; ++j)
-                    if (on[j]) a.out[oi[j]] = ov[j];
-            } else if constexpr (EPI == 1) {
-                float num[RPT];
+#pragma unroll
+                    for (int k = 0; k < S; ++k) val[j] = fmaf(fz[k], acc[j][k], val[j]);
+            }
+        } else {
+#pragma unroll 1
+            for (int ix = 0; ix < S; ++ix) {
+                float v[RPT][S];
 #pragma unroll
                 for (int j = 0; j < RPT; ++j)
-                    num[j] = on[j] ? (a.epi_in_u16 ? (float)((const uint16_t*)a.epi_in)[oi[j]] : ((const float*)a.epi_in)[oi[j]]) : 1.0f;
 #pragma unroll
-                for (int j = 0; j < RPT; ++j)
-                    if (on[j]) a.out[oi[j]] = num[j] / ov[j];
-            } else {
-                float uo[RPT];
+                    for (int i = 0; i < S; ++i) v[j][i] = V[(wv + NWAVE * j + ix) * WY + lane + i];
 #pragma unroll
-                for (int j = 0; j < RPT; ++j) uo[j] = on[j] ? a.out[oi[j]] : 0.0f;
+                for (int i = 0; i < S; ++i)
 #pragma unroll
-                for (int j = 0; j < RPT; ++j)
-                    if (on[j]) {
-                        const float nu = uo[j] * ov[j];
-                        const double d = (double)nu - (double)uo[j];
-                        n1 += d * d;
-                        n2 += (double)uo[j] * (double)uo[j];
-                        a.out[oi[j]] = nu;
+                    for (int k = 0; k < S; ++k) {
+                        const float wk = w[(k * S + ix) * S + i];
+#pragma unroll
+                        for (int j = 0; j < RPT; ++j) acc[j][k] += v[j][i] * wk;
                     }
+            }
+#pragma unroll
+            for (int j = 0; j < RPT; ++j) {
+                val[j] = acc[j][S - 1];
+#pragma unroll
+                for (int k = S - 1; k > 0; --k) acc[j][k] = acc[j][k - 1];
+                acc[j][0] = 0.0f;
+            }
+        }
+        if (emit) {
+#pragma unroll
+            for (int j = 0; j < RPT; ++j) {
+                const float r = __shfl(val[j], (oy[j] - (int)y0) & 63, 64);
+                if (lane < oc[j]) {
+                    const uint64_t i = ob[j] + (uint64_t)lane;
+                    if constexpr (EPI == 0) {
+                        a.out[i] = r;
+                    } else if constexpr (EPI == 1) {
+                        a.out[i] = ov[j] / r;
+                    } else {
+                        const float nu = ov[j] * r;
+                        const double d = (double)nu - (double)ov[j];
+                        n1 += d * d;
+                        n2 += (double)ov[j] * (double)ov[j];
+                        a.out[i] = nu;
+                    }
+                }
             }
         }
     }
     if constexpr (EPI == 2) {
-        __syncthreads();
-        double* red = (double*)smem;
         red[threadIdx.x] = n1;
         red[CT + threadIdx.x] = n2;
         __syncthreads();
@@ -784,13 +718,6 @@ __global__ __launch_bounds__(CT) void k_conv_sep(ConvArgs<TIn> a) {
             a.part[2 * (int64_t)blockIdx.x + 1] = red[CT];
         }
     }
-}
-
-size_t conv_sep_lds_bytes(int tx, int sy, int sx, int sz) {
-    const int WX = tx + (sx - 1), WYS = TY + (sy - 1), SZR = sz + 1;
-    size_t b = (size_t)SZR * tx * 8 + (size_t)2 * WX * 8 + (size_t)(pow2_above(2 * WX) + 2) * 4 + (size_t)WX * WYS * 4 + (size_t)WX * TY * 4 +
-               (size_t)((WX + 3) & ~3) * 4 + (size_t)SZR * tx * TY;
-    return std::max<size_t>(b, 2 * CT * sizeof(double));
 }
 
 size_t conv_lds_bytes(int tx, bool sep, int sy, int sx, int sz) {
@@ -978,51 +905,33 @@ void launch_conv_tile(const ConvArgs<TIn>& args, unsigned grid, size_t lds, hipS
     HIP_LAUNCH_CHECK();
 }
 
-template <typename TIn, int TX, int SZ, int EPI, bool TOP>
-void launch_conv_sep_k(const ConvArgs<TIn>& args, unsigned grid, size_t lds, hipStream_t st) {
-    if (lds > 65536)
-        (void)hipFuncSetAttribute((const void*)k_conv_sep<TIn, TX, SZ, EPI, TOP>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    hipLaunchKernelGGL((k_conv_sep<TIn, TX, SZ, EPI, TOP>), dim3(grid), dim3(CT), lds, st, args);
+template <int S, bool SEP>
+void launch_conv_dense_s(const DenseArgs& d, int epi, unsigned grid, hipStream_t st) {
+    if (epi == 0) hipLaunchKernelGGL((k_conv_dense<S, SEP, 0>), dim3(grid), dim3(CT), 0, st, d);
+    else if (epi == 1) hipLaunchKernelGGL((k_conv_dense<S, SEP, 1>), dim3(grid), dim3(CT), 0, st, d);
+    else hipLaunchKernelGGL((k_conv_dense<S, SEP, 2>), dim3(grid), dim3(CT), 0, st, d);
     HIP_LAUNCH_CHECK();
 }
-
-/* the variant for the launch's epilogue and level: the finest level has no tree nodes and no
-   next-level image; u16 particles only ever feed the plain store */
-template <typename TIn, int TX, int SZ>
-void launch_conv_sep_tile(const ConvArgs<TIn>& a, unsigned grid, size_t lds, hipStream_t st) {
-    const bool top = a.L.t_row_begin < 0 && a.vout == nullptr;
-    if constexpr (std::is_same<TIn, uint16_t>::value) {
-        if (a.epi != 0) throw Error(APRH_ERR_UNSUPPORTED, "convolution epilogue needs float particles");
-        if (top) launch_conv_sep_k<TIn, TX, SZ, 0, true>(a, grid, lds, st);
-        else launch_conv_sep_k<TIn, TX, SZ, 0, false>(a, grid, lds, st);
-    } else {
-        switch (a.epi * 2 + (top ? 1 : 0)) {
-            case 0: launch_conv_sep_k<TIn, TX, SZ, 0, false>(a, grid, lds, st); break;
-            case 1: launch_conv_sep_k<TIn, TX, SZ, 0, true>(a, grid, lds, st); break;
-            case 2: launch_conv_sep_k<TIn, TX, SZ, 1, false>(a, grid, lds, st); break;
-            case 3: launch_conv_sep_k<TIn, TX, SZ, 1, true>(a, grid, lds, st); break;
-            case 4: launch_conv_sep_k<TIn, TX, SZ, 2, false>(a, grid, lds, st); break;
-            default: launch_conv_sep_k<TIn, TX, SZ, 2, true>(a, grid, lds, st); break;
-        }
+void launch_conv_dense(const DenseArgs& d, int S, bool sep, int epi, unsigned grid, hipStream_t st) {
+    switch (sep ? S : -S) {
+        case 1: launch_conv_dense_s<1, true>(d, epi, grid, st); return;
+        case 3: launch_conv_dense_s<3, true>(d, epi, grid, st); return;
+        case 5: launch_conv_dense_s<5, true>(d, epi, grid, st); return;
+        case 7: launch_conv_dense_s<7, true>(d, epi, grid, st); return;
+        case 9: launch_conv_dense_s<9, true>(d, epi, grid, st); return;
+        case 11: launch_conv_dense_s<11, true>(d, epi, grid, st); return;
+        case 13: launch_conv_dense_s<13, true>(d, epi, grid, st); return;
+        case -3: launch_conv_dense_s<3, false>(d, epi, grid, st); return;
+        case -5: launch_conv_dense_s<5, false>(d, epi, grid, st); return;
+        case -7: launch_conv_dense_s<7, false>(d, epi, grid, st); return;
+        case -9: launch_conv_dense_s<9, false>(d, epi, grid, st); return;
+        default: throw Error(APRH_ERR_UNSUPPORTED, "dense convolution: stencil size not instantiated");
     }
 }
-
-template <typename TIn, int TX>
-void launch_conv_sep_sz(const ConvArgs<TIn>& ca, unsigned grid, size_t lds, hipStream_t st) {
-    switch (ca.L.sz) {
-        case 1: launch_conv_sep_tile<TIn, TX, 1>(ca, grid, lds, st); return;
-        case 3: launch_conv_sep_tile<TIn, TX, 3>(ca, grid, lds, st); return;
-        case 5: launch_conv_sep_tile<TIn, TX, 5>(ca, grid, lds, st); return;
-        case 7: launch_conv_sep_tile<TIn, TX, 7>(ca, grid, lds, st); return;
-        case 9: launch_conv_sep_tile<TIn, TX, 9>(ca, grid, lds, st); return;
-        case 11: launch_conv_sep_tile<TIn, TX, 11>(ca, grid, lds, st); return;
-        case 13: launch_conv_sep_tile<TIn, TX, 13>(ca, grid, lds, st); return;
-        default: throw Error(APRH_ERR_UNSUPPORTED, "register z ring: stencil depth not instantiated");
-    }
+/* stencils the dense kernel is compiled for */
+bool dense_size(const HostStencil& s, bool sep) {
+    return s.sy == s.sz && s.sx == s.sz && (s.sz & 1) && (sep ? s.sz <= 13 : s.sz >= 3 && s.sz <= 9);
 }
-
-/* z sizes with a register-ring separable kernel */
-bool sep_regz_size(int sz) { return sz >= 1 && sz <= 13 && (sz & 1); }
 
 /* the kernel for one level: separable or reference order, tile width, unrolled y taps */
 template <typename TIn>
@@ -1075,6 +984,94 @@ void conv_levels(aprh_context* ctx, aprh_apr& a, const std::vector<HostStencil>&
     }
     Buf W(ctx->pool, flat.size() * 4);
     HIP_CHECK(hipMemcpyAsync(W.ptr(), flat.data(), flat.size() * 4, hipMemcpyHostToDevice, st));
+    auto stencil_of = [&](int l) { return (size_t)std::min((int)stencils.size() - 1, a.l_max - l); };
+    /* the block partials of `blocks` more blocks in *part */
+    auto grow_parts = [&](int64_t blocks) -> double* {
+        if (epi != 2) return nullptr;
+        const int64_t need = (*nparts) + blocks;
+        if ((int64_t)(part->bytes() / 16) < need) {
+            Buf nb(ctx->pool, (size_t)need * 16);
+            if (*nparts > 0) HIP_CHECK(hipMemcpyAsync(nb.ptr(), part->ptr(), (size_t)(*nparts) * 16, hipMemcpyDeviceToDevice, st));
+            *part = std::move(nb);
+        }
+        double* p = part->as<double>() + 2 * (*nparts);
+        *nparts = need;
+        return p;
+    };
+    bool dense = a.l_max - a.l_min < CONV_LEVELS;
+    for (int l = a.l_min; l <= a.l_max; ++l) dense = dense && dense_size(stencils[stencil_of(l)], off_sep[stencil_of(l)] >= 0);
+    if (dense) {
+        /* the images of all levels, then one launch per stencil form and size, the finest level first */
+        std::vector<float*> img((size_t)a.l_max + 1, nullptr);
+        int64_t total = 0;
+        std::vector<int64_t> at((size_t)a.l_max + 1, 0);
+        for (int l = a.l_min; l <= a.l_max; ++l) {
+            at[(size_t)l] = total;
+            total += cdiv(a.y_num[l] * a.x_num[l] * a.z_num[l], 64) * 64;
+        }
+        Buf V(ctx->pool, (size_t)total * 4);
+        for (int l = a.l_min; l <= a.l_max; ++l) img[(size_t)l] = V.as<float>() + at[(size_t)l];
+        level_images<T>(ctx, a, in, tree, img);
+        DenseArgs d;
+        std::memset(&d, 0, sizeof(d));
+        d.xz_end = a.xz_end.as<uint64_t>();
+        d.y_vec = a.y_vec.as<uint16_t>();
+        d.yidx = a.yidx.as<uint16_t>();
+        d.W = W.as<float>();
+        d.out = out;
+        d.epi_in = epi_in;
+        d.reflect = reflect ? 1 : 0;
+        d.epi_in_u16 = epi_u16 ? 1 : 0;
+        std::vector<bool> done((size_t)a.l_max + 1, false);
+        struct Group {
+            DenseArgs d;
+            int S;
+            bool sep;
+            int64_t blocks;
+        };
+        std::vector<Group> groups;
+        int64_t all = 0;
+        for (int first = a.l_max; first >= a.l_min; --first) {
+            if (done[(size_t)first]) continue;
+            Group g{d, stencils[stencil_of(first)].sz, off_sep[stencil_of(first)] >= 0, 0};
+            for (int l = first; l >= a.l_min; --l) {
+                const size_t sn = stencil_of(l);
+                if (done[(size_t)l] || stencils[sn].sz != g.S || (off_sep[sn] >= 0) != g.sep) continue;
+                done[(size_t)l] = true;
+                DenseLevel& L = g.d.L[g.d.n];
+                L.Y = a.y_num[l];
+                L.X = a.x_num[l];
+                L.Z = a.z_num[l];
+                L.row_begin = (int64_t)a.level_xz_vec[l];
+                L.yidx_off = a.yidx_off[l];
+                L.V = img[(size_t)l];
+                L.nyb = nyb_of(L.Y);
+                L.ntx = (int)cdiv(L.X, 16);
+                L.w_off = g.sep ? off_sep[sn] : off_exact[sn];
+                const int64_t nxy = (int64_t)L.ntx * L.nyb;
+                if (nxy == 0 || L.Z == 0) continue;
+                /* about 4096 blocks, in runs of at least twice the stencil's halo planes: a run reads its
+                   halo too, and a block marches its planes one after another */
+                const int64_t H2 = g.S - 1;
+                L.zc = (int)std::max<int64_t>(1, std::min(L.Z, std::max(cdiv(L.Z * nxy, 4096), 2 * H2)));
+                L.ntz = (int)cdiv(L.Z, L.zc);
+                L.block0 = g.blocks;
+                g.blocks += nxy * L.ntz;
+                ++g.d.n;
+            }
+            if (g.blocks > 0x7FFFFFFF) throw Error(APRH_ERR_UNSUPPORTED, "too many convolution tiles");
+            all += g.blocks;
+            groups.push_back(g);
+        }
+        double* pp = grow_parts(all);
+        for (Group& g : groups) {
+            if (g.blocks == 0) continue;
+            g.d.part = pp;
+            launch_conv_dense(g.d, g.S, g.sep, epi, (unsigned)g.blocks, st);
+            if (pp) pp += 2 * g.blocks;
+        }
+        return;
+    }
     /* images of consecutive levels (ping-pong): level l's launch reads V(l-1), writes V(l) */
     const size_t vmax = a.l_max > a.l_min ? (size_t)(a.y_num[a.l_max - 1] * a.x_num[a.l_max - 1] * a.z_num[a.l_max - 1]) : 1;
     Buf V0(ctx->pool, vmax * 4), V1(ctx->pool, a.l_max > a.l_min + 1 ? vmax * 4 : 4);
@@ -1083,7 +1080,7 @@ void conv_levels(aprh_context* ctx, aprh_apr& a, const std::vector<HostStencil>&
     struct Plan {
         LevelDesc L;
         int tx;
-        bool sep, regz;
+        bool sep;
         size_t lds;
         unsigned grid;
     };
@@ -1110,44 +1107,24 @@ void conv_levels(aprh_context* ctx, aprh_apr& a, const std::vector<HostStencil>&
         L.sz = s.sz;
         pl.sep = off_sep[(size_t)sn] >= 0;
         L.w_off = pl.sep ? off_sep[(size_t)sn] : off_exact[(size_t)sn];
-        /* the register-ring kernel addresses a coarse plane with 32-bit offsets */
-        pl.regz = pl.sep && sep_regz_size(s.sz) && s.sy == s.sz && s.sx == s.sz && L.cX * L.cY <= 0x7FFFFFFF;
-        if (pl.regz) {
-            /* 16-row tiles: more blocks per CU hide the plane's global reads better than the
-               smaller x halo of 32-row tiles saves (measured on the 9x9x9 RL workload) */
-            pl.tx = 16;
-            pl.lds = conv_sep_lds_bytes(pl.tx, s.sy, s.sx, s.sz);
-        } else {
-            pl.tx = 16;
-            pl.lds = conv_lds_bytes(16, pl.sep, s.sy, s.sx, s.sz);
-            if (pl.lds > 96 * 1024) {
-                pl.tx = 8;
-                pl.lds = conv_lds_bytes(8, pl.sep, s.sy, s.sx, s.sz);
-            }
+        pl.tx = 16;
+        pl.lds = conv_lds_bytes(16, pl.sep, s.sy, s.sx, s.sz);
+        if (pl.lds > 96 * 1024) {
+            pl.tx = 8;
+            pl.lds = conv_lds_bytes(8, pl.sep, s.sy, s.sx, s.sz);
         }
         if (pl.lds > 160 * 1024) throw Error(APRH_ERR_UNSUPPORTED, "stencil too large for the tile convolution");
         L.ntx = (int)cdiv(L.X, pl.tx);
         L.nty = L.nyb;
         const int64_t nxy = (int64_t)L.ntx * L.nty;
         const int hz = (s.sz - 1) / 2;
-        int64_t zc;
-        if (pl.regz) {
-            /* about 4096 blocks (8192 for 3-plane stencils, whose short halo makes shorter runs
-               cheap: 3x3x3 passes of the 1024x1024x256 RL-TV workload 2 % faster); runs of at
-               least 4 hz planes unless that leaves fewer than ~1024 */
-            zc = cdiv(L.Z * nxy, hz <= 1 ? 8192 : 4096);
-            const int64_t zmin = std::min<int64_t>(L.Z, std::max(8, 4 * hz));
-            if (nxy * cdiv(L.Z, zmin) >= 1024) zc = std::max(zc, zmin);
-            zc = std::max<int64_t>(1, std::min<int64_t>(zc, L.Z));
-        } else {
-            /* at most about 8192 blocks, and at least about 1024 unless runs would exceed 4 hz
-               planes: a block marches its planes one after another, so a small level wants short
-               runs, a large one runs long enough to amortise the 2 hz halo planes */
-            const int64_t W = L.Z * nxy;
-            const int64_t zmin = std::min<int64_t>(L.Z, std::max(8, 4 * hz));
-            zc = std::max(cdiv(W, 8192), std::min(zmin, cdiv(W, 1024)));
-            zc = std::max<int64_t>(1, std::min<int64_t>(zc, L.Z));
-        }
+        /* at most about 8192 blocks, and at least about 1024 unless runs would exceed 4 hz
+           planes: a block marches its planes one after another, so a small level wants short
+           runs, a large one runs long enough to amortise the 2 hz halo planes */
+        const int64_t Wk = L.Z * nxy;
+        const int64_t zmin = std::min<int64_t>(L.Z, std::max(8, 4 * hz));
+        int64_t zc = std::max(cdiv(Wk, 8192), std::min(zmin, cdiv(Wk, 1024)));
+        zc = std::max<int64_t>(1, std::min<int64_t>(zc, L.Z));
         L.zc = (int)zc;
         L.ntz = (int)cdiv(L.Z, zc);
         const int64_t g = nxy * L.ntz;
@@ -1156,17 +1133,7 @@ void conv_levels(aprh_context* ctx, aprh_apr& a, const std::vector<HostStencil>&
         total_blocks += g;
         plans.push_back(pl);
     }
-    double* pbase = nullptr;
-    if (epi == 2) {
-        const int64_t need = (*nparts) + total_blocks;
-        if ((int64_t)(part->bytes() / 16) < need) {
-            Buf nb(ctx->pool, (size_t)need * 16);
-            if (*nparts > 0) HIP_CHECK(hipMemcpyAsync(nb.ptr(), part->ptr(), (size_t)(*nparts) * 16, hipMemcpyDeviceToDevice, st));
-            *part = std::move(nb);
-        }
-        pbase = part->as<double>() + 2 * (*nparts);
-        *nparts = need;
-    }
+    double* pbase = grow_parts(total_blocks);
     int64_t boff = 0;
     for (int l = a.l_min; l <= a.l_max; ++l) {
         const Plan& pl = plans[(size_t)(l - a.l_min)];
@@ -1192,10 +1159,6 @@ void conv_levels(aprh_context* ctx, aprh_apr& a, const std::vector<HostStencil>&
         ca.epi_in_u16 = epi_u16 ? 1 : 0;
         boff += pl.grid;
         if (pl.grid == 0) continue;
-        if (pl.regz) {
-            launch_conv_sep_sz<T, 16>(ca, pl.grid, pl.lds, st);
-            continue;
-        }
         launch_conv_level<T>(ca, pl.tx, pl.sep, pl.grid, pl.lds, st);
     }
 }

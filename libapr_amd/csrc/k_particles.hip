@@ -261,26 +261,36 @@ __global__ __launch_bounds__(1024) void k_tree_small(Rows AR, Rows TR, int t_hi,
 }
 
 /* ---------------- piecewise-constant images ---------------- */
-/* Where the pixels of an image at level L come from: the particles of levels l_min .. L, then the tree
-   nodes of L (where finer particles live).  Source i's cell (z, x, y) covers 2^sh[i] pixels a side. */
+/* Where the pixels of an image at APR level li (counted from l_min) come from: the particles of levels
+   0 .. li, then the tree nodes of li (where finer particles live).  A cell of level s covers 2^(li - s)
+   pixels a side. */
 struct ReconArgs {
-    int n;                     /* sources                                       */
-    int tree;                  /* source that is the tree level, or -1          */
-    int l_lo;                  /* level of source 0                             */
-    int level;                 /* L                                             */
-    int64_t rb[MAXL + 1];      /* index in xz_end (t_xz_end) of the row (0, 0)  */
-    int64_t xn[MAXL + 1];
-    int sh[MAXL + 1];
+    int l_lo;                  /* l_min                                          */
+    int64_t rb[MAXL];          /* index in xz_end of the level's row (0, 0)      */
+    int64_t trb[MAXL];         /* index in t_xz_end of the same tree row, or -1: no tree nodes wanted there */
+    int64_t xn[MAXL];
     const uint64_t* xz;
     const uint16_t* yv;
     const void* parts;
     const uint64_t* txz;
     const uint16_t* tyv;
     const float* tv;
-    uint32_t X, rows;          /* x_num of L, rows (z, x) of L                  */
+};
+/* the image of one level */
+struct ReconImage {
+    int li;
+    uint32_t X, rows;          /* x_num, rows (z, x)                            */
     int64_t Y;
-    void* out;                 /* image, or nullptr                             */
+    void* out;
     uint8_t* lev;              /* level of the covering particle, or nullptr    */
+};
+/* the images of levels l_min .. in one buffer */
+struct LevelImages {
+    int n;
+    int64_t row0[MAXL + 1];    /* first row of each level, counted over all     */
+    uint32_t X[MAXL];
+    int64_t Y[MAXL];
+    float* out[MAXL];
 };
 
 constexpr int RC_BYTES = 4096;   /* of a row's values in LDS, per wave */
@@ -311,88 +321,112 @@ __device__ __forceinline__ void store_staged(E* dst, const E* lds, int head, int
 template <typename E>
 __device__ __forceinline__ int vec_head(const E* p) { return (int)(((uintptr_t)p & 15u) / sizeof(E)); }
 
-/* The image in one pass: a wave takes one row (z, x) of the image (blockIdx.y: 4096 bytes of it), finds
-   the row of every level above it, and writes the levels' values into LDS coarse to fine, a lane per
-   pixel, so a finer level stands where two overlap; then the row leaves in 16-byte words.  Bound by
-   memory: particles and y are read once at the finest level and from L2 by the 4^d rows below a coarser
-   one, and the image is written once.  (Before, a level's image was the coarser one upsampled, then
-   its particles scattered over it: three passes over the finest level, 1.12 ms for 1000 x 1023 x 255
-   u16 against 0.38 ms.)  VALS: values from parts / tree to out, else the levels themselves to out;
-   LEV: the levels to lev as bytes. */
+/* Pixels [c0, c0 + cn) of row (z, x) of level li's image: the wave finds the row of every level above it
+   and writes the levels' values into LDS coarse to fine, a lane per pixel, so a finer level stands where
+   two overlap; then the piece leaves in 16-byte words.  search: the row is longer than the piece.
+   VALS: values from parts / tree to dst, else the levels themselves; LEV: the levels to ldst as bytes */
 template <typename T, typename D, bool VALS, bool LEV>
-__global__ __launch_bounds__(256) void k_recon(ReconArgs a) {
-    constexpr int CHUNK = RC_BYTES / (int)sizeof(D);
+__device__ __forceinline__ void recon_piece(const ReconArgs& a, int li, uint32_t z, uint32_t x, int64_t c0, int cn, bool search, D* st,
+                                            uint8_t* ls, D* dst, uint8_t* ldst, int lane) {
     constexpr int LOG = sizeof(D) == 2 ? 11 : 10;
-    static_assert(CHUNK == 1 << LOG, "chunk size");
+    const int head = vec_head(dst), lhead = LEV ? vec_head(ldst) : 0;
+    const int tree = a.trb[li] >= 0 ? li + 1 : -1;
+    /* lane s: the entries of source s under this row (under the piece) */
+    uint64_t b = 0, e = 0;
+    if (lane <= li || lane == tree) {
+        const bool tr = lane == tree;
+        const int s = tr ? li : lane, d = li - s;
+        const int64_t r = (tr ? a.trb[s] : a.rb[s]) + (int64_t)(z >> d) * a.xn[s] + (x >> d);
+        const uint64_t* xz = tr ? a.txz : a.xz;
+        b = xz[r - 1];
+        e = xz[r];
+        if (search && e > b) {
+            const uint16_t* yv = tr ? a.tyv : a.yv;
+            b = row_lower(yv, b, e, c0 >> d);
+            e = row_lower(yv, b, e, ((c0 + cn - 1) >> d) + 1);
+        }
+    }
+    uint64_t todo = __ballot(e > b);
+    while (todo) {
+        const int s = __builtin_ctzll(todo);
+        todo &= todo - 1;
+        const uint64_t sb = ((uint64_t)__builtin_amdgcn_readlane((int)(b >> 32), s) << 32) | (uint32_t)__builtin_amdgcn_readlane((int)b, s);
+        const int cnt = __builtin_amdgcn_readlane((int)(e - b), s);
+        const bool tr = s == tree;
+        const int d = tr ? 0 : li - s, de = min(d, LOG);   /* a cell wider than the piece covers all of it */
+        const int lv = a.l_lo + (tr ? li : s);
+        const uint16_t* yv = (tr ? a.tyv : a.yv) + sb;
+        const int items = cnt << de;
+        auto value = [&](int i) -> D {
+            if (!VALS) return Cvt<D>::from((uint16_t)lv);
+            return tr ? Cvt<D>::from(a.tv[sb + i]) : Cvt<D>::from(((const T*)a.parts)[sb + i]);
+        };
+        auto put = [&](int k, int64_t y, D v) {
+            /* the pixel's place in the piece; a cell that starts before it (wider than it) fills it from 0 */
+            const int64_t p = max((y << d) - c0, (int64_t)0) + (k & ((1 << de) - 1));
+            if (p < cn) {
+                st[head + p] = v;
+                if (LEV) ls[lhead + p] = (uint8_t)lv;
+            }
+        };
+        int k = lane;
+        for (; k + 192 < items; k += 256) {   /* four pixels per lane in flight */
+            int64_t yy[4];
+            D vv[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                yy[u] = yv[(k + 64 * u) >> de];
+                vv[u] = value((k + 64 * u) >> de);
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u) put(k + 64 * u, yy[u], vv[u]);
+        }
+        for (; k < items; k += 64) put(k, yv[k >> de], value(k >> de));
+    }
+    /* the wave's own LDS writes are in order; the compiler must not move the reads up */
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    store_staged<D>(dst, st, head, cn, lane);
+    if (LEV) store_staged<uint8_t>(ldst, ls, lhead, cn, lane);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   /* the next piece rewrites the stage */
+}
+
+/* The image of one level in one pass: a wave per row (blockIdx.y: 4096 bytes of it).  Bound by memory:
+   particles and y are read once at the finest level and from L2 by the 4^d rows below a coarser one, and
+   the image is written once.  (Before, a level's image was the coarser one upsampled, then its particles
+   scattered over it: three passes over the finest level, 1.12 ms for 1000 x 1023 x 255 u16 against
+   0.38 ms.) */
+template <typename T, typename D, bool VALS, bool LEV>
+__global__ __launch_bounds__(256) void k_recon(ReconArgs a, ReconImage im) {
+    constexpr int CHUNK = RC_BYTES / (int)sizeof(D);
     __shared__ __align__(16) D stage[4][CHUNK + 16 / sizeof(D)];
     __shared__ __align__(16) uint8_t lstage[4][LEV ? CHUNK + 16 : 16];
     const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int64_t c0 = (int64_t)blockIdx.y * CHUNK;
-    const int cn = (int)min((int64_t)CHUNK, a.Y - c0);
-    D* st = stage[wv];
-    uint8_t* ls = lstage[wv];
-    for (int64_t rowl = xcd_block(blockIdx.x, gridDim.x) * 4 + wv; rowl < (int64_t)a.rows; rowl += (int64_t)gridDim.x * 4) {
-        const uint32_t row = (uint32_t)rowl, z = row / a.X, x = row - z * a.X;
-        D* dst = (D*)a.out + ((int64_t)row * a.Y + c0);
-        uint8_t* ldst = LEV ? a.lev + ((int64_t)row * a.Y + c0) : nullptr;
-        const int head = vec_head(dst), lhead = LEV ? vec_head(ldst) : 0;
-        /* lane i: the entries of source i under this row (under its chunk) */
-        uint64_t b = 0, e = 0;
-        if (lane < a.n) {
-            const int d = a.sh[lane];
-            const bool tr = lane == a.tree;
-            const int64_t r = a.rb[lane] + (int64_t)(z >> d) * a.xn[lane] + (x >> d);
-            const uint64_t* xz = tr ? a.txz : a.xz;
-            b = xz[r - 1];
-            e = xz[r];
-            if (gridDim.y > 1 && e > b) {
-                const uint16_t* yv = tr ? a.tyv : a.yv;
-                b = row_lower(yv, b, e, c0 >> d);
-                e = row_lower(yv, b, e, ((c0 + cn - 1) >> d) + 1);
-            }
-        }
-        uint64_t todo = __ballot(e > b);
-        while (todo) {
-            const int s = __builtin_ctzll(todo);
-            todo &= todo - 1;
-            const uint64_t sb = ((uint64_t)__builtin_amdgcn_readlane((int)(b >> 32), s) << 32) | (uint32_t)__builtin_amdgcn_readlane((int)b, s);
-            const int cnt = __builtin_amdgcn_readlane((int)(e - b), s);
-            const bool tr = s == a.tree;
-            const int d = a.sh[s], de = min(d, LOG);   /* a cell wider than the chunk covers all of it */
-            const int lv = tr ? a.level : a.l_lo + s;
-            const uint16_t* yv = (tr ? a.tyv : a.yv) + sb;
-            const int items = cnt << de;
-            auto value = [&](int i) -> D {
-                if (!VALS) return Cvt<D>::from((uint16_t)lv);
-                return tr ? Cvt<D>::from(a.tv[sb + i]) : Cvt<D>::from(((const T*)a.parts)[sb + i]);
-            };
-            auto put = [&](int k, int64_t y, D v) {
-                /* the pixel's place in the chunk; a cell that starts before it (wider than it) fills it from 0 */
-                const int64_t p = max((y << d) - c0, (int64_t)0) + (k & ((1 << de) - 1));
-                if (p < cn) {
-                    st[head + p] = v;
-                    if (LEV) ls[lhead + p] = (uint8_t)lv;
-                }
-            };
-            int k = lane;
-            for (; k + 192 < items; k += 256) {   /* four pixels per lane in flight */
-                int64_t yy[4];
-                D vv[4];
-    #pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                    yy[u] = yv[(k + 64 * u) >> de];
-                    vv[u] = value((k + 64 * u) >> de);
-                }
-    #pragma unroll
-                for (int u = 0; u < 4; ++u) put(k + 64 * u, yy[u], vv[u]);
-            }
-            for (; k < items; k += 64) put(k, yv[k >> de], value(k >> de));
-        }
-        /* the wave's own LDS writes are in order; the compiler must not move the reads up */
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        store_staged<D>(dst, st, head, cn, lane);
-        if (LEV) store_staged<uint8_t>(ldst, ls, lhead, cn, lane);
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   /* the next row rewrites the stage */
+    const int cn = (int)min((int64_t)CHUNK, im.Y - c0);
+    for (int64_t rowl = xcd_block(blockIdx.x, gridDim.x) * 4 + wv; rowl < (int64_t)im.rows; rowl += (int64_t)gridDim.x * 4) {
+        const uint32_t row = (uint32_t)rowl, z = row / im.X, x = row - z * im.X;
+        const int64_t o = (int64_t)row * im.Y + c0;
+        recon_piece<T, D, VALS, LEV>(a, im.li, z, x, c0, cn, gridDim.y > 1, stage[wv], lstage[wv], (D*)im.out + o, LEV ? im.lev + o : nullptr,
+                                     lane);
+    }
+}
+
+/* the float images of several levels in one launch: none of them needs another, and together they fill the
+   chip where the coarse ones alone would each cost a launch */
+template <typename T>
+__global__ __launch_bounds__(256) void k_level_images(ReconArgs a, LevelImages m) {
+    constexpr int CHUNK = RC_BYTES / 4;
+    __shared__ __align__(16) float stage[4][CHUNK + 4];
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t c0 = (int64_t)blockIdx.y * CHUNK;
+    for (int64_t rg = xcd_block(blockIdx.x, gridDim.x) * 4 + wv; rg < m.row0[m.n]; rg += (int64_t)gridDim.x * 4) {
+        int li = 0;
+        while (rg >= m.row0[li + 1]) ++li;
+        if (c0 >= m.Y[li]) continue;
+        const uint32_t row = (uint32_t)(rg - m.row0[li]), X = m.X[li], z = row / X, x = row - z * X;
+        const int cn = (int)min((int64_t)CHUNK, m.Y[li] - c0);
+        recon_piece<T, float, true, false>(a, li, z, x, c0, cn, m.Y[li] > CHUNK, stage[wv], nullptr, m.out[li] + (int64_t)row * m.Y[li] + c0, nullptr,
+                                           lane);
     }
 }
 
@@ -671,40 +705,35 @@ void convolve(aprh_context* ctx, aprh_apr& a, const std::vector<HostStencil>& st
 }
 
 namespace {
-/* the sources of the image at `level` (see ReconArgs) */
-ReconArgs recon_sources(const aprh_apr& a, int level) {
+/* sources of the images of levels l_min .. hi; tree nodes of level `tree` only, or of all levels below l_max */
+ReconArgs recon_sources(const aprh_apr& a, int hi, int tree = -1) {
     ReconArgs r;
     std::memset(&r, 0, sizeof(r));
-    r.tree = -1;
     r.l_lo = a.l_min;
-    r.level = level;
-    for (int l = a.l_min; l <= level; ++l) {
-        if (r.n >= MAXL) throw Error(APRH_ERR_UNSUPPORTED, "too many levels");
-        r.rb[r.n] = (int64_t)a.level_xz_vec[l];
-        r.xn[r.n] = a.x_num[l];
-        r.sh[r.n++] = level - l;
-    }
-    if (level < a.l_max && level <= a.t_l_max && a.t_total > 0) {
-        r.tree = r.n;
-        r.rb[r.n] = (int64_t)a.t_level_xz[level];
-        r.xn[r.n] = a.t_x[level];
-        r.sh[r.n++] = 0;
+    if (hi - a.l_min >= MAXL) throw Error(APRH_ERR_UNSUPPORTED, "too many levels");
+    for (int l = a.l_min; l <= hi; ++l) {
+        const int i = l - a.l_min;
+        r.rb[i] = (int64_t)a.level_xz_vec[l];
+        r.xn[i] = a.x_num[l];
+        r.trb[i] = l < a.l_max && l <= a.t_l_max && a.t_total > 0 && (tree < 0 || l == tree) ? (int64_t)a.t_level_xz[l] : -1;
     }
     r.xz = a.xz_end.as<uint64_t>();
     r.yv = a.y_vec.as<uint16_t>();
     r.txz = a.t_xz_end.as<uint64_t>();
     r.tyv = a.t_y_vec.as<uint16_t>();
-    r.Y = a.y_num[level];
-    r.X = (uint32_t)a.x_num[level];
-    r.rows = (uint32_t)(a.x_num[level] * a.z_num[level]);   /* dims are at most 65535 */
     return r;
+}
+ReconImage recon_image(const aprh_apr& a, int level, void* out, uint8_t* lev) {
+    /* dims are at most 65535, so a level has fewer than 2^32 rows */
+    return {level - a.l_min, (uint32_t)a.x_num[level], (uint32_t)(a.x_num[level] * a.z_num[level]), a.y_num[level], out, lev};
 }
 
 template <typename T, typename D, bool VALS, bool LEV>
-void launch_recon(aprh_context* ctx, const ReconArgs& r) {
+void launch_recon(aprh_context* ctx, const ReconArgs& r, const ReconImage& im) {
     const int64_t chunk = RC_BYTES / (int64_t)sizeof(D);
-    if (r.rows == 0 || r.Y == 0) return;
-    hipLaunchKernelGGL((k_recon<T, D, VALS, LEV>), dim3((unsigned)std::min<int64_t>(cdiv(r.rows, 4), 1 << 20), (unsigned)cdiv(r.Y, chunk)), kBlock, 0, ctx->stream, r);
+    if (im.rows == 0 || im.Y == 0) return;
+    hipLaunchKernelGGL((k_recon<T, D, VALS, LEV>), dim3((unsigned)std::min<int64_t>(cdiv(im.rows, 4), 1 << 20), (unsigned)cdiv(im.Y, chunk)), kBlock,
+                       0, ctx->stream, r, im);
     HIP_LAUNCH_CHECK();
 }
 
@@ -718,16 +747,38 @@ void reconstruct(aprh_context* ctx, aprh_apr& a, const T* parts, int level, U* i
         tree.reset(ctx->pool, std::max<uint64_t>(a.t_total, 1) * 4);
         tree_mean(ctx, a, parts, tree.as<float>());
     }
-    ReconArgs r = recon_sources(a, level);
+    ReconArgs r = recon_sources(a, level, level);
     r.parts = parts;
     r.tv = tree.as<float>();
-    r.out = img;
-    r.lev = lev;
-    if (lev) launch_recon<T, U, true, true>(ctx, r);
-    else launch_recon<T, U, true, false>(ctx, r);
+    const ReconImage im = recon_image(a, level, img, lev);
+    if (lev) launch_recon<T, U, true, true>(ctx, r, im);
+    else launch_recon<T, U, true, false>(ctx, r, im);
     HIP_CHECK(hipStreamSynchronize(ctx->stream));
 }
 }  // namespace
+
+template <typename T>
+void level_images(aprh_context* ctx, const aprh_apr& a, const T* parts, const float* tree, const std::vector<float*>& out) {
+    ReconArgs r = recon_sources(a, a.l_max);
+    r.parts = parts;
+    r.tv = tree;
+    LevelImages m;
+    std::memset(&m, 0, sizeof(m));
+    int64_t ymax = 1;
+    for (int l = a.l_min; l <= a.l_max; ++l) {
+        const int i = m.n++;
+        m.X[i] = (uint32_t)a.x_num[l];
+        m.Y[i] = a.y_num[l];
+        m.out[i] = out[(size_t)l];
+        m.row0[i + 1] = m.row0[i] + a.x_num[l] * a.z_num[l];
+        ymax = std::max(ymax, a.y_num[l]);
+    }
+    hipLaunchKernelGGL(k_level_images<T>, dim3((unsigned)std::min<int64_t>(cdiv(m.row0[m.n], 4), 1 << 20), (unsigned)cdiv(ymax, RC_BYTES / 4)),
+                       kBlock, 0, ctx->stream, r, m);
+    HIP_LAUNCH_CHECK();
+}
+template void level_images<uint16_t>(aprh_context*, const aprh_apr&, const uint16_t*, const float*, const std::vector<float*>&);
+template void level_images<float>(aprh_context*, const aprh_apr&, const float*, const float*, const std::vector<float*>&);
 
 /* APRReconstruction::reconstruct_level (APRReconstruction.hpp:131-171): every pixel takes the
    level of the particle covering it.  At a coarser level L (the patch form, :397-490) a pixel
@@ -735,10 +786,10 @@ void reconstruct(aprh_context* ctx, aprh_apr& a, const T* parts, int level, U* i
 void reconstruct_level(aprh_context* ctx, aprh_apr& a, int level, void* img, int idt) {
     if (level < a.l_min || level > a.l_max) throw Error(APRH_ERR_INVALID_ARGUMENT, "reconstruction level out of range");
     if (level < a.l_max) ensure_tree(ctx, a);
-    ReconArgs r = recon_sources(a, level);
-    r.out = img;
-    if (idt == APRH_DTYPE_U16) launch_recon<uint16_t, uint16_t, false, false>(ctx, r);
-    else launch_recon<uint16_t, float, false, false>(ctx, r);
+    const ReconArgs r = recon_sources(a, level, level);
+    const ReconImage im = recon_image(a, level, img, nullptr);
+    if (idt == APRH_DTYPE_U16) launch_recon<uint16_t, uint16_t, false, false>(ctx, r, im);
+    else launch_recon<uint16_t, float, false, false>(ctx, r, im);
     HIP_CHECK(hipStreamSynchronize(ctx->stream));
 }
 
