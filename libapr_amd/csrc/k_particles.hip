@@ -8,10 +8,10 @@
  *    maps are OR-ed upward through the (0,0,0) child, and the linear tree
  *    access is built by row counts + scan + fill.
  *  - fill_tree_mean (APRTreeNumerics.hpp:63-202): tree levels from the top
- *    down; the children level is scattered into a dense value/type scratch and
- *    each tree node accumulates scale*value/8 over its particle children first
- *    and its tree children second, both in (z, x, y) order -- the order in which
- *    the reference's two passes reach every node -- so the sums are bit-equal.
+ *    down; a wave holds the children of one tree row in LDS and each node
+ *    accumulates scale*value/8 over its particle children first and its tree
+ *    children second, both in (z, x, y) order -- the order in which the
+ *    reference's two passes reach every node -- so the sums are bit-equal.
  *  - piecewise-constant images (APRReconstruction::reconstruct_constant,
  *    APRReconstruction.hpp:80-120, :297-394): at level l_max + level_delta,
  *    one wave per image row over the particles of every level above it and,
@@ -164,99 +164,161 @@ __global__ void k_rows_to_xz(Rows R, const uint64_t* __restrict__ excl, const ui
     xz_end[R.row_begin[li] + (r - R.prefix[li])] = excl[r] + cnt[r];
 }
 
-/* ---------------- dense level images ---------------- */
-/* values (and optionally a type tag) of every particle / tree node of one level into a dense
-   image: wave `wid` of `nw` takes rows wid, wid + nw, ..., its lanes the row's entries */
-template <typename T, typename D>
-__device__ __forceinline__ void scatter_rows_body(const Rows& R, int li, const uint64_t* __restrict__ xz_end,
-                                                  const uint16_t* __restrict__ y_vec, const T* __restrict__ vals, D* V, uint8_t* Ty,
-                                                  uint8_t type, int64_t wid, int64_t nw, int lane) {
-    const int64_t nrows = R.x_num[li] * R.z_num[li];
-    for (int64_t row = wid; row < nrows; row += nw) {
-        const uint64_t b = xz_end[R.row_begin[li] + row - 1], e = xz_end[R.row_begin[li] + row];
-        D* vr = V + row * R.y_num[li];
-        uint8_t* tr = Ty ? Ty + row * R.y_num[li] : nullptr;
-        for (uint64_t i = b + lane; i < e; i += 64) {
-            const uint16_t y = y_vec[i];
-            vr[y] = Cvt<D>::from(vals[i]);
-            if (tr) tr[y] = type;
-        }
+/* first index in [b, e) with y_vec >= y */
+__device__ __forceinline__ uint64_t row_lower(const uint16_t* __restrict__ yv, uint64_t b, uint64_t e, int64_t y) {
+    while (b < e) {
+        const uint64_t mid = (b + e) >> 1;
+        if ((int64_t)yv[mid] < y) b = mid + 1;
+        else e = mid;
     }
-}
-template <typename T, typename D>
-__global__ __launch_bounds__(256) void k_scatter_rows(Rows R, int li, const uint64_t* __restrict__ xz_end,
-                                                      const uint16_t* __restrict__ y_vec, const T* __restrict__ vals, D* V,
-                                                      uint8_t* Ty, uint8_t type) {
-    scatter_rows_body<T, D>(R, li, xz_end, y_vec, vals, V, Ty, type, ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / 64,
-                            ((int64_t)gridDim.x * blockDim.x) / 64, threadIdx.x & 63);
+    return b;
 }
 
-/* one tree level of fill_tree_mean: children (level t+1) are in the dense V/Ty scratch */
-__device__ __forceinline__ void tree_mean_level_body(const Rows& TR, int ti, const uint64_t* __restrict__ txz,
-                                                     const uint16_t* __restrict__ ty, const float* __restrict__ V,
-                                                     const uint8_t* __restrict__ Ty, int64_t cyn, int64_t cxn, int64_t czn, float* tree,
-                                                     int64_t wid, int64_t nw, int lane) {
-    const int64_t pxn = TR.x_num[ti], pzn = TR.z_num[ti], pyn = TR.y_num[ti];
-    const int64_t nrows = pxn * pzn;
-    for (int64_t row = wid; row < nrows; row += nw) {
-        const int64_t zp = row / pxn, xp = row % pxn;
-        const uint64_t b = txz[TR.row_begin[ti] + row - 1], e = txz[TR.row_begin[ti] + row];
-        /* boundary scale factors (APRTreeNumerics.hpp:99-113) */
-        float sxz = (float)((((2 * pxn != cxn) && (xp == pxn - 1)) + ((2 * pzn != czn) && (zp == pzn - 1))) * 2);
-        if (sxz == 0) sxz = 1;
-        const float syxz = (2 * pyn != cyn) ? sxz * 2 : sxz;
-        const int nz = (int)min((int64_t)2, czn - 2 * zp), nx = (int)min((int64_t)2, cxn - 2 * xp);
-        for (uint64_t i = b + lane; i < e; i += 64) {
-            const int64_t yp = ty[i];
-            const float s = (yp == pyn - 1) ? syxz : sxz;
-            const int ny = (int)min((int64_t)2, cyn - 2 * yp);
-            float acc = 0.0f;
-            for (int pass = 1; pass <= 2; ++pass) {
-                for (int a = 0; a < nz; ++a)
-                    for (int bb = 0; bb < nx; ++bb)
-                        for (int c = 0; c < ny; ++c) {
-                            const int64_t ci = ((2 * zp + a) * cxn + (2 * xp + bb)) * cyn + (2 * yp + c);
-                            if (Ty[ci] == pass) acc = s * V[ci] / 8.0f + acc;
-                        }
+/* ---------------- tree means ---------------- */
+/* The tree nodes of one row (zp, xp) of tree level t under child cells [c0, c0 + P): a wave puts the four
+   child rows' particles and tree nodes (level t + 1) into LDS by their y, then takes one node per lane.
+   The children's order is the reference's: its two passes, particles then tree nodes, each in (z, x, y)
+   order.  Bound by the latency of row ends, children, then nodes, and on the largest level by its bytes;
+   eight 64-entry loads are in flight.  (Before, a level's children went through a dense scratch image of the
+   whole level, a clear, two scatters and a gather: the levels below the finest of a 1024 x 1024 x 256 APR
+   took 0.39 ms, now 0.17; of 256 x 256 x 128 87 us, now 58.) */
+template <typename T, int P>
+struct TreeStage {
+    float v[4][P];
+    uint8_t t[4][P];
+};
+struct TreeArgs {
+    Rows AR, TR;
+    int l_min, t_l_max;
+    const uint64_t* xz;
+    const uint16_t* yv;
+    const void* parts;
+    const uint64_t* txz;
+    const uint16_t* tyv;
+    float* tree;
+};
+template <typename T, int P>
+__device__ __forceinline__ void tree_mean_piece(const TreeArgs& a, int t, int64_t row, int64_t c0, TreeStage<T, P>& st, int lane) {
+    const Rows& TR = a.TR;
+    const int c = t + 1;   /* child level; APR and tree levels share the level geometry */
+    const bool tree_child = c <= a.t_l_max;
+    /* the child level's dims: the APR's where it has the level, else the tree's */
+    const int ai = c - a.l_min;
+    const int64_t cyn = ai >= 0 ? a.AR.y_num[ai] : TR.y_num[c], cxn = ai >= 0 ? a.AR.x_num[ai] : TR.x_num[c],
+                  czn = ai >= 0 ? a.AR.z_num[ai] : TR.z_num[c];
+    const int64_t pxn = TR.x_num[t], pzn = TR.z_num[t], pyn = TR.y_num[t];
+    const int64_t zp = row / pxn, xp = row % pxn;
+    const int nz = (int)min((int64_t)2, czn - 2 * zp), nx = (int)min((int64_t)2, cxn - 2 * xp);
+    /* lanes 0..3: particle rows (a, b) of the children, 4..7: their tree rows, 8: this row's nodes */
+    uint64_t b = 0, e = 0;
+    if (lane < 9) {
+        const int r = lane & 3, za = r >> 1, xb = r & 1;
+        const bool part = lane < 4, node = lane == 8;
+        if (node || (za < nz && xb < nx && (part ? ai >= 0 : tree_child))) {
+            const int64_t cr = (2 * zp + za) * cxn + (2 * xp + xb);
+            const int64_t id = node ? TR.row_begin[t] + row : part ? a.AR.row_begin[ai] + cr : TR.row_begin[c] + cr;
+            const uint64_t* xz = part ? a.xz : a.txz;
+            b = xz[id - 1];
+            e = xz[id];
+            if (cyn > P && e > b) {
+                const uint16_t* yv = part ? a.yv : a.tyv;
+                b = row_lower(yv, b, e, node ? c0 / 2 : c0);
+                e = row_lower(yv, b, e, node ? (c0 + P) / 2 : c0 + P);
             }
-            tree[i] = acc;
         }
     }
-}
-__global__ __launch_bounds__(256) void k_tree_mean_level(Rows TR, int ti, const uint64_t* __restrict__ txz, const uint16_t* __restrict__ ty,
-                                                         const float* __restrict__ V, const uint8_t* __restrict__ Ty, int64_t cyn,
-                                                         int64_t cxn, int64_t czn, float* tree) {
-    tree_mean_level_body(TR, ti, txz, ty, V, Ty, cyn, cxn, czn, tree, ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / 64,
-                         ((int64_t)gridDim.x * blockDim.x) / 64, threadIdx.x & 63);
+    const uint64_t nb = ((uint64_t)__builtin_amdgcn_readlane((int)(b >> 32), 8) << 32) | (uint32_t)__builtin_amdgcn_readlane((int)b, 8);
+    const int np = __builtin_amdgcn_readlane((int)(e - b), 8);
+    if (np == 0) return;
+#pragma unroll
+    for (int k = 0; k < P / 64; ++k) ((uint32_t*)st.t)[k * 64 + lane] = 0;
+    /* batches of 64 children of one list, eight in flight */
+    constexpr int U = 8;
+    uint64_t todo = __ballot(lane < 8 && e > b), sb = 0;
+    int k = 0, items = 0, list = 0;
+    for (;;) {
+        uint64_t qb[U];
+        int qn[U], ql[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (k >= items) {
+                k = items = 0;
+                if (todo) {
+                    list = __builtin_ctzll(todo);
+                    todo &= todo - 1;
+                    sb = ((uint64_t)__builtin_amdgcn_readlane((int)(b >> 32), list) << 32) | (uint32_t)__builtin_amdgcn_readlane((int)b, list);
+                    items = __builtin_amdgcn_readlane((int)(e - b), list);
+                }
+            }
+            qb[u] = sb + (uint64_t)k;
+            qn[u] = items - k;
+            ql[u] = list;
+            k += 64;
+        }
+        if (qn[0] <= 0) break;
+        int yy[U];
+        float vv[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            yy[u] = 0;
+            vv[u] = 0.0f;
+            if (lane < qn[u]) {
+                const uint64_t i = qb[u] + (uint64_t)lane;
+                yy[u] = (ql[u] < 4 ? a.yv : a.tyv)[i];
+                vv[u] = ql[u] < 4 ? Cvt<float>::from(((const T*)a.parts)[i]) : a.tree[i];
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (lane < qn[u]) {
+                const int p = yy[u] - (int)c0;
+                if (p >= 0 && p < P) {
+                    st.v[ql[u] & 3][p] = vv[u];
+                    st.t[ql[u] & 3][p] = ql[u] < 4 ? 1 : 2;
+                }
+            }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   /* the lanes read each other's writes below */
+    /* boundary scale factors (APRTreeNumerics.hpp:99-113) */
+    float sxz = (float)((((2 * pxn != cxn) && (xp == pxn - 1)) + ((2 * pzn != czn) && (zp == pzn - 1))) * 2);
+    if (sxz == 0) sxz = 1;
+    const float syxz = (2 * pyn != cyn) ? sxz * 2 : sxz;
+    for (int n = lane; n < np; n += 64) {
+        const int64_t yp = a.tyv[nb + (uint64_t)n];
+        const float s = (yp == pyn - 1) ? syxz : sxz;
+        const int ny = (int)min((int64_t)2, cyn - 2 * yp), p = (int)(2 * yp - c0);
+        float acc = 0.0f;
+        for (int pass = 1; pass <= 2; ++pass)
+            for (int za = 0; za < nz; ++za)
+                for (int xb = 0; xb < nx; ++xb)
+                    for (int cc = 0; cc < ny; ++cc)
+                        if (st.t[za * 2 + xb][p + cc] == pass) acc = s * st.v[za * 2 + xb][p + cc] / 8.0f + acc;
+        a.tree[nb + (uint64_t)n] = acc;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   /* the next piece rewrites the stage */
 }
 
-/* the block's writes to global memory visible to its own later reads: a workgroup-scope fence
-   and barrier (__syncthreads).  All waves of a workgroup run on one CU and share its vector L1,
-   so no cache maintenance is needed at this scope (an agent-scope fence would write back L2) */
-__device__ __forceinline__ void block_sync_global() { __syncthreads(); }
-
-/* the small tree levels t_hi .. 0 in one block of 1024 threads (each level's rows are few, so
-   separate launches would cost more than their work): per level, clear the type tags of the
-   children level, scatter its particles and tree nodes, take the means; the same bodies as the
-   per-level kernels, so the results are identical */
+constexpr int TREE_P = 512, TREE_P_SMALL = 128;   /* child cells per piece */
 template <typename T>
-__global__ __launch_bounds__(1024) void k_tree_small(Rows AR, Rows TR, int t_hi, int l_min, int t_l_max, const uint64_t* __restrict__ xz_end,
-                                                     const uint16_t* __restrict__ y_vec, const T* __restrict__ parts,
-                                                     const uint64_t* __restrict__ txz, const uint16_t* __restrict__ ty, float* tree, float* V,
-                                                     uint8_t* Ty) {
-    const int64_t wid = threadIdx.x / 64, nw = blockDim.x / 64;
-    const int lane = threadIdx.x & 63;
+__global__ __launch_bounds__(256) void k_tree_mean(TreeArgs a, int t) {
+    __shared__ TreeStage<T, TREE_P> st[4];
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t rows = a.TR.x_num[t] * a.TR.z_num[t];
+    for (int64_t r = xcd_block(blockIdx.x, gridDim.x) * 4 + wv; r < rows; r += (int64_t)gridDim.x * 4)
+        tree_mean_piece<T, TREE_P>(a, t, r, (int64_t)blockIdx.y * TREE_P, st[wv], lane);
+}
+/* the small tree levels t_hi .. 0 in one block, a barrier between levels (its waves share a CU's vector L1,
+   so a level's values are visible to the next): separate launches would cost more than their work */
+constexpr int TREE_SMALL_THREADS = 1024;
+template <typename T>
+__global__ __launch_bounds__(TREE_SMALL_THREADS) void k_tree_small(TreeArgs a, int t_hi) {
+    __shared__ TreeStage<T, TREE_P_SMALL> st[TREE_SMALL_THREADS / 64];
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     for (int t = t_hi; t >= 0; --t) {
-        const int c = t + 1;
-        const int64_t cyn = TR.y_num[c], cxn = TR.x_num[c], czn = TR.z_num[c];
-        const int64_t n = cyn * cxn * czn;
-        for (int64_t i = threadIdx.x; i < n; i += blockDim.x) Ty[i] = 0;
-        block_sync_global();
-        if (c >= l_min) scatter_rows_body<T, float>(AR, c - l_min, xz_end, y_vec, parts, V, Ty, (uint8_t)1, wid, nw, lane);
-        if (c <= t_l_max) scatter_rows_body<float, float>(TR, c, txz, ty, (const float*)tree, V, Ty, (uint8_t)2, wid, nw, lane);
-        block_sync_global();
-        tree_mean_level_body(TR, t, txz, ty, V, Ty, cyn, cxn, czn, tree, wid, nw, lane);
-        block_sync_global();
+        const int64_t rows = a.TR.x_num[t] * a.TR.z_num[t], pieces = (2 * a.TR.y_num[t] + TREE_P_SMALL - 1) / TREE_P_SMALL;
+        for (int64_t i = wv; i < rows * pieces; i += TREE_SMALL_THREADS / 64)
+            tree_mean_piece<T, TREE_P_SMALL>(a, t, i / pieces, (i % pieces) * TREE_P_SMALL, st[wv], lane);
+        __syncthreads();
     }
 }
 
@@ -294,16 +356,6 @@ struct LevelImages {
 };
 
 constexpr int RC_BYTES = 4096;   /* of a row's values in LDS, per wave */
-
-/* first index in [b, e) with y_vec >= y */
-__device__ __forceinline__ uint64_t row_lower(const uint16_t* __restrict__ yv, uint64_t b, uint64_t e, int64_t y) {
-    while (b < e) {
-        const uint64_t mid = (b + e) >> 1;
-        if ((int64_t)yv[mid] < y) b = mid + 1;
-        else e = mid;
-    }
-    return b;
-}
 
 /* n elements staged in LDS (element i at lds[head + i]) to dst, whole 16-byte words inside */
 template <typename E>
@@ -457,8 +509,6 @@ __global__ void k_validate_rows(Rows R, const uint64_t* __restrict__ xz_end, con
 
 const dim3 kGrid(4096), kBlock(256);
 
-size_t level_elems(const aprh_apr& a, int l) { return (size_t)(a.y_num[l] * a.x_num[l] * a.z_num[l]); }
-
 }  // namespace
 
 /* ======================================================================== */
@@ -565,41 +615,32 @@ void tree_mean(aprh_context* ctx, aprh_apr& a, const T* parts, float* tree) {
     Rows AR = make_rows(a.y_num, a.x_num, a.z_num, a.level_xz_vec, a.l_min, a.l_max);
     Rows TR = make_rows(a.t_y, a.t_x, a.t_z, a.t_level_xz, 0, a.t_l_max);
     /* the top tree level straight from the particle rows of l_max when they have the regular
-       shape; the levels below through dense scratch of the children level */
+       shape; the levels below from the rows of their children */
     const bool top = tree_mean_top<T>(ctx, a, parts, tree);
     const int t_first = top ? a.t_l_max - 1 : a.t_l_max;
     if (t_first < 0) return;
-    const size_t maxn = level_elems(a, t_first + 1);
-    Buf V(ctx->pool, maxn * 4), Ty(ctx->pool, maxn);
-    /* tree levels whose children level has at most 256 rows go to one single-block launch */
-    int t_small = -1;
-    for (int t = t_first; t >= 0; --t)
-        if (a.x_num[t + 1] * a.z_num[t + 1] <= 256) {
-            t_small = t;
-            break;
-        }
+    TreeArgs ta;
+    ta.AR = AR;
+    ta.TR = TR;
+    ta.l_min = a.l_min;
+    ta.t_l_max = a.t_l_max;
+    ta.xz = a.xz_end.as<uint64_t>();
+    ta.yv = a.y_vec.as<uint16_t>();
+    ta.parts = parts;
+    ta.txz = a.t_xz_end.as<uint64_t>();
+    ta.tyv = a.t_y_vec.as<uint16_t>();
+    ta.tree = tree;
+    /* tree levels of at most 16 rows, a row per wave of one block, go to one launch */
+    int t_small = t_first;
+    while (t_small >= 0 && a.t_x[t_small] * a.t_z[t_small] > TREE_SMALL_THREADS / 64) --t_small;
     for (int t = t_first; t > t_small; --t) {
-        const int c = t + 1;   /* children level; APR and tree levels share the level geometry */
-        const int64_t cyn = a.y_num[c], cxn = a.x_num[c], czn = a.z_num[c];
-        HIP_CHECK(hipMemsetAsync(Ty.ptr(), 0, level_elems(a, c), st));
-        if (c >= a.l_min) {
-            hipLaunchKernelGGL((k_scatter_rows<T, float>), kGrid, kBlock, 0, st, AR, c - a.l_min, a.xz_end.as<uint64_t>(),
-                               a.y_vec.as<uint16_t>(), parts, V.as<float>(), Ty.as<uint8_t>(), (uint8_t)1);
-            HIP_LAUNCH_CHECK();
-        }
-        if (c <= a.t_l_max) {
-            hipLaunchKernelGGL((k_scatter_rows<float, float>), kGrid, kBlock, 0, st, TR, c, a.t_xz_end.as<uint64_t>(),
-                               a.t_y_vec.as<uint16_t>(), (const float*)tree, V.as<float>(), Ty.as<uint8_t>(), (uint8_t)2);
-            HIP_LAUNCH_CHECK();
-        }
-        hipLaunchKernelGGL(k_tree_mean_level, kGrid, kBlock, 0, st, TR, t, a.t_xz_end.as<uint64_t>(), a.t_y_vec.as<uint16_t>(),
-                           V.as<float>(), Ty.as<uint8_t>(), cyn, cxn, czn, tree);
+        const int64_t rows = a.t_x[t] * a.t_z[t];
+        hipLaunchKernelGGL(k_tree_mean<T>, dim3((unsigned)std::min<int64_t>(cdiv(rows, 4), 1 << 20), (unsigned)cdiv(2 * a.t_y[t], TREE_P)), kBlock, 0,
+                           st, ta, t);
         HIP_LAUNCH_CHECK();
     }
     if (t_small >= 0) {
-        hipLaunchKernelGGL((k_tree_small<T>), dim3(1), dim3(1024), 0, st, AR, TR, t_small, a.l_min, a.t_l_max, a.xz_end.as<uint64_t>(),
-                           a.y_vec.as<uint16_t>(), parts, a.t_xz_end.as<uint64_t>(), a.t_y_vec.as<uint16_t>(), tree, V.as<float>(),
-                           Ty.as<uint8_t>());
+        hipLaunchKernelGGL(k_tree_small<T>, dim3(1), dim3(TREE_SMALL_THREADS), 0, st, ta, t_small);
         HIP_LAUNCH_CHECK();
     }
 }

@@ -56,6 +56,51 @@ def test_tree_and_tree_mean(oracle, ctx, shape, nb, seed):
     assert np.array_equal(_bits(A.APRTreeNumerics.fill_tree_mean(g, pf)), _bits(o.fill_tree_mean(pf)))
 
 
+@pytest.mark.parametrize("shape,nb,seed", [((3, 9, 511), 6, 1), ((5, 4, 513), 6, 2), ((18, 35, 129), 9, 3), ((4, 7, 1026), 9, 4), ((3, 5, 4133), 9, 5)])
+def test_tree_mean_pieces(oracle, ctx, shape, nb, seed):
+    """child rows of one piece and a cell more (512; 128 in the launch of the small levels), rows of several
+    pieces, and odd dims, whose last children are scaled"""
+    img, o, g = _pair(oracle, ctx, shape, nb, seed)
+    parts = o.sample(img)
+    for p in (parts, parts.astype(np.float32) * np.float32(0.83)):
+        assert np.array_equal(_bits(A.APRTreeNumerics.fill_tree_mean(g, p)), _bits(o.fill_tree_mean(p)))
+
+
+# y one short of, at and past a block's 64 and a row image's 1024; x about a block's 16; few and many planes
+EDGES = [((8, 17, 63), 5, 1), ((7, 15, 65), 5, 2), ((41, 16, 64), 8, 3), ((9, 33, 129), 8, 4), ((8, 7, 1027), 9, 5)]
+
+
+def _wide(o, stack):
+    """particles of the levels whose lines are longer than half their stencil: in shorter ones the oracle's
+    window holds what the level before left there"""
+    y, x, z = o.dims
+    keep = []
+    for l, n in _particles_per_level(o):
+        s, k = 1 << (o.l_max - l), stack[min(o.l_max - l, len(stack) - 1)].shape
+        keep.append(np.full(n, all(-(-d // s) > m // 2 for d, m in zip((z, x, y), k))))
+    return np.concatenate(keep)
+
+
+@pytest.mark.parametrize("shape,nb,seed", EDGES)
+@pytest.mark.parametrize("size", [3, 5, 7, 9])
+@pytest.mark.parametrize("reflect", [True, False])
+def test_convolve_cubic_edges(oracle, ctx, shape, nb, seed, size, reflect):
+    """cubic stencils without symmetry in reference order; and one level's stencil of another form, which
+    takes the list of all levels to the other kernels"""
+    img, o, g = _pair(oracle, ctx, shape, nb, seed)
+    parts = o.sample(img)
+    rng = np.random.default_rng(seed)
+    stack = oracle.downsampled_stencils(rng.uniform(-1, 1, (size,) * 3).astype(np.float32), o.l_max - o.l_min, False, "oracle")
+    w = _wide(o, stack)
+    assert w.mean() > 0.5
+    for p in (parts, parts.astype(np.float32) * np.float32(0.83)):
+        got = A.APRFilter.convolve_pencil(g, stack, p, reflect_boundary=reflect)
+        assert np.array_equal(_bits(got)[w], _bits(o.convolve_pencil(stack, p, reflect))[w])
+    stack[-1] = rng.uniform(-1, 1, (3, 1, 3)).astype(np.float32)
+    got = A.APRFilter.convolve_pencil(g, stack, parts, reflect_boundary=reflect)
+    assert np.array_equal(_bits(got)[w], _bits(o.convolve_pencil(stack, parts, reflect))[w])
+
+
 @pytest.mark.parametrize("shape,nb,seed", CASES)
 @pytest.mark.parametrize("kind", ["mean3", "gauss5", "aniso"])
 @pytest.mark.parametrize("reflect", [True, False])
@@ -246,6 +291,39 @@ def test_convolve_separable_mode(oracle, sep_ctx, shape, nb, seed, kind, reflect
         e_exact, e_sep = _rel(exp, gt).max(), _rel(got, gt).max()
         print(f"vs float64 ground truth: reference order {e_exact:.2e}, separable {e_sep:.2e}")
         assert e_sep < 1e-5 and e_exact < 1e-5
+
+
+@pytest.mark.parametrize("shape,nb,seed", EDGES)
+@pytest.mark.parametrize("size", [1, 3, 5, 7, 9, 11, 13])
+@pytest.mark.parametrize("reflect", [True, False])
+def test_convolve_separable_edges(oracle, sep_ctx, shape, nb, seed, size, reflect):
+    """every cubic size; weights and values are positive, so the reference order's size^3 roundings and the
+    three passes' 3 size bound the difference, with 3 more for the factors"""
+    img, o, g = _pair(oracle, sep_ctx, shape, nb, seed)
+    parts = o.sample(img).astype(np.float32)
+    stack = oracle.downsampled_stencils(oracle.gaussian_stencil((size / 4.0,) * 3, (size,) * 3, True), o.l_max - o.l_min, True, "oracle")
+    exp = o.convolve_pencil(stack, parts, reflect)
+    got = A.APRFilter.convolve_pencil(g, stack, parts, reflect_boundary=reflect)
+    w = _wide(o, stack)
+    assert w.any()
+    assert _rel(got, exp)[w].max() <= 2 * (max(size, 3) ** 3 + 3 * max(size, 3) + 3) * 2.0 ** -24
+
+
+@pytest.mark.parametrize("size", [5, 9])
+@pytest.mark.parametrize("separable", [False, True])
+def test_richardson_lucy_edges(oracle, ctx, sep_ctx, size, separable):
+    """the ratio and the update, made where the convolutions write their results"""
+    c = sep_ctx if separable else ctx
+    img, o, g = _pair(oracle, c, (21, 33, 65), 20, 6)
+    psf = oracle.gaussian_stencil((1.0, 1.0, 1.5), (size,) * 3, True)
+    assert _wide(o, oracle.downsampled_stencils(psf, o.l_max - o.l_min, True, "oracle")).all()
+    for parts in (o.sample(img), o.sample(img).astype(np.float32) * np.float32(0.83)):
+        uo, _, _ = o.richardson_lucy(parts, psf, 2)
+        ug, _ = A.APRNumerics.richardson_lucy(g, parts, None, psf, 2, normalize=True)
+        if separable:
+            assert _rel(ug, uo).max() < 1e-5
+        else:
+            assert np.array_equal(_bits(ug), _bits(uo))
 
 
 def test_richardson_lucy_tv_separable_mode(oracle, sep_ctx):
