@@ -483,8 +483,8 @@ __global__ __launch_bounds__(CT) void k_conv_tile(ConvArgs<TIn> a) {
  * over 1000 x 1024 x 250, 1.6 ms of them), the separable form instruction issue and the latency left
  * between two barriers a plane.  Levels of one stencil size share a launch.  With windows assembled from
  * the particle rows in every block, level after level: 5x5x5 in reference order on 1000 x 1024 x 250 6.7 ms
- * for the levels' launches, now 2.05 and 0.74 for the images; 9x9x9 separable on 1024 x 1024 x 256 3.2 ms,
- * now 1.45 and 0.77; 3x3x3 on 256 x 256 x 128 0.39 ms in eight launches, now 0.047 and 0.036. */
+ * for the levels' launches, now 2.05 and 0.5 for the images; 9x9x9 separable on 1024 x 1024 x 256 3.2 ms,
+ * now 1.45 and 0.5; 3x3x3 on 256 x 256 x 128 0.39 ms in eight launches, now 0.047 and 0.030. */
 constexpr int CONV_LEVELS = 24;
 struct DenseLevel {
     int64_t Y, X, Z;
