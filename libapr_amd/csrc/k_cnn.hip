@@ -87,28 +87,18 @@ __device__ __forceinline__ void decompose(int v, int s, int& z, int& x, int& y) 
     y = r - x * s;
 }
 
-/* the four voxels vp .. vp + 3 of one channel of a planar activation, n of them inside the row: one
-   8-byte store (any alignment) where the row holds all four */
-__device__ __forceinline__ void store_planar4(uint16_t* p, const uint16_t (&h)[4], int n) {
-    if (n >= 4) {
-        const uint32_t w[2] = {pack2(h[0], h[1]), pack2(h[2], h[3])};
-        __builtin_memcpy(p, w, 8);
-    } else {
-#pragma unroll
-        for (int i = 0; i < 3; ++i)
-            if (i < n) p[i] = h[i];
-    }
+/* four channels of a channel-last activation */
+__device__ __forceinline__ void store_channels(uint16_t* p, const uint16_t (&h)[4]) {
+    *(uint2*)p = make_uint2(pack2(h[0], h[1]), pack2(h[2], h[3]));
 }
 
 /* ---------------- forward ---------------- */
 
 /* The forward layers run over bricks of 16 (y) x 8 (x) x 4 (z) output voxels.  A block stages the
-   brick's input, (brick + 2)^3 voxels, in LDS once, and its four waves take
-   the brick's 32 y rows of 16 voxels in turn: row (kx, kz) is one 16 x 16 x 32 MFMA chain with the
-   row's 16 voxels as M.  Every brick has the full layout, so a voxel's place is a shift and a mask;
-   rows past the output's x or z edge are skipped, lanes past its y edge compute rows that are never
-   stored (an MFMA row depends on its own A row only).  The one tap that does not exist (27, in the
-   odd half of pair 13) reads tap 26's data against zero weights. */
+   brick's input, (brick + 2)^3 voxels, in LDS once, and its four waves take the brick's 32 y rows of 16
+   voxels: a row is the N of its MFMAs.  Every brick has the full layout, so a voxel's place is a shift
+   and a mask; rows past the output's x or z edge and lanes past its y edge are never stored (an MFMA
+   column depends on its own operand column only). */
 constexpr int BY = 16, BX = 8, BZ = 4, IY = BY + 2, IX = BX + 2, IZ = BZ + 2, ROWS = BX * BZ;
 
 /* brick br of a launch over T tiles of nby x nbx x nbz bricks, y fastest.  The kernels number
@@ -129,36 +119,85 @@ __device__ __forceinline__ void brick_origin(uint32_t br, uint32_t nby, uint32_t
 /* LDS offset (in voxels of the staged brick) of tap t */
 __host__ __device__ constexpr int tap_vox(int t) { return ((t / 9) * IX + (t / 3) % 3) * IY + t % 3; }
 __device__ __forceinline__ int tap_lds(int tap) { return tap_vox(min(tap, NT - 1)); }
-/* odd tap 2p + 1 minus even tap 2p in voxels: 1, IY - 2 or IX * IY - 2 IY - 2; 0 for pair 13,
-   whose odd half (tap 27) re-reads tap 26 */
-__host__ __device__ constexpr int pair_step(int p) { return p == NPAIR - 1 ? 0 : tap_vox(2 * p + 1) - tap_vox(2 * p); }
+/* The 27 taps of a 16 -> 16 layer in 14 pairs, one MFMA each (K = 2 taps x 16 channels), such that one A
+   operand serves many outputs: pairs 0-8 are dy = 0, 1 of row (dz, dx); 9-11 are dy = 2 of (dz, 0) and
+   (dz, 1); 12 is dy = 2 of (0, 2) and (1, 2); 13 is tap 26 alone (its odd half has zero weights and reads
+   tap 26 again).  Tap of half h of pair p, NT for none: */
+__host__ __device__ constexpr int pair_tap(int p, int h) {
+    return p < 9 ? 3 * p + h : p < 12 ? 9 * (p - 9) + 3 * h + 2 : p == 12 ? 9 * h + 8 : h ? NT : 26;
+}
 
-/* one y row of a 16 -> 16 layer: lane (g, m) reads channels (g & 1) * 8 .. + 7 of tap
-   2p + (g >> 1) of voxel m as the A operand of pair p.  lb[k] is the lane's offset in the brick
-   plus its odd-tap step of class k (steps 0, 1, IY - 2, IX * IY - 2 IY - 2), so every read is a
-   per-row base and an immediate offset */
-__device__ __forceinline__ f32x4 row_mfma(const uint16_t* tile, int R, const int (&lb)[4], const u32x4 (&w)[NPAIR]) {
-    const uint16_t* b0 = tile + R + lb[0];
-    const uint16_t* b1 = tile + R + lb[1];
-    const uint16_t* b2 = tile + R + lb[2];
-    const uint16_t* b3 = tile + R + lb[3];
-    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+/* Outputs of a wave: WZ x WX rows of 16 voxels from (kz0, kx0) of the brick.  A row (z, x) of the input is
+   read once for each kind of pair and meets every output it belongs to: 56 LDS reads for 112 MFMAs (one
+   read per MFMA asks for twice the LDS rate that the matrix cores then leave).  The weights are the A
+   operand, so lane (g, m), which reads channels (g & 1) * 8 .. + 7 of half g >> 1 of the pair, voxel m,
+   gets channels 4 g .. 4 g + 3 of voxel m: 8 bytes of a channel-last store or mask, where voxels 4 g .. of
+   channel m made four 2-byte accesses of each.  16 tiles of 64^3, forward layers with planar copies
+   245 -> 162 us, input gradients 339 -> 222, first layer 169 -> 85. */
+constexpr int WZ = 2, WX = 4;
+static_assert(4 * WZ * WX == ROWS && BX == 2 * WX && BZ == 2 * WZ, "the four waves' rows make up the brick");
+__device__ __forceinline__ void rows_mfma(const uint16_t* tile, int kz0, int kx0, int lane, const u32x4 (&w)[NPAIR], f32x4 (&acc)[WZ][WX]) {
+    const int g = lane >> 4, lo = ((kz0 * IX + kx0) * IY + (lane & 15)) * CH + (g & 1) * 8, th = g >> 1;
+    const uint16_t* ba = tile + lo + th * CH;                        /* dy 0, 1               */
+    const uint16_t* bb = tile + lo + 2 * CH + th * IY * CH;          /* dy 2 of x, x + 1      */
+    const uint16_t* bc = tile + lo + 2 * CH + th * IX * IY * CH;     /* dy 2 of z, z + 1      */
+    const uint16_t* bd = tile + lo + 2 * CH;                         /* dy 2 alone            */
+    auto add = [&](f32x4& c, u32x4 a, int p) { c = mfma(w[p], a, c); };
+    auto at = [&](const uint16_t* b, int z, int x) { return *(const u32x4*)(b + (z * IX + x) * IY * CH); };
 #pragma unroll
-    for (int p = 0; p < NPAIR; ++p) {
-        const int st = pair_step(p);
-        const uint16_t* b = st == 0 ? b0 : st == 1 ? b1 : st == IY - 2 ? b2 : b3;
-        acc = mfma(*(const u32x4*)(b + tap_vox(2 * p) * CH), w[p], acc);
-    }
-    return acc;
+    for (int z = 0; z < WZ; ++z)
+#pragma unroll
+        for (int x = 0; x < WX; ++x) acc[z][x] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int z = 0; z < WZ + 2; ++z)
+#pragma unroll
+        for (int x = 0; x < WX + 2; ++x) {
+            const u32x4 a = at(ba, z, x);
+#pragma unroll
+            for (int dz = 0; dz < 3; ++dz)
+#pragma unroll
+                for (int dx = 0; dx < 3; ++dx)
+                    if (z - dz >= 0 && z - dz < WZ && x - dx >= 0 && x - dx < WX) add(acc[z - dz][x - dx], a, 3 * dz + dx);
+            if (x < WX) {
+                const u32x4 b = at(bb, z, x);
+#pragma unroll
+                for (int dz = 0; dz < 3; ++dz)
+                    if (z - dz >= 0 && z - dz < WZ) add(acc[z - dz][x], b, 9 + dz);
+            }
+            if (x >= 2 && z < WZ) add(acc[z][x - 2], at(bc, z, x), 12);
+            if (x >= 2 && z >= 2) add(acc[z - 2][x - 2], at(bd, z, x), 13);
+        }
 }
-__device__ __forceinline__ void row_lane_offsets(int m, int g, int (&lb)[4]) {
-    const int lo = m * CH + (g & 1) * 8, th = g >> 1;
-    lb[0] = lo;
-    lb[1] = lo + th * CH;
-    lb[2] = lo + th * (IY - 2) * CH;
-    lb[3] = lo + th * (IX * IY - 2 * IY - 2) * CH;
+
+/* The part of the tiles' outputs that is wanted: tile t covers an image of (y, x, z) from org[3 t ..], and a
+   layer's outputs are wanted `extra` voxels past the image's end (org nullptr: all).  Bricks wholly outside
+   are skipped: nothing wanted depends on what they would hold. */
+struct Need {
+    const int* org;
+    int y, x, z, extra;
+};
+__device__ __forceinline__ bool needed(const Need& n, int t, int z0, int x0, int y0) {
+    if (!n.org) return true;
+    return y0 < n.y - n.org[3 * t] + n.extra && x0 < n.x - n.org[3 * t + 1] + n.extra && z0 < n.z - n.org[3 * t + 2] + n.extra;
 }
-static_assert(pair_step(0) == 1 && pair_step(1) == IY - 2 && pair_step(4) == IX * IY - 2 * IY - 2, "tap steps");
+/* an image whose tiles the network reads and writes in place of tile buffers */
+struct Volume {
+    const void* img;
+    int64_t yn, xn, zn;
+    const int* org;
+    float inv_scale, scale, floor_v;
+    float* out;
+};
+
+__device__ __forceinline__ int64_t refl_any(int64_t q, int64_t n) {
+    /* reflection about the edge samples, repeated for windows wider than the volume */
+    if (q >= 0 && q < n) return q;
+    if (n == 1) return 0;
+    const int64_t per = 2 * (n - 1);
+    q %= per;
+    if (q < 0) q += per;
+    return q < n ? q : per - q;
+}
 
 /* stages the brick's input, IZ x IX x IY voxels of 16 channels from (z0, x0, y0) + off of a tile
    of side sin, as tile[(lz * IX + lx) * IY + ly][16], 16-byte chunk c at tile[8 c].
@@ -202,16 +241,18 @@ __device__ __forceinline__ void stage_brick(uint16_t* tile, const uint16_t* __re
 
 /* layer 1: x (f32, side s0) -> a (bf16, side s1 = s0 - 2), ReLU(conv + b1).  The brick's input goes
    straight to LDS as f32 (global_load_lds_dword, clamped at the far edges as in stage_brick) and
-   is rounded to bf16 when the A operand is built; lane (g, m) holds taps g * 8 .. g * 8 + 7 of
-   voxel m */
+   is rounded to bf16 when the operand is built; lane (g, m) holds taps g * 8 .. g * 8 + 7 of
+   voxel m.  IMG: the input is read from an image of T, reflected past its ends and scaled (before, a pass
+   of its own made the tiles: 74 us per 32 of 72^3) */
 constexpr int NIN1 = IZ * IX * IY, NIN1_PT = (NIN1 + 255) / 256;
+template <typename T, bool IMG>
 __global__ __launch_bounds__(256) void k_l1_lds(const float* __restrict__ x, int s0, int s1, const u32x4* __restrict__ W1p,
                                                 const float* __restrict__ b1, uint16_t* a_cl, uint16_t* a_pl, uint32_t nbricks, uint32_t nby,
-                                                uint32_t nbx, uint32_t nbz) {
+                                                uint32_t nbx, uint32_t nbz, Need need, Volume vol) {
     __shared__ __attribute__((aligned(16))) float tile[NIN1_PT * 256];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), m = lane & 15, g = lane >> 4;
     const u32x4 wb = W1p[lane];
-    const float bias = b1[m];
+    const f32x4 bias = *(const f32x4*)(b1 + g * 4);
     int toff[8];
 #pragma unroll
     for (int j = 0; j < 8; ++j) toff[j] = tap_lds(g * 8 + j);
@@ -219,18 +260,32 @@ __global__ __launch_bounds__(256) void k_l1_lds(const float* __restrict__ x, int
     for (uint32_t br = (uint32_t)xcd_block(blockIdx.x, gridDim.x); br < nbricks; br += gridDim.x) {
         int t, z0, x0, y0;
         brick_origin(br, nby, nbx, nbz, t, z0, x0, y0);
+        if (!needed(need, t, z0, x0, y0)) continue;
         const float* xt = x + (int64_t)t * nin;
         __syncthreads();   /* the previous brick's waves are done with the tile */
+        float in[NIN1_PT];
 #pragma unroll
         for (int j = 0; j < NIN1_PT; ++j) {
             const int c = threadIdx.x + 256 * j;
+            in[j] = 0.0f;
             if (c < NIN1) {
                 const int ly = c % IY, r = c / IY, lx = r % IX, lz = r / IX;
                 const int zi = min(z0 + lz, s0 - 1), xi = min(x0 + lx, s0 - 1), yi = min(y0 + ly, s0 - 1);
-                __builtin_amdgcn_global_load_lds((const void*)(xt + (zi * s0 + xi) * s0 + yi), LDS_PTR(tile + wave * 64 + 256 * j), 4, 0, 0);
+                if constexpr (IMG) {
+                    const int64_t gy = refl_any(vol.org[3 * t] - 4 + yi, vol.yn), gx = refl_any(vol.org[3 * t + 1] - 4 + xi, vol.xn),
+                                  gz = refl_any(vol.org[3 * t + 2] - 4 + zi, vol.zn);
+                    in[j] = (float)((const T*)vol.img)[(gz * vol.xn + gx) * vol.yn + gy] * vol.inv_scale;
+                } else {
+                    __builtin_amdgcn_global_load_lds((const void*)(xt + (zi * s0 + xi) * s0 + yi), LDS_PTR(tile + wave * 64 + 256 * j), 4, 0, 0);
+                }
             }
         }
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        if constexpr (IMG) {
+#pragma unroll
+            for (int j = 0; j < NIN1_PT; ++j) tile[threadIdx.x + 256 * j] = in[j];
+        } else {
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        }
         __syncthreads();
         for (int row = wave; row < ROWS; row += 4) {
             const int kx = row % BX, kz = row / BX;
@@ -241,122 +296,154 @@ __global__ __launch_bounds__(256) void k_l1_lds(const float* __restrict__ x, int
             for (int j = 0; j < 8; ++j) f[j] = base[toff[j]];
             const u32x4 av = {pack2_bf16(f[0], f[1]), pack2_bf16(f[2], f[3]), pack2_bf16(f[4], f[5]), pack2_bf16(f[6], f[7])};
             f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-            acc = mfma(av, wb, acc);
-            const int vrow = ((z0 + kz) * s1 + x0 + kx) * s1 + y0 + g * 4;
-            const int64_t vc = ((int64_t)t * nv + vrow) * CH + m;
-            const int64_t vp = ((int64_t)t * CH + m) * nv + vrow;
+            acc = mfma(wb, av, acc);
+            if (y0 + m >= s1) continue;
+            /* channels 4 g .. of voxel m */
+            const int v = ((z0 + kz) * s1 + x0 + kx) * s1 + y0 + m;
             uint16_t hv[4];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                hv[i] = f2bf_hw(fmaxf(acc[i] + bias, 0.0f));
-                if (y0 + g * 4 + i < s1) a_cl[vc + i * CH] = hv[i];
+            for (int i = 0; i < 4; ++i) hv[i] = f2bf_hw(fmaxf(acc[i] + bias[i], 0.0f));
+            store_channels(a_cl + ((int64_t)t * nv + v) * CH + g * 4, hv);
+            if (a_pl) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) a_pl[((int64_t)t * CH + g * 4 + i) * nv + v] = hv[i];
             }
-            if (a_pl) store_planar4(a_pl + vp, hv, s1 - (y0 + g * 4));
         }
     }
 }
 
 /* 16 -> 16 convolution: out(v) = sum_tap W[tap] in(v + tap + off) (zero outside the input), then
    + bias, ReLU, and / or the mask (ReLU derivative of a stored activation).  K of an MFMA is a pair
-   of taps x 16 input channels: lane (g, m) holds channels (g & 1) * 8 .. + 7 of tap 2p + (g >> 1) */
+   of taps x 16 input channels (rows_mfma) */
 template <bool DIRECT>
-__global__ __launch_bounds__(256) void k_conv16_lds(const uint16_t* __restrict__ in_cl, int sin, int sout, int off,
+__global__ __launch_bounds__(256, 3) void k_conv16_lds(const uint16_t* __restrict__ in_cl, int sin, int sout, int off,
                                                     const u32x4* __restrict__ Wp, const float* __restrict__ bias,
                                                     const uint16_t* __restrict__ mask_cl, uint16_t* out_cl, uint16_t* out_pl, int relu,
-                                                    uint32_t nbricks, uint32_t nby, uint32_t nbx, uint32_t nbz) {
+                                                    uint32_t nbricks, uint32_t nby, uint32_t nbx, uint32_t nbz, Need need) {
     __shared__ __attribute__((aligned(16))) uint16_t tile[IZ * IX * IY * CH];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), m = lane & 15, g = lane >> 4;
+    const int kz0 = (wave >> 1) * WZ, kx0 = (wave & 1) * WX;
     u32x4 w[NPAIR];
 #pragma unroll
     for (int p = 0; p < NPAIR; ++p) w[p] = Wp[p * 64 + lane];
-    const float bv = bias ? bias[m] : 0.0f;
-    int lb[4];
-    row_lane_offsets(m, g, lb);
+    f32x4 bv = {0.f, 0.f, 0.f, 0.f};
+    if (bias) bv = *(const f32x4*)(bias + g * 4);
     const int nv = sout * sout * sout;
     for (uint32_t br = (uint32_t)xcd_block(blockIdx.x, gridDim.x); br < nbricks; br += gridDim.x) {
         int t, z0, x0, y0;
         brick_origin(br, nby, nbx, nbz, t, z0, x0, y0);
+        if (!needed(need, t, z0, x0, y0)) continue;
         stage_brick<DIRECT>(tile, in_cl + (int64_t)t * sin * sin * sin * CH, sin, off, z0, x0, y0);
-        for (int row = wave; row < ROWS; row += 4) {
-            const int kx = row % BX, kz = row / BX;
-            if (x0 + kx >= sout || z0 + kz >= sout) continue;
-            const f32x4 acc = row_mfma(tile, (kz * IX + kx) * IY * CH, lb, w);
-            /* this lane's four outputs: voxels vrow + g * 4 + i, channel m */
-            const int vrow = ((z0 + kz) * sout + x0 + kx) * sout + y0 + g * 4;
-            const int64_t vc = ((int64_t)t * nv + vrow) * CH + m;
-            const int64_t vp = ((int64_t)t * CH + m) * nv + vrow;
-            uint16_t hv[4] = {0, 0, 0, 0};
+        if (x0 + kx0 >= sout || z0 + kz0 >= sout) continue;
+        f32x4 acc[WZ][WX];
+        rows_mfma(tile, kz0, kx0, lane, w, acc);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                if (y0 + g * 4 + i < sout) {
-                    float val = acc[i] + bv;
+        for (int kz = 0; kz < WZ; ++kz)
+#pragma unroll
+            for (int kx = 0; kx < WX; ++kx) {
+                const int zo = z0 + kz0 + kz, xo = x0 + kx0 + kx;
+                if (xo >= sout || zo >= sout) continue;
+                const int vrow = (zo * sout + xo) * sout + y0;
+                uint16_t hv[4];
+                /* channels 4 g .. of voxel m */
+                if (y0 + m >= sout) continue;
+                const int64_t vc = ((int64_t)t * nv + vrow + m) * CH + g * 4;
+                uint16_t mk[4];
+                if (mask_cl) __builtin_memcpy(mk, __builtin_assume_aligned(mask_cl + vc, 8), 8);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    float val = acc[kz][kx][i] + bv[i];
                     if (relu) val = fmaxf(val, 0.0f);
-                    if (mask_cl && !(bf2f(mask_cl[vc + i * CH]) > 0.0f)) val = 0.0f;
+                    if (mask_cl && !(bf2f(mk[i]) > 0.0f)) val = 0.0f;
                     hv[i] = f2bf_hw(val);
-                    if (out_cl) out_cl[vc + i * CH] = hv[i];
+                }
+                if (out_cl) store_channels(out_cl + vc, hv);
+                if (out_pl) {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) out_pl[((int64_t)t * CH + g * 4 + i) * nv + vrow + m] = hv[i];
                 }
             }
-            if (out_pl) store_planar4(out_pl + vp, hv, sout - (y0 + g * 4));
-        }
     }
 }
 
 /* layer 4 + residual (+ loss gradient): y = x(centre) + b4 + sum W4 a3, on the MFMA.  The weights
-   keep f32 accuracy as two bf16 parts: W4p holds bf16(W4) in output columns 0-7 and
-   bf16(W4 - bf16(W4)) in columns 8-15, so column 0 + column 8 is the layer's output.  Lane
-   (g, m < 4) takes voxel g * 4 + m of its row, and a row's 16 outputs leave in one coalesced store.
+   keep f32 accuracy as two bf16 parts: W4p holds bf16(W4) in output channels 0-7 and
+   bf16(W4 - bf16(W4)) in channels 8-15, so channel 0 + channel 8 is the layer's output.  Lane
+   m < 16 takes voxel m of each row.
    With a target, also the loss gradient g4 = 2 (y - tgt) gscale and per-block partial sums of
-   (y - tgt)^2 and g4 */
-__global__ __launch_bounds__(256) void k_l4_lds(const uint16_t* __restrict__ a3_cl, int S, const float* __restrict__ x,
+   (y - tgt)^2 and g4.  IMG: the residual comes from an image of T and the output goes to one, scaled and
+   floored (before, a pass of its own wrote the tiles back: 27 us per 32 of 64^3) */
+template <typename T, bool IMG>
+__global__ __launch_bounds__(256, 3) void k_l4_lds(const uint16_t* __restrict__ a3_cl, int S, const float* __restrict__ x,
                                                 const u32x4* __restrict__ W4p, const float* __restrict__ b4, const float* __restrict__ tgt,
                                                 float* y, float* g4, float gscale, double* part, uint32_t nbricks, uint32_t nby, uint32_t nbx,
-                                                uint32_t nbz) {
+                                                uint32_t nbz, Need need, Volume vol) {
     __shared__ __attribute__((aligned(16))) uint16_t tile[IZ * IX * IY * CH];
-    __shared__ double red[2][256];
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), m = lane & 15, g = lane >> 4;
+    __shared__ double red[2][IMG ? 1 : 256];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int kz0 = (wave >> 1) * WZ, kx0 = (wave & 1) * WX;
     u32x4 w[NPAIR];
 #pragma unroll
     for (int p = 0; p < NPAIR; ++p) w[p] = W4p[p * 64 + lane];
     const float bv = b4[0];
-    int lb[4];
-    row_lane_offsets(m, g, lb);
     const int s3 = S + 2, s0 = S + 8;
     const int nv = S * S * S, n3 = s3 * s3 * s3, n0 = s0 * s0 * s0;
     double dsum = 0, gsum = 0;
     for (uint32_t br = (uint32_t)xcd_block(blockIdx.x, gridDim.x); br < nbricks; br += gridDim.x) {
         int t, z0, x0, y0;
         brick_origin(br, nby, nbx, nbz, t, z0, x0, y0);
+        if (!needed(need, t, z0, x0, y0)) continue;
         stage_brick<true>(tile, a3_cl + (int64_t)t * n3 * CH, s3, 0, z0, x0, y0);
-        for (int row = wave; row < ROWS; row += 4) {
-            const int kx = row % BX, kz = row / BX;
-            if (x0 + kx >= S || z0 + kz >= S) continue;
-            /* the residual (and target) loads go out before the MFMA chain */
-            const int zo = z0 + kz, xo = x0 + kx, yo = y0 + g * 4 + m;
-            const bool mine = m < 4 && yo < S;
-            const int64_t i = (int64_t)t * nv + (zo * S + xo) * S + yo;
-            float xv = 0.0f, tv = 0.0f;
-            if (mine) {
-                xv = x[(int64_t)t * n0 + ((zo + 4) * s0 + xo + 4) * s0 + yo + 4];
-                if (tgt) tv = tgt[i];
-            }
-            const f32x4 acc = row_mfma(tile, (kz * IX + kx) * IY * CH, lb, w);
-            float sum[4];
+        if (x0 + kx0 >= S || z0 + kz0 >= S) continue;
+        /* the residual (and target) loads go out before the MFMA chains */
+        const int yo = y0 + lane;
+        float xv[WZ][WX], tv[WZ][WX];
+        int64_t at[WZ][WX];
 #pragma unroll
-            for (int k = 0; k < 4; ++k) sum[k] = acc[k] + __shfl_down(acc[k], 8, 16);
-            if (mine) {
-                const float a = m == 0 ? sum[0] : m == 1 ? sum[1] : m == 2 ? sum[2] : sum[3];
-                const float out = xv + bv + a;
-                y[i] = out;
-                if (tgt) {
-                    const float d = out - tv;
-                    const float gv = 2.0f * d * gscale;
-                    g4[i] = gv;
-                    dsum += (double)d * (double)d;
-                    gsum += (double)gv;
+        for (int kz = 0; kz < WZ; ++kz)
+#pragma unroll
+            for (int kx = 0; kx < WX; ++kx) {
+                const int zo = z0 + kz0 + kz, xo = x0 + kx0 + kx;
+                bool mine = lane < 16 && yo < S && xo < S && zo < S;
+                xv[kz][kx] = tv[kz][kx] = 0.0f;
+                if constexpr (IMG) {
+                    const int64_t gy = vol.org[3 * t] + yo, gx = vol.org[3 * t + 1] + xo, gz = vol.org[3 * t + 2] + zo;
+                    mine = mine && gy < vol.yn && gx < vol.xn && gz < vol.zn;
+                    at[kz][kx] = mine ? (gz * vol.xn + gx) * vol.yn + gy : -1;
+                    if (mine) xv[kz][kx] = (float)((const T*)vol.img)[at[kz][kx]] * vol.inv_scale;
+                } else {
+                    at[kz][kx] = mine ? (int64_t)t * nv + (zo * S + xo) * S + yo : -1;
+                    if (mine) {
+                        xv[kz][kx] = x[(int64_t)t * n0 + ((zo + 4) * s0 + xo + 4) * s0 + yo + 4];
+                        if (tgt) tv[kz][kx] = tgt[at[kz][kx]];
+                    }
                 }
             }
-        }
+        f32x4 acc[WZ][WX];
+        rows_mfma(tile, kz0, kx0, lane, w, acc);
+#pragma unroll
+        for (int kz = 0; kz < WZ; ++kz)
+#pragma unroll
+            for (int kx = 0; kx < WX; ++kx) {
+                const float a = acc[kz][kx][0] + __shfl_down(acc[kz][kx][0], 32, 64);
+                const int64_t i = at[kz][kx];
+                if (i < 0) continue;
+                const float out = xv[kz][kx] + bv + a;
+                if constexpr (IMG) {
+                    vol.out[i] = fmaxf(out * vol.scale, vol.floor_v);
+                } else {
+                    y[i] = out;
+                    if (tgt) {
+                        const float d = out - tv[kz][kx];
+                        const float gv = 2.0f * d * gscale;
+                        g4[i] = gv;
+                        dsum += (double)d * (double)d;
+                        gsum += (double)gv;
+                    }
+                }
+            }
     }
+    if constexpr (IMG) return;
     if (!part) return;
     red[0][threadIdx.x] = dsum;
     red[1][threadIdx.x] = gsum;
@@ -713,7 +800,7 @@ __global__ void k_pack(const float* __restrict__ P, u32x4* W1p, u32x4* W2p, u32x
         /* layer 4: bf16(W4[tap][cin]) in output columns 0-7, the bf16 remainder in columns 8-15 */
         const int q = idx - 64 - 4 * NPAIR * 64;
         const int p = q / 64, l = q % 64, n = l & 15, g = l >> 4;
-        const int tap = 2 * p + (g >> 1), c0 = (g & 1) * 8;
+        const int tap = pair_tap(p, g >> 1), c0 = (g & 1) * 8;
         for (int j = 0; j < 8; ++j) {
             const float wv = tap < NT ? P[OFF_W4 + tap * CH + c0 + j] : 0.0f;
             const uint16_t hi = f2bf(wv);
@@ -724,7 +811,7 @@ __global__ void k_pack(const float* __restrict__ P, u32x4* W1p, u32x4* W2p, u32x
         const int r = idx - 64;
         const int which = r / (NPAIR * 64), q = r % (NPAIR * 64);
         const int p = q / 64, l = q % 64, n = l & 15, g = l >> 4;
-        const int tap = 2 * p + (g >> 1), c0 = (g & 1) * 8;
+        const int tap = pair_tap(p, g >> 1), c0 = (g & 1) * 8;
         const int offw = (which == 0 || which == 2) ? OFF_W2 : OFF_W3;
         const bool transposed = which >= 2;
         for (int j = 0; j < 8; ++j) {
@@ -741,44 +828,20 @@ __global__ void k_pack(const float* __restrict__ P, u32x4* W1p, u32x4* W2p, u32x
     *dst = (u32x4){pack2(h[0], h[1]), pack2(h[2], h[3]), pack2(h[4], h[5]), pack2(h[6], h[7])};
 }
 
-__device__ __forceinline__ int64_t refl_any(int64_t q, int64_t n) {
-    /* reflection about the edge samples, repeated for windows wider than the volume */
-    if (n == 1) return 0;
-    const int64_t per = 2 * (n - 1);
-    q %= per;
-    if (q < 0) q += per;
-    return q < n ? q : per - q;
-}
-
-/* tiles of side s = size + 2 * halo starting at (origin - halo), reflect-padded, divided by scale */
+/* tiles of side s = size + 2 * halo starting at (origin - halo), reflect-padded, divided by scale; tiles along
+   the grid's y */
 template <typename T>
 __global__ void k_extract(const T* __restrict__ img, int64_t yn, int64_t xn, int64_t zn, const int* __restrict__ org, int ntiles, int s, int halo,
                           float inv_scale, float* out) {
     const int64_t nv = (int64_t)s * s * s;
-    const int64_t total = nv * ntiles;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += (int64_t)gridDim.x * blockDim.x) {
-        const int t = (int)(i / nv);
-        const int v = (int)(i % nv);
-        int z, x, y;
-        decompose(v, s, z, x, y);
-        const int64_t gy = refl_any((int64_t)org[3 * t] - halo + y, yn);
-        const int64_t gx = refl_any((int64_t)org[3 * t + 1] - halo + x, xn);
-        const int64_t gz = refl_any((int64_t)org[3 * t + 2] - halo + z, zn);
-        out[i] = (float)img[(gz * xn + gx) * yn + gy] * inv_scale;
-    }
-}
-
-/* tile outputs back into the image (voxels inside the volume), times scale, floored at `floor_v` */
-__global__ void k_scatter_tiles(const float* __restrict__ yt, int S, const int* __restrict__ org, int ntiles, int64_t yn, int64_t xn,
-                                int64_t zn, float scale, float floor_v, float* img) {
-    const int64_t nv = (int64_t)S * S * S;
-    const int64_t total = nv * ntiles;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += (int64_t)gridDim.x * blockDim.x) {
-        const int t = (int)(i / nv);
-        int z, x, y;
-        decompose((int)(i % nv), S, z, x, y);
-        const int64_t gy = org[3 * t] + y, gx = org[3 * t + 1] + x, gz = org[3 * t + 2] + z;
-        if (gy < yn && gx < xn && gz < zn) img[(gz * xn + gx) * yn + gy] = fmaxf(yt[i] * scale, floor_v);
+    for (int t = blockIdx.y; t < ntiles; t += gridDim.y) {
+        for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < nv; i += (int64_t)gridDim.x * blockDim.x) {
+            const uint32_t v = (uint32_t)i, row = v / (uint32_t)s, y = v - row * (uint32_t)s, z = row / (uint32_t)s, x = row - z * (uint32_t)s;
+            const int64_t gy = refl_any((int64_t)org[3 * t] - halo + y, yn);
+            const int64_t gx = refl_any((int64_t)org[3 * t + 1] - halo + x, xn);
+            const int64_t gz = refl_any((int64_t)org[3 * t + 2] - halo + z, zn);
+            out[t * nv + i] = (float)img[(gz * xn + gx) * yn + gy] * inv_scale;
+        }
     }
 }
 
@@ -845,14 +908,14 @@ Bricks bricks(int T, int s, int64_t cap) {
 
 /* 16 -> 16 convolution of T tiles (input side sin, output side sout, input offset off) */
 void conv16(hipStream_t st, const uint16_t* in_cl, int sin, int sout, int off, const u32x4* Wp, const float* bias,
-            const uint16_t* mask_cl, uint16_t* out_cl, uint16_t* out_pl, int relu, int T) {
+            const uint16_t* mask_cl, uint16_t* out_cl, uint16_t* out_pl, int relu, int T, Need need = Need()) {
     const Bricks b = bricks(T, sout, 65536);
-    if (off == 0)
-        hipLaunchKernelGGL(k_conv16_lds<true>, dim3(b.grid), kBlk, 0, st, in_cl, sin, sout, off, Wp, bias, mask_cl, out_cl, out_pl, relu, b.n, b.ny,
-                           b.nx, b.nz);
-    else
-        hipLaunchKernelGGL(k_conv16_lds<false>, dim3(b.grid), kBlk, 0, st, in_cl, sin, sout, off, Wp, bias, mask_cl, out_cl, out_pl, relu, b.n,
-                           b.ny, b.nx, b.nz);
+    auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(b.grid), kBlk, 0, st, in_cl, sin, sout, off, Wp, bias, mask_cl, out_cl, out_pl, relu, b.n, b.ny, b.nx, b.nz,
+                           need);
+    };
+    if (off == 0) launch(k_conv16_lds<true>);
+    else launch(k_conv16_lds<false>);
     HIP_LAUNCH_CHECK();
 }
 
@@ -870,8 +933,10 @@ struct Acts {
 int l4_blocks(int T, int S) { return (int)bricks(T, S, 4096).grid; }
 
 /* forward of T tiles (input side S + 8); planar copies when training; part holds l4_blocks(T, S)
-   pairs of loss partials */
-void forward(aprh_cnn* n, const float* x, int T, int S, float* y, Acts& A, bool train, const float* tgt, float* g4, double* part) {
+   pairs of loss partials.  With an image (dt its type) the tiles at vol->org are read from it and written
+   to its output instead of x and y */
+void forward(aprh_cnn* n, const float* x, int T, int S, float* y, Acts& A, bool train, const float* tgt, float* g4, double* part,
+             const Volume* vol = nullptr, int dt = APRH_DTYPE_F32) {
     hipStream_t st = n->ctx->stream;
     const int s0 = S + 8, s1 = S + 6, s2 = S + 4, s3 = S + 2;
     auto vox = [&](int s) { return (size_t)T * s * s * s; };
@@ -883,20 +948,32 @@ void forward(aprh_cnn* n, const float* x, int T, int S, float* y, Acts& A, bool 
         A.a2p.reset(n->ctx->pool, vox(s2) * CH * 2 + PL_PAD);
         A.a3p.reset(n->ctx->pool, vox(s3) * CH * 2 + PL_PAD);
     }
+    const Volume v = vol ? *vol : Volume();
+    auto need = [&](int extra) { return vol ? Need{v.org, (int)v.yn, (int)v.xn, (int)v.zn, extra} : Need(); };
     const float* P = n->P.as<float>();
     {
         const Bricks b = bricks(T, s1, 65536);
-        hipLaunchKernelGGL(k_l1_lds, dim3(b.grid), kBlk, 0, st, x, s0, s1, (const u32x4*)n->W1p.as<u32x4>(), P + OFF_B1, A.a1c.as<uint16_t>(),
-                           train ? A.a1p.as<uint16_t>() : (uint16_t*)nullptr, b.n, b.ny, b.nx, b.nz);
+        auto launch = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, dim3(b.grid), kBlk, 0, st, x, s0, s1, (const u32x4*)n->W1p.as<u32x4>(), P + OFF_B1, A.a1c.as<uint16_t>(),
+                               train ? A.a1p.as<uint16_t>() : (uint16_t*)nullptr, b.n, b.ny, b.nx, b.nz, need(6), v);
+        };
+        if (!vol) launch(k_l1_lds<float, false>);
+        else if (dt == APRH_DTYPE_U16) launch(k_l1_lds<uint16_t, true>);
+        else launch(k_l1_lds<float, true>);
         HIP_LAUNCH_CHECK();
     }
     conv16(st, A.a1c.as<uint16_t>(), s1, s2, 0, n->W2p.as<u32x4>(), P + OFF_B2, nullptr, A.a2c.as<uint16_t>(),
-           train ? A.a2p.as<uint16_t>() : nullptr, 1, T);
+           train ? A.a2p.as<uint16_t>() : nullptr, 1, T, need(4));
     conv16(st, A.a2c.as<uint16_t>(), s2, s3, 0, n->W3p.as<u32x4>(), P + OFF_B3, nullptr, A.a3c.as<uint16_t>(),
-           train ? A.a3p.as<uint16_t>() : nullptr, 1, T);
-    const Bricks b4 = bricks(T, S, 4096);
-    hipLaunchKernelGGL(k_l4_lds, dim3(b4.grid), kBlk, 0, st, (const uint16_t*)A.a3c.as<uint16_t>(), S, x, (const u32x4*)n->W4p.as<u32x4>(),
-                       P + OFF_B4, tgt, y, g4, 1.0f / (float)vox(S), part, b4.n, b4.ny, b4.nx, b4.nz);
+           train ? A.a3p.as<uint16_t>() : nullptr, 1, T, need(2));
+    const Bricks b4 = bricks(T, S, vol ? 65536 : 4096);
+    auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(b4.grid), kBlk, 0, st, (const uint16_t*)A.a3c.as<uint16_t>(), S, x, (const u32x4*)n->W4p.as<u32x4>(),
+                           P + OFF_B4, tgt, y, g4, 1.0f / (float)vox(S), part, b4.n, b4.ny, b4.nx, b4.nz, need(0), v);
+    };
+    if (!vol) launch(k_l4_lds<float, false>);
+    else if (dt == APRH_DTYPE_U16) launch(k_l4_lds<uint16_t, true>);
+    else launch(k_l4_lds<float, true>);
     HIP_LAUNCH_CHECK();
 }
 
@@ -989,11 +1066,13 @@ double device_mean(aprh_context* ctx, const void* v, int dt, size_t n) {
     return n ? s / (double)n : 0.0;
 }
 
-/* the network over a whole volume in 64^3 tiles; out = y * scale (floored) */
+/* the network over a whole volume in tiles; out = y * scale (floored).  Every output depends on its own
+   neighbourhood alone, so the tiles' size is free: the layers of 74^3 tiles (80^3, 78^3, 76^3) fill their
+   bricks of 16 x 8 x 4 where those of 64^3 (70^3, 68^3, 66^3) leave a fifth of their work outside */
 void apply_volume(aprh_cnn* n, const void* img, int dt, int64_t yn, int64_t xn, int64_t zn, float scale, float floor_v, float* out) {
     hipStream_t st = n->ctx->stream;
     Pool* pool = n->ctx->pool;
-    const int S = 64, s0 = S + 8;
+    const int S = 74;
     const int ty = (int)cdiv(yn, S), tx = (int)cdiv(xn, S), tz = (int)cdiv(zn, S);
     const int ntiles = ty * tx * tz;
     std::vector<int> org((size_t)ntiles * 3);
@@ -1006,22 +1085,12 @@ void apply_volume(aprh_cnn* n, const void* img, int dt, int64_t yn, int64_t xn, 
             }
     Buf dorg(pool, org.size() * 4);
     HIP_CHECK(hipMemcpyAsync(dorg.ptr(), org.data(), org.size() * 4, hipMemcpyHostToDevice, st));
-    const int B = 32;   /* tiles per batch */
-    Buf xin(pool, (size_t)B * s0 * s0 * s0 * 4), y(pool, (size_t)B * S * S * S * 4);
+    const int B = 16;   /* tiles per batch */
     for (int t0 = 0; t0 < ntiles; t0 += B) {
         const int T = std::min(B, ntiles - t0);
-        const int* o = dorg.as<int>() + 3 * t0;
-        if (dt == APRH_DTYPE_U16)
-            hipLaunchKernelGGL(k_extract<uint16_t>, dim3(8192), kBlk, 0, st, (const uint16_t*)img, yn, xn, zn, o, T, s0, 4, 1.0f / scale,
-                               xin.as<float>());
-        else
-            hipLaunchKernelGGL(k_extract<float>, dim3(8192), kBlk, 0, st, (const float*)img, yn, xn, zn, o, T, s0, 4, 1.0f / scale,
-                               xin.as<float>());
-        HIP_LAUNCH_CHECK();
+        const Volume vol{img, yn, xn, zn, dorg.as<int>() + 3 * t0, 1.0f / scale, scale, floor_v, out};
         Acts A;
-        forward(n, xin.as<float>(), T, S, y.as<float>(), A, false, nullptr, nullptr, nullptr);
-        hipLaunchKernelGGL(k_scatter_tiles, dim3(8192), kBlk, 0, st, (const float*)y.as<float>(), S, o, T, yn, xn, zn, scale, floor_v, out);
-        HIP_LAUNCH_CHECK();
+        forward(n, nullptr, T, S, nullptr, A, false, nullptr, nullptr, nullptr, &vol, dt);
     }
     HIP_CHECK(hipStreamSynchronize(st));
 }
@@ -1163,11 +1232,12 @@ int aprh_cnn_extract_tiles(aprh_context* ctx, const void* image, int dtype, int6
     DevIn im(ctx, image, n * (dtype == APRH_DTYPE_U16 ? 2 : 4));
     DevIn org(ctx, origins, (size_t)T * 3 * 4);
     DevOut o(ctx, out, (size_t)T * s * s * s * 4);
+    const dim3 grid((unsigned)std::min<int64_t>(cdiv((int64_t)s * s * s, 256), 8192), (unsigned)std::min(T, 65535));
     if (dtype == APRH_DTYPE_U16)
-        hipLaunchKernelGGL(k_extract<uint16_t>, dim3(8192), kBlk, 0, ctx->stream, (const uint16_t*)im.ptr, y, x, z, (const int*)org.ptr, T, s,
-                           halo, 1.0f / scale, (float*)o.ptr);
+        hipLaunchKernelGGL(k_extract<uint16_t>, grid, kBlk, 0, ctx->stream, (const uint16_t*)im.ptr, y, x, z, (const int*)org.ptr, T, s, halo,
+                           1.0f / scale, (float*)o.ptr);
     else
-        hipLaunchKernelGGL(k_extract<float>, dim3(8192), kBlk, 0, ctx->stream, (const float*)im.ptr, y, x, z, (const int*)org.ptr, T, s, halo,
+        hipLaunchKernelGGL(k_extract<float>, grid, kBlk, 0, ctx->stream, (const float*)im.ptr, y, x, z, (const int*)org.ptr, T, s, halo,
                            1.0f / scale, (float*)o.ptr);
     HIP_LAUNCH_CHECK();
     o.finish(ctx);

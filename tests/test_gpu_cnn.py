@@ -137,6 +137,22 @@ def test_apply_equals_tiles(ctx):
         np.testing.assert_allclose(blk, yt[k][:blk.shape[0], :blk.shape[1], :blk.shape[2]], rtol=1e-6, atol=1e-3)
 
 
+@pytest.mark.parametrize("shape", [(1, 1, 1), (3, 75, 74), (9, 73, 149), (76, 5, 80), (2, 10, 17)])
+@pytest.mark.parametrize("dtype", [np.uint16, np.float32])
+def test_apply_ragged(ctx, shape, dtype):
+    """volumes that end just past, at and before a tile's or a brick's end, and shorter than the halo: each
+    output depends on its reflected neighbourhood alone, so tiles of another size give the same values"""
+    net = A.WarmStartCNN(ctx, params=rand_params(9))
+    img = (np.random.default_rng(3).random(shape) * 500 + 100).astype(dtype)
+    out = net.apply(img, scale=250.0)
+    S, (z, x, y) = 20, shape
+    org = [(oy, ox, oz) for oz in range(0, z, S) for ox in range(0, x, S) for oy in range(0, y, S)]
+    yt = net.forward_tiles(A.extract_tiles(img, (y, x, z), org, S, 4, 250.0), S) * 250.0
+    for k, (oy, ox, oz) in enumerate(org):
+        blk = out[oz:oz + S, ox:ox + S, oy:oy + S]
+        np.testing.assert_allclose(blk, yt[k][:blk.shape[0], :blk.shape[1], :blk.shape[2]], rtol=1e-6, atol=1e-3)
+
+
 def test_sample_image_f32_matches_oracle(oracle, ctx):
     img16 = A.synth_blobs((29, 45, 61), 3, 12)
     o = oracle.get_apr(img16, oracle.params(rel_error=0.1, sigma_th=50, Ip_th=120, grad_th=10), "oracle")
