@@ -1017,9 +1017,14 @@ void conv_levels(aprh_context* ctx, aprh_apr& a, const std::vector<HostStencil>&
         *nparts = need;
         return p;
     };
+    /* the images of all levels take four times the memory of k_conv_tile's two: up to 2^34 cells (64 GiB) */
     bool dense = a.l_max - a.l_min < CONV_LEVELS;
-    for (int l = a.l_min; l <= a.l_max; ++l) dense = dense && dense_size(stencils[stencil_of(l)], off_sep[stencil_of(l)] >= 0);
-    if (dense) {
+    int64_t cells = 0;
+    for (int l = a.l_min; l <= a.l_max; ++l) {
+        dense = dense && dense_size(stencils[stencil_of(l)], off_sep[stencil_of(l)] >= 0);
+        cells += a.y_num[l] * a.x_num[l] * a.z_num[l];
+    }
+    if (dense && cells <= ((int64_t)1 << 34)) {
         /* the images of all levels, then one launch per stencil form and size, the finest level first */
         std::vector<float*> img((size_t)a.l_max + 1, nullptr);
         int64_t total = 0;
