@@ -5,7 +5,8 @@
  *
  * Network: four "valid" 3x3x3 convolutions, 1 -> 16 -> 16 -> 16 -> 1
  * channels, ReLU after the first three, residual output y = x + conv4.  A
- * tile of side S + 8 gives an output tile of side S (S = 64 in use).
+ * tile of side S + 8 gives an output tile of side S (64 in training, 74
+ * over a whole volume).
  * Parameters (f32 master copy, 14737 values): W1[27][16] b1[16]
  * W2[27][16][16] b2[16] W3[27][16][16] b3[16] W4[27][16] b4, tap =
  * (dz * 3 + dx) * 3 + dy.
@@ -21,8 +22,8 @@
  * MFMA operand layout (16x16x32 bf16, verified on the device): lane l holds
  * A[l % 16][(l / 16) * 8 + j] and B[(l / 16) * 8 + j][l % 16] for j < 8, and
  * the result D[(l / 16) * 4 + i][l % 16] for i < 4.
- *  - convolution (forward and input gradient): M = 16 output voxels, N = 16
- *    output channels, K = pairs of taps x 16 input channels (14 MFMAs);
+ *  - convolution (forward and input gradient): M = 16 output channels, N = 16
+ *    output voxels, K = pairs of taps x 16 input channels (14 MFMAs);
  *  - weight gradient: M = 16 input channels (or taps), N = 16 output
  *    channels (or taps), K = 32 voxels along y.
  */
