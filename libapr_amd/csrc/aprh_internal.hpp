@@ -210,6 +210,11 @@ struct aprh_apr {
     aprh::Buf yidx, t_yidx;                        /* u16                       */
     std::vector<int64_t> yidx_off, t_yidx_off;     /* per level                 */
     int top_tree_regular = -1;                     /* top tree level readable straight from the particle rows: -1 unknown */
+    /* xz_end and y_vec hold another structure now: all that was derived from the last one is made again on next use */
+    void structure_changed() {
+        tree_built = yidx_built = false;
+        top_tree_regular = -1;
+    }
 };
 
 namespace aprh {

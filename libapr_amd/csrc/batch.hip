@@ -262,10 +262,12 @@ void read_slots(aprh_batch* b) {
     for (int i = 0; i < b->n; ++i) {
         b->aprs[i]->total = tot[i];
         b->aprs[i]->bspline_offset = off[i];
-        b->aprs[i]->tree_built = false;
+        b->aprs[i]->structure_changed();
+    }
+    /* the other volumes' APRs are whole also where one overflowed */
+    for (int i = 0; i < b->n; ++i)
         if (err[3 * i] || err[3 * i + 1] || err[3 * i + 2])
             throw Error(APRH_ERR_OVERFLOW, "integer under-/overflow in the B-spline smoothing of batch volume " + std::to_string(i));
-    }
 }
 
 }  // namespace

@@ -87,6 +87,33 @@ def test_batch_mixes_long_and_short_rows(oracle, ctx):
     batch.close()
 
 
+def test_batch_particles_after_each_run(ctx):
+    """the tree, the y-block index and the row shapes that filters derive from a structure belong to one run:
+    dims with several blocks of 64 along y, other images in each run; the same as an APR of its own gives"""
+    dims = [(129, 33, 17), (200, 40, 24)]
+    batch = A.APRBatch(dims, par=_apar(), ctx=ctx)
+    conv = A.APRConverter(ctx)
+    conv.par = _apar()
+    for seed0, blobs in ((10, 3), (50, 40), (90, 8)):
+        imgs = [A.synth_blobs((z, x, y), seed0 + i, blobs) for i, (y, x, z) in enumerate(dims)]
+        for i, img in enumerate(imgs):
+            batch.set_input(i, img)
+        batch.run()
+        for i, img in enumerate(imgs):
+            got, single = batch.get(i), conv.get_apr(img)
+            print(f"seed {seed0} volume {i}: P={got.total} single={single.total}", flush=True)
+            assert got.total == single.total
+            parts = A.ParticleData().sample_image(single, img).astype(np.float32)
+            assert np.array_equal(A.APRTreeNumerics.fill_tree_mean(got, parts), A.APRTreeNumerics.fill_tree_mean(single, parts))
+            for shape in ((3, 3, 3), (3, 5, 3)):
+                st = np.random.default_rng(i).uniform(0, 1, shape).astype(np.float32)
+                g, e = (A.APRFilter.convolve_pencil(a, st, parts) for a in (got, single))
+                assert np.array_equal(g.view(np.uint32), e.view(np.uint32))
+            single.close()
+            got.close()
+    batch.close()
+
+
 def test_batch_rejects_small_volumes(ctx):
     with pytest.raises(A.AprhError) as e:
         A.APRBatch([(64, 64, 64), (4, 4, 4)], ctx=ctx)
