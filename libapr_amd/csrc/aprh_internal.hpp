@@ -192,6 +192,7 @@ struct aprh_apr {
     bool borrowed = false;                         /* owned by a batch plan     */
     aprh::Buf xz_end;                              /* u64[n_xz]                 */
     aprh::Buf y_vec;                               /* u16[total]                */
+    bool complete = true;                          /* every voxel lies in a particle's cell (a conversion's always does) */
     /* optional stage outputs (context keep_intermediates) */
     aprh::Buf smoothed, grad_raw, lis_raw, grad, lis, levels;
     std::vector<aprh::Buf> pct;                    /* final particle-cell tree  */
@@ -337,7 +338,7 @@ struct HostStencil {
 /* APRStencil::get_downsampled_stencils (APRStencil.hpp:81-97) on the host */
 std::vector<HostStencil> downsampled_stencils(const HostStencil& in, int nlevels, bool normalize);
 /* throws APRH_ERR_INVALID_ARGUMENT unless xz_end / y_vec describe a.org's level geometry */
-void validate_structure(aprh_context* ctx, const aprh_apr& a);
+void validate_structure(aprh_context* ctx, aprh_apr& a);
 void ensure_tree(aprh_context* ctx, aprh_apr& a);
 template <typename T>
 void tree_mean(aprh_context* ctx, aprh_apr& a, const T* parts, float* tree);

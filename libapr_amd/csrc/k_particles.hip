@@ -376,17 +376,27 @@ __device__ __forceinline__ void store_staged(E* dst, const E* lds, int n, int la
    piece leaves in 16-byte words.  A lane takes four pixels at a time from one load of y and one of values:
    four entries of level li, two of the next, else a quarter, half or all of one (a lane per pixel issued
    four times the instructions, which bound it: the images of 1024 x 1024 x 256 0.77 ms, now 0.50).  search: the row is longer than the piece.
-   VALS: values from parts / tree to dst, else the levels themselves; LEV: the levels to ldst as bytes */
-template <typename T, typename D, bool VALS, bool LEV>
-__device__ __forceinline__ void recon_piece(const ReconArgs& a, int li, uint32_t z, uint32_t x, int64_t c0, int cn, bool search, D* st,
-                                            uint8_t* ls, D* dst, uint8_t* ldst, int lane) {
+   VALS: values from parts / tree, else the levels themselves; LEV: the levels to ls as bytes.
+   HOLES: the structure's particles need not cover the image: a pixel without any is 0 (as is its level), or
+   takes the coarser tree nodes that are wanted and reach it */
+template <typename T, typename D, bool VALS, bool LEV, bool HOLES>
+__device__ __forceinline__ void recon_stage(const ReconArgs& a, int li, uint32_t z, uint32_t x, int64_t c0, int cn, bool search, D* st,
+                                            uint8_t* ls, int lane) {
     constexpr int LOG = sizeof(D) == 2 ? 11 : 10;
+    if constexpr (HOLES) {
+        for (int i = lane; i < RC_BYTES / (int)sizeof(D); i += 64) {
+            st[i] = (D)0;
+            if (LEV) ls[i] = 0;
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    }
     const int tree = a.trb[li] >= 0 ? li + 1 : -1;
-    /* lane s: the entries of source s under this row (under the piece) */
+    /* lane s: the entries of source s under this row (under the piece), and of the tree nodes of li after them;
+       HOLES: lane 2 s those of level s, lane 2 s + 1 those of its tree nodes */
     uint64_t b = 0, e = 0;
-    if (lane <= li || lane == tree) {
-        const bool tr = lane == tree;
-        const int s = tr ? li : lane, d = li - s;
+    const bool tr = HOLES ? lane & 1 : lane == tree;
+    const int s = HOLES ? lane >> 1 : tr ? li : lane, d = li - s;
+    if (s <= li && (!HOLES || !tr || a.trb[s] >= 0)) {
         const int64_t r = (tr ? a.trb[s] : a.rb[s]) + (int64_t)(z >> d) * a.xn[s] + (x >> d);
         const uint64_t* xz = tr ? a.txz : a.xz;
         b = xz[r - 1];
@@ -400,13 +410,13 @@ __device__ __forceinline__ void recon_piece(const ReconArgs& a, int li, uint32_t
     const int base = (int)c0;
     uint64_t todo = __ballot(e > b);
     while (todo) {
-        const int s = __builtin_ctzll(todo);
+        const int q = __builtin_ctzll(todo);
         todo &= todo - 1;
-        const uint64_t sb = ((uint64_t)__builtin_amdgcn_readlane((int)(b >> 32), s) << 32) | (uint32_t)__builtin_amdgcn_readlane((int)b, s);
-        const int cnt = __builtin_amdgcn_readlane((int)(e - b), s);
-        const bool tr = s == tree;
-        const int d = tr ? 0 : li - s;
-        const int lv = a.l_lo + (tr ? li : s);
+        const uint64_t sb = ((uint64_t)__builtin_amdgcn_readlane((int)(b >> 32), q) << 32) | (uint32_t)__builtin_amdgcn_readlane((int)b, q);
+        const int cnt = __builtin_amdgcn_readlane((int)(e - b), q);
+        const bool tr = HOLES ? q & 1 : q == tree;
+        const int s = HOLES ? q >> 1 : tr ? li : q, d = li - s;
+        const int lv = a.l_lo + s;
         const uint16_t* yv = (tr ? a.tyv : a.yv) + sb;
         /* entries i .. i + E - 1 */
         auto load = [&](auto& y, auto& v, int i) {
@@ -472,6 +482,12 @@ __device__ __forceinline__ void recon_piece(const ReconArgs& a, int li, uint32_t
     }
     /* the wave's own LDS writes are in order; the compiler must not move the reads up */
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+}
+/* the same, and the piece to dst (its levels to ldst) */
+template <typename T, typename D, bool VALS, bool LEV, bool HOLES>
+__device__ __forceinline__ void recon_piece(const ReconArgs& a, int li, uint32_t z, uint32_t x, int64_t c0, int cn, bool search, D* st,
+                                            uint8_t* ls, D* dst, uint8_t* ldst, int lane) {
+    recon_stage<T, D, VALS, LEV, HOLES>(a, li, z, x, c0, cn, search, st, ls, lane);
     store_staged<D>(dst, st, cn, lane);
     if (LEV) store_staged<uint8_t>(ldst, ls, cn, lane);
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   /* the next piece rewrites the stage */
@@ -482,7 +498,7 @@ __device__ __forceinline__ void recon_piece(const ReconArgs& a, int li, uint32_t
    the image is written once.  (Before, a level's image was the coarser one upsampled, then its particles
    scattered over it: three passes over the finest level, 1.12 ms for 1000 x 1023 x 255 u16 against
    0.29 ms, 4.6 TB/s.) */
-template <typename T, typename D, bool VALS, bool LEV>
+template <typename T, typename D, bool VALS, bool LEV, bool HOLES>
 __global__ __launch_bounds__(256) void k_recon(ReconArgs a, ReconImage im) {
     constexpr int CHUNK = RC_BYTES / (int)sizeof(D);
     __shared__ __align__(16) D stage[4][CHUNK];
@@ -493,14 +509,31 @@ __global__ __launch_bounds__(256) void k_recon(ReconArgs a, ReconImage im) {
     for (int64_t rowl = xcd_block(blockIdx.x, gridDim.x) * 4 + wv; rowl < (int64_t)im.rows; rowl += (int64_t)gridDim.x * 4) {
         const uint32_t row = (uint32_t)rowl, z = row / im.X, x = row - z * im.X;
         const int64_t o = (int64_t)row * im.Y + c0;
-        recon_piece<T, D, VALS, LEV>(a, im.li, z, x, c0, cn, gridDim.y > 1, stage[wv], lstage[wv], (D*)im.out + o, LEV ? im.lev + o : nullptr,
-                                     lane);
+        recon_piece<T, D, VALS, LEV, HOLES>(a, im.li, z, x, c0, cn, gridDim.y > 1, stage[wv], lstage[wv], (D*)im.out + o,
+                                            LEV ? im.lev + o : nullptr, lane);
     }
+}
+
+/* *holes when a pixel of the image has no particle */
+__global__ __launch_bounds__(256) void k_holes(ReconArgs a, ReconImage im, int* holes) {
+    constexpr int CHUNK = RC_BYTES / 2;
+    __shared__ __align__(16) uint16_t stage[4][CHUNK];
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t c0 = (int64_t)blockIdx.y * CHUNK;
+    const int cn = (int)min((int64_t)CHUNK, im.Y - c0);
+    bool found = false;
+    for (int64_t rowl = xcd_block(blockIdx.x, gridDim.x) * 4 + wv; rowl < (int64_t)im.rows; rowl += (int64_t)gridDim.x * 4) {
+        const uint32_t row = (uint32_t)rowl, z = row / im.X, x = row - z * im.X;
+        recon_stage<uint16_t, uint16_t, false, false, true>(a, im.li, z, x, c0, cn, gridDim.y > 1, stage[wv], nullptr, lane);
+        for (int i = lane; i < cn; i += 64) found = found || stage[wv][i] == 0;   /* levels start at 1 */
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    }
+    if (found) atomicOr(holes, 1);
 }
 
 /* the float images of several levels in one launch: none of them needs another, and together they fill the
    chip where the coarse ones alone would each cost a launch */
-template <typename T>
+template <typename T, bool HOLES>
 __global__ __launch_bounds__(256) void k_level_images(ReconArgs a, LevelImages m) {
     constexpr int CHUNK = RC_BYTES / 4;
     __shared__ __align__(16) float stage[4][CHUNK];
@@ -512,8 +545,8 @@ __global__ __launch_bounds__(256) void k_level_images(ReconArgs a, LevelImages m
         if (c0 >= m.Y[li]) continue;
         const uint32_t row = (uint32_t)(rg - m.row0[li]), X = m.X[li], z = row / X, x = row - z * X;
         const int cn = (int)min((int64_t)CHUNK, m.Y[li] - c0);
-        recon_piece<T, float, true, false>(a, li, z, x, c0, cn, m.Y[li] > CHUNK, stage[wv], nullptr, m.out[li] + (int64_t)row * m.Y[li] + c0, nullptr,
-                                           lane);
+        recon_piece<T, float, true, false, HOLES>(a, li, z, x, c0, cn, m.Y[li] > CHUNK, stage[wv], nullptr,
+                                                  m.out[li] + (int64_t)row * m.Y[li] + c0, nullptr, lane);
     }
 }
 
@@ -548,7 +581,32 @@ const dim3 kGrid(4096), kBlock(256);
 
 /* ======================================================================== */
 
-void validate_structure(aprh_context* ctx, const aprh_apr& a) {
+namespace {
+/* sources of the images of levels l_min .. hi; tree nodes of level `tree` only, or of all levels below l_max */
+ReconArgs recon_sources(const aprh_apr& a, int hi, int tree = -1) {
+    ReconArgs r;
+    std::memset(&r, 0, sizeof(r));
+    r.l_lo = a.l_min;
+    if (hi - a.l_min >= MAXL) throw Error(APRH_ERR_UNSUPPORTED, "too many levels");
+    for (int l = a.l_min; l <= hi; ++l) {
+        const int i = l - a.l_min;
+        r.rb[i] = (int64_t)a.level_xz_vec[l];
+        r.xn[i] = a.x_num[l];
+        r.trb[i] = l < a.l_max && l <= a.t_l_max && a.t_total > 0 && (tree < 0 || l == tree) ? (int64_t)a.t_level_xz[l] : -1;
+    }
+    r.xz = a.xz_end.as<uint64_t>();
+    r.yv = a.y_vec.as<uint16_t>();
+    r.txz = a.t_xz_end.as<uint64_t>();
+    r.tyv = a.t_y_vec.as<uint16_t>();
+    return r;
+}
+ReconImage recon_image(const aprh_apr& a, int level, void* out, uint8_t* lev) {
+    /* dims are at most 65535, so a level has fewer than 2^32 rows */
+    return {level - a.l_min, (uint32_t)a.x_num[level], (uint32_t)(a.x_num[level] * a.z_num[level]), a.y_num[level], out, lev};
+}
+}  // namespace
+
+void validate_structure(aprh_context* ctx, aprh_apr& a) {
     hipStream_t st = ctx->stream;
     Rows R = make_rows(a.y_num, a.x_num, a.z_num, a.level_xz_vec, a.l_min, a.l_max);
     const int64_t nrows = R.prefix[R.n_levels];
@@ -567,6 +625,15 @@ void validate_structure(aprh_context* ctx, const aprh_apr& a) {
     HIP_CHECK(hipStreamSynchronize(st));
     if (h_err || first != 0 || last != a.total)
         throw Error(APRH_ERR_INVALID_ARGUMENT, "malformed APR structure (xz_end_vec / y_vec do not describe the given dimensions)");
+    /* the particles of a stored structure need not cover the image */
+    const ReconImage im = recon_image(a, a.l_max, nullptr, nullptr);
+    HIP_CHECK(hipMemsetAsync(err.ptr(), 0, 4, st));
+    hipLaunchKernelGGL(k_holes, dim3((unsigned)std::min<int64_t>(cdiv(im.rows, 4), 1 << 20), (unsigned)cdiv(im.Y, RC_BYTES / 2)), kBlock, 0, st,
+                       recon_sources(a, a.l_max), im, err.as<int>());
+    HIP_LAUNCH_CHECK();
+    HIP_CHECK(hipMemcpyAsync(&h_err, err.ptr(), 4, hipMemcpyDeviceToHost, st));
+    HIP_CHECK(hipStreamSynchronize(st));
+    a.complete = h_err == 0;
 }
 
 void ensure_tree(aprh_context* ctx, aprh_apr& a) {
@@ -781,35 +848,12 @@ void convolve(aprh_context* ctx, aprh_apr& a, const std::vector<HostStencil>& st
 }
 
 namespace {
-/* sources of the images of levels l_min .. hi; tree nodes of level `tree` only, or of all levels below l_max */
-ReconArgs recon_sources(const aprh_apr& a, int hi, int tree = -1) {
-    ReconArgs r;
-    std::memset(&r, 0, sizeof(r));
-    r.l_lo = a.l_min;
-    if (hi - a.l_min >= MAXL) throw Error(APRH_ERR_UNSUPPORTED, "too many levels");
-    for (int l = a.l_min; l <= hi; ++l) {
-        const int i = l - a.l_min;
-        r.rb[i] = (int64_t)a.level_xz_vec[l];
-        r.xn[i] = a.x_num[l];
-        r.trb[i] = l < a.l_max && l <= a.t_l_max && a.t_total > 0 && (tree < 0 || l == tree) ? (int64_t)a.t_level_xz[l] : -1;
-    }
-    r.xz = a.xz_end.as<uint64_t>();
-    r.yv = a.y_vec.as<uint16_t>();
-    r.txz = a.t_xz_end.as<uint64_t>();
-    r.tyv = a.t_y_vec.as<uint16_t>();
-    return r;
-}
-ReconImage recon_image(const aprh_apr& a, int level, void* out, uint8_t* lev) {
-    /* dims are at most 65535, so a level has fewer than 2^32 rows */
-    return {level - a.l_min, (uint32_t)a.x_num[level], (uint32_t)(a.x_num[level] * a.z_num[level]), a.y_num[level], out, lev};
-}
-
 template <typename T, typename D, bool VALS, bool LEV>
-void launch_recon(aprh_context* ctx, const ReconArgs& r, const ReconImage& im) {
-    const int64_t chunk = RC_BYTES / (int64_t)sizeof(D);
+void launch_recon(aprh_context* ctx, const ReconArgs& r, const ReconImage& im, bool complete) {
     if (im.rows == 0 || im.Y == 0) return;
-    hipLaunchKernelGGL((k_recon<T, D, VALS, LEV>), dim3((unsigned)std::min<int64_t>(cdiv(im.rows, 4), 1 << 20), (unsigned)cdiv(im.Y, chunk)), kBlock,
-                       0, ctx->stream, r, im);
+    const dim3 grid((unsigned)std::min<int64_t>(cdiv(im.rows, 4), 1 << 20), (unsigned)cdiv(im.Y, RC_BYTES / (int64_t)sizeof(D)));
+    if (complete) hipLaunchKernelGGL((k_recon<T, D, VALS, LEV, false>), grid, kBlock, 0, ctx->stream, r, im);
+    else hipLaunchKernelGGL((k_recon<T, D, VALS, LEV, true>), grid, kBlock, 0, ctx->stream, r, im);
     HIP_LAUNCH_CHECK();
 }
 
@@ -827,8 +871,8 @@ void reconstruct(aprh_context* ctx, aprh_apr& a, const T* parts, int level, U* i
     r.parts = parts;
     r.tv = tree.as<float>();
     const ReconImage im = recon_image(a, level, img, lev);
-    if (lev) launch_recon<T, U, true, true>(ctx, r, im);
-    else launch_recon<T, U, true, false>(ctx, r, im);
+    if (lev) launch_recon<T, U, true, true>(ctx, r, im, a.complete);
+    else launch_recon<T, U, true, false>(ctx, r, im, a.complete);
     HIP_CHECK(hipStreamSynchronize(ctx->stream));
 }
 }  // namespace
@@ -849,8 +893,9 @@ void level_images(aprh_context* ctx, const aprh_apr& a, const T* parts, const fl
         m.row0[i + 1] = m.row0[i] + a.x_num[l] * a.z_num[l];
         ymax = std::max(ymax, a.y_num[l]);
     }
-    hipLaunchKernelGGL(k_level_images<T>, dim3((unsigned)std::min<int64_t>(cdiv(m.row0[m.n], 4), 1 << 20), (unsigned)cdiv(ymax, RC_BYTES / 4)),
-                       kBlock, 0, ctx->stream, r, m);
+    const dim3 grid((unsigned)std::min<int64_t>(cdiv(m.row0[m.n], 4), 1 << 20), (unsigned)cdiv(ymax, RC_BYTES / 4));
+    if (a.complete) hipLaunchKernelGGL((k_level_images<T, false>), grid, kBlock, 0, ctx->stream, r, m);
+    else hipLaunchKernelGGL((k_level_images<T, true>), grid, kBlock, 0, ctx->stream, r, m);
     HIP_LAUNCH_CHECK();
 }
 template void level_images<uint16_t>(aprh_context*, const aprh_apr&, const uint16_t*, const float*, const std::vector<float*>&);
@@ -864,8 +909,8 @@ void reconstruct_level(aprh_context* ctx, aprh_apr& a, int level, void* img, int
     if (level < a.l_max) ensure_tree(ctx, a);
     const ReconArgs r = recon_sources(a, level, level);
     const ReconImage im = recon_image(a, level, img, nullptr);
-    if (idt == APRH_DTYPE_U16) launch_recon<uint16_t, uint16_t, false, false>(ctx, r, im);
-    else launch_recon<uint16_t, float, false, false>(ctx, r, im);
+    if (idt == APRH_DTYPE_U16) launch_recon<uint16_t, uint16_t, false, false>(ctx, r, im, a.complete);
+    else launch_recon<uint16_t, float, false, false>(ctx, r, im, a.complete);
     HIP_CHECK(hipStreamSynchronize(ctx->stream));
 }
 

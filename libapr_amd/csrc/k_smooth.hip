@@ -56,7 +56,8 @@ __device__ __forceinline__ int sm_offset(int level, float scale, int om, int d_m
     return max((int)(a < b ? a : b), 0);   /* never below 0, whatever the scale: the sums' indices stay inside */
 }
 
-/* half-widths by level, in LDS: the division is done once per level and block */
+/* half-widths by level, in LDS: the division is done once per level and block.  Levels are at most 16 (dims
+   are at most 65535), and 0 where no particle covers the pixel */
 constexpr int SM_LEVELS = 32;
 template <typename T>
 __device__ __forceinline__ void sm_offsets(int* tab, float scale, int om, int d_max) {

@@ -646,3 +646,92 @@ def test_face_neighbour_filters(oracle, ctx, shape, nb, seed):
         got = A.APRNumerics.seperable_face_neighbour_filter(g, pf, f, rep)
         assert np.array_equal(_bits(got), _bits(o.face_neighbour_filter(pf, f, 0, rep))), rep
 
+
+
+def _with_holes(oracle, shape, nb, seed, keep):
+    """a converted APR's structure with only the particles that keep(level, z, x, y) wants: (dims, xz_end, y_vec)"""
+    o = oracle.get_apr(A.synth_blobs(shape, seed, nb), oracle.params(rel_error=0.1, sigma_th=50, Ip_th=120, grad_th=10), "oracle")
+    ends, yv = o.xz_end_vec.astype(np.int64), o.y_vec
+    y, x, z = o.dims
+    new, out, row = [0], [], 1
+    for l in range(o.l_min, o.l_max + 1):
+        s = 1 << (o.l_max - l)
+        for zz in range(-(-z // s)):
+            for xx in range(-(-x // s)):
+                ys = yv[ends[row - 1]:ends[row]]
+                out.append(np.array([v for v in ys if keep(l, zz, xx, int(v))], np.uint16))
+                new.append(new[-1] + len(out[-1]))
+                row += 1
+    assert row == len(ends)
+    return o.dims, np.array(new, np.uint64), np.concatenate(out)
+
+
+def _images(apr, parts, tree_values):
+    """per level (image of its particles, coarser ones and its tree nodes' values, with 0 where nothing is;
+    the particles' (z, x, y)): what a convolution at that level reads"""
+    y, x, z = apr.org_dims
+    _, ends, yv = apr.structure()
+    tree = apr.tree()
+    tends, tyv, tlxz = tree["xz_end_vec"], tree["y_vec"], tree["level_xz_vec"]
+    res, row, prev = {}, 1, None
+    for l in range(apr.l_min, apr.l_max + 1):
+        s = 1 << (apr.l_max - l)
+        d = (-(-z // s), -(-x // s), -(-y // s))
+        v = np.zeros(d, np.float32) if prev is None else prev.repeat(2, 0).repeat(2, 1).repeat(2, 2)[:d[0], :d[1], :d[2]].copy()
+        at = []
+        for r in range(d[0] * d[1]):
+            for i in range(int(ends[row - 1]), int(ends[row])):
+                at.append((r // d[1], r % d[1], int(yv[i])))
+                v[at[-1]] = parts[i]
+            row += 1
+        if tree_values is not None and l < apr.l_max:
+            for r in range(d[0] * d[1]):
+                q = int(tlxz[l]) + r
+                for i in range(int(tends[q - 1]), int(tends[q])):
+                    v[r // d[1], r % d[1], int(tyv[i])] = tree_values[i]
+        res[l] = (v, at)
+        prev = v
+    return res
+
+
+@pytest.mark.parametrize("shape,nb,seed", [((9, 17, 70), 5, 1), ((20, 6, 33), 4, 2), ((3, 3, 2100), 9, 3)])
+@pytest.mark.parametrize("what", ["scattered", "rows", "coarse", "nothing"])
+def test_structure_with_uncovered_cells(oracle, ctx, shape, nb, seed, what):
+    """a stored structure's particles need not cover the image: a cell without any reads the nearest tree node
+    above it in a convolution, else 0, and is 0 in a reconstruction, whatever the memory held before"""
+    keep = {"scattered": lambda l, z, x, y: (7 * y + 3 * x + z) % 5 != 0, "rows": lambda l, z, x, y: (x + z) % 3 != 0,
+            "coarse": lambda l, z, x, y: l >= 5, "nothing": lambda l, z, x, y: False}[what]
+    dims, xz, yv = _with_holes(oracle, shape, nb, seed, keep)
+    A.APRReconstruction.reconstruct_constant(*(lambda i, o, g: (g, o.sample(i)))(*_pair(oracle, ctx, shape, nb, seed)))   # leaves values in LDS
+    g = A.APR.from_structure(dims, xz, yv, ctx=ctx)
+    parts = np.random.default_rng(seed).uniform(1, 100, len(yv)).astype(np.float32)
+    tv = A.APRTreeNumerics.fill_tree_mean(g, parts) if what != "nothing" else np.zeros(0, np.float32)
+    images = _images(g, parts, tv)
+    nlev = g.l_max - g.l_min + 1
+    for tap in ((0, 1, 2), (1, 1, 1), (2, 0, 1)):
+        st = np.zeros((3, 3, 3), np.float32)
+        st[tap] = 1.0
+        exp = []
+        for l in range(g.l_min, g.l_max + 1):
+            v, at = images[l]
+            w = np.pad(v, 1)
+            exp += [w[z + tap[0], x + tap[1], y + tap[2]] for z, x, y in at]
+        exp = np.array(exp, np.float32)
+        got = A.APRFilter.convolve_pencil(g, [st] * nlev, parts, reflect_boundary=False)
+        assert np.array_equal(got, exp)
+        wide = np.zeros((3, 5, 3), np.float32)   # the same tap in a stencil that other kernels take
+        wide[tap[0], tap[1] + 1, tap[2]] = 1.0
+        assert np.array_equal(A.APRFilter.convolve_pencil(g, [wide] * nlev, parts, reflect_boundary=False), exp)
+    plain = _images(g, parts, None)[g.l_max][0]
+    for dt in (np.uint16, np.float32):
+        assert np.array_equal(A.APRReconstruction.reconstruct_constant(g, parts, 0, dt), plain.astype(dt))
+    levels = _images(g, np.concatenate([np.full(len(images[l][1]), l, np.float32) for l in images]), None)[g.l_max][0]
+    assert np.array_equal(A.APRReconstruction.reconstruct_level(g), levels.astype(np.uint16))
+    for dt in (np.uint16, np.float32):
+        s0 = A.APRReconstruction.reconstruct_smooth(g, parts, out_dtype=dt)
+        # half-widths of 0 everywhere leave the running sums' differences: the image up to their rounding
+        s1 = A.APRReconstruction.reconstruct_smooth(g, parts, scale_d=(1e9,) * 3, out_dtype=dt)
+        assert np.isfinite(s0.astype(np.float64)).all() and s0.max() <= 101
+        tol = 3 * max(shape) * 100 * max(shape) * 2.0 ** -24 if dt == np.float32 else 3
+        assert np.abs(s1.astype(np.float64) - plain.astype(dt)).max() <= tol
+    g.close()
