@@ -1271,14 +1271,16 @@ void launch_iir_outer(aprh_context* ctx, T* img, int64_t y, int64_t x, int64_t z
                thousand lanes of 16 bytes) and z (98 thousand) 0.86 ms together with 16 bytes, 0.47 this way */
             int vl = V;
             while (vl > 4 / (int)sizeof(T) && (y / vl) * outer < OUTER_LANES) vl >>= 1;
-            auto pass = [&](auto cc, auto vv, int chunk) {
+            /* the chunk states of whichever form runs, whose size does not depend on the width: held until the
+               launch is queued (stream order keeps the block's later users behind it); a batch plan's
+               alternatives share it, since the launch takes one of them */
+            const bool alts = ctx->recorder && std::is_same<T, uint16_t>::value;
+            const int64_t most_chunks = cdiv(n - 4, alts ? 8 : OUTER_CK);
+            Buf ck(ctx->pool, ((size_t)(most_chunks - 1) * 2 * sizeof(T) + 16) * (size_t)(y * outer));
+            auto pass = [&](auto cc, auto vv) {
                 constexpr int C = decltype(cc)::value, VL = decltype(vv)::value;
                 IirArgs<T> q = a;
                 q.ck_lanes = (y / VL) * outer;
-                /* the chunk states live until the launch ends: from the pool, returned after the
-                   launch is queued (stream order keeps later users behind it) */
-                const int64_t chunks = (n - 4 + chunk - 1) / chunk;
-                Buf ck(ctx->pool, ((size_t)(chunks - 1) * 2 * sizeof(Pack<T, VL>) + 16 * VL) * (size_t)q.ck_lanes);
                 q.ck = ck.as<uint4>();
                 return tile_alt<IirOuterCk<T, C, VL>>(q, cdiv(q.ck_lanes, 256), C == 8 ? "checkpoint every 8, 16 bytes"
                                                                                 : VL == V ? "checkpoint every 16, 16 bytes"
@@ -1286,18 +1288,18 @@ void launch_iir_outer(aprh_context* ctx, T* img, int64_t y, int64_t x, int64_t z
             };
             auto run = [&](const TileAlt& alt) { launch_tiles_alts(ctx, {alt}, 0); };
             using C16 = std::integral_constant<int, OUTER_CK>;
-            if (ctx->recorder && std::is_same<T, uint16_t>::value) {
+            if (alts) {
                 /* a batch plan times the widths and a denser spacing over all its volumes */
                 launch_tiles_alts(ctx,
-                                  {pass(C16{}, std::integral_constant<int, V>{}, OUTER_CK), pass(std::integral_constant<int, 8>{}, std::integral_constant<int, V>{}, 8),
-                                   pass(C16{}, std::integral_constant<int, V / 2>{}, OUTER_CK)},
+                                  {pass(C16{}, std::integral_constant<int, V>{}), pass(std::integral_constant<int, 8>{}, std::integral_constant<int, V>{}),
+                                   pass(C16{}, std::integral_constant<int, V / 2>{})},
                                   0);
             } else if (vl == V) {
-                run(pass(C16{}, std::integral_constant<int, V>{}, OUTER_CK));
+                run(pass(C16{}, std::integral_constant<int, V>{}));
             } else if (vl == V / 2) {
-                run(pass(C16{}, std::integral_constant<int, V / 2>{}, OUTER_CK));
+                run(pass(C16{}, std::integral_constant<int, V / 2>{}));
             } else {
-                run(pass(C16{}, std::integral_constant<int, V / 4>{}, OUTER_CK));
+                run(pass(C16{}, std::integral_constant<int, V / 4>{}));
             }
             return;
         }

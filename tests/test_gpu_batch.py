@@ -6,6 +6,7 @@ import ctypes as C
 
 import numpy as np
 import pytest
+import torch
 
 import libapr_amd as A
 
@@ -112,6 +113,21 @@ def test_batch_particles_after_each_run(ctx):
             single.close()
             got.close()
     batch.close()
+
+
+def test_batch_scratch_holds_one_set_of_line_states(ctx):
+    """an x or z smoothing pass is recorded in several forms of which the launch takes one: they share one buffer of
+    line states, (len / 8) states of 2 u16 per line, half a byte per voxel and axis.  The plan has 9.5 bytes per
+    voxel with that; a buffer for each form would make it 10.6"""
+    y, x, z = 1024, 512, 256
+    ctx.release_cache()
+    torch.cuda.synchronize()
+    before = torch.cuda.mem_get_info()[0]
+    batch = A.APRBatch([(y, x, z)], par=_apar(), ctx=ctx)
+    ctx.release_cache()
+    used = (before - torch.cuda.mem_get_info()[0]) / (y * x * z)
+    batch.close()
+    assert 9.0 < used < 10.0, used
 
 
 def test_batch_rejects_small_volumes(ctx):
