@@ -309,6 +309,41 @@ def test_convolve_separable_edges(oracle, sep_ctx, shape, nb, seed, size, reflec
     assert _rel(got, exp)[w].max() <= 2 * (max(size, 3) ** 3 + 3 * max(size, 3) + 3) * 2.0 ** -24
 
 
+@pytest.mark.parametrize("shape,nb,seed", EDGES)
+@pytest.mark.parametrize("size", [1, 3, 5, 7, 9, 11, 13])
+@pytest.mark.parametrize("reflect", [True, False])
+def test_convolve_separable_lists(oracle, sep_ctx, shape, nb, seed, size, reflect):
+    """lists of which one level's stencil is of another form: the cubic ones, the finest or the coarser, take the
+    kernel with the z ring in registers (bound as above).  The finest level's stencil is the widest: the oracle's
+    windows have its size"""
+    img, o, g = _pair(oracle, sep_ctx, shape, nb, seed)
+    wide = oracle.gaussian_stencil((1.0, 1.0, 1.0), (size + 2, size, size + 2), True)
+    narrow = oracle.gaussian_stencil((1.0, 1.0, 1.0), (min(size, 3), 1, min(size, 3)), True)
+    stack = oracle.downsampled_stencils(oracle.gaussian_stencil((size / 4.0,) * 3, (size,) * 3, True), o.l_max - o.l_min, True, "oracle")
+    for at, other in ((0, wide), (-1, narrow)):
+        st = list(stack)
+        st[at] = other
+        w = _wide(o, st)
+        assert w.any()
+        for parts in (o.sample(img), o.sample(img).astype(np.float32) * np.float32(0.83)):
+            exp = o.convolve_pencil(st, parts, reflect)
+            got = A.APRFilter.convolve_pencil(g, st, parts, reflect_boundary=reflect)
+            assert _rel(got, exp)[w].max() <= 2 * ((size + 2) ** 3 + 3 * (size + 2) + 3) * 2.0 ** -24
+
+
+def test_richardson_lucy_wide_psf(oracle, sep_ctx):
+    """a PSF of 15 taps a side: its finest level and the coarser ones (9, 5 and 3 taps) take different
+    kernels, with the ratio and the update at their outputs"""
+    img, o, g = _pair(oracle, sep_ctx, (40, 48, 66), 30, 6)
+    psf = oracle.gaussian_stencil((2.0, 2.0, 2.5), (15, 15, 15), True)
+    w = _wide(o, oracle.downsampled_stencils(psf, o.l_max - o.l_min, True, "oracle"))
+    assert w.mean() > 0.9
+    for parts in (o.sample(img), o.sample(img).astype(np.float32) * np.float32(0.83)):
+        uo, _, _ = o.richardson_lucy(parts, psf, 2)
+        ug, _ = A.APRNumerics.richardson_lucy(g, parts, None, psf, 2, normalize=True)
+        assert _rel(ug, uo)[w].max() < 1e-5
+
+
 @pytest.mark.parametrize("size", [5, 9])
 @pytest.mark.parametrize("separable", [False, True])
 def test_richardson_lucy_edges(oracle, ctx, sep_ctx, size, separable):
