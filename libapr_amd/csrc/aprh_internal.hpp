@@ -47,6 +47,9 @@ public:
     explicit Pool(int device) : device_(device) {}
     ~Pool();
     void* get(size_t bytes);
+    /* nullptr where the device has not the memory (64 MiB left over included), without giving up cached blocks
+       for nothing */
+    void* try_get(size_t bytes);
     void put(void* p);
     void release_all();
     size_t bytes_cached() const { return cached_; }
@@ -85,6 +88,14 @@ public:
         pool_ = pool;
         bytes_ = bytes;
         p_ = bytes ? pool->get(bytes) : nullptr;
+    }
+    bool try_reset(Pool* pool, size_t bytes) {
+        release();
+        p_ = pool->try_get(bytes);
+        if (!p_) return false;
+        pool_ = pool;
+        bytes_ = bytes;
+        return true;
     }
     void release() {
         if (p_ && pool_) pool_->put(p_);

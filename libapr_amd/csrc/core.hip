@@ -60,6 +60,22 @@ void* Pool::get(size_t bytes) {
     return p;
 }
 
+void* Pool::try_get(size_t bytes) {
+    const size_t b = bucket(bytes);
+    const auto it = free_.lower_bound(b);
+    if (it == free_.end() || it->first > b + b / 4) {
+        size_t free = 0, total = 0;
+        HIP_CHECK(hipMemGetInfo(&free, &total));
+        if (b + ((size_t)64 << 20) > free + cached_) return nullptr;
+    }
+    try {
+        return get(bytes);
+    } catch (const Error&) {   /* enough memory, but in pieces */
+        (void)hipGetLastError();
+        return nullptr;
+    }
+}
+
 void Pool::put(void* p) {
     if (keep_) return;
     auto it = live_.find(p);

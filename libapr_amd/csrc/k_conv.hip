@@ -9,9 +9,10 @@
  * update_lower_level, :743-849; reflective or zero ends, :384-504), summing taps
  * in (z, x, y) order (run_convolution_pencil, :705-736).
  *
- * Cubic stencils: k_conv_dense over dense images of all levels (see there).
+ * Lists of cubic stencils: k_conv_dense over dense images of all levels (see there), where the device has
+ * room for them.
  *
- * Other stencils (k_conv_tile): one launch per level walks tiles of TX x 64 cells (x, y) through a run of
+ * Other lists (k_conv_tile; k_conv_sep for their cubic separable stencils): one launch per level walks tiles of TX x 64 cells (x, y) through a run of
  * z planes.  For each plane the block assembles the tile and its halo in LDS:
  *   1. the coarser level's image V(l-1) upsampled (every cell not covered by a
  *      level-l particle or tree node lies inside a coarser particle),
@@ -1392,23 +1393,20 @@ void conv_levels(aprh_context* ctx, aprh_apr& a, const std::vector<HostStencil>&
         *nparts = need;
         return p;
     };
-    /* the images of all levels take four times the memory of k_conv_tile's two: up to 2^34 cells (64 GiB) */
     bool dense = a.l_max - a.l_min < CONV_LEVELS;
-    int64_t cells = 0;
+    std::vector<int64_t> at((size_t)a.l_max + 1, 0);
+    int64_t total = 0;
     for (int l = a.l_min; l <= a.l_max; ++l) {
         dense = dense && dense_size(stencils[stencil_of(l)], off_sep[stencil_of(l)] >= 0);
-        cells += a.y_num[l] * a.x_num[l] * a.z_num[l];
+        at[(size_t)l] = total;
+        total += cdiv(a.y_num[l] * a.x_num[l] * a.z_num[l], 64) * 64;
     }
-    if (dense && cells <= ((int64_t)1 << 34)) {
+    /* the images of all levels take four times the memory of the other kernels' two: where the device has not
+       that much, those run */
+    Buf V;
+    if (dense && V.try_reset(ctx->pool, (size_t)total * 4)) {
         /* the images of all levels, then one launch per stencil form and size, the finest level first */
         std::vector<float*> img((size_t)a.l_max + 1, nullptr);
-        int64_t total = 0;
-        std::vector<int64_t> at((size_t)a.l_max + 1, 0);
-        for (int l = a.l_min; l <= a.l_max; ++l) {
-            at[(size_t)l] = total;
-            total += cdiv(a.y_num[l] * a.x_num[l] * a.z_num[l], 64) * 64;
-        }
-        Buf V(ctx->pool, (size_t)total * 4);
         for (int l = a.l_min; l <= a.l_max; ++l) img[(size_t)l] = V.as<float>() + at[(size_t)l];
         level_images<T>(ctx, a, in, tree, img);
         DenseArgs d;

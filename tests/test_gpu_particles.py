@@ -12,6 +12,7 @@ particles back.
 """
 import numpy as np
 import pytest
+import torch
 
 import libapr_amd as A
 
@@ -770,3 +771,45 @@ def test_structure_with_uncovered_cells(oracle, ctx, shape, nb, seed, what):
         tol = 3 * max(shape) * 100 * max(shape) * 2.0 ** -24 if dt == np.float32 else 3
         assert np.abs(s1.astype(np.float64) - plain.astype(dt)).max() <= tol
     g.close()
+
+
+@pytest.mark.parametrize("y,left", [(4096, 12 << 30), (65535, None)])
+def test_convolve_without_room_for_level_images(sep_ctx, y, left):
+    """y x 1024 x 1024 with all particles at the level of 16-voxel cells, where the images of all levels would take
+    19.6 GB of 12 that are left, or 314 GB.  The other kernels' two (4.3 GB, 69 GB) have room, and give what the same
+    cells give as an APR of y / 16 x 64 x 64"""
+    sep_ctx.release_cache()
+    torch.cuda.empty_cache()
+    free, total = torch.cuda.mem_get_info()
+    if left is None and total > 4 * 8 * y * 1024 * 1024 // 7:
+        pytest.skip("a device with room for the images")
+    n, side = -(-y // 16), 64
+
+    def one_level(dims, level):
+        """(xz_end, y_vec) of particles in all cells of one level, n x 64 x 64 of them"""
+        top = int(np.ceil(np.log2(max(dims))))
+        rows = [-(-dims[1] // 2 ** (top - l)) * -(-dims[2] // 2 ** (top - l)) for l in range(1, top + 1)]
+        assert rows[level - 1] == side * side and -(-dims[0] // 2 ** (top - level)) == n
+        ends = np.concatenate([np.zeros(1 + sum(rows[:level - 1])), np.arange(1, side * side + 1) * n, np.full(sum(rows[level:]), side * side * n)])
+        return ends.astype(np.uint64), np.tile(np.arange(n, dtype=np.uint16), side * side)
+
+    top = int(np.ceil(np.log2(y)))
+    parts = np.random.default_rng(0).uniform(50, 150, n * side * side).astype(np.float32)
+    small = A.APR.from_structure((n, side, side), *one_level((n, side, side), top - 4), sep_ctx)
+    big = A.APR.from_structure((y, 1024, 1024), *one_level((y, 1024, 1024), top - 4), sep_ctx)
+    print("structures made", flush=True)
+    g3 = A.APRStencil.create_gaussian_filter((0.75,) * 3, (3,) * 3, True)
+    g5 = A.APRStencil.create_gaussian_filter((1.25,) * 3, (5,) * 3, True)
+    taken = torch.empty(torch.cuda.mem_get_info()[0] - left, dtype=torch.uint8, device="cuda") if left else None
+    got = A.APRFilter.convolve_pencil(big, [g3] * 4 + [g5], parts)
+    ug, _ = A.APRNumerics.richardson_lucy(big, parts, None, g3, 1, use_stencil_downsample=False)
+    print("done", flush=True)
+    big.close()
+    sep_ctx.release_cache()
+    del taken
+    torch.cuda.empty_cache()
+    exp = A.APRFilter.convolve_pencil(small, [g5], parts)
+    assert _rel(got, exp).max() <= 2 * (5 ** 3 + 3 * 5 + 3) * 2.0 ** -24
+    us, _ = A.APRNumerics.richardson_lucy(small, parts, None, g3, 1, use_stencil_downsample=False)
+    assert _rel(ug, us).max() < 1e-5
+    small.close()
