@@ -1264,7 +1264,16 @@ int aprh_cnn_apply(aprh_context* ctx, aprh_cnn* n, const void* image, int dtype,
     DevOut o(ctx, out, nv * 4);
     if (!(scale > 0)) scale = (float)device_mean(ctx, im.ptr, dtype, nv);
     if (!(scale > 0)) scale = 1.0f;
-    apply_volume(n, im.ptr, dtype, y, x, z, scale, -INFINITY, (float*)o.ptr);
+    /* tiles read their neighbours' voxels while finished ones are written: in place needs a copy of the image */
+    const size_t bytes = nv * (dtype == APRH_DTYPE_U16 ? 2 : 4);
+    const void* src = im.ptr;
+    Buf copy;
+    if ((const char*)src < (const char*)o.ptr + nv * 4 && (const char*)o.ptr < (const char*)src + bytes) {
+        copy.reset(ctx->pool, bytes);
+        HIP_CHECK(hipMemcpyAsync(copy.ptr(), src, bytes, hipMemcpyDeviceToDevice, ctx->stream));
+        src = copy.ptr();
+    }
+    apply_volume(n, src, dtype, y, x, z, scale, -INFINITY, (float*)o.ptr);
     o.finish(ctx);
     APRH_CATCH
 }

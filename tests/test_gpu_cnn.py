@@ -153,6 +153,19 @@ def test_apply_ragged(ctx, shape, dtype):
         np.testing.assert_allclose(blk, yt[k][:blk.shape[0], :blk.shape[1], :blk.shape[2]], rtol=1e-6, atol=1e-3)
 
 
+def test_apply_in_place(ctx):
+    """the output over the image, in more tiles than one batch takes"""
+    net = A.WarmStartCNN(ctx, params=rand_params(4))
+    z, x, y = 80, 160, 300
+    img = np.random.default_rng(3).uniform(100, 600, (z, x, y)).astype(np.float32)
+    exp = net.apply(img, scale=250.0)
+    d = A.DeviceArray(img.nbytes, ctx=ctx)
+    d.from_host(img)
+    net.apply(d.data_ptr(), dims=(y, x, z), scale=250.0, out=d.data_ptr(), dtype="float32")
+    assert np.array_equal(d.to_host(np.float32, img.size).reshape(img.shape), exp)
+    d.free()
+
+
 def test_sample_image_f32_matches_oracle(oracle, ctx):
     img16 = A.synth_blobs((29, 45, 61), 3, 12)
     o = oracle.get_apr(img16, oracle.params(rel_error=0.1, sigma_th=50, Ip_th=120, grad_th=10), "oracle")
