@@ -318,7 +318,7 @@ int aprh_cnn_train_step(aprh_context* ctx, aprh_cnn* net, const float* in, const
    volume border, divided by scale */
 int aprh_cnn_extract_tiles(aprh_context* ctx, const void* image, int dtype, int64_t y_num, int64_t x_num, int64_t z_num,
                            const int32_t* origins, int32_t T, int32_t size, int32_t halo, float scale, float* out);
-/* the network over a whole image in 64^3 tiles (4-voxel reflect halo at the border);
+/* the network over a whole image, tile by tile (4-voxel reflect halo at the border; out may be the image);
    the image is divided by scale (<= 0: its mean) and the result multiplied back */
 int aprh_cnn_apply(aprh_context* ctx, aprh_cnn* net, const void* image, int dtype, int64_t y_num, int64_t x_num, int64_t z_num,
                    float scale, float* out);

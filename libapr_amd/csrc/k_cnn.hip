@@ -5,8 +5,8 @@
  *
  * Network: four "valid" 3x3x3 convolutions, 1 -> 16 -> 16 -> 16 -> 1
  * channels, ReLU after the first three, residual output y = x + conv4.  A
- * tile of side S + 8 gives an output tile of side S (64 in training, 74
- * over a whole volume).
+ * tile of side S + 8 gives an output tile of side S (64 in training; over
+ * a whole volume as its size suggests).
  * Parameters (f32 master copy, 14737 values): W1[27][16] b1[16]
  * W2[27][16][16] b2[16] W3[27][16][16] b3[16] W4[27][16] b4, tap =
  * (dz * 3 + dx) * 3 + dy.
@@ -170,16 +170,26 @@ __device__ __forceinline__ void rows_mfma(const uint16_t* tile, int kz0, int kx0
         }
 }
 
-/* The part of the tiles' outputs that is wanted: tile t covers an image of (y, x, z) from org[3 t ..], and a
-   layer's outputs are wanted `extra` voxels past the image's end (org nullptr: all).  Bricks wholly outside
-   are skipped: nothing wanted depends on what they would hold. */
-struct Need {
-    const int* org;
-    int y, x, z, extra;
+/* The bricks of a layer over the tiles of an image, of which the last ones end within a tile: tile t has the
+   y x z bricks tab[t].y x tab[t].z x tab[t].w from number tab[t].x on, and what lies outside them nothing wanted
+   depends on (tab nullptr: all tiles alike).  The wanted bricks are numbered without gaps: launched over whole
+   tiles, the XCDs whose share was the image's ends had nothing to do (128^3 in eight tiles of 74^3: 0.30 ms,
+   0.26 this way; 150^3 0.70, 0.44). */
+struct BrickMap {
+    const int4* tab;
+    int T;
 };
-__device__ __forceinline__ bool needed(const Need& n, int t, int z0, int x0, int y0) {
-    if (!n.org) return true;
-    return y0 < n.y - n.org[3 * t] + n.extra && x0 < n.x - n.org[3 * t + 1] + n.extra && z0 < n.z - n.org[3 * t + 2] + n.extra;
+__device__ __forceinline__ void wanted_brick(const BrickMap& m, uint32_t br, uint32_t nby, uint32_t nbx, uint32_t nbz, int& t, int& z0, int& x0,
+                                             int& y0) {
+    if (!m.tab) return brick_origin(br, nby, nbx, nbz, t, z0, x0, y0);
+    const int lane = threadIdx.x & 63;
+    int4 e = make_int4(0x7FFFFFFF, 1, 1, 1);
+    if (lane < m.T) e = m.tab[lane];
+    const int own = __popcll(__ballot((uint32_t)e.x <= br)) - 1;
+    int none;
+    brick_origin(br - (uint32_t)__builtin_amdgcn_readlane(e.x, own), (uint32_t)__builtin_amdgcn_readlane(e.y, own),
+                 (uint32_t)__builtin_amdgcn_readlane(e.z, own), (uint32_t)__builtin_amdgcn_readlane(e.w, own), none, z0, x0, y0);
+    t = own;
 }
 /* an image whose tiles the network reads and writes in place of tile buffers */
 struct Volume {
@@ -249,7 +259,7 @@ constexpr int NIN1 = IZ * IX * IY, NIN1_PT = (NIN1 + 255) / 256;
 template <typename T, bool IMG>
 __global__ __launch_bounds__(256) void k_l1_lds(const float* __restrict__ x, int s0, int s1, const u32x4* __restrict__ W1p,
                                                 const float* __restrict__ b1, uint16_t* a_cl, uint16_t* a_pl, uint32_t nbricks, uint32_t nby,
-                                                uint32_t nbx, uint32_t nbz, Need need, Volume vol) {
+                                                uint32_t nbx, uint32_t nbz, BrickMap map, Volume vol) {
     __shared__ __attribute__((aligned(16))) float tile[NIN1_PT * 256];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), m = lane & 15, g = lane >> 4;
     const u32x4 wb = W1p[lane];
@@ -260,8 +270,7 @@ __global__ __launch_bounds__(256) void k_l1_lds(const float* __restrict__ x, int
     const int nv = s1 * s1 * s1, nin = s0 * s0 * s0;
     for (uint32_t br = (uint32_t)xcd_block(blockIdx.x, gridDim.x); br < nbricks; br += gridDim.x) {
         int t, z0, x0, y0;
-        brick_origin(br, nby, nbx, nbz, t, z0, x0, y0);
-        if (!needed(need, t, z0, x0, y0)) continue;
+        wanted_brick(map, br, nby, nbx, nbz, t, z0, x0, y0);
         const float* xt = x + (int64_t)t * nin;
         __syncthreads();   /* the previous brick's waves are done with the tile */
         float in[NIN1_PT];
@@ -320,7 +329,7 @@ template <bool DIRECT>
 __global__ __launch_bounds__(256, 3) void k_conv16_lds(const uint16_t* __restrict__ in_cl, int sin, int sout, int off,
                                                     const u32x4* __restrict__ Wp, const float* __restrict__ bias,
                                                     const uint16_t* __restrict__ mask_cl, uint16_t* out_cl, uint16_t* out_pl, int relu,
-                                                    uint32_t nbricks, uint32_t nby, uint32_t nbx, uint32_t nbz, Need need) {
+                                                    uint32_t nbricks, uint32_t nby, uint32_t nbx, uint32_t nbz, BrickMap map) {
     __shared__ __attribute__((aligned(16))) uint16_t tile[IZ * IX * IY * CH];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), m = lane & 15, g = lane >> 4;
     const int kz0 = (wave >> 1) * WZ, kx0 = (wave & 1) * WX;
@@ -332,8 +341,7 @@ __global__ __launch_bounds__(256, 3) void k_conv16_lds(const uint16_t* __restric
     const int nv = sout * sout * sout;
     for (uint32_t br = (uint32_t)xcd_block(blockIdx.x, gridDim.x); br < nbricks; br += gridDim.x) {
         int t, z0, x0, y0;
-        brick_origin(br, nby, nbx, nbz, t, z0, x0, y0);
-        if (!needed(need, t, z0, x0, y0)) continue;
+        wanted_brick(map, br, nby, nbx, nbz, t, z0, x0, y0);
         stage_brick<DIRECT>(tile, in_cl + (int64_t)t * sin * sin * sin * CH, sin, off, z0, x0, y0);
         if (x0 + kx0 >= sout || z0 + kz0 >= sout) continue;
         f32x4 acc[WZ][WX];
@@ -378,7 +386,7 @@ template <typename T, bool IMG>
 __global__ __launch_bounds__(256, 3) void k_l4_lds(const uint16_t* __restrict__ a3_cl, int S, const float* __restrict__ x,
                                                 const u32x4* __restrict__ W4p, const float* __restrict__ b4, const float* __restrict__ tgt,
                                                 float* y, float* g4, float gscale, double* part, uint32_t nbricks, uint32_t nby, uint32_t nbx,
-                                                uint32_t nbz, Need need, Volume vol) {
+                                                uint32_t nbz, BrickMap map, Volume vol) {
     __shared__ __attribute__((aligned(16))) uint16_t tile[IZ * IX * IY * CH];
     __shared__ double red[2][IMG ? 1 : 256];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -392,8 +400,7 @@ __global__ __launch_bounds__(256, 3) void k_l4_lds(const uint16_t* __restrict__ 
     double dsum = 0, gsum = 0;
     for (uint32_t br = (uint32_t)xcd_block(blockIdx.x, gridDim.x); br < nbricks; br += gridDim.x) {
         int t, z0, x0, y0;
-        brick_origin(br, nby, nbx, nbz, t, z0, x0, y0);
-        if (!needed(need, t, z0, x0, y0)) continue;
+        wanted_brick(map, br, nby, nbx, nbz, t, z0, x0, y0);
         stage_brick<true>(tile, a3_cl + (int64_t)t * n3 * CH, s3, 0, z0, x0, y0);
         if (x0 + kx0 >= S || z0 + kz0 >= S) continue;
         /* the residual (and target) loads go out before the MFMA chains */
@@ -895,12 +902,17 @@ struct Bricks {
     uint32_t n, ny, nx, nz;
     unsigned grid;
 };
-Bricks bricks(int T, int s, int64_t cap) {
+/* one layer of a pass over an image's tiles: their wanted bricks */
+struct LayerBricks {
+    BrickMap map;
+    int64_t n;
+};
+Bricks bricks(int T, int s, int64_t cap, const LayerBricks* wanted = nullptr) {
     Bricks b;
     b.ny = (uint32_t)cdiv(s, BY);
     b.nx = (uint32_t)cdiv(s, BX);
     b.nz = (uint32_t)cdiv(s, BZ);
-    const int64_t n = (int64_t)T * b.ny * b.nx * b.nz;
+    const int64_t n = wanted ? wanted->n : (int64_t)T * b.ny * b.nx * b.nz;
     if (n > 0x7FFFFFFF) throw Error(APRH_ERR_INVALID_ARGUMENT, "too many tiles in one network pass");
     b.n = (uint32_t)n;
     b.grid = (unsigned)std::min<int64_t>(n, cap);
@@ -909,11 +921,11 @@ Bricks bricks(int T, int s, int64_t cap) {
 
 /* 16 -> 16 convolution of T tiles (input side sin, output side sout, input offset off) */
 void conv16(hipStream_t st, const uint16_t* in_cl, int sin, int sout, int off, const u32x4* Wp, const float* bias,
-            const uint16_t* mask_cl, uint16_t* out_cl, uint16_t* out_pl, int relu, int T, Need need = Need()) {
-    const Bricks b = bricks(T, sout, 65536);
+            const uint16_t* mask_cl, uint16_t* out_cl, uint16_t* out_pl, int relu, int T, const LayerBricks* wanted = nullptr) {
+    const Bricks b = bricks(T, sout, 65536, wanted);
     auto launch = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, dim3(b.grid), kBlk, 0, st, in_cl, sin, sout, off, Wp, bias, mask_cl, out_cl, out_pl, relu, b.n, b.ny, b.nx, b.nz,
-                           need);
+                           wanted ? wanted->map : BrickMap());
     };
     if (off == 0) launch(k_conv16_lds<true>);
     else launch(k_conv16_lds<false>);
@@ -935,9 +947,9 @@ int l4_blocks(int T, int S) { return (int)bricks(T, S, 4096).grid; }
 
 /* forward of T tiles (input side S + 8); planar copies when training; part holds l4_blocks(T, S)
    pairs of loss partials.  With an image (dt its type) the tiles at vol->org are read from it and written
-   to its output instead of x and y */
+   to its output instead of x and y, at the layers' wanted bricks */
 void forward(aprh_cnn* n, const float* x, int T, int S, float* y, Acts& A, bool train, const float* tgt, float* g4, double* part,
-             const Volume* vol = nullptr, int dt = APRH_DTYPE_F32) {
+             const Volume* vol = nullptr, int dt = APRH_DTYPE_F32, const LayerBricks* wanted = nullptr) {
     hipStream_t st = n->ctx->stream;
     const int s0 = S + 8, s1 = S + 6, s2 = S + 4, s3 = S + 2;
     auto vox = [&](int s) { return (size_t)T * s * s * s; };
@@ -950,13 +962,14 @@ void forward(aprh_cnn* n, const float* x, int T, int S, float* y, Acts& A, bool 
         A.a3p.reset(n->ctx->pool, vox(s3) * CH * 2 + PL_PAD);
     }
     const Volume v = vol ? *vol : Volume();
-    auto need = [&](int extra) { return vol ? Need{v.org, (int)v.yn, (int)v.xn, (int)v.zn, extra} : Need(); };
+    auto layer = [&](int k) { return wanted ? wanted + k : nullptr; };
+    auto map = [&](int k) { return wanted ? wanted[k].map : BrickMap(); };
     const float* P = n->P.as<float>();
     {
-        const Bricks b = bricks(T, s1, 65536);
+        const Bricks b = bricks(T, s1, 65536, layer(0));
         auto launch = [&](auto kernel) {
             hipLaunchKernelGGL(kernel, dim3(b.grid), kBlk, 0, st, x, s0, s1, (const u32x4*)n->W1p.as<u32x4>(), P + OFF_B1, A.a1c.as<uint16_t>(),
-                               train ? A.a1p.as<uint16_t>() : (uint16_t*)nullptr, b.n, b.ny, b.nx, b.nz, need(6), v);
+                               train ? A.a1p.as<uint16_t>() : (uint16_t*)nullptr, b.n, b.ny, b.nx, b.nz, map(0), v);
         };
         if (!vol) launch(k_l1_lds<float, false>);
         else if (dt == APRH_DTYPE_U16) launch(k_l1_lds<uint16_t, true>);
@@ -964,13 +977,13 @@ void forward(aprh_cnn* n, const float* x, int T, int S, float* y, Acts& A, bool 
         HIP_LAUNCH_CHECK();
     }
     conv16(st, A.a1c.as<uint16_t>(), s1, s2, 0, n->W2p.as<u32x4>(), P + OFF_B2, nullptr, A.a2c.as<uint16_t>(),
-           train ? A.a2p.as<uint16_t>() : nullptr, 1, T, need(4));
+           train ? A.a2p.as<uint16_t>() : nullptr, 1, T, layer(1));
     conv16(st, A.a2c.as<uint16_t>(), s2, s3, 0, n->W3p.as<u32x4>(), P + OFF_B3, nullptr, A.a3c.as<uint16_t>(),
-           train ? A.a3p.as<uint16_t>() : nullptr, 1, T, need(2));
-    const Bricks b4 = bricks(T, S, vol ? 65536 : 4096);
+           train ? A.a3p.as<uint16_t>() : nullptr, 1, T, layer(2));
+    const Bricks b4 = bricks(T, S, vol ? 65536 : 4096, layer(3));
     auto launch = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, dim3(b4.grid), kBlk, 0, st, (const uint16_t*)A.a3c.as<uint16_t>(), S, x, (const u32x4*)n->W4p.as<u32x4>(),
-                           P + OFF_B4, tgt, y, g4, 1.0f / (float)vox(S), part, b4.n, b4.ny, b4.nx, b4.nz, need(0), v);
+                           P + OFF_B4, tgt, y, g4, 1.0f / (float)vox(S), part, b4.n, b4.ny, b4.nx, b4.nz, map(3), v);
     };
     if (!vol) launch(k_l4_lds<float, false>);
     else if (dt == APRH_DTYPE_U16) launch(k_l4_lds<uint16_t, true>);
@@ -1067,31 +1080,83 @@ double device_mean(aprh_context* ctx, const void* v, int dt, size_t n) {
     return n ? s / (double)n : 0.0;
 }
 
-/* the network over a whole volume in tiles; out = y * scale (floored).  Every output depends on its own
-   neighbourhood alone, so the tiles' size is free: the layers of 74^3 tiles (80^3, 78^3, 76^3) fill their
-   bricks of 16 x 8 x 4 where those of 64^3 (70^3, 68^3, 66^3) leave a fifth of their work outside */
+/* the wanted bricks of layer l along an axis of n voxels in tiles of side S, of which the output is wanted
+   e = 6 - 2 l voxels past the axis' end */
+int64_t bricks_along(int64_t n, int S, int l, int b) {
+    const int e = 6 - 2 * l;
+    const int64_t tiles = cdiv(n, S);
+    return (tiles - 1) * cdiv(S + e, b) + cdiv(n - (tiles - 1) * S + e, b);
+}
+
+/* tiles per batch: their activations (32 bytes a voxel and layer) are to stay in the 256 MB cache from one layer
+   to the next (512 x 500 x 130 in 74^3 tiles, 6 / 16 / 32 a batch: 3.99 / 3.62 / 3.68 ms) */
+int tiles_per_batch(int S) { return (int)std::max<int64_t>(1, std::min<int64_t>(64, (int64_t)16 * 74 * 74 * 74 / ((int64_t)S * S * S))); }
+
+/* The side of the tiles.  Every output depends on its own neighbourhood alone, so it is free; what counts is the
+   bricks of 16 x 8 x 4 that the layers need, which overhang the tiles' and the image's ends.  Their cost, per
+   brick as measured in ns, and 20 us of each batch's launches and last waves decide: 128^3 takes one tile
+   (0.23 ms; 74^3 tiles 0.26, 64^3 tiles 0.25), 512 x 500 x 130 takes 136^3 (3.23 ms; 74^3 3.39), 333 x 250 x 77
+   138^3 (0.70 ms; 74^3 0.76). */
+int tile_side(int64_t yn, int64_t xn, int64_t zn) {
+    constexpr double ns[4] = {6.5, 10.7, 10.7, 13.0};
+    int best = 0;
+    double least = 0;
+    for (int S = 32; S <= 138; S += 2) {
+        double cost = 20000.0 * (double)cdiv(cdiv(yn, S) * cdiv(xn, S) * cdiv(zn, S), tiles_per_batch(S));
+        for (int l = 0; l < 4; ++l)
+            cost += ns[l] * (double)bricks_along(yn, S, l, BY) * (double)bricks_along(xn, S, l, BX) * (double)bricks_along(zn, S, l, BZ);
+        if (best == 0 || cost < least) {
+            best = S;
+            least = cost;
+        }
+    }
+    return best;
+}
+
+/* the network over a whole volume in tiles; out = y * scale (floored) */
 void apply_volume(aprh_cnn* n, const void* img, int dt, int64_t yn, int64_t xn, int64_t zn, float scale, float floor_v, float* out) {
     hipStream_t st = n->ctx->stream;
     Pool* pool = n->ctx->pool;
-    const int S = 74;
+    const int S = tile_side(yn, xn, zn);
     const int ty = (int)cdiv(yn, S), tx = (int)cdiv(xn, S), tz = (int)cdiv(zn, S);
     const int ntiles = ty * tx * tz;
+    const bool whole = yn % S == 0 && xn % S == 0 && zn % S == 0;   /* all tiles alike */
+    const int B = tiles_per_batch(S);   /* at most 64: wanted_brick looks a tile up in one wave */
+    /* per layer and tile the wanted bricks (layer l's output is wanted 6 - 2 l voxels past the image's end), then
+       the tiles' origins */
+    std::vector<int4> tab((size_t)ntiles * 4);
     std::vector<int> org((size_t)ntiles * 3);
+    std::vector<int64_t> count((size_t)cdiv(ntiles, B) * 4, 0);
     for (int k = 0, z = 0; z < tz; ++z)
         for (int x = 0; x < tx; ++x)
             for (int y = 0; y < ty; ++y, ++k) {
                 org[3 * k] = y * S;
                 org[3 * k + 1] = x * S;
                 org[3 * k + 2] = z * S;
+                for (int l = 0; l < 4; ++l) {
+                    const int e = 6 - 2 * l;
+                    auto along = [&](int64_t n, int o, int b) { return (int)cdiv(std::min<int64_t>(S, n - o) + e, b); };
+                    int64_t& c = count[(size_t)(k / B) * 4 + l];
+                    const int4 q = make_int4((int)c, along(yn, y * S, BY), along(xn, x * S, BX), along(zn, z * S, BZ));
+                    tab[(size_t)l * ntiles + k] = q;
+                    c += (int64_t)q.y * q.z * q.w;
+                }
             }
-    Buf dorg(pool, org.size() * 4);
-    HIP_CHECK(hipMemcpyAsync(dorg.ptr(), org.data(), org.size() * 4, hipMemcpyHostToDevice, st));
-    const int B = 16;   /* tiles per batch */
+    std::vector<uint8_t> host(tab.size() * 16 + org.size() * 4);
+    std::memcpy(host.data(), tab.data(), tab.size() * 16);
+    std::memcpy(host.data() + tab.size() * 16, org.data(), org.size() * 4);
+    Buf dev(pool, host.size());
+    HIP_CHECK(hipMemcpyAsync(dev.ptr(), host.data(), host.size(), hipMemcpyHostToDevice, st));
+    const int4* dtab = dev.as<int4>();
+    const int* dorg = (const int*)(dtab + tab.size());
     for (int t0 = 0; t0 < ntiles; t0 += B) {
         const int T = std::min(B, ntiles - t0);
-        const Volume vol{img, yn, xn, zn, dorg.as<int>() + 3 * t0, 1.0f / scale, scale, floor_v, out};
+        const Volume vol{img, yn, xn, zn, dorg + 3 * t0, 1.0f / scale, scale, floor_v, out};
+        LayerBricks wanted[4];
+        for (int l = 0; l < 4 && !whole; ++l)
+            wanted[l] = {{dtab + (size_t)l * ntiles + t0, T}, count[(size_t)(t0 / B) * 4 + l]};
         Acts A;
-        forward(n, nullptr, T, S, nullptr, A, false, nullptr, nullptr, nullptr, &vol, dt);
+        forward(n, nullptr, T, S, nullptr, A, false, nullptr, nullptr, nullptr, &vol, dt, whole ? nullptr : wanted);
     }
     HIP_CHECK(hipStreamSynchronize(st));
 }

@@ -137,7 +137,7 @@ def test_apply_equals_tiles(ctx):
         np.testing.assert_allclose(blk, yt[k][:blk.shape[0], :blk.shape[1], :blk.shape[2]], rtol=1e-6, atol=1e-3)
 
 
-@pytest.mark.parametrize("shape", [(1, 1, 1), (3, 75, 74), (9, 73, 149), (76, 5, 80), (2, 10, 17)])
+@pytest.mark.parametrize("shape", [(1, 1, 1), (3, 75, 74), (9, 73, 149), (76, 5, 80), (2, 10, 17), (5, 139, 285), (139, 6, 140), (32, 64, 96)])
 @pytest.mark.parametrize("dtype", [np.uint16, np.float32])
 def test_apply_ragged(ctx, shape, dtype):
     """volumes that end just past, at and before a tile's or a brick's end, and shorter than the halo: each
