@@ -349,8 +349,8 @@ struct ReconImage {
 /* the images of levels l_min .. in one buffer */
 struct LevelImages {
     int n;
-    int64_t row0[MAXL + 1];    /* first row of each level, counted over all     */
-    uint32_t X[MAXL];
+    int64_t block0[MAXL], blocks;   /* first block (four rows) of each level, the finest level first; their number */
+    uint32_t X[MAXL], rows[MAXL];
     int64_t Y[MAXL];
     float* out[MAXL];
 };
@@ -539,11 +539,13 @@ __global__ __launch_bounds__(256) void k_level_images(ReconArgs a, LevelImages m
     __shared__ __align__(16) float stage[4][CHUNK];
     const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int64_t c0 = (int64_t)blockIdx.y * CHUNK;
-    for (int64_t rg = xcd_block(blockIdx.x, gridDim.x) * 4 + wv; rg < m.row0[m.n]; rg += (int64_t)gridDim.x * 4) {
-        int li = 0;
-        while (rg >= m.row0[li + 1]) ++li;
-        if (c0 >= m.Y[li]) continue;
-        const uint32_t row = (uint32_t)(rg - m.row0[li]), X = m.X[li], z = row / X, x = row - z * X;
+    for (int64_t v = blockIdx.x; v < m.blocks; v += gridDim.x) {
+        int li = m.n - 1;
+        while (li > 0 && v >= m.block0[li - 1]) --li;
+        /* each level is dealt out over the XCDs by itself: the rows of a coarse one cost little */
+        const int64_t rowl = xcd_block(v - m.block0[li], (m.rows[li] + 3) / 4) * 4 + wv;
+        if (c0 >= m.Y[li] || rowl >= m.rows[li]) continue;
+        const uint32_t row = (uint32_t)rowl, X = m.X[li], z = row / X, x = row - z * X;
         const int cn = (int)min((int64_t)CHUNK, m.Y[li] - c0);
         recon_piece<T, float, true, false, HOLES>(a, li, z, x, c0, cn, m.Y[li] > CHUNK, stage[wv], nullptr,
                                                   m.out[li] + (int64_t)row * m.Y[li] + c0, nullptr, lane);
@@ -890,10 +892,14 @@ void level_images(aprh_context* ctx, const aprh_apr& a, const T* parts, const fl
         m.X[i] = (uint32_t)a.x_num[l];
         m.Y[i] = a.y_num[l];
         m.out[i] = out[(size_t)l];
-        m.row0[i + 1] = m.row0[i] + a.x_num[l] * a.z_num[l];
+        m.rows[i] = (uint32_t)(a.x_num[l] * a.z_num[l]);   /* dims are at most 65535 */
         ymax = std::max(ymax, a.y_num[l]);
     }
-    const dim3 grid((unsigned)std::min<int64_t>(cdiv(m.row0[m.n], 4), 1 << 20), (unsigned)cdiv(ymax, RC_BYTES / 4));
+    for (int i = m.n - 1; i >= 0; --i) {
+        m.block0[i] = m.blocks;
+        m.blocks += cdiv(m.rows[i], 4);
+    }
+    const dim3 grid((unsigned)std::min<int64_t>(m.blocks, 1 << 20), (unsigned)cdiv(ymax, RC_BYTES / 4));
     if (a.complete) hipLaunchKernelGGL((k_level_images<T, false>), grid, kBlock, 0, ctx->stream, r, m);
     else hipLaunchKernelGGL((k_level_images<T, true>), grid, kBlock, 0, ctx->stream, r, m);
     HIP_LAUNCH_CHECK();
