@@ -349,8 +349,9 @@ struct ReconImage {
 /* the images of levels l_min .. in one buffer */
 struct LevelImages {
     int n;
-    int64_t block0[MAXL], blocks;   /* first block (four rows) of each level, the finest level first; their number */
+    int64_t block0[MAXL], blocks;   /* first block of each level, the finest level first; their number */
     uint32_t X[MAXL], rows[MAXL];
+    int G[MAXL];               /* lanes per row                                 */
     int64_t Y[MAXL];
     float* out[MAXL];
 };
@@ -358,10 +359,10 @@ struct LevelImages {
 constexpr int RC_BYTES = 4096;   /* of a row's values in LDS, per wave */
 
 /* n elements staged in LDS to dst in 16-byte words at any alignment, the last ones singly */
-template <typename E>
+template <typename E, int G>
 __device__ __forceinline__ void store_staged(E* dst, const E* lds, int n, int lane) {
     constexpr int V = 16 / sizeof(E);
-    for (int i = lane * V; i < n; i += 64 * V) {
+    for (int i = lane * V; i < n; i += G * V) {
         if (i + V <= n) {
             const uint4 w = *(const uint4*)(lds + i);
             __builtin_memcpy(dst + i, &w, 16);
@@ -378,11 +379,14 @@ __device__ __forceinline__ void store_staged(E* dst, const E* lds, int n, int la
    four times the instructions, which bound it: the images of 1024 x 1024 x 256 0.77 ms, now 0.50).  search: the row is longer than the piece.
    VALS: values from parts / tree, else the levels themselves; LEV: the levels to ls as bytes.
    HOLES: the structure's particles need not cover the image: a pixel without any is 0 (as is its level), or
-   takes the coarser tree nodes that are wanted and reach it */
-template <typename T, typename D, bool VALS, bool LEV, bool HOLES>
+   takes the coarser tree nodes that are wanted and reach it.
+   G < 64: each G lanes take a row of their own, with its (z, x) and stage; whole rows only (c0 = 0, no search) */
+template <typename T, typename D, bool VALS, bool LEV, bool HOLES, int G>
 __device__ __forceinline__ void recon_stage(const ReconArgs& a, int li, uint32_t z, uint32_t x, int64_t c0, int cn, bool search, D* st,
                                             uint8_t* ls, int lane) {
     constexpr int LOG = sizeof(D) == 2 ? 11 : 10;
+    static_assert(!HOLES || G == 64, "incomplete structures take one row per wave");
+    const int sl = G == 64 ? lane : lane & (G - 1);
     if constexpr (HOLES) {
         for (int i = lane; i < RC_BYTES / (int)sizeof(D); i += 64) {
             st[i] = (D)0;
@@ -394,9 +398,9 @@ __device__ __forceinline__ void recon_stage(const ReconArgs& a, int li, uint32_t
     /* lane s: the entries of source s under this row (under the piece), and of the tree nodes of li after them;
        HOLES: lane 2 s those of level s, lane 2 s + 1 those of its tree nodes */
     uint64_t b = 0, e = 0;
-    const bool tr = HOLES ? lane & 1 : lane == tree;
-    const int s = HOLES ? lane >> 1 : tr ? li : lane, d = li - s;
-    if (s <= li && (!HOLES || !tr || a.trb[s] >= 0)) {
+    const bool tr = HOLES ? lane & 1 : sl == tree;
+    const int s = HOLES ? lane >> 1 : tr ? li : sl, d = li - s;
+    if (cn > 0 && s <= li && (!HOLES || !tr || a.trb[s] >= 0)) {
         const int64_t r = (tr ? a.trb[s] : a.rb[s]) + (int64_t)(z >> d) * a.xn[s] + (x >> d);
         const uint64_t* xz = tr ? a.txz : a.xz;
         b = xz[r - 1];
@@ -409,11 +413,24 @@ __device__ __forceinline__ void recon_stage(const ReconArgs& a, int li, uint32_t
     }
     const int base = (int)c0;
     uint64_t todo = __ballot(e > b);
+    if constexpr (G < 64) {   /* sources that any of the wave's rows has */
+#pragma unroll
+        for (int o = 32; o >= G; o >>= 1) todo |= todo >> o;
+        todo &= ((uint64_t)1 << G) - 1;
+    }
     while (todo) {
         const int q = __builtin_ctzll(todo);
         todo &= todo - 1;
-        const uint64_t sb = ((uint64_t)__builtin_amdgcn_readlane((int)(b >> 32), q) << 32) | (uint32_t)__builtin_amdgcn_readlane((int)b, q);
-        const int cnt = __builtin_amdgcn_readlane((int)(e - b), q);
+        uint64_t sb;
+        int cnt;
+        if constexpr (G == 64) {
+            sb = ((uint64_t)__builtin_amdgcn_readlane((int)(b >> 32), q) << 32) | (uint32_t)__builtin_amdgcn_readlane((int)b, q);
+            cnt = __builtin_amdgcn_readlane((int)(e - b), q);
+        } else {
+            const int from = (lane & ~(G - 1)) | q;
+            sb = ((uint64_t)(uint32_t)__shfl((int)(b >> 32), from, 64) << 32) | (uint32_t)__shfl((int)b, from, 64);
+            cnt = __shfl((int)(e - b), from, 64);
+        }
         const bool tr = HOLES ? q & 1 : q == tree;
         const int s = HOLES ? q >> 1 : tr ? li : q, d = li - s;
         const int lv = a.l_lo + s;
@@ -454,7 +471,7 @@ __device__ __forceinline__ void recon_stage(const ReconArgs& a, int li, uint32_t
         /* E entries per lane; the last lane's end with the row's last one, so it may repeat some */
         auto entries = [&](auto n, auto w) {
             constexpr int E = decltype(n)::value;
-            for (int k = lane * E; k < cnt; k += 64 * E) {
+            for (int k = sl * E; k < cnt; k += G * E) {
                 uint16_t y[E];
                 D v[E];
                 load(y, v, min(k, cnt - E));
@@ -472,7 +489,7 @@ __device__ __forceinline__ void recon_stage(const ReconArgs& a, int li, uint32_t
         } else {
             /* four pixels per lane; a cell that starts before the piece (wider than it) fills it from 0 */
             const int m = min(d, LOG) - 2;
-            for (int k = lane; k < cnt << m; k += 64) {
+            for (int k = sl; k < cnt << m; k += G) {
                 uint16_t y[1];
                 D v[1];
                 load(y, v, k >> m);
@@ -484,12 +501,12 @@ __device__ __forceinline__ void recon_stage(const ReconArgs& a, int li, uint32_t
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 }
 /* the same, and the piece to dst (its levels to ldst) */
-template <typename T, typename D, bool VALS, bool LEV, bool HOLES>
+template <typename T, typename D, bool VALS, bool LEV, bool HOLES, int G>
 __device__ __forceinline__ void recon_piece(const ReconArgs& a, int li, uint32_t z, uint32_t x, int64_t c0, int cn, bool search, D* st,
                                             uint8_t* ls, D* dst, uint8_t* ldst, int lane) {
-    recon_stage<T, D, VALS, LEV, HOLES>(a, li, z, x, c0, cn, search, st, ls, lane);
-    store_staged<D>(dst, st, cn, lane);
-    if (LEV) store_staged<uint8_t>(ldst, ls, cn, lane);
+    recon_stage<T, D, VALS, LEV, HOLES, G>(a, li, z, x, c0, cn, search, st, ls, lane);
+    store_staged<D, G>(dst, st, cn, lane & (G - 1));
+    if (LEV) store_staged<uint8_t, G>(ldst, ls, cn, lane & (G - 1));
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   /* the next piece rewrites the stage */
 }
 
@@ -498,19 +515,21 @@ __device__ __forceinline__ void recon_piece(const ReconArgs& a, int li, uint32_t
    the image is written once.  (Before, a level's image was the coarser one upsampled, then its particles
    scattered over it: three passes over the finest level, 1.12 ms for 1000 x 1023 x 255 u16 against
    0.29 ms, 4.6 TB/s.) */
-template <typename T, typename D, bool VALS, bool LEV, bool HOLES>
+template <typename T, typename D, bool VALS, bool LEV, bool HOLES, int G>
 __global__ __launch_bounds__(256) void k_recon(ReconArgs a, ReconImage im) {
-    constexpr int CHUNK = RC_BYTES / (int)sizeof(D);
+    constexpr int CHUNK = RC_BYTES / (int)sizeof(D), R = 64 / G;
     __shared__ __align__(16) D stage[4][CHUNK];
     __shared__ __align__(16) uint8_t lstage[4][LEV ? CHUNK : 16];
     const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int64_t c0 = (int64_t)blockIdx.y * CHUNK;
     const int cn = (int)min((int64_t)CHUNK, im.Y - c0);
-    for (int64_t rowl = xcd_block(blockIdx.x, gridDim.x) * 4 + wv; rowl < (int64_t)im.rows; rowl += (int64_t)gridDim.x * 4) {
-        const uint32_t row = (uint32_t)rowl, z = row / im.X, x = row - z * im.X;
+    for (int64_t row0 = (xcd_block(blockIdx.x, gridDim.x) * 4 + wv) * R; row0 < (int64_t)im.rows; row0 += (int64_t)gridDim.x * 4 * R) {
+        const int sub = G == 64 ? 0 : lane / G;
+        const bool on = row0 + sub < (int64_t)im.rows;
+        const uint32_t row = (uint32_t)row0 + (on ? sub : 0), z = row / im.X, x = row - z * im.X;
         const int64_t o = (int64_t)row * im.Y + c0;
-        recon_piece<T, D, VALS, LEV, HOLES>(a, im.li, z, x, c0, cn, gridDim.y > 1, stage[wv], lstage[wv], (D*)im.out + o,
-                                            LEV ? im.lev + o : nullptr, lane);
+        recon_piece<T, D, VALS, LEV, HOLES, G>(a, im.li, z, x, c0, on ? cn : 0, G == 64 && gridDim.y > 1, stage[wv] + sub * (CHUNK / R),
+                                               lstage[wv] + (LEV ? sub * (CHUNK / R) : 0), (D*)im.out + o, LEV ? im.lev + o : nullptr, lane);
     }
 }
 
@@ -524,7 +543,7 @@ __global__ __launch_bounds__(256) void k_holes(ReconArgs a, ReconImage im, int* 
     bool found = false;
     for (int64_t rowl = xcd_block(blockIdx.x, gridDim.x) * 4 + wv; rowl < (int64_t)im.rows; rowl += (int64_t)gridDim.x * 4) {
         const uint32_t row = (uint32_t)rowl, z = row / im.X, x = row - z * im.X;
-        recon_stage<uint16_t, uint16_t, false, false, true>(a, im.li, z, x, c0, cn, gridDim.y > 1, stage[wv], nullptr, lane);
+        recon_stage<uint16_t, uint16_t, false, false, true, 64>(a, im.li, z, x, c0, cn, gridDim.y > 1, stage[wv], nullptr, lane);
         for (int i = lane; i < cn; i += 64) found = found || stage[wv][i] == 0;   /* levels start at 1 */
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     }
@@ -533,7 +552,7 @@ __global__ __launch_bounds__(256) void k_holes(ReconArgs a, ReconImage im, int* 
 
 /* the float images of several levels in one launch: none of them needs another, and together they fill the
    chip where the coarse ones alone would each cost a launch */
-template <typename T, bool HOLES>
+template <typename T, bool HOLES, bool SHORT>
 __global__ __launch_bounds__(256) void k_level_images(ReconArgs a, LevelImages m) {
     constexpr int CHUNK = RC_BYTES / 4;
     __shared__ __align__(16) float stage[4][CHUNK];
@@ -543,12 +562,25 @@ __global__ __launch_bounds__(256) void k_level_images(ReconArgs a, LevelImages m
         int li = m.n - 1;
         while (li > 0 && v >= m.block0[li - 1]) --li;
         /* each level is dealt out over the XCDs by itself: the rows of a coarse one cost little */
-        const int64_t rowl = xcd_block(v - m.block0[li], (m.rows[li] + 3) / 4) * 4 + wv;
-        if (c0 >= m.Y[li] || rowl >= m.rows[li]) continue;
-        const uint32_t row = (uint32_t)rowl, X = m.X[li], z = row / X, x = row - z * X;
+        const int G = SHORT ? m.G[li] : 64, per = 256 / G;
+        const int64_t row0 = xcd_block(v - m.block0[li], ((int64_t)m.rows[li] + per - 1) / per) * per + wv * (64 / G);
+        if (c0 >= m.Y[li] || row0 >= m.rows[li]) continue;
         const int cn = (int)min((int64_t)CHUNK, m.Y[li] - c0);
-        recon_piece<T, float, true, false, HOLES>(a, li, z, x, c0, cn, m.Y[li] > CHUNK, stage[wv], nullptr,
-                                                  m.out[li] + (int64_t)row * m.Y[li] + c0, nullptr, lane);
+        auto rows = [&](auto g) {
+            constexpr int GG = decltype(g)::value, R = 64 / GG;
+            const int sub = GG == 64 ? 0 : lane / GG;
+            const bool on = row0 + sub < (int64_t)m.rows[li];
+            const uint32_t row = (uint32_t)row0 + (on ? sub : 0), X = m.X[li], z = row / X, x = row - z * X;
+            recon_piece<T, float, true, false, HOLES, GG>(a, li, z, x, c0, on ? cn : 0, GG == 64 && m.Y[li] > CHUNK, stage[wv] + sub * (CHUNK / R),
+                                                          nullptr, m.out[li] + (int64_t)row * m.Y[li] + c0, nullptr, lane);
+        };
+        if constexpr (!SHORT) {
+            rows(std::integral_constant<int, 64>());
+        } else {
+            if (G == 64) rows(std::integral_constant<int, 64>());
+            else if (G == 32) rows(std::integral_constant<int, 32>());
+            else rows(std::integral_constant<int, 16>());
+        }
     }
 }
 
@@ -850,12 +882,25 @@ void convolve(aprh_context* ctx, aprh_apr& a, const std::vector<HostStencil>& st
 }
 
 namespace {
+/* lanes per row of an image at `level`: what a short row's entries fill, four a lane, if they hold its sources
+   (a wave's time is its chain of loads, however few lanes have one: 30 x 1000 x 1000 u16 0.43 ms with a wave per
+   row, 0.12 with 16 lanes; 128 x 600 x 600 0.18, 0.09 with 32; rows of 160 take one pass of a wave either way) */
+int recon_lanes(const aprh_apr& a, int level, int64_t y) {
+    const int sources = level - a.l_min + 2;
+    if (!a.complete) return 64;
+    if (y <= 64 && sources <= 16) return 16;
+    return y <= 128 && sources <= 32 ? 32 : 64;
+}
+
 template <typename T, typename D, bool VALS, bool LEV>
-void launch_recon(aprh_context* ctx, const ReconArgs& r, const ReconImage& im, bool complete) {
+void launch_recon(aprh_context* ctx, const aprh_apr& a, const ReconArgs& r, const ReconImage& im) {
     if (im.rows == 0 || im.Y == 0) return;
-    const dim3 grid((unsigned)std::min<int64_t>(cdiv(im.rows, 4), 1 << 20), (unsigned)cdiv(im.Y, RC_BYTES / (int64_t)sizeof(D)));
-    if (complete) hipLaunchKernelGGL((k_recon<T, D, VALS, LEV, false>), grid, kBlock, 0, ctx->stream, r, im);
-    else hipLaunchKernelGGL((k_recon<T, D, VALS, LEV, true>), grid, kBlock, 0, ctx->stream, r, im);
+    const int G = recon_lanes(a, im.li + a.l_min, im.Y);
+    const dim3 grid((unsigned)std::min<int64_t>(cdiv(im.rows, 256 / G), 1 << 20), (unsigned)cdiv(im.Y, RC_BYTES / (int64_t)sizeof(D)));
+    if (!a.complete) hipLaunchKernelGGL((k_recon<T, D, VALS, LEV, true, 64>), grid, kBlock, 0, ctx->stream, r, im);
+    else if (G == 64) hipLaunchKernelGGL((k_recon<T, D, VALS, LEV, false, 64>), grid, kBlock, 0, ctx->stream, r, im);
+    else if (G == 32) hipLaunchKernelGGL((k_recon<T, D, VALS, LEV, false, 32>), grid, kBlock, 0, ctx->stream, r, im);
+    else hipLaunchKernelGGL((k_recon<T, D, VALS, LEV, false, 16>), grid, kBlock, 0, ctx->stream, r, im);
     HIP_LAUNCH_CHECK();
 }
 
@@ -873,8 +918,8 @@ void reconstruct(aprh_context* ctx, aprh_apr& a, const T* parts, int level, U* i
     r.parts = parts;
     r.tv = tree.as<float>();
     const ReconImage im = recon_image(a, level, img, lev);
-    if (lev) launch_recon<T, U, true, true>(ctx, r, im, a.complete);
-    else launch_recon<T, U, true, false>(ctx, r, im, a.complete);
+    if (lev) launch_recon<T, U, true, true>(ctx, a, r, im);
+    else launch_recon<T, U, true, false>(ctx, a, r, im);
     HIP_CHECK(hipStreamSynchronize(ctx->stream));
 }
 }  // namespace
@@ -895,13 +940,17 @@ void level_images(aprh_context* ctx, const aprh_apr& a, const T* parts, const fl
         m.rows[i] = (uint32_t)(a.x_num[l] * a.z_num[l]);   /* dims are at most 65535 */
         ymax = std::max(ymax, a.y_num[l]);
     }
+    /* with the short rows' forms in it the kernel runs 5 % slower over long ones (1024 x 1024 x 256: 0.56, 0.59 ms) */
+    const bool shrt = recon_lanes(a, a.l_max, a.y_num[a.l_max]) < 64;
     for (int i = m.n - 1; i >= 0; --i) {
+        m.G[i] = shrt ? recon_lanes(a, i + a.l_min, a.y_num[i + a.l_min]) : 64;
         m.block0[i] = m.blocks;
-        m.blocks += cdiv(m.rows[i], 4);
+        m.blocks += cdiv(m.rows[i], 256 / m.G[i]);
     }
     const dim3 grid((unsigned)std::min<int64_t>(m.blocks, 1 << 20), (unsigned)cdiv(ymax, RC_BYTES / 4));
-    if (a.complete) hipLaunchKernelGGL((k_level_images<T, false>), grid, kBlock, 0, ctx->stream, r, m);
-    else hipLaunchKernelGGL((k_level_images<T, true>), grid, kBlock, 0, ctx->stream, r, m);
+    if (!a.complete) hipLaunchKernelGGL((k_level_images<T, true, false>), grid, kBlock, 0, ctx->stream, r, m);
+    else if (shrt) hipLaunchKernelGGL((k_level_images<T, false, true>), grid, kBlock, 0, ctx->stream, r, m);
+    else hipLaunchKernelGGL((k_level_images<T, false, false>), grid, kBlock, 0, ctx->stream, r, m);
     HIP_LAUNCH_CHECK();
 }
 template void level_images<uint16_t>(aprh_context*, const aprh_apr&, const uint16_t*, const float*, const std::vector<float*>&);
@@ -915,8 +964,8 @@ void reconstruct_level(aprh_context* ctx, aprh_apr& a, int level, void* img, int
     if (level < a.l_max) ensure_tree(ctx, a);
     const ReconArgs r = recon_sources(a, level, level);
     const ReconImage im = recon_image(a, level, img, nullptr);
-    if (idt == APRH_DTYPE_U16) launch_recon<uint16_t, uint16_t, false, false>(ctx, r, im, a.complete);
-    else launch_recon<uint16_t, float, false, false>(ctx, r, im, a.complete);
+    if (idt == APRH_DTYPE_U16) launch_recon<uint16_t, uint16_t, false, false>(ctx, a, r, im);
+    else launch_recon<uint16_t, float, false, false>(ctx, a, r, im);
     HIP_CHECK(hipStreamSynchronize(ctx->stream));
 }
 
