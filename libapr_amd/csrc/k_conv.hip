@@ -1449,10 +1449,12 @@ void conv_levels(aprh_context* ctx, aprh_apr& a, const std::vector<HostStencil>&
                 L.w_off = g.sep ? off_sep[sn] : off_exact[sn];
                 const int64_t nxy = (int64_t)L.ntx * L.nyb;
                 if (nxy == 0 || L.Z == 0) continue;
-                /* about 4096 blocks, in runs of at least twice the stencil's halo planes: a run reads its
-                   halo too, and a block marches its planes one after another */
-                const int64_t H2 = g.S - 1;
-                L.zc = (int)std::max<int64_t>(1, std::min(L.Z, std::max(cdiv(L.Z * nxy, 4096), 2 * H2)));
+                /* about 4096 blocks, in runs of at least twice the stencil's halo planes (a run reads its halo
+                   too), but down to one plane while there are fewer than 512 blocks: a block marches its planes one
+                   after another (9x9x9 in reference order on 64^3: 16 blocks 610 us, 256 blocks 376; with 1024 as the
+                   bound 128^3 takes 583, with 512 490, with 256 505) */
+                const int64_t H2 = g.S - 1, W = L.Z * nxy;
+                L.zc = (int)std::max<int64_t>(1, std::min(L.Z, std::max(cdiv(W, 4096), std::min(2 * H2, cdiv(W, 512)))));
                 L.ntz = (int)cdiv(L.Z, L.zc);
                 L.block0 = g.blocks;
                 g.blocks += nxy * L.ntz;
