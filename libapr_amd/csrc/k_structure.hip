@@ -844,20 +844,21 @@ template <typename T> __device__ __forceinline__ T pyr_store(float m);
 template <> __device__ __forceinline__ uint16_t pyr_store<uint16_t>(float m) { return (uint16_t)(int32_t)m; }
 template <> __device__ __forceinline__ float pyr_store<float>(float m) { return m; }
 
-/* a lane takes the coarse cells of 16 bytes of a fine row (4 u16 cells, 2 float cells) from four fine
-   rows, loaded at any alignment; the sums of a u16 cell are exact in any order, those of a float cell
+/* a lane takes the coarse cells of 8 bytes of a fine row (2 u16 cells, a float cell) from four fine
+   rows (16 bytes of floats: 1024 x 1024 x 20 23 us for the first level, 15 with 8; u16 is alike with both), loaded at any alignment; the sums of a u16 cell are exact in any order, those of a float cell
    run in the order above.  fg, fx: division by the groups of a row and by cd.x (32-bit indices), or
    fits == 0 */
+constexpr int PYR_BYTES = 8;
 struct PyrDiv {
     FastDiv fg, fx;
     int fits;
 };
 template <typename T>
 __global__ __launch_bounds__(256) void k_pyr_down(const T* __restrict__ fine, Dims fd, T* coarse, Dims cd, PyrDiv dv) {
-    constexpr int NF = 16 / sizeof(T), NC = NF / 2;
+    constexpr int NF = PYR_BYTES / sizeof(T), NC = NF / 2;
     const int64_t ng = (cd.y + NC - 1) / NC;
     const int64_t total = ng * cd.x * cd.z;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += (int64_t)gridDim.x * blockDim.x) {
+    for (int64_t i = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x; i < total; i += (int64_t)gridDim.x * blockDim.x) {
         int64_t g, x, z;
         if (dv.fits) {
             const uint32_t r = dv.fg.div((uint32_t)i), zz = dv.fx.div(r);
@@ -873,17 +874,17 @@ __global__ __launch_bounds__(256) void k_pyr_down(const T* __restrict__ fine, Di
         const int64_t x0 = 2 * x, x1 = min(2 * x + 1, fd.x - 1), z0 = 2 * z, z1 = min(2 * z + 1, fd.z - 1), y0 = NF * g;
         const T* rows[4] = {fine + (z0 * fd.x + x0) * fd.y, fine + (z0 * fd.x + x1) * fd.y, fine + (z1 * fd.x + x0) * fd.y,
                             fine + (z1 * fd.x + x1) * fd.y};
-        uint32_t w[4][4];
+        uint32_t w[4][PYR_BYTES / 4];
         if (y0 + NF <= fd.y) {
 #pragma unroll
-            for (int q = 0; q < 4; ++q) __builtin_memcpy(w[q], rows[q] + y0, 16);
+            for (int q = 0; q < 4; ++q) __builtin_memcpy(w[q], rows[q] + y0, PYR_BYTES);
         } else {
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
                 T e[NF];
 #pragma unroll
                 for (int j = 0; j < NF; ++j) e[j] = rows[q][min(y0 + j, fd.y - 1)];
-                __builtin_memcpy(w[q], e, 16);
+                __builtin_memcpy(w[q], e, PYR_BYTES);
             }
         }
         T o[NC];
@@ -1370,7 +1371,7 @@ void pyramid_levels(aprh_context* ctx, const aprh_apr& a, const T* img, T* Pyr, 
         const T* fine = (l == lmax - 1) ? img : Pyr + off[l + 1];
         const Dims fd{a.y_num[l + 1], a.x_num[l + 1], a.z_num[l + 1]}, cd{a.y_num[l], a.x_num[l], a.z_num[l]};
         T* coarse = Pyr + off[l];
-        const int64_t ng = cdiv(cd.y, 8 / (int64_t)sizeof(T)), work = ng * cd.x * cd.z;
+        const int64_t ng = cdiv(cd.y, PYR_BYTES / 2 / (int64_t)sizeof(T)), work = ng * cd.x * cd.z;
         PyrDiv dv;
         dv.fits = fits32(work) ? 1 : 0;
         if (dv.fits) {
