@@ -40,6 +40,7 @@ namespace {
 /* the merged launch of one tile-shape alternative: arguments and tile prefix of every volume */
 struct GroupAlt {
     const TileAlt* proto = nullptr;           /* body, block size, launcher, name, shape */
+    size_t index = 0;                         /* of the alternative in the volumes' records */
     int64_t tiles = 0;
     Buf d_args, d_prefix;
 };
@@ -162,21 +163,33 @@ void merge(aprh_batch* b) {
                 break;
             }
         }
-        g.alts.resize(std::max<size_t>(na, 1));
-        g.alt = std::min<int>(g.recs.front()->prefer, (int)g.alts.size() - 1);
+        /* an alternative that is an earlier one again for every volume is not timed */
+        auto equal = [](const TileAlt& p, const TileAlt& q) { return p.body == q.body && p.tiles == q.tiles && p.args == q.args; };
+        for (size_t k = 0; k < std::max<size_t>(na, 1); ++k) {
+            bool again = false;
+            for (size_t j = 0; j < k && !again; ++j) {
+                again = true;
+                for (const TileRec* r : g.recs) again = again && equal(r->alts[j], r->alts[k]);
+            }
+            if (again) continue;
+            if ((int)k == g.recs.front()->prefer) g.alt = (int)g.alts.size();
+            GroupAlt ga;
+            ga.index = k;
+            g.alts.push_back(std::move(ga));
+        }
         b->groups.push_back(std::move(g));
     }
     /* arguments and tile prefixes of each launch and alternative, uploaded once */
     for (auto& g : b->groups) {
         for (size_t k = 0; k < g.alts.size(); ++k) {
             GroupAlt& ga = g.alts[k];
-            ga.proto = &g.recs.front()->alts[k];
+            ga.proto = &g.recs.front()->alts[ga.index];
             const size_t as = ga.proto->args.size();
             std::vector<uint8_t> args(as * g.recs.size());
             std::vector<int64_t> prefix(g.recs.size() + 1, 0);
             for (size_t v = 0; v < g.recs.size(); ++v) {
-                std::memcpy(args.data() + v * as, g.recs[v]->alts[k].args.data(), as);
-                prefix[v + 1] = prefix[v] + g.recs[v]->alts[k].tiles;
+                std::memcpy(args.data() + v * as, g.recs[v]->alts[ga.index].args.data(), as);
+                prefix[v + 1] = prefix[v] + g.recs[v]->alts[ga.index].tiles;
             }
             ga.tiles = prefix.back();
             ga.d_args.reset(b->pool, args.size());

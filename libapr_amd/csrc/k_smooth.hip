@@ -18,7 +18,7 @@
  * Each pass is one kernel that reads and writes the image once and keeps the
  * sums in LDS: whole lines along y, a ring of 2 offset_max + 2 sums per lane
  * along x and z.  A 512 x 480 x 200 f32 image, its reconstruction included:
- * 2.02 ms with the sums in a scratch image and a second kernel per pass, 0.70 ms
+ * 2.02 ms with the sums in a scratch image and a second kernel per pass, 0.64 ms
  * now.
  */
 #include <type_traits>

@@ -65,7 +65,7 @@ __device__ __forceinline__ uint8_t seed_of(uint8_t m, int level, int mode) {
 struct DownArgs {
     const uint8_t* fine;
     Dims fd;
-    uint8_t* coarse;   /* nullptr: not wanted */
+    uint8_t* coarse;
     Dims cd;
     uint8_t* pct;
     int level, mode;
@@ -121,7 +121,7 @@ __device__ __forceinline__ void level_down_body(const DownArgs& a, int64_t G, in
                 m[k] = h[0] | (h[1] << 16);
             }
             const uint32_t sd[2] = {seed4(m[0], a.level, a.mode), seed4(m[1], a.level, a.mode)};
-            if (a.coarse) __builtin_memcpy(a.coarse + o, m, 8);
+            __builtin_memcpy(a.coarse + o, m, 8);
             __builtin_memcpy(a.pct + o, sd, 8);
         } else {
             for (int j = 0; j < 8 && c0 + j < cd.y; ++j) {
@@ -136,7 +136,7 @@ __device__ __forceinline__ void level_down_body(const DownArgs& a, int64_t G, in
                         a.fpct[rows[q] + yb] = seed_of(vb, a.level + 1, 0);
                     }
                 }
-                if (a.coarse) a.coarse[o + j] = m;
+                a.coarse[o + j] = m;
                 a.pct[o + j] = seed_of(m, a.level, a.mode);
             }
         }
@@ -449,7 +449,6 @@ constexpr int CPL = 16;   /* cells per lane per chunk: a wave covers 1024 cells 
 
 /* weights of the CPL cells [c0, c0 + CPL) of a row (0 beyond its end) */
 __device__ __forceinline__ void chunk_weights(const RowTable& t, int li, const uint8_t* p, int ylen, int c0, int w[CPL]) {
-    const bool top = (li == t.n_levels - 1);
     if (c0 + CPL <= ylen) {   /* one 16-byte load at any alignment */
         uint4 v;
         __builtin_memcpy(&v, p + c0, 16);
@@ -460,7 +459,6 @@ __device__ __forceinline__ void chunk_weights(const RowTable& t, int li, const u
 #pragma unroll
         for (int j = 0; j < CPL; ++j) w[j] = (c0 + j < ylen) ? cell_weight(t, li, p[c0 + j], c0 + j) : 0;
     }
-    (void)top;
 }
 
 /* the APR rows of work item w (1, or up to 4 sharing a pct row at l_max) and its cells */
@@ -681,8 +679,6 @@ struct LevelDown {
     static const char* name() { return "pulling_level_down"; }
     static __device__ __forceinline__ void run(const Args& a, int64_t t) { level_down_body(a, a.G, t); }
 };
-/* planes per lane: a batch plan times the alternatives against each other */
-template <int ALT>
 struct PullLevel {
     using Args = PullArgs;
     static constexpr int THREADS = 256;
@@ -1237,10 +1233,10 @@ void build_structure_seeded(aprh_context* ctx, aprh_apr& a, const uint8_t* level
         const PullArgs p = pargs(zc);
         if (ctx->recorder) {
             const PullArgs p4 = pargs(4);
-            launch_tiles_alts(ctx, {tile_alt<PullLevel<0>>(p, p.G, "planes per lane by size"), tile_alt<PullLevel<4>>(p4, p4.G, "4 planes per lane")},
+            launch_tiles_alts(ctx, {tile_alt<PullLevel>(p, p.G, "planes per lane by size"), tile_alt<PullLevel>(p4, p4.G, "4 planes per lane")},
                               0);
         } else {
-            launch_tiles<PullLevel<0>>(ctx, p, p.G);
+            launch_tiles<PullLevel>(ctx, p, p.G);
         }
     }
     if (small >= lmin) {
