@@ -306,7 +306,7 @@ def test_convolve_separable_edges(oracle, sep_ctx, shape, nb, seed, size, reflec
     exp = o.convolve_pencil(stack, parts, reflect)
     got = A.APRFilter.convolve_pencil(g, stack, parts, reflect_boundary=reflect)
     w = _wide(o, stack)
-    assert w.any()
+    assert w.mean() > 0.9   # the two finest levels at least
     assert _rel(got, exp)[w].max() <= 2 * (max(size, 3) ** 3 + 3 * max(size, 3) + 3) * 2.0 ** -24
 
 
@@ -318,14 +318,14 @@ def test_convolve_separable_lists(oracle, sep_ctx, shape, nb, seed, size, reflec
     kernel with the z ring in registers (bound as above).  The finest level's stencil is the widest: the oracle's
     windows have its size"""
     img, o, g = _pair(oracle, sep_ctx, shape, nb, seed)
-    wide = oracle.gaussian_stencil((1.0, 1.0, 1.0), (size + 2, size, size + 2), True)
+    wide = oracle.gaussian_stencil((1.0, 1.0, 1.0), (size + 2, size, size), True)
     narrow = oracle.gaussian_stencil((1.0, 1.0, 1.0), (min(size, 3), 1, min(size, 3)), True)
     stack = oracle.downsampled_stencils(oracle.gaussian_stencil((size / 4.0,) * 3, (size,) * 3, True), o.l_max - o.l_min, True, "oracle")
     for at, other in ((0, wide), (-1, narrow)):
         st = list(stack)
         st[at] = other
         w = _wide(o, st)
-        assert w.any()
+        assert w.mean() > 0.9
         for parts in (o.sample(img), o.sample(img).astype(np.float32) * np.float32(0.83)):
             exp = o.convolve_pencil(st, parts, reflect)
             got = A.APRFilter.convolve_pencil(g, st, parts, reflect_boundary=reflect)
