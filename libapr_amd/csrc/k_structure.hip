@@ -1313,14 +1313,14 @@ void build_structure_seeded(aprh_context* ctx, aprh_apr& a, const uint8_t* level
         ri.parts = sr->parts;
         sr->done = true;
     }
-    /* a wave per work item when the longest rows have more than half again the 256 cells that 16 lanes take
-       at once: rows of 501 cells (1001 x 777 x 203, sampling included) 0.62 ms with 16 lanes, 0.41 with
-       64; rows of 320 cells (640 x 513 x 250) 0.08 ms with 16 lanes, 0.13 with 64 */
+    /* a wave per work item for long rows, 16 lanes (256 cells at once) for short ones.  Measured with rows of 100 to
+       1500 cells in 40 M voxels, 16 / 64 lanes: 320 cells 46 / 49 us, 384 44 / 43, 512 42 / 37; with the sampling, whose
+       gathers want more lanes, 200 cells 110 / 127, 256 155 / 136, 384 164 / 109 */
     {
         const int64_t FG16 = stride_tiles(t.n_work, FILL_WAVES * 4, 16384), FG64 = stride_tiles(t.n_work, FILL_WAVES, 16384);
         const typename RowFill<16>::Args f16{P, t, rp, rowoff.as<uint64_t>(), a.y_vec.as<uint16_t>(), FG16, ri};
         const typename RowFill<64>::Args f64{P, t, rp, rowoff.as<uint64_t>(), a.y_vec.as<uint16_t>(), FG64, ri};
-        const int prefer = t.map_y[t.n_levels - 1] > 24 * CPL ? 1 : 0;
+        const int prefer = t.map_y[t.n_levels - 1] > (ri.parts ? 14 : 24) * CPL ? 1 : 0;
         if (ctx->recorder)
             launch_tiles_alts(ctx, {tile_alt<RowFill<16>>(f16, FG16, "16 lanes per item"), tile_alt<RowFill<64>>(f64, FG64, "64 lanes per item")},
                               prefer);
