@@ -144,8 +144,8 @@ void richardson_lucy_tv(aprh_context* ctx, aprh_apr& a, const T* in, float* u, c
     if (has_x) gx.reset(ctx->pool, P * 4);
     if (has_z) gz.reset(ctx->pool, P * 4);
     /* gradient_cfd's rescaled central differences (unit pixel size).  In separable mode each is
-       embedded in a 3x3x3 stencil (its taps on the centre line, zeros elsewhere), which the
-       register-ring kernel takes; in the reference's tap order they stay 1-D */
+       embedded in a 3x3x3 stencil (its taps on the centre line, zeros elsewhere), which the kernel over
+       dense level images takes; in the reference's tap order they stay 1-D */
     std::vector<HostStencil> cfd[3];
     for (int d = 0; d < 3; ++d) cfd[d] = rescaled_stencils(sep ? cube3(cfd_stencil(d, 1.0f)) : cfd_stencil(d, 1.0f), a.l_max - a.l_min);
     float* tr = tree.as<float>();

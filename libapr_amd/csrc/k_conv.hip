@@ -474,7 +474,7 @@ constexpr int pow2_above(int n) {
     return p;
 }
 
-/* Cubic separable stencils of a list that k_conv_dense does not take, with the z pass in registers.  Each thread owns one y (its lane) in TX / 4
+/* Cubic separable stencils where k_conv_dense does not run, with the z pass in registers.  Each thread owns one y (its lane) in TX / 4
    rows of the tile and keeps the x-passed values of the last SZ planes of those cells in
    registers; a per-plane map from interior cells to their particle (offset in the row's block,
    0xFF for none) sits in an LDS ring of SZ + 1 planes, so the tile needs no LDS ring of planes
@@ -806,8 +806,8 @@ __global__ __launch_bounds__(CT) void k_conv_sep(ConvArgs<TIn> a) {
  * over 1000 x 1024 x 250, 1.6 ms of them), the separable form instruction issue and the latency left
  * between two barriers a plane.  Levels of one stencil size share a launch.  With windows assembled from
  * the particle rows in every block, level after level: 5x5x5 in reference order on 1000 x 1024 x 250 6.7 ms
- * for the levels' launches, now 2.05 and 0.5 for the images; 9x9x9 separable on 1024 x 1024 x 256 3.2 ms,
- * now 1.45 and 0.5; 3x3x3 on 256 x 256 x 128 0.39 ms in eight launches, now 0.047 and 0.030. */
+ * for the levels' launches, now 2.05 and 0.55 for the images; 9x9x9 separable on 1024 x 1024 x 256 3.2 ms,
+ * now 1.45 and 0.5; 3x3x3 on 256 x 256 x 128 0.39 ms in eight launches, now 0.047 and 0.028. */
 constexpr int CONV_LEVELS = 24;
 struct DenseLevel {
     int64_t Y, X, Z;
@@ -1508,8 +1508,8 @@ void conv_levels(aprh_context* ctx, aprh_apr& a, const std::vector<HostStencil>&
         L.sz = s.sz;
         pl.sep = off_sep[(size_t)sn] >= 0;
         L.w_off = pl.sep ? off_sep[(size_t)sn] : off_exact[(size_t)sn];
-        /* the register-ring kernel (twice as fast as k_conv_tile on separable levels) addresses a coarse plane
-           with 32-bit offsets */
+        /* the register-ring kernel addresses a coarse plane with 32-bit offsets (9 taps on 1024 x 1024 x 256 3.5 ms,
+           14.5 with k_conv_tile) */
         pl.ring = pl.sep && sep_ring_size(s) && L.cX * L.cY <= 0x7FFFFFFF;
         pl.tx = 16;
         if (pl.ring) {
