@@ -192,7 +192,8 @@ typedef struct aprh_rl_stats {
 
 /* APR from a stored structure, as APRFile::read_apr restores LinearAccess
    (LinearAccess.hpp:33-35): xz_end_vec[xz_end_size] for the GenInfo of (y, x, z) and
-   y_vec[total].  Host or device pointers; the structure is validated. */
+   y_vec[total].  Host or device pointers; the structure is validated.  Its particles need not
+   cover the image: what they leave out is 0 in reconstructions. */
 int aprh_apr_from_structure(aprh_context* ctx, int64_t y_num, int64_t x_num, int64_t z_num, const uint64_t* xz_end_vec,
                             uint64_t xz_end_size, const uint16_t* y_vec, uint64_t total, aprh_apr** out);
 /* APR::initialize_tree_dense (APR.hpp:633-689) on first use; tree GenInfo + sizes */
